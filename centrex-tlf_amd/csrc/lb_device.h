@@ -15,6 +15,14 @@
 // where a_s folds the time-independent terms that read the slot's own element
 // (computed once per trajectory), and the "gather" terms read other elements
 // that the owning threads publish to LDS.
+//
+// Couplings.  The gather terms of an output that read the same element (with
+// the same conjugation) are merged into one coupling v * x_in, v = sum f_g
+// c_g(t); on a diagonal output, whose imaginary part is zero, a term and its
+// conjugate merge into twice the one (their sum is twice its real part).  The
+// distinct values v of a plan are its entries.  They are evaluated once per
+// stage into LDS (the time-independent ones once per trajectory), so a
+// coupling is four FMAs on two 16-byte LDS reads, and its table is one word.
 #pragma once
 
 #ifndef __HIPCC_RTC__
@@ -48,6 +56,17 @@ __host__ __device__ inline uint32_t lb_gword(uint32_t pub, bool real_in, bool co
                                              uint32_t coef) {
   return (pub & 0xFFFFFu) | (real_in ? (1u << 20) : 0u) | (conj_in ? (1u << 21) : 0u) |
          (conj_c ? (1u << 22) : 0u) | (coef << 24);
+}
+
+// Coupling word: bits 4..15 byte offset of the entry's value (16 x its index;
+// the time-independent entries first), bit 0 time-dependent entry, bit 1
+// conjugated input, bits 16..31 byte offset of the input in the publication
+// buffer (16 x its publication index).
+#define LB_MAX_ENTRIES 4095
+#define LB_MAX_COUPLED 4096
+#define LB_ENT_ROWS 6  // rows of time-dependent entry values: one per stage time of a step
+__host__ __device__ inline uint32_t lb_cword(uint32_t pub, bool conj_in, bool dyn, uint32_t entry) {
+  return (pub << 20) | (entry << 4) | (conj_in ? 2u : 0u) | (dyn ? 1u : 0u);
 }
 
 // One bytecode instruction (rust/src/lindblad/eval.rs:11-60 opcodes).  Op 20
@@ -94,13 +113,26 @@ struct DevPlan {
   const int32_t* self_coef;  // S*max_self, coefficient id or -1 (constant) ; -2 unused
   const uint8_t* self_conj;  // S*max_self
   const double* self_f;      // S*max_self*2
-  // gather ELL, rows grouped per block
+  // couplings, rows grouped per block (0: the plan's entries do not fit in
+  // LDS and the kernels read the gather tables below instead)
+  int32_t couplings;
+  int32_t nv_stat, nv_dyn;   // time-independent and time-dependent entries
+  int32_t nv_terms;          // terms of the time-dependent entries
+  int32_t c_rows_total;
+  const int32_t* c_row0;     // nblk
+  const int32_t* c_rows;     // nblk
+  const uint32_t* c_word;    // c_rows_total * 64
+  const int32_t* ent_ptr;    // nv_dyn + nv_stat + 1, the time-dependent entries first
+  const uint32_t* ent_coef;  // coefficient row index (K: the constant 1), bit 31 conjugated
+  const double* ent_f;       // factors
+  // gather ELL, rows grouped per block (plans without couplings, and the
+  // adjoint, which needs every term's own coefficient)
   const int32_t* blk_row0;   // nblk
   const int32_t* blk_rows;   // nblk
   const uint32_t* g_word;    // rows*64
   const double* g_f;         // rows*64*2
   int32_t g_rows;            // total gather rows
-  int32_t lds_tables;        // 1: kernels copy the gather tables into LDS
+  int32_t lds_tables;        // 1: kernels copy the coupling words (or gather tables) into LDS
   // restricted plans hold only the elements reachable from an initial support;
   // the others are written as zeros
   int32_t restricted;
@@ -127,6 +159,60 @@ struct DevPlan {
   int32_t vm_depth;             // deepest expression stack
   const double* base;           // n_base*2
 };
+
+// LDS of the multi-wave kernels, in bytes from the start: one layout for the
+// host, which sizes the launch, and the device.
+struct LbLds {
+  uint32_t pub, ent, selfc, wts, coef, slots, red, vm, park, ef, ecoef, eptr, gf, word, misc, evv, total;
+};
+__host__ __device__ inline LbLds lb_lds_layout(const DevPlan& P) {
+  LbLds l;
+  uint32_t q = 0;
+  const uint32_t cells = P.lds_tables ? 64u * (uint32_t)(P.couplings ? P.c_rows_total : P.g_rows) : 0u;
+  const uint32_t nt = P.couplings ? (uint32_t)P.nv_terms : 0u;
+  l.pub = q; q += 2u * 16u * (uint32_t)P.n_pub;
+  l.ent = q; q += P.couplings ? 16u * (uint32_t)(P.nv_stat + LB_ENT_ROWS * P.nv_dyn) : 0u;
+  l.selfc = q; q += 16u * (uint32_t)P.S;
+  l.coef = q; q += 8u * 16u * (uint32_t)(P.K + 1);
+  l.slots = q; q += 8u * 16u * (uint32_t)P.n_slots;
+  l.vm = q; q += 8u * 16u * (uint32_t)P.vm_depth;
+  l.park = q; q += 16u * 128u;
+  l.ef = q; q += 16u * nt;
+  l.gf = q; q += P.couplings ? 0u : 16u * cells;
+  l.wts = q; q += 8u * (uint32_t)((P.n + 1) & ~1);
+  l.red = q; q += 8u * 4u * (uint32_t)P.nblk;
+  l.evv = q; q += 8u * (uint32_t)((P.n + 3) & ~1);
+  l.word = q; q += 4u * cells;
+  l.ecoef = q; q += 4u * nt;
+  l.eptr = q; q += P.couplings ? 4u * (uint32_t)(P.nv_dyn + 1) : 0u;
+  q = (q + 15u) & ~15u;
+  l.misc = q; q += 16u;
+  l.total = q;
+  return l;
+}
+
+// LDS of the paired kernel: the entry definitions once, the rest per half.
+struct LbLdsPair {
+  uint32_t ent, coef, slots, vm, pub, park, ef, wts, ecoef, eptr, misc, total;
+};
+__host__ __device__ inline LbLdsPair lb_lds_pair(const DevPlan& P) {
+  LbLdsPair l;
+  uint32_t q = 0;
+  l.ent = q; q += 2u * 16u * (uint32_t)(P.nv_stat + LB_ENT_ROWS * P.nv_dyn);
+  l.coef = q; q += 2u * 8u * 16u * (uint32_t)(P.K + 1);
+  l.slots = q; q += 2u * 8u * 16u * (uint32_t)P.n_slots;
+  l.vm = q; q += 2u * 8u * 16u * (uint32_t)P.vm_depth;
+  l.pub = q; q += 64u * 16u;
+  l.park = q; q += 128u * 16u;
+  l.ef = q; q += 16u * (uint32_t)P.nv_terms;
+  l.wts = q; q += 8u * (uint32_t)((P.n + 1) & ~1);
+  l.ecoef = q; q += 4u * (uint32_t)P.nv_terms;
+  l.eptr = q; q += 4u * (uint32_t)(P.nv_dyn + 1);
+  q = (q + 15u) & ~15u;
+  l.misc = q; q += 16u;
+  l.total = q;
+  return l;
+}
 
 // Waves that sweep a checkpoint segment of the single-block adjoint (each
 // applies its share of the transposed rows of every reverse stage).

@@ -17,6 +17,7 @@
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "lb_device.h"
@@ -292,26 +293,13 @@ void pick_config(int S, int rows, int* id_out, int* W_out) {
   *W_out = bestW;
 }
 
-// Gather tables up to this size are copied into LDS by every workgroup.
+// Coupling words (or gather tables) up to this size are copied into LDS by every workgroup.
 constexpr int64_t kLdsTableBytes = 32 * 1024;
 // LDS of one workgroup on gfx950.
 constexpr int64_t kMaxLdsBytes = 160 * 1024;
 
-// Must match carve() in lb_kernels.hip.
-int64_t lds_bytes_for(const DevPlan& P) {
-  const int64_t cells = P.lds_tables ? (int64_t)P.g_rows * 64 : 0;
-  return 8 * (int64_t)(4 * P.n_pub) + 8 * 2 * (int64_t)P.S + 8 * (int64_t)((P.n + 1) & ~1) +
-         16 * 8 * (int64_t)(P.K + 1) + 16 * 8 * (int64_t)P.n_slots + 8 * 4 * (int64_t)P.nblk +
-         16 * 8 * (int64_t)P.vm_depth + 16 * 128 + 16 * cells + 4 * ((cells + 3) & ~3) + 16 +
-         8 * (int64_t)(P.n + 2);
-}
-
-// Must match carve_pair() in lb_kernels.hip.
-int64_t lds_bytes_pair(const DevPlan& P) {
-  const int64_t g = P.g_rows;  // one block: its rows
-  return g * 64 * 16 + 2 * 8 * (int64_t)(P.K + 1) * 16 + 2 * 8 * (int64_t)P.n_slots * 16 +
-         2 * 8 * (int64_t)P.vm_depth * 16 + 64 * 16 + 128 * 16 + 8 * (int64_t)((P.n + 1) & ~1) + g * 64 * 4 + 16;
-}
+int64_t lds_bytes_for(const DevPlan& P) { return lb_lds_layout(P).total; }
+int64_t lds_bytes_pair(const DevPlan& P) { return lb_lds_pair(P).total; }
 
 int set_lds_limit(const void* fn, size_t lds) {
   if (lds > 65536)
@@ -342,6 +330,102 @@ std::vector<uint8_t> active_closure(const PlanSource& S, std::vector<uint8_t> ac
   return act;
 }
 
+// The gather terms of the active outputs merged into couplings (lb_device.h).
+struct Coupling {
+  int in;        // upper index of the input
+  bool conj;     // conjugated input (false for a diagonal one, which is real)
+  int entry;     // index into Couplings::entries
+};
+struct EntryTerm {
+  uint32_t coef;  // coefficient row index (K: the constant 1), bit 31 conjugated
+  double re, im;
+  bool operator<(const EntryTerm& o) const { return std::tie(coef, re, im) < std::tie(o.coef, o.re, o.im); }
+  bool operator==(const EntryTerm& o) const { return coef == o.coef && re == o.re && im == o.im; }
+};
+struct Couplings {
+  std::vector<std::vector<Coupling>> of;        // per upper output
+  std::vector<std::vector<EntryTerm>> entries;  // time-dependent entries first
+  int n_dyn = 0;
+  int64_t dyn_terms = 0;
+};
+
+Couplings merge_couplings(const PlanSource& src, const std::vector<uint8_t>& act) {
+  struct Raw {
+    int in;
+    bool conj;
+    std::vector<EntryTerm> v;
+  };
+  Couplings out;
+  out.of.resize(src.U);
+  std::map<std::vector<EntryTerm>, int> dyn_id, stat_id;
+  auto is_dyn = [&](const std::vector<EntryTerm>& v) {
+    for (const EntryTerm& t : v) {
+      const uint32_t k = t.coef & 0x7FFFFFFFu;
+      if (k < (uint32_t)src.K && src.coef_dyn[k]) return true;
+    }
+    return false;
+  };
+  auto conj_of = [&](const EntryTerm& t) {
+    const uint32_t k = t.coef & 0x7FFFFFFFu;
+    return EntryTerm{k == (uint32_t)src.K ? t.coef : t.coef ^ 0x80000000u, t.re, -t.im};
+  };
+  std::vector<std::vector<std::pair<bool, int>>> ids(src.U);  // (time-dependent, index of its kind)
+  for (int o = 0; o < src.U; ++o) {
+    if (!act[o]) continue;
+    std::vector<Raw> raw;
+    for (int64_t k = src.output_ptrs[o]; k < src.output_ptrs[o + 1]; ++k) {
+      const int in = (int)src.input_indices[k];
+      const int64_t ci = src.coeff_indices[k];
+      if (in == o && !(ci >= 0 && src.coef_dyn[ci]) && !src.input_conj[k]) continue;  // a self term
+      const bool conj = src.up_im[in] >= 0 && src.input_conj[k];
+      EntryTerm t{ci < 0 ? (uint32_t)src.K : ((uint32_t)ci | (src.coeff_conj[k] ? 0x80000000u : 0u)),
+                  src.factors_re[k], src.factors_im[k]};
+      auto it = std::find_if(raw.begin(), raw.end(), [&](const Raw& r) { return r.in == in && r.conj == conj; });
+      if (it == raw.end()) raw.push_back(Raw{in, conj, {t}});
+      else it->v.push_back(t);
+    }
+    if (src.up_im[o] < 0) {
+      // a diagonal output keeps the real part only: x v and its conjugate are twice the one
+      for (size_t i = 0; i < raw.size(); ++i) {
+        for (size_t j = i + 1; j < raw.size(); ++j) {
+          if (raw[i].in != raw[j].in || raw[i].conj == raw[j].conj) continue;
+          std::vector<EntryTerm> a = raw[i].v, b;
+          for (const EntryTerm& t : raw[j].v) b.push_back(conj_of(t));
+          std::sort(a.begin(), a.end());
+          std::sort(b.begin(), b.end());
+          if (!(a == b)) continue;
+          Raw& keep = raw[i].conj ? raw[j] : raw[i];
+          for (EntryTerm& t : keep.v) {
+            t.re *= 2.0;
+            t.im *= 2.0;
+          }
+          if (raw[i].conj) raw[i] = raw[j];
+          raw.erase(raw.begin() + j);
+          break;
+        }
+      }
+    }
+    for (const Raw& r : raw) {
+      const bool dyn = is_dyn(r.v);
+      auto& table = dyn ? dyn_id : stat_id;
+      const int id = table.emplace(r.v, (int)table.size()).first->second;
+      out.of[o].push_back(Coupling{r.in, r.conj, 0});
+      ids[o].push_back({dyn, id});
+    }
+  }
+  out.n_dyn = (int)dyn_id.size();
+  out.entries.resize(dyn_id.size() + stat_id.size());
+  for (const auto& kv : dyn_id) {
+    out.entries[kv.second] = kv.first;
+    out.dyn_terms += (int64_t)kv.first.size();
+  }
+  for (const auto& kv : stat_id) out.entries[dyn_id.size() + kv.second] = kv.first;
+  for (int o = 0; o < src.U; ++o)
+    for (size_t j = 0; j < ids[o].size(); ++j)
+      out.of[o][j].entry = ids[o][j].first ? ids[o][j].second : out.n_dyn + ids[o][j].second;
+  return out;
+}
+
 // Lane layout and device tables for the active elements `act` (lb_device.h).
 int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage* im) {
   const int n = src.n, U = src.U;
@@ -368,12 +452,42 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
       }
     }
   }
-  // slots: active outputs ordered by gather count (descending), then index
+  const int S = std::max(64, (n_act + 63) / 64 * 64), nblk = S / 64;
+  const bool one_block = S == 64;
+  DevPlan& P = im->dev;
+  P.n = n;
+  P.dim = n * n;
+  P.upper_len = U;
+  P.S = S;
+  P.nblk = nblk;
+  P.K = src.K;
+  P.KD = src.K * (1 + src.n_diff);
+  P.n_slots = src.prog.n_slots;
+  P.vm_depth = std::max(src.prog.max_depth, 1);
+  P.n_pub = one_block ? n_act : (int)std::count(published.begin(), published.end(), (uint8_t)1);
+  // Couplings, when their entries (and the rest of a workgroup's LDS) fit;
+  // the gather tables otherwise.
+  const Couplings cpl = merge_couplings(src, act);
+  const int n_stat = (int)cpl.entries.size() - cpl.n_dyn + 1;  // and the zero of padding rows
+  P.couplings = 1;
+  P.nv_dyn = cpl.n_dyn;
+  P.nv_stat = n_stat;
+  P.nv_terms = (int32_t)std::min<int64_t>(cpl.dyn_terms, 1 << 20);
+  P.lds_tables = 0;
+  P.c_rows_total = P.g_rows = 0;
+  if (P.nv_dyn + P.nv_stat > LB_MAX_ENTRIES || P.n_pub > LB_MAX_COUPLED ||
+      16 * (int64_t)(P.nv_stat + LB_ENT_ROWS * P.nv_dyn) + 20 * (int64_t)P.nv_terms > kMaxLdsBytes ||
+      lds_bytes_for(P) > kMaxLdsBytes) {
+    P.couplings = 0;
+    P.nv_dyn = P.nv_stat = P.nv_terms = 0;
+  }
+  std::vector<int> n_rows(U, 0);  // table rows of an output in the solve's table
+  for (int o = 0; o < U; ++o) n_rows[o] = P.couplings ? (int)cpl.of[o].size() : n_gather[o];
+  // slots: active outputs ordered by their rows (descending), then index
   std::vector<int> order;
   for (int o = 0; o < U; ++o)
     if (act[o]) order.push_back(o);
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return n_gather[a] > n_gather[b]; });
-  const int S = std::max(64, (n_act + 63) / 64 * 64), nblk = S / 64;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return n_rows[a] > n_rows[b]; });
   // Blocks of 64 consecutive elements of that order, placed so that the
   // default launch's waves get about equal gather rows: wave w of nw holds
   // blocks w, w + nw, w + 2 nw, ..., so the blocks go, longest first, to the
@@ -384,7 +498,7 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
     std::vector<int> brows(nblk, 0);
     int rows_sum = 0;
     for (int b = 0; b < nblk; ++b) {
-      for (int l = 0; l < 64 && 64 * b + l < n_act; ++l) brows[b] = std::max(brows[b], n_gather[order[64 * b + l]]);
+      for (int l = 0; l < 64 && 64 * b + l < n_act; ++l) brows[b] = std::max(brows[b], n_rows[order[64 * b + l]]);
       rows_sum += brows[b];
     }
     std::vector<int> pos_of(nblk);
@@ -418,7 +532,6 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   // A plan of one block publishes every element at its slot index, so the
   // gather words name the owning lane (the single-wave kernels read inputs
   // by cross-lane permutes).
-  const bool one_block = S == 64;
   for (int s = 0; s < S; ++s) {
     const int o = slot_el[s];
     if (o < 0) continue;
@@ -469,6 +582,55 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
         g_f[2 * e + 1] = src.factors_im[k];
       }
     }
+  }
+  // coupling words, rows grouped per block; padding rows read entry zero
+  std::vector<int32_t> c_row0(nblk, 0), c_rows(nblk, 0), ent_ptr;
+  std::vector<uint32_t> c_word, ent_coef;
+  std::vector<double> ent_f;
+  int c_total = 0;
+  if (P.couplings) {
+    auto word = [&](int in, bool conj, int entry) {
+      const bool dyn = entry < P.nv_dyn;
+      // values in LDS: the time-independent entries, then the rows of the others
+      const int at = dyn ? P.nv_stat + entry : entry - P.nv_dyn;
+      return lb_cword((uint32_t)(in < 0 ? 0 : pub_of_upper[in]), conj, dyn, (uint32_t)at);
+    };
+    for (int b = 0; b < nblk; ++b) {
+      int rows = 0;
+      for (int l = 0; l < 64; ++l)
+        if (slot_el[64 * b + l] >= 0) rows = std::max(rows, n_rows[slot_el[64 * b + l]]);
+      c_row0[b] = c_total;
+      c_rows[b] = rows;
+      c_total += rows;
+    }
+    const int zero = P.nv_dyn + P.nv_stat - 1;
+    c_word.assign((size_t)c_total * 64, word(-1, false, zero));
+    for (int s = 0; s < S; ++s) {
+      const int o = slot_el[s], b = s / 64, l = s % 64;
+      if (o < 0) continue;
+      for (size_t j = 0; j < cpl.of[o].size(); ++j)
+        c_word[(size_t)(c_row0[b] + (int)j) * 64 + l] = word(cpl.of[o][j].in, cpl.of[o][j].conj, cpl.of[o][j].entry);
+    }
+    ent_ptr.push_back(0);
+    auto add = [&](const std::vector<EntryTerm>& v) {
+      for (const EntryTerm& t : v) {
+        ent_coef.push_back(t.coef);
+        ent_f.push_back(t.re);
+        ent_f.push_back(t.im);
+      }
+      ent_ptr.push_back((int32_t)ent_coef.size());
+    };
+    for (const auto& v : cpl.entries) add(v);
+    add({EntryTerm{(uint32_t)src.K, 0.0, 0.0}});
+    P.c_rows_total = c_total;
+    P.lds_tables = 1;
+    if (4 * 64 * (int64_t)c_total > kLdsTableBytes || lds_bytes_for(P) > kMaxLdsBytes) P.lds_tables = 0;
+  }
+  // the gather tables: plans without couplings, and differentiable ones
+  const bool gather = !P.couplings || src.n_diff > 0;
+  if (!gather) {
+    g_word.clear();
+    g_f.clear();
   }
   // transposed tables of a differentiable plan: for each input slot, the terms
   // that read it (self-folded terms excluded), output named by its slot
@@ -523,23 +685,13 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
     if (src.up_im[u] >= 0) packed_upper[src.up_im[u]] = u;
   }
 
-  DevPlan& P = im->dev;
-  P.n = n;
-  P.dim = n * n;
-  P.upper_len = U;
-  P.S = S;
-  P.nblk = nblk;
   P.n_pub = n_pub;
-  P.K = src.K;
-  P.KD = src.K * (1 + src.n_diff);
   P.n_diff = src.n_diff;
   P.diff_time = src.diff_time;
-  P.n_slots = src.prog.n_slots;
   P.n_base = src.n_base;
   P.n_compounds = src.prog.n_compounds;
-  P.vm_depth = std::max(src.prog.max_depth, 1);
   P.g_rows = rows_total;
-  P.lds_tables = (int64_t)rows_total * 64 * 20 <= kLdsTableBytes ? 1 : 0;
+  if (!P.couplings) P.lds_tables = (int64_t)rows_total * 64 * 20 <= kLdsTableBytes ? 1 : 0;
   P.max_self = max_self;
   P.time_dependent = src.time_dependent ? 1 : 0;
   P.restricted = n_act < U ? 1 : 0;
@@ -554,6 +706,12 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   up(self_coef, &P.self_coef);
   up(self_conj, &P.self_conj);
   up(self_f, &P.self_f);
+  up(c_row0, &P.c_row0);
+  up(c_rows, &P.c_rows);
+  up(c_word, &P.c_word);
+  up(ent_ptr, &P.ent_ptr);
+  up(ent_coef, &P.ent_coef);
+  up(ent_f, &P.ent_f);
   up(blk_row0, &P.blk_row0);
   up(blk_rows, &P.blk_rows);
   up(g_word, &P.g_word);
@@ -625,19 +783,20 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   up(t_word, &P.t_word);
   up(t_f, &P.t_f);
   if (rc != LB_OK) return rc;
-  pick_config(S, rows_total, &im->default_variant, &im->default_W);
+  const int solve_rows = P.couplings ? c_total : rows_total;
+  pick_config(S, solve_rows, &im->default_variant, &im->default_W);
   // paired variant: the fewest register rows holding a one-block plan of <= 32 elements
   im->pair_variant = -1;
-  if (nblk == 1 && n_act <= 32) {
+  if (nblk == 1 && n_act <= 32 && P.couplings) {
     int best_g = 1 << 30;
     for (int id = 0; id < lb_dev_variant_count(); ++id) {
       const int g = lb_dev_variant_rows(id);
-      if (lb_dev_variant_pair(id) && rows_total <= g && g < best_g) { best_g = g; im->pair_variant = id; }
+      if (lb_dev_variant_pair(id) && solve_rows <= g && g < best_g) { best_g = g; im->pair_variant = id; }
     }
   }
   im->lds_bytes = lds_bytes_for(P);
   im->n_pub = n_pub;
-  im->rows_total = rows_total;
+  im->rows_total = solve_rows;
   im->g_rows_host = blk_rows;
   im->t_rows_host = t_rows.empty() ? 0 : t_rows[0];
   im->flops = flops;
@@ -924,8 +1083,8 @@ int resolve_config(const DevImage* p, int variant, int threads, bool pair_ok, in
   if (variant > 0) {
     *id = variant - 1;
     if (!lb_dev_variant(*id, &R, &maxw, &waves)) return fail(LB_ERR_INVALID, "unknown kernel variant");
-    *W = threads ? threads : variant_threads(*id, p->dev.S, p->dev.g_rows);
-    if (lb_dev_variant_rows(*id) && (*W != 64 || !variant_threads(*id, p->dev.S, p->dev.g_rows)))
+    *W = threads ? threads : variant_threads(*id, p->dev.S, (int)p->rows_total);
+    if (lb_dev_variant_rows(*id) && (*W != 64 || !variant_threads(*id, p->dev.S, (int)p->rows_total)))
       return fail(LB_ERR_UNSUPPORTED, "single-wave variant needs a plan of at most 64 elements");
     if (!*W || *W > maxw || (int64_t)R * *W < p->dev.S)
       return fail(LB_ERR_UNSUPPORTED, "kernel variant does not cover the plan with this workgroup size");
@@ -1238,6 +1397,7 @@ int launch_table(const lb_plan* p, const lb_solve_args* a, const DevImage* im, D
   hipStream_t s = (hipStream_t)stream;
   DevPlan P = im->dev;
   P.vm_depth = std::max(P.vm_depth, ev_depth);  // the stop-event expression runs on lane 0's stack
+  if (lds_bytes_for(P) > kMaxLdsBytes && P.couplings) P.lds_tables = 0;  // a deep expression's stack
   const size_t lds = (size_t)lds_bytes_for(P);
   int rc = set_lds_limit(fn, lds);
   if (rc) return rc;

@@ -457,29 +457,131 @@ struct Lds {
   double* red;    // 4 x nblk block sums
   dcpx* vm;       // 8 lanes x vm_depth expression stacks
   double2* park;  // 128 entries: single-wave state parked around the expression machine
-  double2* gf;    // gather factors (when the plan stages its tables in LDS)
-  uint32_t* gw;   // gather words
+  dcpx* ent;      // entry values: nv_stat time-independent, then LB_ENT_ROWS x nv_dyn
+  double2* ef;    // factors, coefficient rows and extents of the time-dependent entries
+  uint32_t* ecoef;
+  int* eptr;
+  double2* gf;    // gather factors (plans without couplings that stage their tables in LDS)
+  uint32_t* gw;   // coupling or gather words
   int* misc;      // [0] queue value
   double* evv;    // n + 2: stop-event populations, [n] expression value, [n + 1] complex flag
 };
 
 __device__ __forceinline__ Lds carve(const DevPlan& P) {
   extern __shared__ double smem[];
+  char* const base = reinterpret_cast<char*>(smem);
+  const LbLds l = lb_lds_layout(P);
   Lds L;
-  L.pub = smem;
-  L.selfc = L.pub + 4 * (size_t)P.n_pub;
-  L.wts = L.selfc + 2 * (size_t)P.S;
-  L.coef = reinterpret_cast<dcpx*>(L.wts + ((P.n + 1) & ~1));
-  L.slots = L.coef + 8 * (P.K + 1);
-  L.red = reinterpret_cast<double*>(L.slots + 8 * P.n_slots);
-  L.vm = reinterpret_cast<dcpx*>(L.red + 4 * P.nblk);
-  L.park = reinterpret_cast<double2*>(L.vm + 8 * P.vm_depth);
-  L.gf = L.park + 128;
-  const size_t cells = P.lds_tables ? (size_t)P.g_rows * 64 : 0;
-  L.gw = reinterpret_cast<uint32_t*>(L.gf + cells);
-  L.misc = reinterpret_cast<int*>(L.gw + ((cells + 3) & ~(size_t)3));
-  L.evv = reinterpret_cast<double*>(L.misc + 4);
+  L.pub = reinterpret_cast<double*>(base + l.pub);
+  L.ent = reinterpret_cast<dcpx*>(base + l.ent);
+  L.selfc = reinterpret_cast<double*>(base + l.selfc);
+  L.wts = reinterpret_cast<double*>(base + l.wts);
+  L.coef = reinterpret_cast<dcpx*>(base + l.coef);
+  L.slots = reinterpret_cast<dcpx*>(base + l.slots);
+  L.red = reinterpret_cast<double*>(base + l.red);
+  L.vm = reinterpret_cast<dcpx*>(base + l.vm);
+  L.park = reinterpret_cast<double2*>(base + l.park);
+  L.ef = reinterpret_cast<double2*>(base + l.ef);
+  L.ecoef = reinterpret_cast<uint32_t*>(base + l.ecoef);
+  L.eptr = reinterpret_cast<int*>(base + l.eptr);
+  L.gf = reinterpret_cast<double2*>(base + l.gf);
+  L.gw = reinterpret_cast<uint32_t*>(base + l.word);
+  L.misc = reinterpret_cast<int*>(base + l.misc);
+  L.evv = reinterpret_cast<double*>(base + l.evv);
   return L;
+}
+
+// One term of an entry: f c, c the coefficient (conjugated when bit 31 of
+// its index is set) -- rhs.rs:815-876 factor semantics.
+__device__ __forceinline__ dcpx entry_term(double2 f, uint32_t id, const dcpx* coef) {
+  dcpx c = coef[id & 0x7FFFFFFFu];
+  c.im = (id & 0x80000000u) ? -c.im : c.im;
+  return mk(fma(f.x, c.re, -(f.y * c.im)), fma(f.x, c.im, f.y * c.re));
+}
+
+// Values of the time-dependent entries for NR coefficient rows (`coef`, KK
+// apart) into the entry rows `out` (nv_dyn apart): one lane per entry, its
+// definition read once for all rows.
+template <int NR>
+__device__ __forceinline__ void fill_entries(int nv_dyn, const int* eptr, const uint32_t* ecoef, const double2* ef,
+                                             const dcpx* coef, int KK, dcpx* out, int tid, int W) {
+  for (int e = tid; e < nv_dyn; e += W) {
+    const int p0 = eptr[e], p1 = eptr[e + 1];
+    dcpx v[NR];
+    {
+      const double2 f = ef[p0];
+      const uint32_t id = ecoef[p0];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) v[r] = entry_term(f, id, coef + r * KK);
+    }
+    for (int t = p0 + 1; t < p1; ++t) {
+      const double2 f = ef[t];
+      const uint32_t id = ecoef[t];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) v[r] = cadd(v[r], entry_term(f, id, coef + r * KK));
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) out[r * nv_dyn + e] = v[r];
+  }
+}
+
+// The time-independent entries of a trajectory (definitions from global memory).
+__device__ __forceinline__ void fill_static_entries(const DevPlan& P, const dcpx* coef, dcpx* out, int tid, int W) {
+  const double2* ef = reinterpret_cast<const double2*>(P.ent_f);
+  for (int e = tid; e < P.nv_stat; e += W) {
+    const int p0 = P.ent_ptr[P.nv_dyn + e], p1 = P.ent_ptr[P.nv_dyn + e + 1];
+    dcpx v = mk(0.0, 0.0);
+    for (int t = p0; t < p1; ++t) {
+      const dcpx q = entry_term(ef[t], P.ent_coef[t], coef);
+      v = t == p0 ? q : cadd(v, q);
+    }
+    out[e] = v;
+  }
+}
+
+// One coupling: acc += v x_in (or v conj(x_in)).
+__device__ __forceinline__ void couple(uint32_t sign, double2 v, double2 x, double& accr, double& acci) {
+  const double xi = __hiloint2double(__double2hiint(x.y) ^ (int)sign, __double2loint(x.y));
+  // explicit fused operations: the library is built without implicit
+  // contraction, so every kernel variant rounds identically
+  accr = fma(-v.y, xi, fma(v.x, x.x, accr));
+  acci = fma(v.y, x.x, fma(v.x, xi, acci));
+}
+
+// N couplings of one lane: every LDS read first, then the terms in order.
+template <int N, typename WordPtr>
+__device__ __forceinline__ void couple_rows(WordPtr cw, const char* pubbuf, const char* ent, uint32_t dyn,
+                                            double& accr, double& acci) {
+  uint32_t w[N];
+  double2 x[N], v[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) w[j] = cw[64 * j];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    x[j] = *reinterpret_cast<const double2*>(pubbuf + (w[j] >> 16));
+    v[j] = *reinterpret_cast<const double2*>(ent + ((w[j] & 0xFFF0u) + (w[j] & 1u) * dyn));
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) couple((w[j] << 30) & 0x80000000u, v[j], x[j], accr, acci);
+}
+
+// The couplings of one block for entry row `vrow`, in row order.  Latency of
+// the LDS reads bounds a row, so four rows' reads are in flight at once; a
+// row is 4 FMAs, 2 16-byte reads and a 4-byte word against 8 FP64 operations,
+// 3 reads and a 20-byte table cell (often from L2) when every gather term was
+// applied with its own factor and coefficient.  512 + 512 uneven batch (72
+// levels: 48 rows instead of 63, the longest block 14 instead of 21) 727 ->
+// 517 ms.
+template <typename WordPtr>
+__device__ __forceinline__ void couple_block(WordPtr cw, int rows, const char* pubbuf, const char* ent, uint32_t dyn,
+                                             double& accr, double& acci) {
+  int j = 0;
+  for (; j + 4 <= rows; j += 4) couple_rows<4>(cw + 64 * j, pubbuf, ent, dyn, accr, acci);
+  if (rows & 2) {
+    couple_rows<2>(cw + 64 * j, pubbuf, ent, dyn, accr, acci);
+    j += 2;
+  }
+  if (rows & 1) couple_rows<1>(cw + 64 * j, pubbuf, ent, dyn, accr, acci);
 }
 
 // One gather term: acc += f * c * x_in (rhs.rs:815-876 term semantics), with
@@ -574,21 +676,38 @@ __device__ __forceinline__ void gather_block(const uint32_t* gw, const double2* 
 template <int R>
 __device__ __forceinline__ void rhs_eval(const DevPlan& P, const Lds& L, const Slots<R>& S,
                                          const double (&xr)[R], const double (&xi)[R], double (&kr)[R],
-                                         double (&ki)[R], double* pubbuf, const dcpx* coef, int tid,
+                                         double (&ki)[R], double* pubbuf, const dcpx* coef, int vrow, int tid,
                                          int W) {
   const int lane = tid & 63;
   // wave-uniform block index: lets the row counts live in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (S.pub[r] >= 0) reinterpret_cast<double2*>(pubbuf)[S.pub[r]] = double2{xr[r], xi[r]};
+  __syncthreads();
+  if (P.couplings) {
+    const char* const pb = reinterpret_cast<const char*>(pubbuf);
+    const char* const ent = reinterpret_cast<const char*>(L.ent);
+    const uint32_t dyn = 16u * (uint32_t)(vrow * P.nv_dyn);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int blk = wave + (W >> 6) * r;
+      if (blk >= P.nblk) { kr[r] = 0.0; ki[r] = 0.0; continue; }
+      const double2 a = reinterpret_cast<const double2*>(L.selfc)[tid + W * r];
+      double accr = fma(a.x, xr[r], -(a.y * xi[r]));
+      double acci = fma(a.x, xi[r], a.y * xr[r]);
+      const int row0 = cst(P.c_row0)[blk], rows = cst(P.c_rows)[blk];
+      if (P.lds_tables)
+        couple_block(static_cast<const uint32_t*>(L.gw) + (row0 * 64 + lane), rows, pb, ent, dyn, accr, acci);
+      else
+        couple_block(P.c_word + ((size_t)row0 * 64 + lane), rows, pb, ent, dyn, accr, acci);
+      kr[r] = accr;
+      ki[r] = S.diag(r) ? 0.0 : acci;
+    }
+    return;
+  }
   const uint32_t* gw = P.lds_tables ? static_cast<const uint32_t*>(L.gw) : P.g_word;
   const double2* gf = P.lds_tables ? static_cast<const double2*>(L.gf) : reinterpret_cast<const double2*>(P.g_f);
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (S.pub[r] >= 0) {
-      pubbuf[2 * S.pub[r]] = xr[r];
-      pubbuf[2 * S.pub[r] + 1] = xi[r];
-    }
-  }
-  __syncthreads();
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int blk = wave + (W >> 6) * r;
@@ -603,8 +722,19 @@ __device__ __forceinline__ void rhs_eval(const DevPlan& P, const Lds& L, const S
   }
 }
 
-// Copy the gather tables into LDS once per workgroup (plans whose tables fit).
+// Copy the coupling (or gather) tables into LDS once per workgroup (plans
+// whose tables fit), and the definitions of the time-dependent entries.
 __device__ __forceinline__ void stage_tables(const DevPlan& P, const Lds& L, int tid, int W) {
+  if (P.couplings) {
+    for (int i = tid; i < P.nv_terms; i += W) {
+      L.ef[i] = reinterpret_cast<const double2*>(P.ent_f)[i];
+      L.ecoef[i] = P.ent_coef[i];
+    }
+    for (int i = tid; i <= P.nv_dyn; i += W) L.eptr[i] = P.ent_ptr[i];
+    if (P.lds_tables)
+      for (int i = tid; i < P.c_rows_total * 64; i += W) L.gw[i] = P.c_word[i];
+    return;
+  }
   if (!P.lds_tables) return;
   const int cells = P.g_rows * 64;
   const double2* gf = reinterpret_cast<const double2*>(P.g_f);
@@ -889,8 +1019,6 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
   Slots<R> S;
   load_slots<R>(P, S, tid, W);
   stage_tables(P, L, tid, W);
-  const int wrows = G > 0 ? cst(P.blk_rows)[0] : 0;
-  double2 selfv = double2{0.0, 0.0};
 
   for (;;) {
     __syncthreads();
@@ -922,9 +1050,9 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
     for (int i = tid; i < 7 * P.n_slots; i += W) L.slots[P.n_slots + i] = L.slots[i % P.n_slots];
     for (int i = tid; i < 7 * KK; i += W) L.coef[KK + i] = L.coef[i % KK];
     fold_self(P, tid, W, L.coef, L.selfc);
-    if constexpr (G > 0) {
-      __syncthreads();  // coefficient rows and self folds are read below
-      selfv = reinterpret_cast<const double2*>(L.selfc)[tid];
+    if (P.couplings) {  // entry row 5 holds t0 until the last stage needs it
+      fill_static_entries(P, L.coef, L.ent, tid, W);
+      fill_entries<1>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef, KK, L.ent + P.nv_stat + 5 * P.nv_dyn, tid, W);
     }
 
     // ---- state
@@ -995,14 +1123,10 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
     double k_r[8][R], k_i[8][R];
     int buf = 0;
 #define PUB (L.pub + buf * 2 * P.n_pub)
-#define LB_RHS(xr, xi, kr, ki, cf)                                                         \
-  do {                                                                                     \
-    if constexpr (G > 0) {                                                                 \
-      rhs_wave<(G > 0 ? G : 1)>(L, wrows, tid, selfv, S.diag(0), xr[0], xi[0], kr[0], ki[0], cf); \
-    } else {                                                                               \
-      rhs_eval<R>(P, L, S, xr, xi, kr, ki, PUB, cf, tid, W);                               \
-      buf ^= 1;                                                                            \
-    }                                                                                      \
+#define LB_RHS(xr, xi, kr, ki, cf, vrow)                         \
+  do {                                                           \
+    rhs_eval<R>(P, L, S, xr, xi, kr, ki, PUB, cf, vrow, tid, W); \
+    buf ^= 1;                                                    \
   } while (0)
 
     if (bad_support) {
@@ -1016,7 +1140,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
     } else {
       double x = t0, h;
       // ---- k1 = f(t0, y0) (also f0 of hinit); the barrier inside orders the LDS fills above
-      LB_RHS(y_r, y_i, k_r[1], k_i[1], L.coef);
+      LB_RHS(y_r, y_i, k_r[1], k_i[1], L.coef, 5);
       if (isfinite(C.dt) && C.dt > 0.0) {
         h = fmin(C.dt, t1 - t0);
       } else {
@@ -1034,14 +1158,16 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         double h0 = (d0 < 1.0e-10 || d1 < 1.0e-10) ? 1.0e-6 : 0.01 * sqrt(d0 / d1);
         h0 = fmin(h0, hmax);
         if (tid == 0) eval_coefficients(P, L.slots + P.n_slots, L.coef + KK, x + h0, true, L.vm);
-        if constexpr (G > 0) __syncthreads();
+        __syncthreads();
+        if (P.couplings)
+          fill_entries<1>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + KK, KK, L.ent + P.nv_stat, tid, W);
         double yt_r[R], yt_i[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           yt_r[r] = y_r[r] + k_r[1][r] * h0;
           yt_i[r] = y_i[r] + k_i[1][r] * h0;
         }
-        LB_RHS(yt_r, yt_i, k_r[2], k_i[2], L.coef + KK);
+        LB_RHS(yt_r, yt_i, k_r[2], k_i[2], L.coef + KK, 0);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           const double sr = C.abstol + fabs(y_r[r]) * C.reltol, si = C.abstol + fabs(y_i[r]) * C.reltol;
@@ -1105,8 +1231,13 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           eval_coefficients(P, L.slots + s * P.n_slots, L.coef + s * KK, x + h * T::c(s), true,
                             L.vm + tid * P.vm_depth);
         }
-        if constexpr (G > 0) {
+        if (P.time_dependent) {
           __syncthreads();  // stage coefficients are read by every lane
+          // stages 2..6 take entry rows 0..4; stage 7 is at the same time as 6
+          if (P.couplings)
+            fill_entries<5>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + 2 * KK, KK, L.ent + P.nv_stat, tid, W);
+        }
+        if constexpr (G > 0) {
           const double2 py = L.park[tid], pk = L.park[64 + tid];
           y_r[0] = py.x;
           y_i[0] = py.y;
@@ -1152,7 +1283,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
               break;
           }
           double ko_r[R], ko_i[R];
-          LB_RHS(yt_r, yt_i, ko_r, ko_i, L.coef + s * KK);
+          LB_RHS(yt_r, yt_i, ko_r, ko_i, L.coef + s * KK, min(s, 6) - 2);
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             switch (s) {
@@ -1586,6 +1717,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
     for (int i = tid; i < 7 * P.n_slots; i += W) L.slots[P.n_slots + i] = L.slots[i % P.n_slots];
     for (int i = tid; i < 7 * KK; i += W) L.coef[KK + i] = L.coef[i % KK];
     fold_self(P, tid, W, L.coef, L.selfc);
+    if (P.couplings) fill_static_entries(P, L.coef, L.ent, tid, W);
 
     double y_r[R], y_i[R];
     const double* y0 = C.y0 + (C.y0_shared ? 0 : traj * (int64_t)P.dim);
@@ -1644,10 +1776,10 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
     };
     double k_r[7][R], k_i[7][R];
     int buf = 0;
-#define LB_FRHS(xr, xi, kr, ki, cf)                                         \
-  do {                                                                      \
-    rhs_eval<R>(P, L, S, xr, xi, kr, ki, L.pub + buf * 2 * P.n_pub, cf, tid, W); \
-    buf ^= 1;                                                               \
+#define LB_FRHS(xr, xi, kr, ki, s)                                                              \
+  do {                                                                                          \
+    rhs_eval<R>(P, L, S, xr, xi, kr, ki, L.pub + buf * 2 * P.n_pub, L.coef + (s) * KK, (s) - 1, tid, W); \
+    buf ^= 1;                                                                                   \
   } while (0)
 
     if (bad_support) {
@@ -1687,16 +1819,20 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
         if (P.time_dependent && tid < NS)
           eval_coefficients(P, L.slots + (tid + 1) * P.n_slots, L.coef + (tid + 1) * KK, F::time(x, h, tid + 1),
                             true, L.vm + tid * P.vm_depth);
+        if (P.time_dependent && P.couplings) {
+          __syncthreads();
+          fill_entries<NS>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + KK, KK, L.ent + P.nv_stat, tid, W);
+        }
         // (the barrier inside the first RHS orders the rows before the gathers)
         double yt_r[R], yt_i[R], yn_r[R], yn_i[R];
-        LB_FRHS(y_r, y_i, k_r[1], k_i[1], L.coef + KK);
+        LB_FRHS(y_r, y_i, k_r[1], k_i[1], 1);
         if constexpr (ST == 1) {
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             yt_r[r] = y_r[r] + 0.5 * h * k_r[1][r];
             yt_i[r] = y_i[r] + 0.5 * h * k_i[1][r];
           }
-          LB_FRHS(yt_r, yt_i, k_r[2], k_i[2], L.coef + 2 * KK);
+          LB_FRHS(yt_r, yt_i, k_r[2], k_i[2], 2);
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             yn_r[r] = y_r[r] + h * k_r[2][r];
@@ -1708,19 +1844,19 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
             yt_r[r] = y_r[r] + 0.5 * h * k_r[1][r];
             yt_i[r] = y_i[r] + 0.5 * h * k_i[1][r];
           }
-          LB_FRHS(yt_r, yt_i, k_r[2], k_i[2], L.coef + 2 * KK);
+          LB_FRHS(yt_r, yt_i, k_r[2], k_i[2], 2);
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             yt_r[r] = y_r[r] + 0.5 * h * k_r[2][r];
             yt_i[r] = y_i[r] + 0.5 * h * k_i[2][r];
           }
-          LB_FRHS(yt_r, yt_i, k_r[3], k_i[3], L.coef + 3 * KK);
+          LB_FRHS(yt_r, yt_i, k_r[3], k_i[3], 3);
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             yt_r[r] = y_r[r] + h * k_r[3][r];
             yt_i[r] = y_i[r] + h * k_i[3][r];
           }
-          LB_FRHS(yt_r, yt_i, k_r[4], k_i[4], L.coef + 4 * KK);
+          LB_FRHS(yt_r, yt_i, k_r[4], k_i[4], 4);
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             yn_r[r] = y_r[r] + h * (k_r[1][r] + 2.0 * k_r[2][r] + 2.0 * k_r[3][r] + k_r[4][r]) / 6.0;
@@ -1737,23 +1873,23 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
             yt_r[r] = y_r[r] + h * (1.0 / 5.0) * k_r[1][r];
             yt_i[r] = y_i[r] + h * (1.0 / 5.0) * k_i[1][r];
           }
-          LB_FRHS(yt_r, yt_i, k_r[2], k_i[2], L.coef + 2 * KK);
+          LB_FRHS(yt_r, yt_i, k_r[2], k_i[2], 2);
           LB_FSUM((3.0 / 40.0) * k_r[1][r] + (9.0 / 40.0) * k_r[2][r],
                   (3.0 / 40.0) * k_i[1][r] + (9.0 / 40.0) * k_i[2][r])
-          LB_FRHS(yt_r, yt_i, k_r[3], k_i[3], L.coef + 3 * KK);
+          LB_FRHS(yt_r, yt_i, k_r[3], k_i[3], 3);
           LB_FSUM((44.0 / 45.0) * k_r[1][r] - (56.0 / 15.0) * k_r[2][r] + (32.0 / 9.0) * k_r[3][r],
                   (44.0 / 45.0) * k_i[1][r] - (56.0 / 15.0) * k_i[2][r] + (32.0 / 9.0) * k_i[3][r])
-          LB_FRHS(yt_r, yt_i, k_r[4], k_i[4], L.coef + 4 * KK);
+          LB_FRHS(yt_r, yt_i, k_r[4], k_i[4], 4);
           LB_FSUM((19372.0 / 6561.0) * k_r[1][r] - (25360.0 / 2187.0) * k_r[2][r] + (64448.0 / 6561.0) * k_r[3][r] -
                       (212.0 / 729.0) * k_r[4][r],
                   (19372.0 / 6561.0) * k_i[1][r] - (25360.0 / 2187.0) * k_i[2][r] + (64448.0 / 6561.0) * k_i[3][r] -
                       (212.0 / 729.0) * k_i[4][r])
-          LB_FRHS(yt_r, yt_i, k_r[5], k_i[5], L.coef + 5 * KK);
+          LB_FRHS(yt_r, yt_i, k_r[5], k_i[5], 5);
           LB_FSUM((9017.0 / 3168.0) * k_r[1][r] - (355.0 / 33.0) * k_r[2][r] + (46732.0 / 5247.0) * k_r[3][r] +
                       (49.0 / 176.0) * k_r[4][r] - (5103.0 / 18656.0) * k_r[5][r],
                   (9017.0 / 3168.0) * k_i[1][r] - (355.0 / 33.0) * k_i[2][r] + (46732.0 / 5247.0) * k_i[3][r] +
                       (49.0 / 176.0) * k_i[4][r] - (5103.0 / 18656.0) * k_i[5][r])
-          LB_FRHS(yt_r, yt_i, k_r[6], k_i[6], L.coef + 6 * KK);
+          LB_FRHS(yt_r, yt_i, k_r[6], k_i[6], 6);
 #undef LB_FSUM
 #pragma unroll
           for (int r = 0; r < R; ++r) {
@@ -1869,73 +2005,78 @@ __device__ __forceinline__ double half_sum(double x, int lane) {
 // only non-zero lane of a second wave sum.
 __device__ __forceinline__ double half_total(double x, int lane) { return half_sum(x, lane) + 0.0; }
 
-// The single-wave RHS for the element in slot `sl` of this half: inputs from
-// the lanes of the same half.  A kernel compiled for one plan (LB_GEN_COEF)
-// holds exactly its rows, so its loops have no row checks; the words are
-// loaded first, then every permute, then the factors and coefficients, so
-// each group of loads issues together.
+// The couplings of one lane, unpacked once per launch: byte offset of the
+// input in the half's publication buffer, byte offset and row stride of the
+// entry's value, and the sign bit of a conjugated input.
 template <int G>
-__device__ __forceinline__ void rhs_pair(const uint32_t* gw, const double2* gf, int rows, int sl, int base,
-                                         double2 selfv, bool diag, double xr, double xi, double& kr, double& ki,
-                                         const dcpx* coef) {
+struct PairRows {
+  uint32_t x[G], v[G], dv[G], sign[G];
+};
+
+// The single-wave RHS for the element in slot `sl` of this half: the lanes
+// publish the stage input to LDS and read each other's (one wave: its LDS
+// operations complete in order, no barrier).  A kernel compiled for one plan
+// (LB_GEN_COEF) holds exactly its rows, so its loops have no row checks.
+// Every read issues before the first term.
+template <int G>
+__device__ __forceinline__ void rhs_pair(const PairRows<G>& T, int rows, char* pub, const char* ent, int vrow, int sl,
+                                         double2 selfv, bool diag, double xr, double xi, double& kr, double& ki) {
 #ifdef LB_GEN_COEF
   (void)rows;
   constexpr bool exact = true;
 #else
   constexpr bool exact = false;
 #endif
+  reinterpret_cast<double2*>(pub)[sl] = double2{xr, xi};
+  wave_sync();
   double accr = fma(selfv.x, xr, -(selfv.y * xi));
   double acci = fma(selfv.x, xi, selfv.y * xr);
-  uint32_t w[G];
-  double2 f[G];
-  double sr[G], si[G];
-#pragma unroll
-  for (int j = 0; j < G; ++j)
-    if (exact || j < rows) w[j] = gw[j * 64 + sl];
+  double2 x[G], v[G];
 #pragma unroll
   for (int j = 0; j < G; ++j) {
     if (exact || j < rows) {
-      const int src = (int)(w[j] & 31u) | base;
-      sr[j] = __shfl(xr, src, 64);
-      si[j] = __shfl(xi, src, 64);
+      x[j] = *reinterpret_cast<const double2*>(pub + T.x[j]);
+      v[j] = *reinterpret_cast<const double2*>(ent + (T.v[j] + (uint32_t)vrow * T.dv[j]));
     }
   }
 #pragma unroll
   for (int j = 0; j < G; ++j)
-    if (exact || j < rows) f[j] = gf[j * 64 + sl];
-#pragma unroll
-  for (int j = 0; j < G; ++j)
-    if (exact || j < rows) gather_apply(w[j], f[j], coef, sr[j], si[j], accr, acci);
+    if (exact || j < rows) couple(T.sign[j], v[j], x[j], accr, acci);
+  wave_sync();
   kr = accr;
   ki = diag ? 0.0 : acci;
 }
 
 struct LdsPair {
-  double2* gf;    // g_rows x 64 gather factors
+  dcpx* ent;      // 2 halves x (nv_stat + LB_ENT_ROWS x nv_dyn) entry values
   dcpx* coef;     // 2 halves x 8 rows x (K + 1): [0] t0, [2..7] stage times
   dcpx* slots;    // 2 halves x 8 x n_slots
   dcpx* vm;       // 2 halves x 8 lanes x vm_depth
-  double2* selfc; // 2 halves x 32 folded self coefficients
+  char* pub;      // 2 halves x 32 published stage inputs
   double2* park;  // 2 x 64: y and k1 around the expression machine
+  double2* ef;    // factors, coefficient rows and extents of the time-dependent entries
+  uint32_t* ecoef;
+  int* eptr;
   double* wts;    // n integral weights
-  uint32_t* gw;   // g_rows x 64 gather words
   int* misc;      // [0..1] queue values, [2..3] support flags
 };
 
 __device__ __forceinline__ LdsPair carve_pair(const DevPlan& P) {
   extern __shared__ double smem[];
-  const int g = cst(P.blk_rows)[0];
-  char* q = reinterpret_cast<char*>(smem);
+  char* const base = reinterpret_cast<char*>(smem);
+  const LbLdsPair l = lb_lds_pair(P);
   LdsPair L;
-  L.gf = reinterpret_cast<double2*>(q); q += (size_t)g * 64 * 16;
-  L.coef = reinterpret_cast<dcpx*>(q); q += (size_t)2 * 8 * (P.K + 1) * 16;
-  L.slots = reinterpret_cast<dcpx*>(q); q += (size_t)2 * 8 * P.n_slots * 16;
-  L.vm = reinterpret_cast<dcpx*>(q); q += (size_t)2 * 8 * P.vm_depth * 16;
-  L.selfc = reinterpret_cast<double2*>(q); q += (size_t)64 * 16;
-  L.park = reinterpret_cast<double2*>(q); q += (size_t)128 * 16;
-  L.wts = reinterpret_cast<double*>(q); q += (size_t)((P.n + 1) & ~1) * 8;
-  L.gw = reinterpret_cast<uint32_t*>(q); q += (size_t)g * 64 * 4;
-  L.misc = reinterpret_cast<int*>(q);
+  L.ent = reinterpret_cast<dcpx*>(base + l.ent);
+  L.coef = reinterpret_cast<dcpx*>(base + l.coef);
+  L.slots = reinterpret_cast<dcpx*>(base + l.slots);
+  L.vm = reinterpret_cast<dcpx*>(base + l.vm);
+  L.pub = base + l.pub;
+  L.park = reinterpret_cast<double2*>(base + l.park);
+  L.ef = reinterpret_cast<double2*>(base + l.ef);
+  L.ecoef = reinterpret_cast<uint32_t*>(base + l.ecoef);
+  L.eptr = reinterpret_cast<int*>(base + l.eptr);
+  L.wts = reinterpret_cast<double*>(base + l.wts);
+  L.misc = reinterpret_cast<int*>(base + l.misc);
   return L;
 }
 
@@ -1956,16 +2097,28 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
   const int lane = threadIdx.x, half = lane >> 5, sl = lane & 31, base = lane & 32;
   const LdsPair L = carve_pair(P);
   const int KK = P.K + 1;
-  const int grows = cst(P.blk_rows)[0];
+  const int crows = cst(P.c_rows)[0];
   dcpx* const coef = L.coef + half * 8 * KK;
   dcpx* const slots = L.slots + half * 8 * P.n_slots;
+  dcpx* const ent = L.ent + half * (P.nv_stat + LB_ENT_ROWS * P.nv_dyn);
+  char* const pub = L.pub + half * 32 * 16;
+  PairRows<G> rows;
+#pragma unroll
+  for (int j = 0; j < G; ++j) {
+    const uint32_t w = j < crows ? P.c_word[j * 64 + sl] : 0u;
+    rows.x[j] = w >> 16;
+    rows.v[j] = w & 0xFFF0u;
+    rows.dv[j] = (w & 1u) * 16u * (uint32_t)P.nv_dyn;
+    rows.sign[j] = (w << 30) & 0x80000000u;
+  }
   Slots<1> S;
   load_slots<1>(P, S, sl, 64);
   const bool diag = S.diag(0);
-  for (int i = lane; i < grows * 64; i += 64) {
-    L.gf[i] = reinterpret_cast<const double2*>(P.g_f)[i];
-    L.gw[i] = P.g_word[i];
+  for (int i = lane; i < P.nv_terms; i += 64) {
+    L.ef[i] = reinterpret_cast<const double2*>(P.ent_f)[i];
+    L.ecoef[i] = P.ent_coef[i];
   }
+  for (int i = lane; i <= P.nv_dyn; i += 64) L.eptr[i] = P.ent_ptr[i];
   for (int i = lane; i < P.n; i += 64) {
     double w = 0.0;
     for (int q = 0; q < C.n_weights; ++q)
@@ -2024,6 +2177,9 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
       for (int i = sl; i < 7 * P.n_slots; i += 32) slots[P.n_slots + i] = slots[i % P.n_slots];
       for (int i = sl; i < 7 * KK; i += 32) coef[KK + i] = coef[i % KK];
       wave_sync();  // the stage rows are read by the expression-machine lanes
+      fill_static_entries(P, coef, ent, sl, 32);
+      fill_entries<1>(P.nv_dyn, L.eptr, L.ecoef, L.ef, coef, KK, ent + P.nv_stat + 5 * P.nv_dyn, sl, 32);
+      wave_sync();
       {  // folded self coefficient of this element (fold_self arithmetic)
         dcpx acc = mk(0.0, 0.0);
         for (int j = 0; j < P.max_self; ++j) {
@@ -2078,7 +2234,8 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
         if (t1 == C.t0) {
           last = true;
         } else {
-          rhs_pair<G>(L.gw, L.gf, grows, sl, base, selfv, diag, y_r[0], y_i[0], k_r[1][0], k_i[1][0], coef);
+          rhs_pair<G>(rows, crows, pub, reinterpret_cast<const char*>(ent), 5, sl, selfv, diag, y_r[0], y_i[0],
+                      k_r[1][0], k_i[1][0]);
           h = fmin(C.dt, t1 - C.t0);
           rhs_calls = 1;
         }
@@ -2116,7 +2273,12 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
                           L.vm + (half * 8 + sl) * P.vm_depth);
 #endif
       }
-      wave_sync();  // stage coefficients are read by every lane of the half
+      if (P.time_dependent) {
+        wave_sync();  // stage coefficients are read by every lane of the half
+        // stages 2..6 take entry rows 0..4; stage 7 is at the same time as 6
+        fill_entries<5>(P.nv_dyn, L.eptr, L.ecoef, L.ef, coef + 2 * KK, KK, ent + P.nv_stat, sl, 32);
+      }
+      wave_sync();
       {
         const double2 py = L.park[lane], pk = L.park[64 + lane];
         y_r[0] = py.x;
@@ -2128,8 +2290,8 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
       double yt_r[1], yt_i[1], yn_r[1], yn_i[1];
 #define LB_PAIR_STAGE(st)                                                                            \
   stage_combo<1, SOLVER, st>(h, y_r, y_i, k_r, k_i, yt_r, yt_i);                                    \
-  rhs_pair<G>(L.gw, L.gf, grows, sl, base, selfv, diag, yt_r[0], yt_i[0], k_r[st][0], k_i[st][0],   \
-              coef + (st) * KK);
+  rhs_pair<G>(rows, crows, pub, reinterpret_cast<const char*>(ent), (st) - 2, sl, selfv, diag, yt_r[0], yt_i[0], \
+              k_r[st][0], k_i[st][0]);
       LB_PAIR_STAGE(2)
       LB_PAIR_STAGE(3)
       LB_PAIR_STAGE(4)
@@ -2142,7 +2304,8 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
         const double a0 = yn_r[0] - yt_r[0], a1 = yn_i[0] - yt_i[0];
         stiff_d = a0 * a0 + a1 * a1;
       }
-      rhs_pair<G>(L.gw, L.gf, grows, sl, base, selfv, diag, yn_r[0], yn_i[0], k_r[7][0], k_i[7][0], coef + 7 * KK);
+      rhs_pair<G>(rows, crows, pub, reinterpret_cast<const char*>(ent), 4, sl, selfv, diag, yn_r[0], yn_i[0],
+                  k_r[7][0], k_i[7][0]);
       rhs_calls += 6;
       // ---- error norm, integrand, stiffness (as the single-wave form)
       double er = T::e(1) * k_r[1][0], ei = T::e(1) * k_i[1][0];
@@ -3513,6 +3676,10 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_rhs_kernel(const DevPlan P, co
     }
     __syncthreads();
     fold_self(P, tid, W, L.coef, L.selfc);
+    if (P.couplings) {
+      fill_static_entries(P, L.coef, L.ent, tid, W);
+      fill_entries<1>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef, P.K + 1, L.ent + P.nv_stat, tid, W);
+    }
     double xr[R], xi[R], kr[R], ki[R];
     const double* y = C.y + b * (int64_t)P.dim;
 #pragma unroll
@@ -3521,7 +3688,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_rhs_kernel(const DevPlan P, co
       xr[r] = S.valid(r) ? y[P.slot_re[s]] : 0.0;
       xi[r] = (S.valid(r) && !S.diag(r)) ? y[P.slot_im[s]] : 0.0;
     }
-    rhs_eval<R>(P, L, S, xr, xi, kr, ki, L.pub, L.coef, tid, W);
+    rhs_eval<R>(P, L, S, xr, xi, kr, ki, L.pub, L.coef, 0, tid, W);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (!S.valid(r)) continue;

@@ -30,7 +30,7 @@ import numpy as np
 
 from . import _driver as D
 from .derivatives import differentiate_flat_plan
-from .native import DevicePlan, Tape
+from .native import DevicePlan, NativeError, Tape
 
 __all__ = ["DifferentiablePhotonCount", "photon_count"]
 
@@ -75,6 +75,11 @@ class DifferentiablePhotonCount:
         self.every = int(ckpt_every)
         self.capacity = int(tape_capacity)
         self.plan = DevicePlan(differentiate_flat_plan(prepared.flat_plan, self.slots, with_time=True))
+        if getattr(prepared, "specialize", True):
+            try:
+                self.plan.specialize()
+            except NativeError:  # an instruction without a generated form: the precompiled kernels run
+                pass
 
     def _common(self, params, y0):
         import torch

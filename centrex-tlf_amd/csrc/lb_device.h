@@ -191,17 +191,23 @@ __host__ __device__ inline LbLds lb_lds_layout(const DevPlan& P) {
   return l;
 }
 
-// LDS of the paired kernel: the entry definitions once, the rest per half.
+// Forms of the paired kernel: save plans and traces, stop events.
+#define LB_LANE_SAVE 1
+#define LB_LANE_EVENT 2
+
+// LDS of the paired kernel with nh trajectories per wave: the entry
+// definitions once, the rest per trajectory.
 struct LbLdsPair {
-  uint32_t ent, coef, slots, vm, pub, park, ef, wts, ecoef, eptr, misc, total;
+  uint32_t ent, coef, slots, vm, pub, evv, park, ef, wts, ecoef, eptr, misc, total;
 };
-__host__ __device__ inline LbLdsPair lb_lds_pair(const DevPlan& P) {
+__host__ __device__ inline LbLdsPair lb_lds_pair(const DevPlan& P, uint32_t nh) {
   LbLdsPair l;
   uint32_t q = 0;
-  l.ent = q; q += 2u * 16u * (uint32_t)(P.nv_stat + LB_ENT_ROWS * P.nv_dyn);
-  l.coef = q; q += 2u * 8u * 16u * (uint32_t)(P.K + 1);
-  l.slots = q; q += 2u * 8u * 16u * (uint32_t)P.n_slots;
-  l.vm = q; q += 2u * 8u * 16u * (uint32_t)P.vm_depth;
+  l.ent = q; q += nh * 16u * (uint32_t)(P.nv_stat + LB_ENT_ROWS * P.nv_dyn);
+  l.coef = q; q += nh * 8u * 16u * (uint32_t)(P.K + 1);
+  l.slots = q; q += nh * 8u * 16u * (uint32_t)P.n_slots;
+  l.vm = q; q += nh * 8u * 16u * (uint32_t)P.vm_depth;
+  l.evv = q; q += nh * 8u * (uint32_t)((P.n + 3) & ~1);
   l.pub = q; q += 64u * 16u;
   l.park = q; q += 128u * 16u;
   l.ef = q; q += 16u * (uint32_t)P.nv_terms;

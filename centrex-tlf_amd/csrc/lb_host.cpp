@@ -168,15 +168,13 @@ struct lb_plan {
   size_t ev_cap = 0;
   hipEvent_t ev_copied = nullptr;
   // plan-specialised paired kernels (lb_plan_specialize): the generated
-  // coefficient function, and (variant | gather rows << 8, solver) -> compiled module
+  // coefficient function, and kernel name -> compiled module
   // A failed compilation leaves a null entry (the precompiled kernel runs)
   // and its reason in spec_failure.
   bool spec = false;
   std::string spec_source, spec_failure;
-  std::map<std::pair<int, int>, std::pair<hipModule_t, hipFunction_t>> spec_kernels;
+  std::map<std::string, std::shared_ptr<LbModule>> spec_kernels;
   ~lb_plan() {
-    for (auto& kv : spec_kernels)
-      if (kv.second.first) (void)hipModuleUnload(kv.second.first);
     auto release = [](DevImage* im) {
       if (!im) return;
       for (void* a : im->allocations) (void)hipFree(a);
@@ -295,11 +293,13 @@ void pick_config(int S, int rows, int* id_out, int* W_out) {
 
 // Coupling words (or gather tables) up to this size are copied into LDS by every workgroup.
 constexpr int64_t kLdsTableBytes = 32 * 1024;
+// Coupling rows a plan-specialised paired kernel holds in registers (4 each).
+constexpr int kMaxLaneRows = 16;
 // LDS of one workgroup on gfx950.
 constexpr int64_t kMaxLdsBytes = 160 * 1024;
 
 int64_t lds_bytes_for(const DevPlan& P) { return lb_lds_layout(P).total; }
-int64_t lds_bytes_pair(const DevPlan& P) { return lb_lds_pair(P).total; }
+int64_t lds_bytes_pair(const DevPlan& P, int nh = 2) { return lb_lds_pair(P, (uint32_t)nh).total; }
 
 int set_lds_limit(const void* fn, size_t lds) {
   if (lds > 65536)
@@ -1435,46 +1435,84 @@ int launch_table(const lb_plan* p, const lb_solve_args* a, const DevImage* im, D
 
 namespace {
 
-// The plan-specialised form of paired variant `id` for `solver`, compiled on
-// first use; nullptr when the plan is not specialised.  (Only the paired
-// kernels take the generated code: a specialised multi-wave kernel launched
-// with 1024-thread workgroups had its queue aborted at dispatch, cause not
-// found, so the single- and multi-wave kernels stay on the precompiled form.)
-int spec_kernel(lb_plan* p, int id, int solver, int rows, hipStream_t stream, hipFunction_t* fn) {
+// The plan-specialised kernel `name` (a template-id), compiled on first use;
+// nullptr when the plan is not specialised.  (Only the paired kernels, one
+// wave per workgroup, take the generated code: a specialised multi-wave
+// kernel launched with 1024-thread workgroups had its queue aborted at
+// dispatch, cause not found, so the multi-wave kernels stay on the
+// precompiled form.)
+int spec_kernel(lb_plan* p, const std::string& name, hipStream_t stream, hipFunction_t* fn) {
   *fn = nullptr;
   std::lock_guard<std::mutex> lock(p->mu);
   if (!p->spec) return LB_OK;
-  // the kernel holds exactly the plan's gather rows in registers (fewer than
-  // the variant's maximum frees registers; the same rows in the same order)
-  const int G = std::max(1, std::min(rows, lb_dev_variant_rows(id)));
-  auto it = p->spec_kernels.find({id | (G << 8), solver});
+  auto it = p->spec_kernels.find(name);
   if (it == p->spec_kernels.end()) {
     // no compilation or module load inside a stream capture: a captured
     // first call takes the precompiled kernel (bitwise the same results)
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(stream, &cs));
     if (cs != hipStreamCaptureStatusNone) return LB_OK;
-    int R, maxw, waves;
-    if (!lb_dev_variant(id, &R, &maxw, &waves)) return fail(LB_ERR_INVALID, "no such kernel variant");
-    if (!lb_dev_variant_pair(id)) return fail(LB_ERR_INVALID, "only paired variants are specialised");
-    char name[96];
-    std::snprintf(name, sizeof name, "lb_solve_pair_kernel<%d, %d, %d>", solver == LB_SOLVER_TSIT5 ? 1 : 0, G,
-                  waves);
-    hipModule_t mod = nullptr;
-    hipFunction_t f = nullptr;
+    std::shared_ptr<LbModule> mod;
     std::string why;
-    if (lb_rtc_compile(p->spec_source, name, &mod, &f, why)) {
+    if (lb_rtc_compile(p->spec_source, name, &mod, why)) {
       // the precompiled kernel computes the same values: run it, remember
       // the failure so that later calls neither recompile nor fail
       (void)hipGetLastError();  // a failed module load leaves its error behind
-      mod = nullptr;
-      f = nullptr;
-      p->spec_failure = std::string(name) + ": " + why;
+      mod.reset();
+      p->spec_failure = name + ": " + why;
     }
-    it = p->spec_kernels.emplace(std::make_pair(id | (G << 8), solver), std::make_pair(mod, f)).first;
+    it = p->spec_kernels.emplace(name, mod).first;
   }
-  *fn = it->second.second;
+  *fn = it->second ? it->second->function : nullptr;
   return LB_OK;
+}
+
+// Launch of a plan-specialised paired kernel for this call, if it has one:
+// *launched says whether the call was launched.  The kernels hold exactly the
+// plan's coupling rows in registers and one or two trajectories per wave
+// (plans of at most 32 elements two).  Against the precompiled kernels that
+// run these calls otherwise (n = 39 grids): the expression machine leaves the
+// step, and a step needs no workgroup barrier.
+int launch_spec(lb_plan* p, const lb_solve_args* a, const DevImage* im, DevCall& c, hipStream_t s, bool event,
+                int ev_depth, bool* launched) {
+  *launched = false;
+  const bool fixed = a->solver >= LB_SOLVER_FIXED_DOPRI5;
+  DevPlan P = im->dev;
+  P.vm_depth = std::max(P.vm_depth, ev_depth);  // the stop-event expression runs on one lane's stack
+  const int rows = (int)im->rows_total, nh = im->active <= 32 ? 2 : 1;
+  if (!p->spec || !P.time_dependent || P.nblk != 1 || !P.couplings || rows > kMaxLaneRows) return LB_OK;
+  if (a->mode != LB_MODE_PERSISTENT || a->replay_h || !(std::isfinite(a->dt) && a->dt > 0.0)) return LB_OK;
+  if (fixed && event) return LB_OK;
+  const size_t lds = (size_t)lds_bytes_pair(P, nh);
+  if (lds > 65536) return LB_OK;  // dynamic LDS within 64 KB: no per-kernel opt-in needed
+  const bool save = a->trace || a->n_saveat > 0 || a->output_kind == LB_OUT_RATE;
+  char name[96];
+  if (fixed)
+    std::snprintf(name, sizeof name, "lb_fixed_pair_kernel<%d, %d, 2, %d>", a->solver - LB_SOLVER_FIXED_DOPRI5,
+                  std::max(1, rows), 64 / nh);
+  else
+    std::snprintf(name, sizeof name, "lb_solve_pair_kernel<%d, %d, 2, %d, %d>", a->solver == LB_SOLVER_TSIT5 ? 1 : 0,
+                  std::max(1, rows), 64 / nh, event ? LB_LANE_SAVE | LB_LANE_EVENT : save ? LB_LANE_SAVE : 0);
+  hipFunction_t fn = nullptr;
+  int rc = spec_kernel(p, name, s, &fn);
+  if (rc || !fn) return rc;
+  int grid = a->workgroups;
+  if (grid <= 0) {
+    int per_cu = 0;
+    HIP_TRY(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64, lds));
+    grid = std::max(1, per_cu) * std::max(1, p->cus);
+  }
+  grid = (int)std::min<int64_t>(grid, (a->n_traj + nh - 1) / nh);
+  c.traj_offset = 0;
+  int slot = 0;
+  if ((rc = p->queues.acquire(s, &c.queue, &slot))) return rc;
+  void* rargs[] = {&c.queue};
+  HIP_TRY(hipLaunchKernel(lb_dev_queue_reset_kernel(), dim3(1), dim3(1), rargs, 0, s));
+  void* args[] = {&P, &c};
+  HIP_TRY(hipModuleLaunchKernel(fn, grid, 1, 1, 64, 1, 1, (unsigned)lds, s, args, nullptr));
+  HIP_TRY(hipGetLastError());
+  *launched = true;
+  return p->queues.retire(slot, s);
 }
 
 }  // namespace
@@ -1489,12 +1527,25 @@ extern "C" int lb_solve(const lb_plan* p, const lb_solve_args* a, void* stream) 
   int ev_depth = 0;
   if ((rc = prepare_event(const_cast<lb_plan*>(p), a, (hipStream_t)stream, c, &ev_depth))) return rc;
   const bool event = a->event_kind != LB_EVENT_NONE;
-  if (event || a->solver >= LB_SOLVER_FIXED_DOPRI5) return launch_table(p, a, im, c, stream, event, ev_depth);
+  if (event || a->solver >= LB_SOLVER_FIXED_DOPRI5) {
+    if (a->tape_h == nullptr && a->threads_per_traj == 0) {
+      bool launched = false;
+      rc = launch_spec(const_cast<lb_plan*>(p), a, im, c, (hipStream_t)stream, event, ev_depth, &launched);
+      if (rc || launched) return rc;
+    }
+    return launch_table(p, a, im, c, stream, event, ev_depth);
+  }
   int id, W;
   const bool pair_ok = a->mode == LB_MODE_PERSISTENT && !a->trace && a->n_saveat == 0 &&
                        !a->replay_h && std::isfinite(a->dt) && a->dt > 0.0 && a->output_kind != LB_OUT_RATE;
   if ((rc = resolve_config(im, a->variant, a->threads_per_traj, pair_ok, &id, &W))) return rc;
   const bool pair = lb_dev_variant_pair(id) != 0;
+  // a single-wave variant named for a plan that pairs is that variant
+  if (pair || (lb_dev_variant_rows(id) && (a->variant <= 0 || im->active > 32))) {
+    bool launched = false;
+    rc = launch_spec(const_cast<lb_plan*>(p), a, im, c, (hipStream_t)stream, false, 0, &launched);
+    if (rc || launched) return rc;
+  }
   void* fn = lb_dev_solve_kernel(id, a->solver);
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "kernel variant is not built");
   void* reset = lb_dev_queue_reset_kernel();
@@ -1535,26 +1586,13 @@ extern "C" int lb_solve(const lb_plan* p, const lb_solve_args* a, void* stream) 
     grid = std::max(1, per_cu) * std::max(1, p->cus);
   }
   grid = (int)std::min<int64_t>(grid, pair ? (a->n_traj + 1) / 2 : a->n_traj);
-  hipFunction_t spec_fn = nullptr;
-  if (pair && P.time_dependent && lds <= 65536 &&
-      (rc = spec_kernel(const_cast<lb_plan*>(p), id, a->solver, (int)im->rows_total, s, &spec_fn)))
-    return rc;
-  if (spec_fn && a->workgroups <= 0) {  // its own register allocation sets its residency
-    int per_cu = 0;
-    HIP_TRY(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, spec_fn, W, lds));
-    grid = (int)std::min<int64_t>((int64_t)std::max(1, per_cu) * std::max(1, p->cus),
-                                  pair ? (a->n_traj + 1) / 2 : a->n_traj);
-  }
   c.traj_offset = 0;
   int slot = 0;
   if ((rc = const_cast<lb_plan*>(p)->queues.acquire(s, &c.queue, &slot))) return rc;
   void* rargs[] = {&c.queue};
   HIP_TRY(hipLaunchKernel(reset, dim3(1), dim3(1), rargs, 0, s));
   void* args[] = {&P, &c};
-  if (spec_fn)  // dynamic LDS within 64 KB: no per-kernel opt-in needed
-    HIP_TRY(hipModuleLaunchKernel(spec_fn, grid, 1, 1, W, 1, 1, (unsigned)lds, s, args, nullptr));
-  else
-    HIP_TRY(hipLaunchKernel(fn, dim3(grid), dim3(W), args, lds, s));
+  HIP_TRY(hipLaunchKernel(fn, dim3(grid), dim3(W), args, lds, s));
   HIP_TRY(hipGetLastError());
   return const_cast<lb_plan*>(p)->queues.retire(slot, s);
 }

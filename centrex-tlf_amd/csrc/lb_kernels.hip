@@ -426,6 +426,31 @@ __device__ __forceinline__ void stage_combo(double h, const double (&y_r)[R], co
   }
 }
 
+// The step-size controller (common.rs:32-70): alpha = 0.2 - 0.75 beta, beta =
+// 0.04, safety 0.9, the step's factor within [1/5, 10].  The reference's h /
+// (err^alpha fac_old^-beta / 0.9) is h times 0.9 exp(beta ln fac_old - alpha
+// ln err): one log of the squared norm and one exp.  ln fac_old = max(ln err,
+// ln 1e-4) is carried from the last accepted step.  As two pow, a square root
+// and three divisions one after another the chain was 3.1k of a paired
+// attempt's 15k cycles.  A NaN error norm is a rejection with the largest cut.
+#define LB_LOG_FAC_MIN -9.210340371976182  // ln 1e-4
+struct StepControl {
+  double err, lerr, raw;  // error norm, its log, the factor before its bounds
+  bool accept;
+  // q = err^2; lfo = ln fac_old
+  __device__ __forceinline__ StepControl(double q, double lfo) {
+    err = sqrt(q);
+    lerr = 0.5 * log(q);
+    accept = err <= 1.0;
+    raw = 0.9 * exp((accept ? 0.04 * lfo : 0.0) - (0.2 - 0.04 * 0.75) * lerr);
+  }
+  __device__ __forceinline__ double factor() const {
+    return accept ? fmax(0.2, fmin(10.0, raw)) : fmax(0.2, raw);
+  }
+  // the factor is one of its bounds (no dependence on err or fac_old)
+  __device__ __forceinline__ bool clamped() const { return accept ? !(raw < 10.0 && raw > 0.2) : !(raw > 0.2); }
+};
+
 template <int R>
 __device__ __forceinline__ void copy_k(const double (&a)[R], const double (&b)[R], double (&ka)[R],
                                        double (&kb)[R]) {
@@ -1198,9 +1223,8 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         push(t0, y_r, y_i, true);
       }
       // ---- controller state (common.rs:32-70)
-      const double beta = 0.04, alpha = 0.2 - beta * 0.75, facc1 = 1.0 / 0.2, facc2 = 1.0 / 10.0;
-      const double safety = 0.9, hmax = fabs(t1 - t0);
-      double fac_old = 1.0e-4;
+      const double hmax = fabs(t1 - t0), inv_dim = 1.0 / (double)P.dim;
+      double fac_old = 1.0e-4, lfo = LB_LOG_FAC_MIN;
       bool reject = false, last = false;
       int64_t ns = 0, nst = 0, ia = 0;
 
@@ -1322,16 +1346,9 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           }
         }
         __syncthreads();
-        const double err = C.replay_h ? 0.0 : sqrt(block_total(P, L.red, 0) / (double)P.dim);
-        // ---- controller (common.rs:48-69); the two powers at once in each
-        // wave (lanes 0-31: err^alpha, lanes 32-63: fac_old^-beta)
-        const int wl = tid & 63;
-        const double pw = pow(wl < 32 ? err : fac_old, wl < 32 ? alpha : -beta);
-        const double fac11 = __shfl(pw, 0, 64), fo = __shfl(pw, 32, 64);
-        double fac = fac11 * fo;
-        const double fac_s = fac / safety;
-        fac = fmax(facc2, fmin(facc1, fac_s));
-        double hn = h / fac;
+        const StepControl ctl(C.replay_h ? 0.0 : block_total(P, L.red, 0) * inv_dim, lfo);
+        const double err = ctl.err;
+        double hn = h * ctl.factor();
         if (C.tape_h && !C.replay_h) {
           // attempt tape: what the adjoint needs to differentiate this attempt
           // and the controller's decision (one record per attempt)
@@ -1339,24 +1356,18 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           if (a < C.tape_cap) {
             if (tid == 0) {
               int fl = clipped ? LB_TAPE_CLIPPED : 0;
-              double h_next;
-              if (err <= 1.0) {
-                h_next = hn;
+              if (ctl.clamped()) fl |= LB_TAPE_CLAMPED;
+              if (ctl.accept) {
                 fl |= LB_TAPE_ACCEPTED | (accepted == 0 ? LB_TAPE_FIRST : 0) | (err > 1.0e-4 ? LB_TAPE_ERRQ : 0);
-                if (!(fac_s > facc2 && fac_s < facc1)) fl |= LB_TAPE_CLAMPED;
                 double hc = hn;
                 if (fabs(hc) > hmax) { hc = hmax; fl |= LB_TAPE_HMAX; }
                 if (reject && fabs(h) < fabs(hc)) fl |= LB_TAPE_MINRULE;
-              } else {
-                const double fr = fac11 / safety;
-                h_next = h / fmin(facc1, fr);
-                if (!(fr < facc1)) fl |= LB_TAPE_CLAMPED;
               }
               const int64_t o = traj * C.tape_cap + a;
               C.tape_t[o] = x;
               C.tape_h[o] = h;
               C.tape_c[3 * o] = err;
-              C.tape_c[3 * o + 1] = h_next;
+              C.tape_c[3 * o + 1] = hn;
               C.tape_c[3 * o + 2] = fac_old;
               C.tape_f[o] = fl;
             }
@@ -1374,8 +1385,9 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
             }
           }
         }
-        if (err <= 1.0) {
+        if (ctl.accept) {
           fac_old = fmax(err, 1.0e-4);
+          lfo = fmax(ctl.lerr, LB_LOG_FAC_MIN);
           if (fabs(hn) > hmax) hn = hmax;
           if (reject) hn = fmin(fabs(hn), fabs(h));
           reject = false;
@@ -1503,7 +1515,6 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           }
           if (last) break;
         } else {
-          hn = h / fmin(facc1, fac11 / safety);
           reject = true;
           last = false;
           if (accepted >= 1) ++rejected;
@@ -1610,6 +1621,91 @@ struct FixedStep {
            : s == 4 ? x + h * (4.0 / 5.0) : s == 5 ? x + h * (8.0 / 9.0) : x + h;
   }
 };
+
+// One step of size h from y: the stage derivatives k (stage s from
+// rhs(x_r, x_i, s, k_r, k_i)) and the new state yn, with the sums in the
+// reference's operation order.
+template <int ST, int R, typename Rhs>
+__device__ __forceinline__ void fixed_step(double h, const double (&y_r)[R], const double (&y_i)[R],
+                                           double (&k_r)[7][R], double (&k_i)[7][R], double (&yt_r)[R],
+                                           double (&yt_i)[R], double (&yn_r)[R], double (&yn_i)[R], Rhs&& rhs) {
+  rhs(y_r, y_i, 1, k_r[1], k_i[1]);
+  if constexpr (ST == 1) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      yt_r[r] = y_r[r] + 0.5 * h * k_r[1][r];
+      yt_i[r] = y_i[r] + 0.5 * h * k_i[1][r];
+    }
+    rhs(yt_r, yt_i, 2, k_r[2], k_i[2]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      yn_r[r] = y_r[r] + h * k_r[2][r];
+      yn_i[r] = y_i[r] + h * k_i[2][r];
+    }
+  } else if constexpr (ST == 2) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      yt_r[r] = y_r[r] + 0.5 * h * k_r[1][r];
+      yt_i[r] = y_i[r] + 0.5 * h * k_i[1][r];
+    }
+    rhs(yt_r, yt_i, 2, k_r[2], k_i[2]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      yt_r[r] = y_r[r] + 0.5 * h * k_r[2][r];
+      yt_i[r] = y_i[r] + 0.5 * h * k_i[2][r];
+    }
+    rhs(yt_r, yt_i, 3, k_r[3], k_i[3]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      yt_r[r] = y_r[r] + h * k_r[3][r];
+      yt_i[r] = y_i[r] + h * k_i[3][r];
+    }
+    rhs(yt_r, yt_i, 4, k_r[4], k_i[4]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      yn_r[r] = y_r[r] + h * (k_r[1][r] + 2.0 * k_r[2][r] + 2.0 * k_r[3][r] + k_r[4][r]) / 6.0;
+      yn_i[r] = y_i[r] + h * (k_i[1][r] + 2.0 * k_i[2][r] + 2.0 * k_i[3][r] + k_i[4][r]) / 6.0;
+    }
+  } else {
+#define LB_FSUM(expr_r, expr_i)            \
+  _Pragma("unroll") for (int r = 0; r < R; ++r) { \
+    yt_r[r] = y_r[r] + h * (expr_r);       \
+    yt_i[r] = y_i[r] + h * (expr_i);       \
+  }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      yt_r[r] = y_r[r] + h * (1.0 / 5.0) * k_r[1][r];
+      yt_i[r] = y_i[r] + h * (1.0 / 5.0) * k_i[1][r];
+    }
+    rhs(yt_r, yt_i, 2, k_r[2], k_i[2]);
+    LB_FSUM((3.0 / 40.0) * k_r[1][r] + (9.0 / 40.0) * k_r[2][r],
+            (3.0 / 40.0) * k_i[1][r] + (9.0 / 40.0) * k_i[2][r])
+    rhs(yt_r, yt_i, 3, k_r[3], k_i[3]);
+    LB_FSUM((44.0 / 45.0) * k_r[1][r] - (56.0 / 15.0) * k_r[2][r] + (32.0 / 9.0) * k_r[3][r],
+            (44.0 / 45.0) * k_i[1][r] - (56.0 / 15.0) * k_i[2][r] + (32.0 / 9.0) * k_i[3][r])
+    rhs(yt_r, yt_i, 4, k_r[4], k_i[4]);
+    LB_FSUM((19372.0 / 6561.0) * k_r[1][r] - (25360.0 / 2187.0) * k_r[2][r] + (64448.0 / 6561.0) * k_r[3][r] -
+                (212.0 / 729.0) * k_r[4][r],
+            (19372.0 / 6561.0) * k_i[1][r] - (25360.0 / 2187.0) * k_i[2][r] + (64448.0 / 6561.0) * k_i[3][r] -
+                (212.0 / 729.0) * k_i[4][r])
+    rhs(yt_r, yt_i, 5, k_r[5], k_i[5]);
+    LB_FSUM((9017.0 / 3168.0) * k_r[1][r] - (355.0 / 33.0) * k_r[2][r] + (46732.0 / 5247.0) * k_r[3][r] +
+                (49.0 / 176.0) * k_r[4][r] - (5103.0 / 18656.0) * k_r[5][r],
+            (9017.0 / 3168.0) * k_i[1][r] - (355.0 / 33.0) * k_i[2][r] + (46732.0 / 5247.0) * k_i[3][r] +
+                (49.0 / 176.0) * k_i[4][r] - (5103.0 / 18656.0) * k_i[5][r])
+    rhs(yt_r, yt_i, 6, k_r[6], k_i[6]);
+#undef LB_FSUM
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      yn_r[r] = y_r[r] + h * ((35.0 / 384.0) * k_r[1][r] + (500.0 / 1113.0) * k_r[3][r] +
+                              (125.0 / 192.0) * k_r[4][r] - (2187.0 / 6784.0) * k_r[5][r] +
+                              (11.0 / 84.0) * k_r[6][r]);
+      yn_i[r] = y_i[r] + h * ((35.0 / 384.0) * k_i[1][r] + (500.0 / 1113.0) * k_i[3][r] +
+                              (125.0 / 192.0) * k_i[4][r] - (2187.0 / 6784.0) * k_i[5][r] +
+                              (11.0 / 84.0) * k_i[6][r]);
+    }
+  }
+}
 
 // Outputs of a finished trajectory (final values, integral, stats), as the
 // adaptive kernel writes them.
@@ -1776,11 +1872,6 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
     };
     double k_r[7][R], k_i[7][R];
     int buf = 0;
-#define LB_FRHS(xr, xi, kr, ki, s)                                                              \
-  do {                                                                                          \
-    rhs_eval<R>(P, L, S, xr, xi, kr, ki, L.pub + buf * 2 * P.n_pub, L.coef + (s) * KK, (s) - 1, tid, W); \
-    buf ^= 1;                                                                                   \
-  } while (0)
 
     if (bad_support) {
       status = LB_TRAJ_BAD_SUPPORT;
@@ -1825,82 +1916,12 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
         }
         // (the barrier inside the first RHS orders the rows before the gathers)
         double yt_r[R], yt_i[R], yn_r[R], yn_i[R];
-        LB_FRHS(y_r, y_i, k_r[1], k_i[1], 1);
-        if constexpr (ST == 1) {
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            yt_r[r] = y_r[r] + 0.5 * h * k_r[1][r];
-            yt_i[r] = y_i[r] + 0.5 * h * k_i[1][r];
-          }
-          LB_FRHS(yt_r, yt_i, k_r[2], k_i[2], 2);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            yn_r[r] = y_r[r] + h * k_r[2][r];
-            yn_i[r] = y_i[r] + h * k_i[2][r];
-          }
-        } else if constexpr (ST == 2) {
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            yt_r[r] = y_r[r] + 0.5 * h * k_r[1][r];
-            yt_i[r] = y_i[r] + 0.5 * h * k_i[1][r];
-          }
-          LB_FRHS(yt_r, yt_i, k_r[2], k_i[2], 2);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            yt_r[r] = y_r[r] + 0.5 * h * k_r[2][r];
-            yt_i[r] = y_i[r] + 0.5 * h * k_i[2][r];
-          }
-          LB_FRHS(yt_r, yt_i, k_r[3], k_i[3], 3);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            yt_r[r] = y_r[r] + h * k_r[3][r];
-            yt_i[r] = y_i[r] + h * k_i[3][r];
-          }
-          LB_FRHS(yt_r, yt_i, k_r[4], k_i[4], 4);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            yn_r[r] = y_r[r] + h * (k_r[1][r] + 2.0 * k_r[2][r] + 2.0 * k_r[3][r] + k_r[4][r]) / 6.0;
-            yn_i[r] = y_i[r] + h * (k_i[1][r] + 2.0 * k_i[2][r] + 2.0 * k_i[3][r] + k_i[4][r]) / 6.0;
-          }
-        } else {
-#define LB_FSUM(expr_r, expr_i)            \
-  _Pragma("unroll") for (int r = 0; r < R; ++r) { \
-    yt_r[r] = y_r[r] + h * (expr_r);       \
-    yt_i[r] = y_i[r] + h * (expr_i);       \
-  }
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            yt_r[r] = y_r[r] + h * (1.0 / 5.0) * k_r[1][r];
-            yt_i[r] = y_i[r] + h * (1.0 / 5.0) * k_i[1][r];
-          }
-          LB_FRHS(yt_r, yt_i, k_r[2], k_i[2], 2);
-          LB_FSUM((3.0 / 40.0) * k_r[1][r] + (9.0 / 40.0) * k_r[2][r],
-                  (3.0 / 40.0) * k_i[1][r] + (9.0 / 40.0) * k_i[2][r])
-          LB_FRHS(yt_r, yt_i, k_r[3], k_i[3], 3);
-          LB_FSUM((44.0 / 45.0) * k_r[1][r] - (56.0 / 15.0) * k_r[2][r] + (32.0 / 9.0) * k_r[3][r],
-                  (44.0 / 45.0) * k_i[1][r] - (56.0 / 15.0) * k_i[2][r] + (32.0 / 9.0) * k_i[3][r])
-          LB_FRHS(yt_r, yt_i, k_r[4], k_i[4], 4);
-          LB_FSUM((19372.0 / 6561.0) * k_r[1][r] - (25360.0 / 2187.0) * k_r[2][r] + (64448.0 / 6561.0) * k_r[3][r] -
-                      (212.0 / 729.0) * k_r[4][r],
-                  (19372.0 / 6561.0) * k_i[1][r] - (25360.0 / 2187.0) * k_i[2][r] + (64448.0 / 6561.0) * k_i[3][r] -
-                      (212.0 / 729.0) * k_i[4][r])
-          LB_FRHS(yt_r, yt_i, k_r[5], k_i[5], 5);
-          LB_FSUM((9017.0 / 3168.0) * k_r[1][r] - (355.0 / 33.0) * k_r[2][r] + (46732.0 / 5247.0) * k_r[3][r] +
-                      (49.0 / 176.0) * k_r[4][r] - (5103.0 / 18656.0) * k_r[5][r],
-                  (9017.0 / 3168.0) * k_i[1][r] - (355.0 / 33.0) * k_i[2][r] + (46732.0 / 5247.0) * k_i[3][r] +
-                      (49.0 / 176.0) * k_i[4][r] - (5103.0 / 18656.0) * k_i[5][r])
-          LB_FRHS(yt_r, yt_i, k_r[6], k_i[6], 6);
-#undef LB_FSUM
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            yn_r[r] = y_r[r] + h * ((35.0 / 384.0) * k_r[1][r] + (500.0 / 1113.0) * k_r[3][r] +
-                                    (125.0 / 192.0) * k_r[4][r] - (2187.0 / 6784.0) * k_r[5][r] +
-                                    (11.0 / 84.0) * k_r[6][r]);
-            yn_i[r] = y_i[r] + h * ((35.0 / 384.0) * k_i[1][r] + (500.0 / 1113.0) * k_i[3][r] +
-                                    (125.0 / 192.0) * k_i[4][r] - (2187.0 / 6784.0) * k_i[5][r] +
-                                    (11.0 / 84.0) * k_i[6][r]);
-          }
-        }
+        fixed_step<ST, R>(h, y_r, y_i, k_r, k_i, yt_r, yt_i, yn_r, yn_i,
+                          [&](const double (&xr)[R], const double (&xi)[R], int s, double (&kr)[R], double (&ki)[R]) {
+                            rhs_eval<R>(P, L, S, xr, xi, kr, ki, L.pub + buf * 2 * P.n_pub, L.coef + s * KK, s - 1,
+                                        tid, W);
+                            buf ^= 1;
+                          });
         rhs_calls += NS;
         ++accepted;
         ++steps;
@@ -1951,7 +1972,6 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
         fail_x = (double)si;
       }
     }
-#undef LB_FRHS
     if (status == 0 && C.trace && n_pushed > C.capacity) status = LB_TRAJ_CAPACITY;
     if constexpr (EV) {
       if (C.out_event_t && tid == 0) C.out_event_t[traj] = ev_t;
@@ -1976,10 +1996,20 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
 // order their LDS traffic with wavefront-scope fences (no workgroup barrier
 // inside the divergent halves).
 //
-// Covered: persistent launches with pushes at every accepted step (final
-// outputs and the weighted integral), a given initial step dt, and the
-// adjoint's attempt tape; trace, save plans and replays take the other
-// kernels.
+// Covered: persistent launches with a given initial step dt: pushes at every
+// accepted step (final outputs and the weighted integral), the adjoint's
+// attempt tape, and in the forms compiled per plan (lb_rtc.cpp) save plans and
+// traces (LB_LANE_SAVE), stop events (LB_LANE_EVENT) and plans of 33..64
+// elements with one trajectory per wave (LPT = 64).  Replays and calls that
+// leave the initial step to the solver take the other kernels.
+//
+// Bound by the latency of one wave's step: the stage chain (publish, read,
+// couple) six times, the generated coefficient code, two half-wave sums and
+// the controller.  With the couplings, one log and one exp for the controller
+// and no expression machine, 64 x 64 grid 2.40 -> 1.61 ms; against the
+// precompiled kernels that ran these calls: rate trace at 201 points 5.56 ->
+// 2.15 ms, stop events 7.45 -> 1.53 ms, RK4 8.59 -> 2.39 ms, x/y scan (41
+// elements) 2.44 -> 0.95 ms, one solve 1.91 -> 1.07 ms.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -1992,7 +2022,9 @@ __device__ __forceinline__ void wave_sync() {
 // Sum over this lane's half-wave, rounded as wave_sum rounds a wave whose
 // other half holds zeros: the 16-lane rows by the same DPP tree, then
 // (row_a + row_b) + (0 + 0).
+template <int LPT>
 __device__ __forceinline__ double half_sum(double x, int lane) {
+  if constexpr (LPT == 64) return wave_sum(x);
   x += dpp_d<0xB1>(x);
   x += dpp_d<0x4E>(x);
   x += dpp_d<0x141>(x);
@@ -2003,7 +2035,10 @@ __device__ __forceinline__ double half_sum(double x, int lane) {
 
 // A block total of the single-wave form (one block): the stored sum is the
 // only non-zero lane of a second wave sum.
-__device__ __forceinline__ double half_total(double x, int lane) { return half_sum(x, lane) + 0.0; }
+template <int LPT>
+__device__ __forceinline__ double half_total(double x, int lane) {
+  return half_sum<LPT>(x, lane) + 0.0;
+}
 
 // The couplings of one lane, unpacked once per launch: byte offset of the
 // input in the half's publication buffer, byte offset and row stride of the
@@ -2048,29 +2083,33 @@ __device__ __forceinline__ void rhs_pair(const PairRows<G>& T, int rows, char* p
 }
 
 struct LdsPair {
-  dcpx* ent;      // 2 halves x (nv_stat + LB_ENT_ROWS x nv_dyn) entry values
-  dcpx* coef;     // 2 halves x 8 rows x (K + 1): [0] t0, [2..7] stage times
-  dcpx* slots;    // 2 halves x 8 x n_slots
-  dcpx* vm;       // 2 halves x 8 lanes x vm_depth
-  char* pub;      // 2 halves x 32 published stage inputs
-  double2* park;  // 2 x 64: y and k1 around the expression machine
-  double2* ef;    // factors, coefficient rows and extents of the time-dependent entries
+  dcpx* ent;      // per trajectory: nv_stat + LB_ENT_ROWS x nv_dyn entry values
+  dcpx* coef;     // 8 rows x (K + 1): [0] t0, [2..7] stage times
+  dcpx* slots;    // 8 x n_slots
+  dcpx* vm;       // 8 lanes x vm_depth
+  char* pub;      // published stage inputs
+  double* evv;    // n + 2: stop-event populations, [n] expression value, [n + 1] complex flag
+  double2* park;  // per lane: y and k1 around the expression machine
+  double2* ef;    // per wave: factors, coefficient rows and extents of the time-dependent entries
   uint32_t* ecoef;
   int* eptr;
   double* wts;    // n integral weights
   int* misc;      // [0..1] queue values, [2..3] support flags
 };
 
-__device__ __forceinline__ LdsPair carve_pair(const DevPlan& P) {
+// The wave's LDS, with the per-trajectory arrays of trajectory `half` of NH.
+template <int LPT>
+__device__ __forceinline__ LdsPair carve_pair(const DevPlan& P, int half) {
   extern __shared__ double smem[];
   char* const base = reinterpret_cast<char*>(smem);
-  const LbLdsPair l = lb_lds_pair(P);
+  const LbLdsPair l = lb_lds_pair(P, 64 / LPT);
   LdsPair L;
-  L.ent = reinterpret_cast<dcpx*>(base + l.ent);
-  L.coef = reinterpret_cast<dcpx*>(base + l.coef);
-  L.slots = reinterpret_cast<dcpx*>(base + l.slots);
-  L.vm = reinterpret_cast<dcpx*>(base + l.vm);
-  L.pub = base + l.pub;
+  L.ent = reinterpret_cast<dcpx*>(base + l.ent) + half * (P.nv_stat + LB_ENT_ROWS * P.nv_dyn);
+  L.coef = reinterpret_cast<dcpx*>(base + l.coef) + half * 8 * (P.K + 1);
+  L.slots = reinterpret_cast<dcpx*>(base + l.slots) + half * 8 * P.n_slots;
+  L.vm = reinterpret_cast<dcpx*>(base + l.vm) + half * 8 * P.vm_depth;
+  L.pub = base + l.pub + half * LPT * 16;
+  L.evv = reinterpret_cast<double*>(base + l.evv) + half * ((P.n + 3) & ~1);
   L.park = reinterpret_cast<double2*>(base + l.park);
   L.ef = reinterpret_cast<double2*>(base + l.ef);
   L.ecoef = reinterpret_cast<uint32_t*>(base + l.ecoef);
@@ -2078,6 +2117,223 @@ __device__ __forceinline__ LdsPair carve_pair(const DevPlan& P) {
   L.wts = reinterpret_cast<double*>(base + l.wts);
   L.misc = reinterpret_cast<int*>(base + l.misc);
   return L;
+}
+
+// Tables of one wave, filled once per launch: the coupling rows of slot `sl`,
+// the entry definitions and the integral weights.
+template <int LPT, int G>
+__device__ __forceinline__ void lane_tables(const DevPlan& P, const DevCall& C, const LdsPair& L, int crows, int lane,
+                                            int sl, PairRows<G>& rows) {
+#pragma unroll
+  for (int j = 0; j < G; ++j) {
+    const uint32_t w = j < crows ? P.c_word[j * 64 + sl] : 0u;
+    rows.x[j] = w >> 16;
+    rows.v[j] = w & 0xFFF0u;
+    rows.dv[j] = (w & 1u) * 16u * (uint32_t)P.nv_dyn;
+    rows.sign[j] = (w << 30) & 0x80000000u;
+  }
+  for (int i = lane; i < P.nv_terms; i += 64) {
+    L.ef[i] = reinterpret_cast<const double2*>(P.ent_f)[i];
+    L.ecoef[i] = P.ent_coef[i];
+  }
+  for (int i = lane; i <= P.nv_dyn; i += 64) L.eptr[i] = P.ent_ptr[i];
+  for (int i = lane; i < P.n; i += 64) {
+    double w = 0.0;
+    for (int q = 0; q < C.n_weights; ++q)
+      if (C.weight_index[q] == i) w += C.weight_value[q];
+    L.wts[i] = w;
+  }
+  wave_sync();
+}
+
+// The next trajectory of the queue for the `need`ing halves: true while it is
+// integrated by this half; `done` when the queue has run out.  Entries of a
+// queue order outside the batch are skipped.
+__device__ __forceinline__ bool lane_take(const DevCall& C, const LdsPair& L, int half, int sl, bool need, bool& done,
+                                          int64_t& traj) {
+  if (need && sl == 0) L.misc[half] = atomicAdd(C.queue, 1);
+  wave_sync();
+  if (!need) return false;
+  const int64_t local = L.misc[half];
+  if (local >= C.n_traj) {
+    done = true;
+    return false;
+  }
+  traj = C.queue_order ? (int64_t)C.queue_order[local + C.traj_offset] : local + C.traj_offset;
+  return traj >= 0 && traj < C.n_total;
+}
+
+// A trajectory's start: parameters and coefficients at t0, entries (the
+// time-dependent ones of t0 in entry row `row0`), the folded self coefficient
+// and the state of this lane's element.  Returns whether y0 leaves the support.
+template <int LPT>
+__device__ __forceinline__ bool lane_start(const DevPlan& P, const DevCall& C, const LdsPair& L, const Slots<1>& S,
+                                           int half, int sl, int64_t traj, int row0, double2& selfv,
+                                           double (&y_r)[1], double (&y_i)[1]) {
+  const int KK = P.K + 1;
+  for (int i = sl; i < P.n_slots; i += LPT)
+    L.slots[i] = i < P.n_base ? mk(P.base[2 * i], P.base[2 * i + 1]) : mk(0.0, 0.0);
+  wave_sync();
+  if (sl == 0) {
+    apply_overrides(C, traj, L.slots);
+    eval_coefficients(P, L.slots, L.coef, C.t0, false, L.vm);
+  }
+  wave_sync();
+  for (int i = sl; i < 7 * P.n_slots; i += LPT) L.slots[P.n_slots + i] = L.slots[i % P.n_slots];
+  for (int i = sl; i < 7 * KK; i += LPT) L.coef[KK + i] = L.coef[i % KK];
+  wave_sync();  // the stage rows are read by the expression-machine lanes
+  fill_static_entries(P, L.coef, L.ent, sl, LPT);
+  fill_entries<1>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef, KK, L.ent + P.nv_stat + row0 * P.nv_dyn, sl, LPT);
+  wave_sync();
+  {  // folded self coefficient of this element (fold_self arithmetic)
+    dcpx acc = mk(0.0, 0.0);
+    for (int j = 0; j < P.max_self; ++j) {
+      const size_t e = (size_t)sl * P.max_self + j;
+      const int id = P.self_coef[e];
+      if (id == -2) break;
+      const dcpx f = mk(P.self_f[2 * e], P.self_f[2 * e + 1]);
+      dcpx c = id < 0 ? mk(1.0, 0.0) : L.coef[id];
+      if (P.self_conj[e]) c.im = -c.im;
+      acc = cadd(acc, cmul(f, c));
+    }
+    selfv = double2{acc.re, acc.im};
+  }
+  const double* y0 = C.y0 + (C.y0_shared ? 0 : traj * (int64_t)P.dim);
+  y_r[0] = S.valid(0) ? y0[P.slot_re[sl]] : 0.0;
+  y_i[0] = (S.valid(0) && !S.diag(0)) ? y0[P.slot_im[sl]] : 0.0;
+  bool bad_support = false;
+  if (P.restricted) {
+    if (sl == 0) L.misc[2 + half] = 0;
+    wave_sync();
+    for (int k = sl; k < P.dim; k += LPT)
+      if (!P.upper_active[P.packed_upper[k]] && y0[k] != 0.0) L.misc[2 + half] = 1;
+    wave_sync();
+    bad_support = L.misc[2 + half] != 0;
+  }
+  return bad_support;
+}
+
+// Outputs of a finished trajectory (the multi-wave kernels').
+template <int LPT>
+__device__ __forceinline__ void lane_finish(const DevPlan& P, const DevCall& C, const Slots<1>& S, int sl, int64_t traj,
+                                            const double (&y_r)[1], const double (&y_i)[1], int status, double fail_x,
+                                            double integral, int64_t n_pushed, int64_t accepted, int64_t rejected,
+                                            int64_t rhs_calls) {
+  const bool ok = status == 0, diag = S.diag(0);
+  const double nanv = __builtin_nan("");
+  if (!C.trace) {  // trace rows were written as the points were pushed
+    if (P.restricted) {
+      if (C.output_kind == LB_OUT_POPULATIONS) {
+        for (int i = sl; i < P.n; i += LPT)
+          if (!P.upper_active[P.packed_upper[i]]) C.out_values[traj * P.n + i] = ok ? 0.0 : nanv;
+      } else if (C.output_kind == LB_OUT_FULL) {
+        for (int k = sl; k < P.dim; k += LPT)
+          if (!P.upper_active[P.packed_upper[k]]) C.out_values[traj * P.dim + k] = ok ? 0.0 : nanv;
+      } else if (C.output_kind == LB_OUT_SELECTED) {
+        for (int q = sl; q < C.n_selected; q += LPT)
+          if (!P.upper_active[C.sel_upper[q]]) {
+            C.out_values[2 * (traj * C.n_selected + q)] = ok ? 0.0 : nanv;
+            C.out_values[2 * (traj * C.n_selected + q) + 1] = ok ? 0.0 : nanv;
+          }
+      }
+    }
+    if (S.valid(0)) {
+      if (C.output_kind == LB_OUT_POPULATIONS) {
+        if (diag) C.out_values[traj * P.n + S.state(0)] = ok ? y_r[0] : nanv;
+      } else if (C.output_kind == LB_OUT_FULL) {
+        C.out_values[traj * P.dim + P.slot_re[sl]] = ok ? y_r[0] : nanv;
+        if (!diag) C.out_values[traj * P.dim + P.slot_im[sl]] = ok ? y_i[0] : nanv;
+      } else if (C.output_kind == LB_OUT_SELECTED) {
+        const int up = P.slot_up[sl];
+        for (int q = 0; q < C.n_selected; ++q) {
+          if (C.sel_upper[q] != up) continue;
+          const double im = (C.sel_flags[q] & 1) ? 0.0 : ((C.sel_flags[q] & 2) ? -y_i[0] : y_i[0]);
+          C.out_values[2 * (traj * C.n_selected + q)] = ok ? y_r[0] : nanv;
+          C.out_values[2 * (traj * C.n_selected + q) + 1] = ok ? im : nanv;
+        }
+      }
+    }
+  }
+  if (sl == 0) {
+    if (C.trace) C.out_counts[traj] = (int32_t)n_pushed;
+    else if (C.output_kind == LB_OUT_INTEGRAL) C.out_values[traj] = ok ? integral : nanv;
+    if (C.out_integral) C.out_integral[traj] = ok ? integral : nanv;
+    C.out_stats[4 * traj + 0] = accepted;
+    C.out_stats[4 * traj + 1] = rejected;
+    C.out_stats[4 * traj + 2] = rhs_calls;
+    C.out_stats[4 * traj + 3] = status;
+    C.out_fail_t[traj] = fail_x;
+  }
+}
+
+// The pushed points of one trajectory (rust/src/ode/output.rs): the weighted
+// trapezoid and the trace rows, as the multi-wave kernels push them.
+template <int LPT>
+struct LanePush {
+  double integral, last_t, last_v, last_pt;
+  int64_t n;
+  __device__ __forceinline__ void reset() {
+    integral = 0.0;
+    last_t = last_pt = __builtin_nan("");
+    last_v = 0.0;
+    n = 0;
+  }
+  // the trapezoid's next node, integrand v at tp
+  __device__ __forceinline__ void node(double tp, double v) {
+    if (isfinite(last_t)) integral += 0.5 * (last_v + v) * (tp - last_t);
+    last_t = tp;
+    last_v = v;
+  }
+  __device__ __forceinline__ void point(const DevPlan& P, const DevCall& C, const Slots<1>& S, int lane, int sl,
+                                        int64_t traj, double my_w, double tp, const double (&vr)[1],
+                                        const double (&vi)[1], bool reduce) {
+    const bool rate = C.output_kind == LB_OUT_RATE;
+    double v = last_v;
+    last_pt = tp;
+    if ((C.want_integral || rate) && reduce) {
+      v = half_total<LPT>(S.valid(0) && S.diag(0) ? my_w * vr[0] : 0.0, lane);
+      if (C.want_integral) node(tp, v);
+    }
+    if (C.trace) {
+      if (n < C.capacity) {
+        const int64_t row = traj * C.capacity + n;
+        if (C.output_kind == LB_OUT_INTEGRAL) {
+          if (sl == 0) C.out_values[row] = integral;
+        } else if (rate) {
+          if (sl == 0) C.out_values[row] = v;
+        } else {
+          write_row<1>(P, C, S, sl, 64, row, vr, vi);
+        }
+        if (sl == 0 && C.out_times) C.out_times[row] = tp;
+      }
+      ++n;
+    }
+  }
+};
+
+// g(t, y) of the stop event for one trajectory (event_value's arithmetic).
+__device__ __forceinline__ double lane_event(const DevPlan& P, const DevCall& C, const LdsPair& L, const Slots<1>& S,
+                                             int sl, double t, const dcpx* slots, double vr, bool& complex_) {
+  double g;
+  if (C.event_kind == LB_EVENT_POPULATION) {
+    if (S.valid(0) && S.diag(0)) L.evv[S.state(0)] = vr;
+    wave_sync();
+    double v = 0.0;
+    for (int k = 0; k < C.n_event; ++k) v += L.evv[cst(C.event_idx)[k]];
+    g = v - C.event_threshold;
+    complex_ = false;
+  } else {
+    if (sl == 0) {
+      const dcpx v = vm_eval(cst(C.event_ops), 0, C.n_event, slots, t, L.vm);
+      L.evv[P.n] = v.re;
+      L.evv[P.n + 1] = fabs(v.im) > 1e-12 ? 1.0 : 0.0;
+    }
+    wave_sync();
+    g = L.evv[P.n];
+    complex_ = L.evv[P.n + 1] != 0.0;
+  }
+  wave_sync();
+  return g;
 }
 
 }  // namespace
@@ -2091,51 +2347,33 @@ __device__ __forceinline__ LdsPair carve_pair(const DevPlan& P) {
 __device__ __forceinline__ void lb_gen_coef(dcpx* sl, dcpx* cf, double t);
 #endif
 
-template <int SOLVER, int G, int WAVES>
+template <int SOLVER, int G, int WAVES, int LPT = 32, int FL = 0>
 __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan P, const DevCall C) {
   using T = Tab<SOLVER>;
-  const int lane = threadIdx.x, half = lane >> 5, sl = lane & 31, base = lane & 32;
-  const LdsPair L = carve_pair(P);
+  constexpr bool SAVE = (FL & LB_LANE_SAVE) != 0, EV = (FL & LB_LANE_EVENT) != 0;
+  const int lane = threadIdx.x, half = LPT == 64 ? 0 : lane >> 5, sl = lane & (LPT - 1);
+  const LdsPair L = carve_pair<LPT>(P, half);
   const int KK = P.K + 1;
   const int crows = cst(P.c_rows)[0];
-  dcpx* const coef = L.coef + half * 8 * KK;
-  dcpx* const slots = L.slots + half * 8 * P.n_slots;
-  dcpx* const ent = L.ent + half * (P.nv_stat + LB_ENT_ROWS * P.nv_dyn);
-  char* const pub = L.pub + half * 32 * 16;
-  PairRows<G> rows;
-#pragma unroll
-  for (int j = 0; j < G; ++j) {
-    const uint32_t w = j < crows ? P.c_word[j * 64 + sl] : 0u;
-    rows.x[j] = w >> 16;
-    rows.v[j] = w & 0xFFF0u;
-    rows.dv[j] = (w & 1u) * 16u * (uint32_t)P.nv_dyn;
-    rows.sign[j] = (w << 30) & 0x80000000u;
-  }
+  const char* const ent = reinterpret_cast<const char*>(L.ent);
   Slots<1> S;
   load_slots<1>(P, S, sl, 64);
   const bool diag = S.diag(0);
-  for (int i = lane; i < P.nv_terms; i += 64) {
-    L.ef[i] = reinterpret_cast<const double2*>(P.ent_f)[i];
-    L.ecoef[i] = P.ent_coef[i];
-  }
-  for (int i = lane; i <= P.nv_dyn; i += 64) L.eptr[i] = P.ent_ptr[i];
-  for (int i = lane; i < P.n; i += 64) {
-    double w = 0.0;
-    for (int q = 0; q < C.n_weights; ++q)
-      if (C.weight_index[q] == i) w += C.weight_value[q];
-    L.wts[i] = w;
-  }
-  wave_sync();
+  PairRows<G> rows;
+  lane_tables<LPT, G>(P, C, L, crows, lane, sl, rows);
   const double my_w = (S.valid(0) && diag) ? L.wts[S.state(0)] : 0.0;
 
-  // per-half trajectory state
+  // per-trajectory state
   bool active = false, done = false;
   int64_t traj = 0;
-  double t1 = 0.0, x = 0.0, h = 0.0, hmax = 0.0, fac_old = 1.0e-4;
-  double integral = 0.0, last_t = 0.0, last_v = 0.0, fail_x = 0.0;
+  double t1 = 0.0, x = 0.0, h = 0.0, hmax = 0.0, fac_old = 1.0e-4, lfo = LB_LOG_FAC_MIN, fail_x = 0.0;
+  LanePush<LPT> pts;
+  pts.reset();
   int64_t accepted = 0, rejected = 0, rhs_calls = 0, ns = 0, nst = 0, ia = 0;
-  int status = 0;
-  bool reject = false, last = false;
+  int status = 0, si = 0;
+  bool reject = false, last = false, ev_fired = false;
+  double ev_old = 0.0, ev_t = __builtin_nan("");
+  const bool step_push = !SAVE || C.n_saveat == 0;
   double2 selfv = double2{0.0, 0.0};
   double y_r[1] = {0.0}, y_i[1] = {0.0};
   double k_r[8][1], k_i[8][1];
@@ -2144,79 +2382,38 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
     k_r[j][0] = 0.0;
     k_i[j][0] = 0.0;
   }
-  const double beta = 0.04, alpha = 0.2 - beta * 0.75, facc1 = 1.0 / 0.2, facc2 = 1.0 / 10.0;
-  const double safety = 0.9, nanv = __builtin_nan("");
+  const double inv_dim = 1.0 / (double)P.dim;
+#define LB_POINT(tp, vr, vi, reduce) pts.point(P, C, S, lane, sl, traj, my_w, tp, vr, vi, reduce)
 
   for (;;) {
     // ---- halves without a trajectory take the next one
     const bool need = !active && !done;
-    if (need && sl == 0) L.misc[half] = atomicAdd(C.queue, 1);
-    wave_sync();
-    if (need) {
-      const int64_t local = L.misc[half];
-      if (local >= C.n_traj) {
-        done = true;
-      } else {
-        traj = C.queue_order ? (int64_t)C.queue_order[local + C.traj_offset] : local + C.traj_offset;
-        active = traj >= 0 && traj < C.n_total;  // entries outside the batch are skipped
-      }
-    }
+    const bool starting = lane_take(C, L, half, sl, need, done, traj);
+    if (need) active = starting;
     if (__all(done)) break;
     // ---- initialise a new trajectory (rust/src/ode/dopri5.rs:160-220)
-    const bool starting = need && active;
     if (starting) {
       t1 = C.t1_per_traj ? C.t1_per_traj[traj] : C.t1;
-      for (int i = sl; i < P.n_slots; i += 32)
-        slots[i] = i < P.n_base ? mk(P.base[2 * i], P.base[2 * i + 1]) : mk(0.0, 0.0);
-      wave_sync();
-      if (sl == 0) {
-        apply_overrides(C, traj, slots);
-        eval_coefficients(P, slots, coef, C.t0, false, L.vm + half * 8 * P.vm_depth);
-      }
-      wave_sync();
-      for (int i = sl; i < 7 * P.n_slots; i += 32) slots[P.n_slots + i] = slots[i % P.n_slots];
-      for (int i = sl; i < 7 * KK; i += 32) coef[KK + i] = coef[i % KK];
-      wave_sync();  // the stage rows are read by the expression-machine lanes
-      fill_static_entries(P, coef, ent, sl, 32);
-      fill_entries<1>(P.nv_dyn, L.eptr, L.ecoef, L.ef, coef, KK, ent + P.nv_stat + 5 * P.nv_dyn, sl, 32);
-      wave_sync();
-      {  // folded self coefficient of this element (fold_self arithmetic)
-        dcpx acc = mk(0.0, 0.0);
-        for (int j = 0; j < P.max_self; ++j) {
-          const size_t e = (size_t)sl * P.max_self + j;
-          const int id = P.self_coef[e];
-          if (id == -2) break;
-          const dcpx f = mk(P.self_f[2 * e], P.self_f[2 * e + 1]);
-          dcpx c = id < 0 ? mk(1.0, 0.0) : coef[id];
-          if (P.self_conj[e]) c.im = -c.im;
-          acc = cadd(acc, cmul(f, c));
-        }
-        selfv = double2{acc.re, acc.im};
-      }
-      const double* y0 = C.y0 + (C.y0_shared ? 0 : traj * (int64_t)P.dim);
-      y_r[0] = S.valid(0) ? y0[P.slot_re[sl]] : 0.0;
-      y_i[0] = (S.valid(0) && !diag) ? y0[P.slot_im[sl]] : 0.0;
-      bool bad_support = false;
-      if (P.restricted) {
-        if (sl == 0) L.misc[2 + half] = 0;
-        wave_sync();
-        for (int k = sl; k < P.dim; k += 32)
-          if (!P.upper_active[P.packed_upper[k]] && y0[k] != 0.0) L.misc[2 + half] = 1;
-        wave_sync();
-        bad_support = L.misc[2 + half] != 0;
-      }
+      // entry row 5 holds t0 (the steps use rows 0..4)
+      const bool bad_support = lane_start<LPT>(P, C, L, S, half, sl, traj, 5, selfv, y_r, y_i);
       accepted = rejected = rhs_calls = 0;
       status = 0;
       fail_x = 0.0;
-      integral = 0.0;
-      last_t = __builtin_nan("");
-      last_v = 0.0;
+      pts.reset();
       x = C.t0;
       reject = false;
       last = false;
       fac_old = 1.0e-4;
+      lfo = LB_LOG_FAC_MIN;
       ns = nst = ia = 0;
       hmax = fabs(t1 - C.t0);
+      if constexpr (SAVE) si = 0;
+      if constexpr (EV) {
+        ev_fired = false;
+        ev_t = __builtin_nan("");
+        for (int i = sl; i < P.n; i += LPT) L.evv[i] = 0.0;
+        wave_sync();
+      }
       if (bad_support) {
         status = LB_TRAJ_BAD_SUPPORT;
         fail_x = C.t0;
@@ -2225,19 +2422,32 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
         status = LB_TRAJ_BAD_SPAN;
         fail_x = C.t0;
         last = true;
+      } else if (t1 == C.t0) {
+        if (C.save_start) LB_POINT(C.t0, y_r, y_i, true);
+        last = true;
       } else {
-        // pushed point t0 (save_start): the trapezoid's first node
-        if (C.save_start && C.want_integral) {
-          last_v = half_total(S.valid(0) && diag ? my_w * y_r[0] : 0.0, lane);
-          last_t = C.t0;
+        rhs_pair<G>(rows, crows, L.pub, ent, 5, sl, selfv, diag, y_r[0], y_i[0], k_r[1][0], k_i[1][0]);
+        h = fmin(C.dt, t1 - C.t0);
+        rhs_calls = 1;
+        if constexpr (EV) {
+          bool cpx = false;
+          ev_old = lane_event(P, C, L, S, sl, C.t0, L.slots, y_r[0], cpx);
+          if (cpx) {
+            status = LB_TRAJ_EVENT_COMPLEX;
+            fail_x = C.t0;
+            last = true;
+          }
         }
-        if (t1 == C.t0) {
-          last = true;
-        } else {
-          rhs_pair<G>(rows, crows, pub, reinterpret_cast<const char*>(ent), 5, sl, selfv, diag, y_r[0], y_i[0],
-                      k_r[1][0], k_i[1][0]);
-          h = fmin(C.dt, t1 - C.t0);
-          rhs_calls = 1;
+        // points at t0 (dopri5.rs:212-220)
+        if (!step_push) {
+          if constexpr (SAVE) {
+            while (si < C.n_saveat && fabs(C.saveat[si] - C.t0) <= time_tol(C.t0)) {
+              LB_POINT(C.saveat[si], y_r, y_i, true);
+              ++si;
+            }
+          }
+        } else if (C.save_start) {
+          LB_POINT(C.t0, y_r, y_i, true);
         }
       }
     }
@@ -2262,23 +2472,27 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
         finishing = true;
       }
       ++ns;
+#ifndef LB_GEN_COEF
+      // the expression machine needs registers of its own
       L.park[lane] = double2{y_r[0], y_i[0]};
       L.park[64 + lane] = double2{k_r[1][0], k_i[1][0]};
-      if (P.time_dependent && sl < 6) {
-        const int st = sl + 2;
-#ifdef LB_GEN_COEF
-        lb_gen_coef(slots + st * P.n_slots, coef + st * KK, x + h * T::c(st));
-#else
-        eval_coefficients(P, slots + st * P.n_slots, coef + st * KK, x + h * T::c(st), true,
-                          L.vm + (half * 8 + sl) * P.vm_depth);
 #endif
-      }
       if (P.time_dependent) {
+        if (sl < 6) {
+          const int st = sl + 2;
+#ifdef LB_GEN_COEF
+          lb_gen_coef(L.slots + st * P.n_slots, L.coef + st * KK, x + h * T::c(st));
+#else
+          eval_coefficients(P, L.slots + st * P.n_slots, L.coef + st * KK, x + h * T::c(st), true,
+                            L.vm + sl * P.vm_depth);
+#endif
+        }
         wave_sync();  // stage coefficients are read by every lane of the half
         // stages 2..6 take entry rows 0..4; stage 7 is at the same time as 6
-        fill_entries<5>(P.nv_dyn, L.eptr, L.ecoef, L.ef, coef + 2 * KK, KK, ent + P.nv_stat, sl, 32);
+        fill_entries<5>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + 2 * KK, KK, L.ent + P.nv_stat, sl, LPT);
+        wave_sync();
       }
-      wave_sync();
+#ifndef LB_GEN_COEF
       {
         const double2 py = L.park[lane], pk = L.park[64 + lane];
         y_r[0] = py.x;
@@ -2286,12 +2500,12 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
         k_r[1][0] = pk.x;
         k_i[1][0] = pk.y;
       }
+#endif
       const bool need_stiff = ((accepted + 1) % 1000 == 0) || ia > 0;
       double yt_r[1], yt_i[1], yn_r[1], yn_i[1];
 #define LB_PAIR_STAGE(st)                                                                            \
   stage_combo<1, SOLVER, st>(h, y_r, y_i, k_r, k_i, yt_r, yt_i);                                    \
-  rhs_pair<G>(rows, crows, pub, reinterpret_cast<const char*>(ent), (st) - 2, sl, selfv, diag, yt_r[0], yt_i[0], \
-              k_r[st][0], k_i[st][0]);
+  rhs_pair<G>(rows, crows, L.pub, ent, (st) - 2, sl, selfv, diag, yt_r[0], yt_i[0], k_r[st][0], k_i[st][0]);
       LB_PAIR_STAGE(2)
       LB_PAIR_STAGE(3)
       LB_PAIR_STAGE(4)
@@ -2304,10 +2518,9 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
         const double a0 = yn_r[0] - yt_r[0], a1 = yn_i[0] - yt_i[0];
         stiff_d = a0 * a0 + a1 * a1;
       }
-      rhs_pair<G>(rows, crows, pub, reinterpret_cast<const char*>(ent), 4, sl, selfv, diag, yn_r[0], yn_i[0],
-                  k_r[7][0], k_i[7][0]);
+      rhs_pair<G>(rows, crows, L.pub, ent, 4, sl, selfv, diag, yn_r[0], yn_i[0], k_r[7][0], k_i[7][0]);
       rhs_calls += 6;
-      // ---- error norm, integrand, stiffness (as the single-wave form)
+      // ---- error norm, integrand, stiffness (as the multi-wave form)
       double er = T::e(1) * k_r[1][0], ei = T::e(1) * k_i[1][0];
 #pragma unroll
       for (int j = 2; j <= 7; ++j) {
@@ -2319,67 +2532,58 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
       er *= h;
       ei *= h;
       const double sr = C.abstol + fmax(fabs(y_r[0]), fabs(yn_r[0])) * C.reltol;
-      const double si = C.abstol + fmax(fabs(y_i[0]), fabs(yn_i[0])) * C.reltol;
-      const double qr = er / sr, qi = ei / si;
-      const double e2 = half_total(S.valid(0) ? qr * qr + (diag ? 0.0 : qi * qi) : 0.0, lane);
-      const double err = sqrt(e2 / (double)P.dim);
-      // the controller's two powers at once: lanes 0-15 of the half take
-      // err^alpha, lanes 16-31 fac_old^-beta (the same pow on the same inputs)
-      const double pw = pow(sl < 16 ? err : fac_old, sl < 16 ? alpha : -beta);
-      const double fac11 = __shfl(pw, base, 64), fo = __shfl(pw, base + 16, 64);
-      double fac = fac11 * fo;
-      const double fac_s = fac / safety;
-      fac = fmax(facc2, fmin(facc1, fac_s));
-      double hn = h / fac;
+      const double si_ = C.abstol + fmax(fabs(y_i[0]), fabs(yn_i[0])) * C.reltol;
+      const double qr = er / sr, qi = ei / si_;
+      const double e2 = half_total<LPT>(S.valid(0) ? qr * qr + (diag ? 0.0 : qi * qi) : 0.0, lane);
+      // the candidate's integrand, summed beside the error norm
+      const double pv =
+          C.want_integral && step_push ? half_total<LPT>(S.valid(0) && diag ? my_w * yn_r[0] : 0.0, lane) : 0.0;
+      const StepControl ctl(e2 * inv_dim, lfo);
+      const double err = ctl.err;
+      double hn = h * ctl.factor();
       if (C.tape_h) {
-        // attempt tape, as the single-wave form records it: one record per
-        // attempt by lane 0 of the half, the state every ckpt_every-th attempt
-        const int64_t a = ns - 1;
-        if (a < C.tape_cap) {
+        // attempt tape, as the multi-wave form records it: one record per
+        // attempt by lane 0, the state every ckpt_every-th attempt
+        if (ns - 1 < C.tape_cap) {
+          const uint32_t a = (uint32_t)(ns - 1);
           if (sl == 0) {
             int fl = finishing ? LB_TAPE_CLIPPED : 0;
-            double h_next;
-            if (err <= 1.0) {
-              h_next = hn;
+            if (ctl.clamped()) fl |= LB_TAPE_CLAMPED;
+            if (ctl.accept) {
               fl |= LB_TAPE_ACCEPTED | (accepted == 0 ? LB_TAPE_FIRST : 0) | (err > 1.0e-4 ? LB_TAPE_ERRQ : 0);
-              if (!(fac_s > facc2 && fac_s < facc1)) fl |= LB_TAPE_CLAMPED;
               double hc = hn;
               if (fabs(hc) > hmax) {
                 hc = hmax;
                 fl |= LB_TAPE_HMAX;
               }
               if (reject && fabs(h) < fabs(hc)) fl |= LB_TAPE_MINRULE;
-            } else {
-              const double fr = fac11 / safety;
-              h_next = h / fmin(facc1, fr);
-              if (!(fr < facc1)) fl |= LB_TAPE_CLAMPED;
             }
             const int64_t o = traj * C.tape_cap + a;
             C.tape_t[o] = x;
             C.tape_h[o] = h;
             C.tape_c[3 * o] = err;
-            C.tape_c[3 * o + 1] = h_next;
+            C.tape_c[3 * o + 1] = hn;
             C.tape_c[3 * o + 2] = fac_old;
             C.tape_f[o] = fl;
           }
-          if (a % C.ckpt_every == 0 && sl < P.S) {
+          const uint32_t every = (uint32_t)C.ckpt_every, seg = a / every;
+          if (seg * every == a && sl < P.S) {
             const int64_t ncap = (C.tape_cap + C.ckpt_every - 1) / C.ckpt_every;
-            double* ck = C.tape_y + ((traj * ncap + a / C.ckpt_every) * P.S) * 2;
-            ck[2 * sl] = y_r[0];
-            ck[2 * sl + 1] = y_i[0];
+            reinterpret_cast<double2*>(C.tape_y)[(traj * ncap + seg) * P.S + sl] = double2{y_r[0], y_i[0]};
           }
         }
       }
-      if (err <= 1.0) {
+      if (ctl.accept) {
         fac_old = fmax(err, 1.0e-4);
+        lfo = fmax(ctl.lerr, LB_LOG_FAC_MIN);
         if (fabs(hn) > hmax) hn = hmax;
         if (reject) hn = fmin(fabs(hn), fabs(h));
         reject = false;
         ++accepted;
-        bool stiff = false;
-        if (accepted % 1000 == 0 || ia > 0) {
+        bool stop = false;
+        if (need_stiff) {
           double a0 = k_r[7][0] - k_r[6][0], a1 = k_i[7][0] - k_i[6][0];
-          const double n2 = half_total(a0 * a0 + a1 * a1, lane), dd2 = half_total(stiff_d, lane);
+          const double n2 = half_total<LPT>(a0 * a0 + a1 * a1, lane), dd2 = half_total<LPT>(stiff_d, lane);
           const double hl = dd2 > 0.0 ? h * sqrt(n2 / dd2) : 0.0;
           if (hl > 3.25) {
             ++ia;
@@ -2387,86 +2591,277 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
             if (ia == 15) {
               status = LB_TRAJ_STIFF;
               fail_x = x;
-              stiff = true;
+              stop = true;
             }
           } else {
             ++nst;
             if (nst == 6) ia = 0;
           }
         }
-        if (stiff) {
+        const double xo = x;
+        bool ev_hit = false;
+        double te = x + h;
+        if (!stop) x += h;
+        if constexpr (EV) {
+          // terminal stop event (dopri5.rs:280-317, tsit5.rs:274-309), as in
+          // lb_solve_kernel: the root's state is left in yt
+          if (!stop) {
+            bool cpx = false;
+            const double g1 = lane_event(P, C, L, S, sl, x, L.slots + 7 * P.n_slots, yn_r[0], cpx);
+            if (cpx) {
+              status = LB_TRAJ_EVENT_COMPLEX;
+              fail_x = x;
+              stop = true;
+            } else if (crossed_zero(ev_old, g1)) {
+              ev_hit = true;
+              if (ev_old == 0.0 || g1 == 0.0) {
+                te = ev_old == 0.0 ? xo : x;
+                yt_r[0] = ev_old == 0.0 ? y_r[0] : yn_r[0];
+                yt_i[0] = ev_old == 0.0 ? y_i[0] : yn_i[0];
+              } else {
+                double lo = 0.0, hi = 1.0, glo = ev_old;
+                for (int it = 0; it < 60; ++it) {
+                  const double mid = 0.5 * (lo + hi);
+                  dense_point<1, SOLVER>(mid, h, y_r, y_i, yn_r, yn_i, k_r, k_i, yt_r, yt_i);
+                  // slot copy 0 is free after the trajectory's start
+                  if (C.event_kind == LB_EVENT_EXPRESSION && sl == 0)
+                    eval_compounds(P, L.slots, xo + mid * h, L.vm);
+                  const double gm = lane_event(P, C, L, S, sl, xo + mid * h, L.slots, yt_r[0], cpx);
+                  if (cpx) {
+                    fail_x = xo + mid * h;
+                    break;
+                  }
+                  if (gm == 0.0) {
+                    lo = mid;
+                    hi = mid;
+                    break;
+                  }
+                  if ((glo < 0.0 && gm > 0.0) || (glo > 0.0 && gm < 0.0)) {
+                    hi = mid;
+                  } else {
+                    lo = mid;
+                    glo = gm;
+                  }
+                }
+                if (cpx) {
+                  status = LB_TRAJ_EVENT_COMPLEX;
+                  stop = true;
+                } else {
+                  const double th = 0.5 * (lo + hi);
+                  dense_point<1, SOLVER>(th, h, y_r, y_i, yn_r, yn_i, k_r, k_i, yt_r, yt_i);
+                  te = xo + th * h;
+                }
+              }
+            }
+            ev_old = g1;
+          }
+        }
+        if (stop) {
           last = true;
         } else {
-          x += h;
-          if (C.want_integral) {
-            const double v = half_total(S.valid(0) && diag ? my_w * yn_r[0] : 0.0, lane);
-            if (isfinite(last_t)) integral += 0.5 * (last_v + v) * (x - last_t);
-            last_t = x;
-            last_v = v;
+          if (step_push) {
+            if (!ev_hit) {
+              if (C.want_integral) pts.node(x, pv);
+              pts.last_pt = x;
+              if constexpr (SAVE) {
+                if (C.trace) LB_POINT(x, yn_r, yn_i, C.output_kind == LB_OUT_RATE);
+              }
+            }
+          } else if constexpr (SAVE) {
+            // save plan points inside (xo, x], or up to the root (dopri5.rs:318-344)
+            const double tb = ev_hit ? te : x;
+            while (si < C.n_saveat && C.saveat[si] <= tb + time_tol(tb)) {
+              const double ts = C.saveat[si];
+              if (ts >= xo - time_tol(xo)) {
+                if (fabs(ts - xo) <= time_tol(xo)) {
+                  LB_POINT(ts, y_r, y_i, true);
+                } else if (fabs(ts - x) <= time_tol(x)) {
+                  LB_POINT(ts, yn_r, yn_i, true);
+                } else {
+                  double ds_r[1], ds_i[1];
+                  dense_point<1, SOLVER>((ts - xo) / h, h, y_r, y_i, yn_r, yn_i, k_r, k_i, ds_r, ds_i);
+                  LB_POINT(ts, ds_r, ds_i, true);
+                }
+              }
+              ++si;
+            }
           }
-          y_r[0] = yn_r[0];
-          y_i[0] = yn_i[0];
-          k_r[1][0] = k_r[7][0];
-          k_i[1][0] = k_i[7][0];
-          if (finishing) last = true;
-          h = hn;
+          if (EV && ev_hit) {
+            if (!(isfinite(pts.last_pt) && fabs(pts.last_pt - te) <= time_tol(te))) LB_POINT(te, yt_r, yt_i, true);
+            // a final state output whose time t1 lies within time_tol of the
+            // root holds the state at t1 (dopri5.rs:318-352)
+            if (!C.trace && C.output_kind != LB_OUT_INTEGRAL && step_push && t1 <= te + time_tol(te)) {
+              if (fabs(t1 - xo) <= time_tol(xo)) {
+                yt_r[0] = y_r[0];
+                yt_i[0] = y_i[0];
+              } else if (fabs(t1 - x) <= time_tol(x)) {
+                yt_r[0] = yn_r[0];
+                yt_i[0] = yn_i[0];
+              } else {
+                dense_point<1, SOLVER>((t1 - xo) / h, h, y_r, y_i, yn_r, yn_i, k_r, k_i, yt_r, yt_i);
+              }
+            }
+            y_r[0] = yt_r[0];
+            y_i[0] = yt_i[0];
+            ev_fired = true;
+            ev_t = te;
+            last = true;
+          } else {
+            y_r[0] = yn_r[0];
+            y_i[0] = yn_i[0];
+            k_r[1][0] = k_r[7][0];
+            k_i[1][0] = k_i[7][0];
+            if (finishing) last = true;
+            h = hn;
+          }
         }
       } else {
-        hn = h / fmin(facc1, fac11 / safety);
         reject = true;
         if (accepted >= 1) ++rejected;
         h = hn;
       }
     }
-    // ---- a finished trajectory writes its outputs (the single-wave form's)
+    // ---- a finished trajectory writes its outputs
     if (active && last) {
+      if constexpr (EV) {
+        if (C.out_event_t && sl == 0) C.out_event_t[traj] = ev_t;
+      }
+      if constexpr (SAVE) {
+        if (status == 0 && !step_push && si != C.n_saveat && !ev_fired) {
+          status = LB_TRAJ_SAVEAT;
+          fail_x = (double)si;  // plan points reached
+        }
+        if (status == 0 && C.trace && pts.n > C.capacity) status = LB_TRAJ_CAPACITY;
+      }
       if (status == 0 && C.tape_h && ns > C.tape_cap) status = LB_TRAJ_CAPACITY;
-      const bool ok = status == 0;
-      if (P.restricted) {
-        if (C.output_kind == LB_OUT_POPULATIONS) {
-          for (int i = sl; i < P.n; i += 32)
-            if (!P.upper_active[P.packed_upper[i]]) C.out_values[traj * P.n + i] = ok ? 0.0 : nanv;
-        } else if (C.output_kind == LB_OUT_FULL) {
-          for (int k = sl; k < P.dim; k += 32)
-            if (!P.upper_active[P.packed_upper[k]]) C.out_values[traj * P.dim + k] = ok ? 0.0 : nanv;
-        } else if (C.output_kind == LB_OUT_SELECTED) {
-          for (int q = sl; q < C.n_selected; q += 32)
-            if (!P.upper_active[C.sel_upper[q]]) {
-              C.out_values[2 * (traj * C.n_selected + q)] = ok ? 0.0 : nanv;
-              C.out_values[2 * (traj * C.n_selected + q) + 1] = ok ? 0.0 : nanv;
-            }
-        }
-      }
-      if (S.valid(0)) {
-        if (C.output_kind == LB_OUT_POPULATIONS) {
-          if (diag) C.out_values[traj * P.n + S.state(0)] = ok ? y_r[0] : nanv;
-        } else if (C.output_kind == LB_OUT_FULL) {
-          C.out_values[traj * P.dim + P.slot_re[sl]] = ok ? y_r[0] : nanv;
-          if (!diag) C.out_values[traj * P.dim + P.slot_im[sl]] = ok ? y_i[0] : nanv;
-        } else if (C.output_kind == LB_OUT_SELECTED) {
-          const int up = P.slot_up[sl];
-          for (int q = 0; q < C.n_selected; ++q) {
-            if (C.sel_upper[q] != up) continue;
-            const double im = (C.sel_flags[q] & 1) ? 0.0 : ((C.sel_flags[q] & 2) ? -y_i[0] : y_i[0]);
-            C.out_values[2 * (traj * C.n_selected + q)] = ok ? y_r[0] : nanv;
-            C.out_values[2 * (traj * C.n_selected + q) + 1] = ok ? im : nanv;
-          }
-        }
-      }
-      if (sl == 0) {
-        if (C.tape_n) C.tape_n[traj] = (int32_t)ns;
-        if (C.output_kind == LB_OUT_INTEGRAL) C.out_values[traj] = ok ? integral : nanv;
-        if (C.out_integral) C.out_integral[traj] = ok ? integral : nanv;
-        C.out_stats[4 * traj + 0] = accepted;
-        C.out_stats[4 * traj + 1] = rejected;
-        C.out_stats[4 * traj + 2] = rhs_calls;
-        C.out_stats[4 * traj + 3] = status;
-        C.out_fail_t[traj] = fail_x;
-      }
+      if (C.tape_n && sl == 0) C.tape_n[traj] = (int32_t)ns;
+      lane_finish<LPT>(P, C, S, sl, traj, y_r, y_i, status, fail_x, pts.integral, pts.n, accepted, rejected,
+                       rhs_calls);
       active = false;
     }
   }
+#undef LB_POINT
 }
+
+#ifdef LB_GEN_COEF
+// Fixed-step integrators for plans of one block, one or two trajectories per
+// wave (lb_fixed_kernel's steps and pushes; no stop events).  Compiled per
+// plan only.
+template <int ST, int G, int WAVES, int LPT>
+__global__ __launch_bounds__(64, WAVES) void lb_fixed_pair_kernel(const DevPlan P, const DevCall C) {
+  using F = FixedStep<ST>;
+  constexpr int NS = F::NS;
+  const int lane = threadIdx.x, half = LPT == 64 ? 0 : lane >> 5, sl = lane & (LPT - 1);
+  const LdsPair L = carve_pair<LPT>(P, half);
+  const int KK = P.K + 1;
+  const int crows = cst(P.c_rows)[0];
+  const char* const ent = reinterpret_cast<const char*>(L.ent);
+  Slots<1> S;
+  load_slots<1>(P, S, sl, 64);
+  const bool diag = S.diag(0);
+  PairRows<G> rows;
+  lane_tables<LPT, G>(P, C, L, crows, lane, sl, rows);
+  const double my_w = (S.valid(0) && diag) ? L.wts[S.state(0)] : 0.0;
+  bool active = false, done = false, last = false;
+  int64_t traj = 0;
+  double t1 = 0.0, x = 0.0, fail_x = 0.0;
+  LanePush<LPT> pts;
+  pts.reset();
+  int64_t steps = 0;
+  int status = 0, si = 0;
+  const bool step_push = C.n_saveat == 0;
+  double2 selfv = double2{0.0, 0.0};
+  double y_r[1] = {0.0}, y_i[1] = {0.0};
+#define LB_POINT(tp, vr, vi) pts.point(P, C, S, lane, sl, traj, my_w, tp, vr, vi, true)
+  for (;;) {
+    const bool need = !active && !done;
+    const bool starting = lane_take(C, L, half, sl, need, done, traj);
+    if (need) active = starting;
+    if (__all(done)) break;
+    if (starting) {
+      t1 = C.t1_per_traj ? C.t1_per_traj[traj] : C.t1;
+      const bool bad_support = lane_start<LPT>(P, C, L, S, half, sl, traj, 0, selfv, y_r, y_i);
+      steps = 0;
+      status = 0;
+      fail_x = 0.0;
+      pts.reset();
+      x = C.t0;
+      si = 0;
+      last = false;
+      if (bad_support || t1 < C.t0 || !(isfinite(C.dt) && C.dt > 0.0)) {
+        status = bad_support ? LB_TRAJ_BAD_SUPPORT : t1 < C.t0 ? LB_TRAJ_BAD_SPAN : LB_TRAJ_BAD_DT;
+        fail_x = C.t0;
+        last = true;
+      } else if (t1 == C.t0) {
+        if (C.save_start) LB_POINT(C.t0, y_r, y_i);
+        last = true;
+      } else if (!step_push) {
+        while (si < C.n_saveat && fabs(C.saveat[si] - C.t0) <= time_tol(C.t0)) {
+          LB_POINT(C.saveat[si], y_r, y_i);
+          ++si;
+        }
+      } else if (C.save_start) {
+        LB_POINT(C.t0, y_r, y_i);
+      }
+    }
+    double h = 0.0;
+    if (active && !last) {
+      if (!(x < t1 - time_tol(t1))) {
+        last = true;
+        if (!step_push && si != C.n_saveat) {
+          status = LB_TRAJ_SAVEAT;
+          fail_x = (double)si;
+        }
+      } else if (steps >= C.maxiters) {
+        status = LB_TRAJ_MAXITERS;
+        fail_x = x;
+        last = true;
+      } else {
+        double target = fmin(x + C.dt, t1);
+        if (!step_push && si < C.n_saveat && C.saveat[si] > x + time_tol(x)) target = fmin(target, C.saveat[si]);
+        h = target - x;
+        if (h <= 0.0 || 0.1 * h <= DBL_EPSILON * fmax(fabs(x), 1.0)) {
+          status = LB_TRAJ_UNDERFLOW;
+          fail_x = x;
+          last = true;
+        }
+      }
+    }
+    if (active && !last) {
+      if (P.time_dependent) {
+        if (sl < NS)
+          lb_gen_coef(L.slots + (sl + 1) * P.n_slots, L.coef + (sl + 1) * KK, F::time(x, h, sl + 1));
+        wave_sync();
+        fill_entries<NS>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + KK, KK, L.ent + P.nv_stat, sl, LPT);
+        wave_sync();
+      }
+      double k_r[7][1], k_i[7][1], yt_r[1], yt_i[1], yn_r[1], yn_i[1];
+      fixed_step<ST, 1>(h, y_r, y_i, k_r, k_i, yt_r, yt_i, yn_r, yn_i,
+                        [&](const double (&xr)[1], const double (&xi)[1], int s, double (&kr)[1], double (&ki)[1]) {
+                          rhs_pair<G>(rows, crows, L.pub, ent, s - 1, sl, selfv, diag, xr[0], xi[0], kr[0], ki[0]);
+                        });
+      ++steps;
+      x += h;
+      if (step_push) {
+        LB_POINT(x, yn_r, yn_i);
+      } else {
+        while (si < C.n_saveat && C.saveat[si] <= x + time_tol(x)) {
+          LB_POINT(C.saveat[si], yn_r, yn_i);
+          ++si;
+        }
+      }
+      y_r[0] = yn_r[0];
+      y_i[0] = yn_i[0];
+    }
+    if (active && last) {
+      if (status == 0 && C.trace && pts.n > C.capacity) status = LB_TRAJ_CAPACITY;
+      lane_finish<LPT>(P, C, S, sl, traj, y_r, y_i, status, fail_x, pts.integral, pts.n, steps, 0, steps * NS);
+      active = false;
+    }
+  }
+#undef LB_POINT
+}
+#endif
 
 // ---------------------------------------------------------------------------
 // Discrete adjoint of the adaptive Dopri5/Tsit5 solve.
@@ -3713,7 +4108,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_rhs_kernel(const DevPlan P, co
 // integrator is the expanded-sparse one: Dopri5 / Tsit5 tableaus,
 // controller, stiffness test, save plan and dense output.
 // ---------------------------------------------------------------------------
-#if LB_PART == 1
+#if LB_PART == 7
 namespace {
 
 struct LdsEff {
@@ -4064,9 +4459,8 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_eff_kernel(const DevEffPlan P,
           push(t0, y);
         }
       }
-      const double beta = 0.04, alpha = 0.2 - beta * 0.75, facc1 = 1.0 / 0.2, facc2 = 1.0 / 10.0;
-      const double safety = 0.9, hmax = fabs(t1 - t0);
-      double fac_old = 1.0e-4;
+      const double hmax = fabs(t1 - t0), inv_dim = 1.0 / (double)P.D;
+      double lfo = LB_LOG_FAC_MIN;
       bool reject = false, last = false;
       int64_t ns = 0, nst = 0, ia = 0;
       while (!last && status == 0) {
@@ -4145,15 +4539,10 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_eff_kernel(const DevEffPlan P,
           }
         }
         __syncthreads();
-        const double err = sqrt(eff_block_total(P, L.red, 0) / (double)P.D);
-        const int wl = tid & 63;
-        const double pw = pow(wl < 32 ? err : fac_old, wl < 32 ? alpha : -beta);
-        const double fac11 = __shfl(pw, 0, 64), fo = __shfl(pw, 32, 64);
-        double fac = fac11 * fo;
-        fac = fmax(facc2, fmin(facc1, fac / safety));
-        double hn = h / fac;
-        if (err <= 1.0) {
-          fac_old = fmax(err, 1.0e-4);
+        const StepControl ctl(eff_block_total(P, L.red, 0) * inv_dim, lfo);
+        double hn = h * ctl.factor();
+        if (ctl.accept) {
+          lfo = fmax(ctl.lerr, LB_LOG_FAC_MIN);
           if (fabs(hn) > hmax) hn = hmax;
           if (reject) hn = fmin(fabs(hn), fabs(h));
           reject = false;
@@ -4198,7 +4587,6 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_eff_kernel(const DevEffPlan P,
           }
           if (last) break;
         } else {
-          hn = h / fmin(facc1, fac11 / safety);
           reject = true;
           last = false;
           if (accepted >= 1) ++rejected;
@@ -4276,7 +4664,7 @@ extern "C" void* lb_dev_eff_rhs_kernel(int id) {
 #undef E
   return nullptr;
 }
-#endif  // LB_PART == 1
+#endif  // LB_PART == 7
 
 #if LB_PART == 0
 __global__ void lb_queue_reset_kernel(int32_t* q) { *q = 0; }

@@ -16,6 +16,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <list>
 #include <map>
 #include <mutex>
 #include <sstream>
@@ -156,6 +157,12 @@ struct CodeObject {
 };
 std::mutex g_code_mu;
 std::map<std::string, CodeObject> g_code;
+// Loaded modules by device and code key; the most recently used ones are held
+// (a plan made again for the same system then loads nothing).  Not destroyed
+// at process exit, when the runtime may be gone.
+constexpr size_t kHeldModules = 16;
+std::map<std::string, std::weak_ptr<LbModule>>& g_modules = *new std::map<std::string, std::weak_ptr<LbModule>>();
+std::list<std::shared_ptr<LbModule>>& g_held = *new std::list<std::shared_ptr<LbModule>>();
 
 int compile_code(const std::string& coef_source, const std::string& name_expr, CodeObject* out,
                  std::string& why) {
@@ -205,13 +212,30 @@ int compile_code(const std::string& coef_source, const std::string& name_expr, C
 
 }  // namespace
 
-int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr, hipModule_t* module,
-                   hipFunction_t* function, std::string& why) {
+int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr, std::shared_ptr<LbModule>* out,
+                   std::string& why) {
   const char* extra = std::getenv("CENTREX_LB_RTC_OPTIONS");
   const std::string key = std::string(extra ? extra : "") + "\n" + name_expr + "\n" + coef_source;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) {
+    why = "no current device";
+    return -1;
+  }
+  const std::string at = std::to_string(device) + "\n" + key;
   CodeObject obj;
+  std::shared_ptr<LbModule> dropped;  // unloaded after the lock is released
   {
     std::lock_guard<std::mutex> lock(g_code_mu);
+    auto loaded = g_modules.find(at);
+    if (loaded != g_modules.end() && (*out = loaded->second.lock())) {
+      g_held.remove(*out);
+      g_held.push_front(*out);
+      if (g_held.size() > kHeldModules) {
+        dropped = g_held.back();
+        g_held.pop_back();
+      }
+      return 0;
+    }
     auto it = g_code.find(key);
     if (it != g_code.end()) obj = it->second;
   }
@@ -221,17 +245,27 @@ int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr,
     g_code.emplace(key, obj);
   }
   const std::string& name = obj.lowered;
-  hipError_t e = hipModuleLoadData(module, obj.code.data());
+  auto m = std::make_shared<LbModule>();
+  hipError_t e = hipModuleLoadData(&m->module, obj.code.data());
   if (e != hipSuccess) {
+    m->module = nullptr;
     why = std::string("hipModuleLoadData: ") + hipGetErrorString(e);
     return -1;
   }
-  e = hipModuleGetFunction(function, *module, name.c_str());
+  e = hipModuleGetFunction(&m->function, m->module, name.c_str());
   if (e != hipSuccess) {
     why = std::string("hipModuleGetFunction: ") + hipGetErrorString(e);
-    (void)hipModuleUnload(*module);
-    *module = nullptr;
     return -1;
   }
+  std::lock_guard<std::mutex> lock(g_code_mu);
+  for (auto it = g_modules.begin(); it != g_modules.end();)
+    it = it->second.expired() ? g_modules.erase(it) : std::next(it);
+  g_modules[at] = m;
+  g_held.push_front(m);
+  if (g_held.size() > kHeldModules) {
+    dropped = g_held.back();
+    g_held.pop_back();
+  }
+  *out = m;
   return 0;
 }

@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -21,6 +22,15 @@ std::string lb_rtc_coef_source(const LbProgram& prog, const std::vector<int32_t>
 // Compiles the kernel sources with `coef_source` for gfx950 and loads the
 // kernel named by `name_expr` (a template-id such as
 // "lb_solve_pair_kernel<0, 8, 2>") from the resulting code object.
-// Returns 0, or -1 with `why` holding the compiler log or the runtime error.
-int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr, hipModule_t* module,
-                   hipFunction_t* function, std::string& why);
+// Plans of one program on one device share the loaded module; the plans that
+// use it hold it, and the last few stay loaded for the next plan.  Returns 0,
+// or -1 with `why` holding the compiler log or the runtime error.
+struct LbModule {
+  hipModule_t module = nullptr;
+  hipFunction_t function = nullptr;
+  ~LbModule() {
+    if (module) (void)hipModuleUnload(module);
+  }
+};
+int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr, std::shared_ptr<LbModule>* out,
+                   std::string& why);

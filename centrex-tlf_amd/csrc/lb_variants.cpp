@@ -6,24 +6,44 @@ extern "C" void* lb_dev_solve_kernel_p0(int, int);
 extern "C" void* lb_dev_solve_kernel_p1(int, int);
 extern "C" void* lb_dev_solve_kernel_p2(int, int);
 extern "C" void* lb_dev_solve_kernel_p3(int, int);
+extern "C" void* lb_dev_solve_kernel_p4(int, int);
+extern "C" void* lb_dev_solve_kernel_p5(int, int);
+extern "C" void* lb_dev_solve_kernel_p6(int, int);
+extern "C" void* lb_dev_solve_kernel_p7(int, int);
 extern "C" void* lb_dev_fixed_kernel_p0(int, int);
 extern "C" void* lb_dev_fixed_kernel_p1(int, int);
 extern "C" void* lb_dev_fixed_kernel_p2(int, int);
 extern "C" void* lb_dev_fixed_kernel_p3(int, int);
+extern "C" void* lb_dev_fixed_kernel_p4(int, int);
+extern "C" void* lb_dev_fixed_kernel_p5(int, int);
+extern "C" void* lb_dev_fixed_kernel_p6(int, int);
+extern "C" void* lb_dev_fixed_kernel_p7(int, int);
 extern "C" void* lb_dev_event_kernel_p0(int, int);
 extern "C" void* lb_dev_event_kernel_p1(int, int);
 extern "C" void* lb_dev_event_kernel_p2(int, int);
 extern "C" void* lb_dev_event_kernel_p3(int, int);
+extern "C" void* lb_dev_event_kernel_p4(int, int);
+extern "C" void* lb_dev_event_kernel_p5(int, int);
+extern "C" void* lb_dev_event_kernel_p6(int, int);
+extern "C" void* lb_dev_event_kernel_p7(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p0(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p1(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p2(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p3(int, int);
+extern "C" void* lb_dev_adjoint_kernel_p4(int, int);
+extern "C" void* lb_dev_adjoint_kernel_p5(int, int);
+extern "C" void* lb_dev_adjoint_kernel_p6(int, int);
+extern "C" void* lb_dev_adjoint_kernel_p7(int, int);
 extern "C" void* lb_dev_rhs_kernel_p0(int);
 extern "C" void* lb_dev_rhs_kernel_p1(int);
 extern "C" void* lb_dev_rhs_kernel_p2(int);
 extern "C" void* lb_dev_rhs_kernel_p3(int);
+extern "C" void* lb_dev_rhs_kernel_p4(int);
+extern "C" void* lb_dev_rhs_kernel_p5(int);
+extern "C" void* lb_dev_rhs_kernel_p6(int);
+extern "C" void* lb_dev_rhs_kernel_p7(int);
 
-static_assert(LB_NPARTS_BUILT == 4, "lb_variants.cpp lists four kernel parts");
+static_assert(LB_NPARTS_BUILT == 8, "lb_variants.cpp lists eight kernel parts");
 
 extern "C" int lb_dev_variant_count(void) {
   int n = 0;
@@ -78,14 +98,12 @@ extern "C" int lb_dev_variant_rows(int id) {
 }
 
 extern "C" void* lb_dev_solve_kernel(int id, int solver) {
-  void* (*parts[])(int, int) = {lb_dev_solve_kernel_p0, lb_dev_solve_kernel_p1, lb_dev_solve_kernel_p2,
-                                lb_dev_solve_kernel_p3};
+  void* (*parts[])(int, int) = {lb_dev_solve_kernel_p0, lb_dev_solve_kernel_p1, lb_dev_solve_kernel_p2, lb_dev_solve_kernel_p3, lb_dev_solve_kernel_p4, lb_dev_solve_kernel_p5, lb_dev_solve_kernel_p6, lb_dev_solve_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);
 }
 
 extern "C" void* lb_dev_rhs_kernel(int id) {
-  void* (*parts[])(int) = {lb_dev_rhs_kernel_p0, lb_dev_rhs_kernel_p1, lb_dev_rhs_kernel_p2,
-                           lb_dev_rhs_kernel_p3};
+  void* (*parts[])(int) = {lb_dev_rhs_kernel_p0, lb_dev_rhs_kernel_p1, lb_dev_rhs_kernel_p2, lb_dev_rhs_kernel_p3, lb_dev_rhs_kernel_p4, lb_dev_rhs_kernel_p5, lb_dev_rhs_kernel_p6, lb_dev_rhs_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id);
 }
 
@@ -105,8 +123,7 @@ extern "C" int lb_dev_adjoint_variant(int id, int* R, int* maxw, int* rows) {
 }
 
 extern "C" void* lb_dev_adjoint_kernel(int id, int solver) {
-  void* (*parts[])(int, int) = {lb_dev_adjoint_kernel_p0, lb_dev_adjoint_kernel_p1, lb_dev_adjoint_kernel_p2,
-                                lb_dev_adjoint_kernel_p3};
+  void* (*parts[])(int, int) = {lb_dev_adjoint_kernel_p0, lb_dev_adjoint_kernel_p1, lb_dev_adjoint_kernel_p2, lb_dev_adjoint_kernel_p3, lb_dev_adjoint_kernel_p4, lb_dev_adjoint_kernel_p5, lb_dev_adjoint_kernel_p6, lb_dev_adjoint_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);
 }
 
@@ -136,13 +153,11 @@ extern "C" int lb_dev_event_variant(int id, int* R, int* maxw) {
 }
 
 extern "C" void* lb_dev_event_kernel(int id, int solver) {
-  void* (*parts[])(int, int) = {lb_dev_event_kernel_p0, lb_dev_event_kernel_p1, lb_dev_event_kernel_p2,
-                                lb_dev_event_kernel_p3};
+  void* (*parts[])(int, int) = {lb_dev_event_kernel_p0, lb_dev_event_kernel_p1, lb_dev_event_kernel_p2, lb_dev_event_kernel_p3, lb_dev_event_kernel_p4, lb_dev_event_kernel_p5, lb_dev_event_kernel_p6, lb_dev_event_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);
 }
 
 extern "C" void* lb_dev_fixed_kernel(int id, int solver) {
-  void* (*parts[])(int, int) = {lb_dev_fixed_kernel_p0, lb_dev_fixed_kernel_p1, lb_dev_fixed_kernel_p2,
-                                lb_dev_fixed_kernel_p3};
+  void* (*parts[])(int, int) = {lb_dev_fixed_kernel_p0, lb_dev_fixed_kernel_p1, lb_dev_fixed_kernel_p2, lb_dev_fixed_kernel_p3, lb_dev_fixed_kernel_p4, lb_dev_fixed_kernel_p5, lb_dev_fixed_kernel_p6, lb_dev_fixed_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);
 }

@@ -43,4 +43,4 @@
 // the first that covers the plan).
 #define LB_ADJ_WAVE_CONFIGS(V) V(4, 12, 2) V(5, 16, 2)
 
-#define LB_NPARTS_BUILT 4
+#define LB_NPARTS_BUILT 8

@@ -93,6 +93,20 @@ struct alignas(16) DevExpr {
   int32_t start, end, dst, pad;
 };
 
+// One operation of the time-dependent programs in three-address form: the
+// multi-wave kernels evaluate them this way, the single expressions of the
+// list above only at t0 and for stop events.  Operands and results are slots
+// of a stage's copy (parameters, then constants, time and temporaries), a
+// result dst < 0 is coefficient row entry -dst-1.  `code` is op | argc << 8 |
+// function << 16 with the bytecode's opcodes; LB_VOP_COPY copies slot a, and
+// op 0 is an idle entry.  A helper's arguments are argc slots from a; POWC's
+// constants are slots b (c, cos c pi) and b + 1 (sin c pi, 0).
+#define LB_VOP_COPY 2
+#define LB_VOP_LANES 8  // operations of one step: the same opcode, no dependence between them
+struct alignas(16) DevVOp {
+  int32_t code, dst, a, b;
+};
+
 struct DevPlan {
   int32_t n, dim, upper_len;
   int32_t S;        // padded slot count (multiple of 64)
@@ -158,12 +172,21 @@ struct DevPlan {
   int32_t n_all_fwd, n_all, n_dyn_fwd, n_dyn;
   int32_t vm_depth;             // deepest expression stack
   const double* base;           // n_base*2
+  // three-address form: slots of a stage's copy (n_slots of the parameter
+  // graph first; 0 steps: the expressions are interpreted one by one), the
+  // time slot, the constants, and the steps of the solve and of the solve and
+  // its derivative programs, LB_VOP_LANES operations each
+  int32_t v_slots, v_time, v_n_const, v_steps, v_steps_all;
+  const int32_t* v_const_slot;
+  const double* v_const;        // v_n_const*2
+  const DevVOp* v_ops;          // v_steps * LB_VOP_LANES
+  const DevVOp* v_ops_all;      // v_steps_all * LB_VOP_LANES
 };
 
 // LDS of the multi-wave kernels, in bytes from the start: one layout for the
 // host, which sizes the launch, and the device.
 struct LbLds {
-  uint32_t pub, ent, selfc, wts, coef, slots, red, vm, park, ef, ecoef, eptr, gf, word, misc, evv, total;
+  uint32_t pub, ent, selfc, wts, coef, slots, red, vm, vops, park, ef, ecoef, eptr, gf, word, misc, evv, total;
 };
 __host__ __device__ inline LbLds lb_lds_layout(const DevPlan& P) {
   LbLds l;
@@ -174,8 +197,9 @@ __host__ __device__ inline LbLds lb_lds_layout(const DevPlan& P) {
   l.ent = q; q += P.couplings ? 16u * (uint32_t)(P.nv_stat + LB_ENT_ROWS * P.nv_dyn) : 0u;
   l.selfc = q; q += 16u * (uint32_t)P.S;
   l.coef = q; q += 8u * 16u * (uint32_t)(P.K + 1);
-  l.slots = q; q += 8u * 16u * (uint32_t)P.n_slots;
+  l.slots = q; q += 8u * 16u * (uint32_t)P.v_slots;
   l.vm = q; q += 8u * 16u * (uint32_t)P.vm_depth;
+  l.vops = q; q += 16u * LB_VOP_LANES * (uint32_t)P.v_steps;
   l.park = q; q += 16u * 128u;
   l.ef = q; q += 16u * nt;
   l.gf = q; q += P.couplings ? 0u : 16u * cells;

@@ -149,6 +149,7 @@ struct DevImage {
   void* ws_c = nullptr;
   size_t ws_y_len = 0, ws_c_len = 0;
   hipEvent_t ws_done = nullptr;  // end of the last adjoint that used the workspace
+  LbVector vec, vec_all;  // three-address form of the solve's programs, and with the derivative ones
   std::vector<int32_t> g_rows_host;  // gather rows per block
   int t_rows_host = 0;               // transposed rows of block 0 (one-block plans)
 };
@@ -295,6 +296,8 @@ void pick_config(int S, int rows, int* id_out, int* W_out) {
 constexpr int64_t kLdsTableBytes = 32 * 1024;
 // Coupling rows a plan-specialised paired kernel holds in registers (4 each).
 constexpr int kMaxLaneRows = 16;
+// The three-address form of the programs is used up to this size (slot copies and table).
+constexpr int64_t kMaxVectorBytes = 24 * 1024;
 // LDS of one workgroup on gfx950.
 constexpr int64_t kMaxLdsBytes = 160 * 1024;
 
@@ -464,6 +467,58 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   P.KD = src.K * (1 + src.n_diff);
   P.n_slots = src.prog.n_slots;
   P.vm_depth = std::max(src.prog.max_depth, 1);
+  // Evaluation order: the compounds the solve needs, the K coefficients,
+  // then the compounds only the derivative programs read and the
+  // derivative programs.  Each part keeps the program's order, so every
+  // expression follows the compounds it reads; a solve evaluates the first
+  // two parts only.
+  std::vector<DevExpr> ex_all, ex_dyn;
+  {
+    const int nc = src.prog.n_compounds, K = src.K, KD = src.K * (1 + src.n_diff);
+    std::vector<int> order;
+    for (int e = 0; e < nc; ++e)
+      if (src.fwd_compound[e]) order.push_back(e);
+    for (int e = nc; e < nc + K; ++e) order.push_back(e);
+    const int n_fwd = (int)order.size();
+    for (int e = 0; e < nc; ++e)
+      if (!src.fwd_compound[e]) order.push_back(e);
+    for (int e = nc + K; e < nc + KD; ++e) order.push_back(e);
+    std::vector<int32_t> list, dst;
+    int n_dyn_fwd = 0;
+    for (int i = 0; i < (int)order.size(); ++i) {
+      const int e = order[i];
+      DevExpr r{};
+      r.start = src.prog.expr_start[e];
+      r.end = src.prog.expr_start[e + 1];
+      if (e < nc) {
+        r.dst = src.prog.compound_slot[e];
+      } else {
+        const int j = e - nc;
+        r.dst = -((j < K ? j : j + 1) + 1);
+      }
+      ex_all.push_back(r);
+      if (src.expr_dyn[e]) {
+        ex_dyn.push_back(r);
+        list.push_back(e);
+        dst.push_back(r.dst);
+        if (i < n_fwd) ++n_dyn_fwd;
+      }
+    }
+    P.n_all_fwd = n_fwd;
+    P.n_all = nc + KD;
+    P.n_dyn_fwd = n_dyn_fwd;
+    P.n_dyn = (int32_t)ex_dyn.size();
+    if (ex_all.empty()) ex_all.push_back(DevExpr{});
+    if (ex_dyn.empty()) ex_dyn.push_back(DevExpr{});
+    // the same time-dependent programs in three-address form
+    const std::vector<int32_t> fwd(list.begin(), list.begin() + n_dyn_fwd), fdst(dst.begin(), dst.begin() + n_dyn_fwd);
+    im->vec = lb_vector_program(src.prog, fwd, fdst, src.prog.n_slots);
+    im->vec_all = src.n_diff > 0 ? lb_vector_program(src.prog, list, dst, src.prog.n_slots) : LbVector{};
+  }
+  P.v_steps = im->vec.steps;
+  P.v_steps_all = im->vec_all.steps;
+  P.v_slots = P.v_steps > 0 ? im->vec.n_slots : P.n_slots;
+  P.v_time = im->vec.time_slot;
   P.n_pub = one_block ? n_act : (int)std::count(published.begin(), published.end(), (uint8_t)1);
   // Couplings, when their entries (and the rest of a workgroup's LDS) fit;
   // the gather tables otherwise.
@@ -475,6 +530,10 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   P.nv_terms = (int32_t)std::min<int64_t>(cpl.dyn_terms, 1 << 20);
   P.lds_tables = 0;
   P.c_rows_total = P.g_rows = 0;
+  if (P.v_steps > 0 && 16 * 8 * (int64_t)(P.v_slots + P.v_steps) > kMaxVectorBytes) {
+    P.v_steps = 0;  // a long program stays interpreted
+    P.v_slots = P.n_slots;
+  }
   if (P.nv_dyn + P.nv_stat > LB_MAX_ENTRIES || P.n_pub > LB_MAX_COUPLED ||
       16 * (int64_t)(P.nv_stat + LB_ENT_ROWS * P.nv_dyn) + 20 * (int64_t)P.nv_terms > kMaxLdsBytes ||
       lds_bytes_for(P) > kMaxLdsBytes) {
@@ -731,49 +790,13 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   up(src.prog.expr_start, &P.expr_start);
   up(src.compound_slot, &P.compound_slot);
   up(src.expr_dyn, &P.expr_dyn);
-  {
-    // Evaluation order: the compounds the solve needs, the K coefficients,
-    // then the compounds only the derivative programs read and the
-    // derivative programs.  Each part keeps the program's order, so every
-    // expression follows the compounds it reads; a solve evaluates the first
-    // two parts only.
-    const int nc = src.prog.n_compounds, K = src.K, KD = src.K * (1 + src.n_diff);
-    std::vector<int> order;
-    for (int e = 0; e < nc; ++e)
-      if (src.fwd_compound[e]) order.push_back(e);
-    for (int e = nc; e < nc + K; ++e) order.push_back(e);
-    const int n_fwd = (int)order.size();
-    for (int e = 0; e < nc; ++e)
-      if (!src.fwd_compound[e]) order.push_back(e);
-    for (int e = nc + K; e < nc + KD; ++e) order.push_back(e);
-    std::vector<DevExpr> all, dyn;
-    int n_dyn_fwd = 0;
-    for (int i = 0; i < (int)order.size(); ++i) {
-      const int e = order[i];
-      DevExpr r{};
-      r.start = src.prog.expr_start[e];
-      r.end = src.prog.expr_start[e + 1];
-      if (e < nc) {
-        r.dst = src.prog.compound_slot[e];
-      } else {
-        const int j = e - nc;
-        r.dst = -((j < K ? j : j + 1) + 1);
-      }
-      all.push_back(r);
-      if (src.expr_dyn[e]) {
-        dyn.push_back(r);
-        if (i < n_fwd) ++n_dyn_fwd;
-      }
-    }
-    P.n_all_fwd = n_fwd;
-    P.n_all = nc + KD;
-    P.n_dyn_fwd = n_dyn_fwd;
-    P.n_dyn = (int32_t)dyn.size();
-    if (all.empty()) all.push_back(DevExpr{});
-    if (dyn.empty()) dyn.push_back(DevExpr{});
-    up(all, &P.ex_all);
-    up(dyn, &P.ex_dyn);
-  }
+  up(ex_all, &P.ex_all);
+  up(ex_dyn, &P.ex_dyn);
+  P.v_n_const = P.v_steps > 0 ? (int32_t)im->vec.const_slot.size() : 0;
+  up(im->vec.const_slot, &P.v_const_slot);
+  up(im->vec.const_value, &P.v_const);
+  up(im->vec.ops, &P.v_ops);
+  up(im->vec_all.ops, &P.v_ops_all);
   up(src.base, &P.base);
   up(act, &P.upper_active);
   up(packed_upper, &P.packed_upper);

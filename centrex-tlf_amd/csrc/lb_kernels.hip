@@ -478,9 +478,10 @@ struct Lds {
   double* selfc;  // 2*S folded self coefficients
   double* wts;    // n integral weights per state
   dcpx* coef;     // 8 x (K+1): [0] t0 and hinit, [1] hinit second point, [2..7] stages
-  dcpx* slots;    // 8 x n_slots
+  dcpx* slots;    // 8 x v_slots
   double* red;    // 4 x nblk block sums
   dcpx* vm;       // 8 lanes x vm_depth expression stacks
+  DevVOp* vops;   // v_steps x LB_VOP_LANES operations
   double2* park;  // 128 entries: single-wave state parked around the expression machine
   dcpx* ent;      // entry values: nv_stat time-independent, then LB_ENT_ROWS x nv_dyn
   double2* ef;    // factors, coefficient rows and extents of the time-dependent entries
@@ -505,6 +506,7 @@ __device__ __forceinline__ Lds carve(const DevPlan& P) {
   L.slots = reinterpret_cast<dcpx*>(base + l.slots);
   L.red = reinterpret_cast<double*>(base + l.red);
   L.vm = reinterpret_cast<dcpx*>(base + l.vm);
+  L.vops = reinterpret_cast<DevVOp*>(base + l.vops);
   L.park = reinterpret_cast<double2*>(base + l.park);
   L.ef = reinterpret_cast<double2*>(base + l.ef);
   L.ecoef = reinterpret_cast<uint32_t*>(base + l.ecoef);
@@ -750,6 +752,7 @@ __device__ __forceinline__ void rhs_eval(const DevPlan& P, const Lds& L, const S
 // Copy the coupling (or gather) tables into LDS once per workgroup (plans
 // whose tables fit), and the definitions of the time-dependent entries.
 __device__ __forceinline__ void stage_tables(const DevPlan& P, const Lds& L, int tid, int W) {
+  for (int i = tid; i < P.v_steps * LB_VOP_LANES; i += W) L.vops[i] = P.v_ops[i];
   if (P.couplings) {
     for (int i = tid; i < P.nv_terms; i += W) {
       L.ef[i] = reinterpret_cast<const double2*>(P.ent_f)[i];
@@ -847,6 +850,70 @@ __device__ __forceinline__ void eval_coefficients(const DevPlan& P, dcpx* sl, dc
   cf[P.K] = mk(1.0, 0.0);
 }
 
+// Lanes of one wave order their LDS traffic with wavefront-scope fences.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The time-dependent programs at up to 8 times by one wave: lane l evaluates
+// operation l >> 3 of every step for time row l & 7 (`row` < 8, `on`: the row
+// is wanted), slots in `sl`, coefficients in `cf`.  The operations of a step
+// are independent and of one opcode, so a step costs one dispatch and one LDS
+// round trip; results are bitwise those of vm_eval, whose operations these
+// are.  On the 72-level plan 25 operations are 12 steps, against 43
+// interpreted instructions of about 600 cycles each.
+__device__ __forceinline__ void vector_eval(const DevVOp* ops, int steps, dcpx* sl, dcpx* cf, int time_slot, double t,
+                                            int lane, bool on) {
+  const int e = lane >> 3;
+  if (on && e == 0) sl[time_slot] = mk(t, 0.0);
+  wave_sync();
+  DevVOp next = ops[e];
+  for (int s = 0; s < steps; ++s) {
+    const DevVOp q = next;
+    if (s + 1 < steps) next = ops[(s + 1) * LB_VOP_LANES + e];
+    const int code = __builtin_amdgcn_readfirstlane(q.code);  // operation 0 of a step is never idle
+    const int op = code & 0xFF;
+    if (on && q.code != 0) {
+      const dcpx a = sl[q.a], b = sl[q.b];
+      dcpx v;
+      switch (op) {
+        case LB_VOP_COPY: v = a; break;
+        case 5: v = cadd(a, b); break;
+        case 6: v = csub(a, b); break;
+        case 7: v = cmul(a, b); break;
+        case 8: v = cdiv(a, b); break;
+        case 9: v = dev_cpow(a, b); break;
+        case 10: v = mk(-a.re, -a.im); break;
+        case 11: v = mk(a.re, -a.im); break;
+        case 12: {
+          const int f = code >> 16;
+          if (f == 4 && a.im == 0.0) v = mk(exp(a.re), 0.0);
+          else v = dev_builtin(f, a);
+          break;
+        }
+        case 13: v = dev_helper(code >> 16, sl + q.a, (code >> 8) & 0xFF); break;
+        case LB_OP_POWC: v = dev_powc(a, b.re, b.im, sl[q.b + 1].re); break;
+        default: {
+          const bool res = op == 14 ? a.re > b.re : op == 15 ? a.re >= b.re : op == 16 ? a.re < b.re
+                         : op == 17 ? a.re <= b.re : op == 18 ? a.re == b.re : a.re != b.re;
+          v = mk(res ? 1.0 : 0.0, 0.0);
+          break;
+        }
+      }
+      if (q.dst >= 0) sl[q.dst] = v;
+      else cf[-q.dst - 1] = v;
+    }
+    wave_sync();
+  }
+}
+
+// The constants of the three-address form into one slot copy.
+__device__ __forceinline__ void fill_constants(const DevPlan& P, dcpx* sl, int tid, int W) {
+  for (int i = tid; i < P.v_n_const; i += W) sl[P.v_const_slot[i]] = mk(P.v_const[2 * i], P.v_const[2 * i + 1]);
+}
+
 template <int R>
 __device__ __forceinline__ void load_slots(const DevPlan& P, Slots<R>& S, int tid, int W) {
 #pragma unroll
@@ -866,6 +933,7 @@ __device__ __forceinline__ void load_slots(const DevPlan& P, Slots<R>& S, int ti
 __device__ __forceinline__ void init_slots(const DevPlan& P, dcpx* sl, int tid, int W) {
   for (int i = tid; i < P.n_slots; i += W)
     sl[i] = i < P.n_base ? mk(P.base[2 * i], P.base[2 * i + 1]) : mk(0.0, 0.0);
+  fill_constants(P, sl, tid, W);
   __syncthreads();
 }
 
@@ -1072,7 +1140,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
       if constexpr (EV) L.evv[i] = 0.0;  // stop-event populations outside a restricted plan stay zero
     }
     __syncthreads();
-    for (int i = tid; i < 7 * P.n_slots; i += W) L.slots[P.n_slots + i] = L.slots[i % P.n_slots];
+    for (int i = tid; i < 7 * P.v_slots; i += W) L.slots[P.v_slots + i] = L.slots[i % P.v_slots];
     for (int i = tid; i < 7 * KK; i += W) L.coef[KK + i] = L.coef[i % KK];
     fold_self(P, tid, W, L.coef, L.selfc);
     if (P.couplings) {  // entry row 5 holds t0 until the last stage needs it
@@ -1182,7 +1250,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         const double d0 = block_total(P, L.red, 0), d1 = block_total(P, L.red, 1), hmax = fabs(t1 - x);
         double h0 = (d0 < 1.0e-10 || d1 < 1.0e-10) ? 1.0e-6 : 0.01 * sqrt(d0 / d1);
         h0 = fmin(h0, hmax);
-        if (tid == 0) eval_coefficients(P, L.slots + P.n_slots, L.coef + KK, x + h0, true, L.vm);
+        if (tid == 0) eval_coefficients(P, L.slots + P.v_slots, L.coef + KK, x + h0, true, L.vm);
         __syncthreads();
         if (P.couplings)
           fill_entries<1>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + KK, KK, L.ent + P.nv_stat, tid, W);
@@ -1250,10 +1318,18 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           L.park[64 + tid] = double2{k_r[1][0], k_i[1][0]};
         }
         // time-dependent coefficients at the six stage times, one lane per stage
-        if (P.time_dependent && tid < 6) {
-          const int s = tid + 2;
-          eval_coefficients(P, L.slots + s * P.n_slots, L.coef + s * KK, x + h * T::c(s), true,
-                            L.vm + tid * P.vm_depth);
+        if (P.time_dependent) {
+          if (P.v_steps > 0) {
+            if (tid < 64) {
+              const int s = min((tid & 7) + 2, 7);
+              vector_eval(L.vops, P.v_steps, L.slots + s * P.v_slots, L.coef + s * KK, P.v_time, x + h * T::c(s), tid,
+                          (tid & 7) < 6);
+            }
+          } else if (tid < 6) {
+            const int s = tid + 2;
+            eval_coefficients(P, L.slots + s * P.v_slots, L.coef + s * KK, x + h * T::c(s), true,
+                              L.vm + tid * P.vm_depth);
+          }
         }
         if (P.time_dependent) {
           __syncthreads();  // stage coefficients are read by every lane
@@ -1414,7 +1490,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           if constexpr (EV) {
             if (C.event_kind) {
               bool cpx = false;
-              const double g1 = event_value<R>(P, C, L, S, tid, W, x, L.slots + 7 * P.n_slots, yn_r, cpx);
+              const double g1 = event_value<R>(P, C, L, S, tid, W, x, L.slots + 7 * P.v_slots, yn_r, cpx);
               if (cpx) { status = LB_TRAJ_EVENT_COMPLEX; fail_x = x; break; }
               if (crossed_zero(ev_old, g1)) {
                 ev_hit = true;
@@ -1810,7 +1886,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
       if constexpr (EV) L.evv[i] = 0.0;
     }
     __syncthreads();
-    for (int i = tid; i < 7 * P.n_slots; i += W) L.slots[P.n_slots + i] = L.slots[i % P.n_slots];
+    for (int i = tid; i < 7 * P.v_slots; i += W) L.slots[P.v_slots + i] = L.slots[i % P.v_slots];
     for (int i = tid; i < 7 * KK; i += W) L.coef[KK + i] = L.coef[i % KK];
     fold_self(P, tid, W, L.coef, L.selfc);
     if (P.couplings) fill_static_entries(P, L.coef, L.ent, tid, W);
@@ -1907,9 +1983,18 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
         const double h = target - x;
         if (h <= 0.0 || 0.1 * h <= DBL_EPSILON * fmax(fabs(x), 1.0)) { status = LB_TRAJ_UNDERFLOW; fail_x = x; break; }
         __syncthreads();  // the previous step's RHS have read their coefficient rows
-        if (P.time_dependent && tid < NS)
-          eval_coefficients(P, L.slots + (tid + 1) * P.n_slots, L.coef + (tid + 1) * KK, F::time(x, h, tid + 1),
-                            true, L.vm + tid * P.vm_depth);
+        if (P.time_dependent) {
+          if (P.v_steps > 0) {
+            if (tid < 64) {
+              const int s = min((tid & 7) + 1, NS);
+              vector_eval(L.vops, P.v_steps, L.slots + s * P.v_slots, L.coef + s * KK, P.v_time, F::time(x, h, s), tid,
+                          (tid & 7) < NS);
+            }
+          } else if (tid < NS) {
+            eval_coefficients(P, L.slots + (tid + 1) * P.v_slots, L.coef + (tid + 1) * KK, F::time(x, h, tid + 1),
+                              true, L.vm + tid * P.vm_depth);
+          }
+        }
         if (P.time_dependent && P.couplings) {
           __syncthreads();
           fill_entries<NS>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + KK, KK, L.ent + P.nv_stat, tid, W);
@@ -2012,12 +2097,6 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
 // elements) 2.44 -> 0.95 ms, one solve 1.91 -> 1.07 ms.
 // ---------------------------------------------------------------------------
 namespace {
-
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Sum over this lane's half-wave, rounded as wave_sum rounds a wave whose
 // other half holds zeros: the 16-lane rows by the same DPP tree, then

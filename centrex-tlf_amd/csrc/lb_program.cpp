@@ -292,3 +292,151 @@ int lb_build_program(const lb_plan_desc* d, const std::vector<uint8_t>& dyn_slot
   if (prog.empty()) prog.push_back(DevInstr{1, 0, 0, 0, 0.0, 0.0, 0.0});
   return 0;
 }
+
+namespace {
+
+struct VNode {
+  DevVOp op;
+  int weight;
+  std::vector<int> after;  // operations whose results this one reads
+  int path = 0;            // weight of the longest chain that starts here
+};
+
+}  // namespace
+
+LbVector lb_vector_program(const LbProgram& prog, const std::vector<int32_t>& list, const std::vector<int32_t>& dst,
+                           int first_slot) {
+  LbVector out;
+  int next = first_slot;
+  out.time_slot = next++;
+  auto constant_at = [&](int slot, double re, double im) {
+    out.const_slot.push_back(slot);
+    out.const_value.push_back(re);
+    out.const_value.push_back(im);
+  };
+  std::map<std::string, int> const_of;
+  auto constant = [&](double re, double im) {
+    std::string key(reinterpret_cast<const char*>(&re), sizeof re);
+    key.append(reinterpret_cast<const char*>(&im), sizeof im);
+    auto it = const_of.find(key);
+    if (it != const_of.end()) return it->second;
+    const int slot = next++;
+    constant_at(slot, re, im);
+    const_of[key] = slot;
+    return slot;
+  };
+  std::vector<VNode> nodes;
+  std::map<int, int> writer;  // slot -> operation that writes it
+  auto emit_op = [&](int code, int d, int a, int b, int weight, const std::vector<int>& reads) {
+    VNode n;
+    n.op = DevVOp{code, d, a, b};
+    n.weight = weight;
+    for (int r : reads) {
+      auto it = writer.find(r);
+      if (it != writer.end()) n.after.push_back(it->second);
+    }
+    nodes.push_back(n);
+    if (d >= 0) writer[d] = (int)nodes.size() - 1;
+  };
+  for (size_t i = 0; i < list.size(); ++i) {
+    const int e = list[i];
+    struct Val {
+      int slot;
+      bool is_const;
+      double re, im;
+    };
+    std::vector<Val> st;
+    auto pop = [&]() {
+      const Val v = st.back();
+      st.pop_back();
+      return v;
+    };
+    const int p1 = prog.expr_start[e + 1];
+    for (int p = prog.expr_start[e]; p < p1; ++p) {
+      const DevInstr& q = prog.instr[p];
+      if (q.op == 1) { st.push_back(Val{-1, true, q.re, q.im}); continue; }
+      if (q.op == 2) { st.push_back(Val{q.index, false, 0, 0}); continue; }
+      if (q.op == 4) { st.push_back(Val{out.time_slot, false, 0, 0}); continue; }
+      auto at = [&](const Val& v) { return v.is_const ? constant(v.re, v.im) : v.slot; };
+      const bool root = p + 1 == p1;
+      int a = 0, b = 0, weight = 1, code = q.op;
+      std::vector<int> reads;
+      if (q.op == 12 || q.op == 13) {
+        const size_t argc = (size_t)std::max(q.argc, 1);
+        std::vector<Val> args(st.end() - argc, st.end());
+        st.resize(st.size() - argc);
+        code |= (q.argc << 8) | (q.function << 16);
+        weight = 5;
+        if (q.op == 12) {
+          a = b = at(args[0]);
+          reads.push_back(a);
+        } else {  // the helper reads its arguments from consecutive slots
+          a = b = next;
+          next += (int)argc;
+          for (size_t k = 0; k < argc; ++k) {
+            if (args[k].is_const) {
+              constant_at(a + (int)k, args[k].re, args[k].im);
+            } else {
+              emit_op(LB_VOP_COPY, a + (int)k, args[k].slot, args[k].slot, 1, {args[k].slot});
+              reads.push_back(a + (int)k);
+            }
+          }
+        }
+      } else if (q.op == 10 || q.op == 11) {
+        a = b = at(pop());
+        reads.push_back(a);
+      } else if (q.op == LB_OP_POWC) {
+        a = at(pop());
+        reads.push_back(a);
+        b = next;
+        next += 2;
+        constant_at(b, q.re, q.im);
+        constant_at(b + 1, q.aux, 0.0);
+        weight = q.re == 2.0 ? 2 : 5;
+      } else {
+        const Val vb = pop(), va = pop();
+        a = at(va);
+        b = at(vb);
+        reads.push_back(a);
+        reads.push_back(b);
+        weight = q.op == 8 ? 2 : q.op == 9 ? 6 : 1;
+      }
+      const int d = root ? dst[i] : next++;
+      emit_op(code, d, a, b, weight, reads);
+      st.push_back(Val{d, false, 0, 0});
+    }
+    if (p1 - prog.expr_start[e] == 1) {  // a single operand: copied
+      const Val v = st.back();
+      const int a = v.is_const ? constant(v.re, v.im) : v.slot;
+      emit_op(LB_VOP_COPY, dst[i], a, a, 1, {a});
+    }
+  }
+  out.n_slots = next;
+  // ---- steps: of the ready operations, the opcode of the one on the longest chain
+  const int n = (int)nodes.size();
+  for (int k = n - 1; k >= 0; --k) {
+    nodes[k].path += nodes[k].weight;
+    for (int p : nodes[k].after) nodes[p].path = std::max(nodes[p].path, nodes[k].path);
+  }
+  std::vector<int> step_of(n, -1);
+  for (int left = n; left > 0; ++out.steps) {
+    std::vector<int> ready;
+    for (int k = 0; k < n; ++k) {
+      bool ok = step_of[k] < 0;
+      for (int p : nodes[k].after) ok = ok && step_of[p] >= 0 && step_of[p] < out.steps;
+      if (ok) ready.push_back(k);
+    }
+    std::stable_sort(ready.begin(), ready.end(), [&](int a, int b) { return nodes[a].path > nodes[b].path; });
+    const int code = nodes[ready[0]].op.code;
+    int used = 0;
+    for (int k : ready) {
+      if (nodes[k].op.code != code || used == LB_VOP_LANES) continue;
+      step_of[k] = out.steps;
+      out.ops.push_back(nodes[k].op);
+      ++used;
+      --left;
+    }
+    for (; used < LB_VOP_LANES; ++used) out.ops.push_back(DevVOp{0, 0, 0, 0});
+  }
+  return out;
+}

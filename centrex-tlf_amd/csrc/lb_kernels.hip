@@ -39,6 +39,22 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T* cst(const 
   return (const __attribute__((address_space(4))) T*)p;
 }
 
+// The kernels' two arguments as they lie in the kernel argument segment.  A
+// field that only a trajectory's start, its end or a tape record reads would
+// stay in scalar registers for the whole launch (and most of them spill);
+// code outside the step reads the arguments through fresh_args() instead,
+// whose result the compiler cannot merge with earlier loads.
+struct KernelArgs {
+  DevPlan P;
+  DevCall C;
+};
+__device__ __forceinline__ const KernelArgs& fresh_args() {
+  typedef const __attribute__((address_space(4))) KernelArgs* Ptr;
+  Ptr p = (Ptr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const KernelArgs*)p;
+}
+
 __device__ __forceinline__ dcpx mk(double r, double i) { return dcpx{r, i}; }
 __device__ __forceinline__ dcpx cadd(dcpx a, dcpx b) { return mk(a.re + b.re, a.im + b.im); }
 __device__ __forceinline__ dcpx csub(dcpx a, dcpx b) { return mk(a.re - b.re, a.im - b.im); }
@@ -699,8 +715,9 @@ __device__ __forceinline__ void gather_block(const uint32_t* gw, const double2* 
 
 // d(rho)/dt for the slots of this thread: publish the cross-coupled elements,
 // barrier, then self term + gathers.  `pubbuf` alternates between two buffers
-// so one barrier per evaluation suffices.
-template <int R>
+// so one barrier per evaluation suffices.  COUPLINGS: the plan is known to
+// have couplings.
+template <int R, bool COUPLINGS = false>
 __device__ __forceinline__ void rhs_eval(const DevPlan& P, const Lds& L, const Slots<R>& S,
                                          const double (&xr)[R], const double (&xi)[R], double (&kr)[R],
                                          double (&ki)[R], double* pubbuf, const dcpx* coef, int vrow, int tid,
@@ -712,7 +729,7 @@ __device__ __forceinline__ void rhs_eval(const DevPlan& P, const Lds& L, const S
   for (int r = 0; r < R; ++r)
     if (S.pub[r] >= 0) reinterpret_cast<double2*>(pubbuf)[S.pub[r]] = double2{xr[r], xi[r]};
   __syncthreads();
-  if (P.couplings) {
+  if (COUPLINGS || P.couplings) {
     const char* const pb = reinterpret_cast<const char*>(pubbuf);
     const char* const ent = reinterpret_cast<const char*>(L.ent);
     const uint32_t dyn = 16u * (uint32_t)(vrow * P.nv_dyn);
@@ -733,6 +750,7 @@ __device__ __forceinline__ void rhs_eval(const DevPlan& P, const Lds& L, const S
     }
     return;
   }
+  if constexpr (COUPLINGS) return;
   const uint32_t* gw = P.lds_tables ? static_cast<const uint32_t*>(L.gw) : P.g_word;
   const double2* gf = P.lds_tables ? static_cast<const double2*>(L.gf) : reinterpret_cast<const double2*>(P.g_f);
 #pragma unroll
@@ -1100,11 +1118,23 @@ __device__ __forceinline__ void write_row(const DevPlan& P, const DevCall& C, co
 // Persistent integrator.
 // ---------------------------------------------------------------------------
 // G > 0 selects the single-wave form (R = 1, 64 threads, G gather rows in
-// registers); G = 0 is the general multi-wave form.
-template <int R, int SOLVER, int MAXW, int WAVES, int G, bool EV = false>
+// registers); G = 0 is the multi-wave form.  LEAN: the multi-wave form of a
+// plan with couplings (and step programs, where it is time-dependent) for a
+// call with a given initial step that pushes at accepted steps at most into
+// the weighted integral: no trace, save plan, replay or stop event.
+//
+// The step of a 72-level plan is 3.1k VALU instructions a wave where the
+// arithmetic needs some 700: most of the others moved spilled scalar and
+// vector registers, whose live ranges came from code that the call does not
+// run.  LEAN leaves that code out, unrolls the stages where they are short,
+// and what runs once a trajectory reads its arguments anew (fresh_args).
+// 512 + 512 uneven batch (72 levels) 390 -> 310 ms, 500 thermal atoms (780
+// elements, kernel) 1.3 -> 0.82 ms.
+template <int R, int SOLVER, int MAXW, int WAVES, int G, bool EV = false, bool LEAN = false>
 __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, const DevCall C) {
   static_assert(G == 0 || (R == 1 && MAXW == 64), "the single-wave form holds one slot per lane");
   static_assert(!EV || G == 0, "stop events run in the multi-wave form");
+  static_assert(!LEAN || (G == 0 && !EV), "the lean form is a multi-wave form without stop events");
   using T = Tab<SOLVER>;
   const int tid = threadIdx.x, W = blockDim.x;
   const Lds L = carve(P);
@@ -1123,50 +1153,56 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
     // the batch are skipped, so a bad order cannot address past the arrays
     const int64_t traj = C.queue_order ? (int64_t)C.queue_order[local + C.traj_offset] : local + C.traj_offset;
     if (traj < 0 || traj >= C.n_total) continue;
-    const double t0 = C.t0;
-    const double t1 = C.t1_per_traj ? C.t1_per_traj[traj] : C.t1;
-
-    // ---- parameters and coefficients at t0, self-term folds, weights
-    init_slots(P, L.slots, tid, W);
-    if (tid == 0) {
-      apply_overrides(C, traj, L.slots);
-      eval_coefficients(P, L.slots, L.coef, t0, false, L.vm);
-    }
-    for (int i = tid; i < P.n; i += W) {
-      double w = 0.0;
-      for (int q = 0; q < C.n_weights; ++q)
-        if (C.weight_index[q] == i) w += C.weight_value[q];
-      L.wts[i] = w;
-      if constexpr (EV) L.evv[i] = 0.0;  // stop-event populations outside a restricted plan stay zero
-    }
-    __syncthreads();
-    for (int i = tid; i < 7 * P.v_slots; i += W) L.slots[P.v_slots + i] = L.slots[i % P.v_slots];
-    for (int i = tid; i < 7 * KK; i += W) L.coef[KK + i] = L.coef[i % KK];
-    fold_self(P, tid, W, L.coef, L.selfc);
-    if (P.couplings) {  // entry row 5 holds t0 until the last stage needs it
-      fill_static_entries(P, L.coef, L.ent, tid, W);
-      fill_entries<1>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef, KK, L.ent + P.nv_stat + 5 * P.nv_dyn, tid, W);
-    }
-
-    // ---- state
-    double y_r[R], y_i[R];
-    const double* y0 = C.y0 + (C.y0_shared ? 0 : traj * (int64_t)P.dim);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int s = tid + W * r;
-      y_r[r] = S.valid(r) ? y0[P.slot_re[s]] : 0.0;
-      y_i[r] = (S.valid(r) && !S.diag(r)) ? y0[P.slot_im[s]] : 0.0;
-    }
-    // a restricted plan needs y0 to vanish outside its elements
+    double t1, y_r[R], y_i[R];
     bool bad_support = false;
-    if (P.restricted) {
-      if (tid == 0) L.misc[1] = 0;
+    {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
+      const double t0 = C.t0;
+      t1 = C.t1_per_traj ? C.t1_per_traj[traj] : C.t1;
+
+      // ---- parameters and coefficients at t0, self-term folds, weights
+      init_slots(P, L.slots, tid, W);
+      if (tid == 0) {
+        apply_overrides(C, traj, L.slots);
+        eval_coefficients(P, L.slots, L.coef, t0, false, L.vm);
+      }
+      for (int i = tid; i < P.n; i += W) {
+        double w = 0.0;
+        for (int q = 0; q < C.n_weights; ++q)
+          if (C.weight_index[q] == i) w += C.weight_value[q];
+        L.wts[i] = w;
+        if constexpr (EV) L.evv[i] = 0.0;  // stop-event populations outside a restricted plan stay zero
+      }
       __syncthreads();
-      for (int k = tid; k < P.dim; k += W)
-        if (!P.upper_active[P.packed_upper[k]] && y0[k] != 0.0) L.misc[1] = 1;
-      __syncthreads();
-      bad_support = L.misc[1] != 0;
+      for (int i = tid; i < 7 * P.v_slots; i += W) L.slots[P.v_slots + i] = L.slots[i % P.v_slots];
+      for (int i = tid; i < 7 * KK; i += W) L.coef[KK + i] = L.coef[i % KK];
+      fold_self(P, tid, W, L.coef, L.selfc);
+      if (P.couplings) {  // entry row 5 holds t0 until the last stage needs it
+        fill_static_entries(P, L.coef, L.ent, tid, W);
+        fill_entries<1>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef, KK, L.ent + P.nv_stat + 5 * P.nv_dyn, tid, W);
+      }
+
+      // ---- state
+      const double* y0 = C.y0 + (C.y0_shared ? 0 : traj * (int64_t)P.dim);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int s = tid + W * r;
+        y_r[r] = S.valid(r) ? y0[P.slot_re[s]] : 0.0;
+        y_i[r] = (S.valid(r) && !S.diag(r)) ? y0[P.slot_im[s]] : 0.0;
+      }
+      // a restricted plan needs y0 to vanish outside its elements
+      if (P.restricted) {
+        if (tid == 0) L.misc[1] = 0;
+        __syncthreads();
+        for (int k = tid; k < P.dim; k += W)
+          if (!P.upper_active[P.packed_upper[k]] && y0[k] != 0.0) L.misc[1] = 1;
+        __syncthreads();
+        bad_support = L.misc[1] != 0;
+      }
     }
+    const double t0 = C.t0;
 
     int64_t accepted = 0, rejected = 0, rhs_calls = 0, attempts = 0;
     int status = 0;
@@ -1180,8 +1216,9 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
     // trace rows.  Pushing at every accepted step folds the integrand into
     // the error-norm reduction; a save plan (saveat) reduces per point.
     int64_t n_pushed = 0, si = 0;
-    const bool step_push = C.n_saveat == 0;
-    const bool rate = C.output_kind == LB_OUT_RATE;
+    const bool step_push = LEAN || C.n_saveat == 0;
+    const bool rate = !LEAN && C.output_kind == LB_OUT_RATE, trace = !LEAN && C.trace;
+    const bool tape = C.tape_h != nullptr, replay = !LEAN && C.replay_h;
     auto push = [&](double tp, const double (&vr)[R], const double (&vi)[R], bool reduce_integrand) {
       double v = last_v;
       if constexpr (EV) last_pt = tp;
@@ -1198,7 +1235,10 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           last_v = v;
         }
       }
-      if (C.trace) {
+      if (trace) {
+        const KernelArgs& A = fresh_args();
+        const DevPlan& P = A.P;
+        const DevCall& C = A.C;
         if (n_pushed < C.capacity) {
           const int64_t row = traj * C.capacity + n_pushed;
           if (C.output_kind == LB_OUT_INTEGRAL) {
@@ -1216,10 +1256,10 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
     double k_r[8][R], k_i[8][R];
     int buf = 0;
 #define PUB (L.pub + buf * 2 * P.n_pub)
-#define LB_RHS(xr, xi, kr, ki, cf, vrow)                         \
-  do {                                                           \
-    rhs_eval<R>(P, L, S, xr, xi, kr, ki, PUB, cf, vrow, tid, W); \
-    buf ^= 1;                                                    \
+#define LB_RHS(xr, xi, kr, ki, cf, vrow)                                \
+  do {                                                                  \
+    rhs_eval<R, LEAN>(P, L, S, xr, xi, kr, ki, PUB, cf, vrow, tid, W); \
+    buf ^= 1;                                                           \
   } while (0)
 
     if (bad_support) {
@@ -1234,9 +1274,12 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
       double x = t0, h;
       // ---- k1 = f(t0, y0) (also f0 of hinit); the barrier inside orders the LDS fills above
       LB_RHS(y_r, y_i, k_r[1], k_i[1], L.coef, 5);
-      if (isfinite(C.dt) && C.dt > 0.0) {
+      if (LEAN || (isfinite(C.dt) && C.dt > 0.0)) {
         h = fmin(C.dt, t1 - t0);
       } else {
+        const KernelArgs& A = fresh_args();
+        const DevPlan& P = A.P;
+        const DevCall& C = A.C;
         // hinit (rust/src/ode/common.rs:72-118)
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -1299,7 +1342,10 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
       while (!last && (!EV || status == 0)) {
         if (ns > C.maxiters) { status = LB_TRAJ_MAXITERS; fail_x = x; break; }
         bool clipped = false;
-        if (C.replay_h) {
+        if (replay) {
+          const KernelArgs& A = fresh_args();
+          const DevPlan& P = A.P;
+          const DevCall& C = A.C;
           // recorded schedule: step sizes of a tape, every step accepted
           const int64_t nrep = C.replay_n[traj];
           if (accepted >= nrep || accepted >= C.tape_cap) { status = LB_TRAJ_CAPACITY; fail_x = x; break; }
@@ -1319,7 +1365,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         }
         // time-dependent coefficients at the six stage times, one lane per stage
         if (P.time_dependent) {
-          if (P.v_steps > 0) {
+          if (LEAN || P.v_steps > 0) {
             if (tid < 64) {
               const int s = min((tid & 7) + 2, 7);
               vector_eval(L.vops, P.v_steps, L.slots + s * P.v_slots, L.coef + s * KK, P.v_time, x + h * T::c(s), tid,
@@ -1334,7 +1380,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         if (P.time_dependent) {
           __syncthreads();  // stage coefficients are read by every lane
           // stages 2..6 take entry rows 0..4; stage 7 is at the same time as 6
-          if (P.couplings)
+          if (LEAN || P.couplings)
             fill_entries<5>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + 2 * KK, KK, L.ent + P.nv_stat, tid, W);
         }
         if constexpr (G > 0) {
@@ -1354,10 +1400,11 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           }
         const bool need_stiff = ((accepted + 1) % 1000 == 0) || ia > 0;
         double yt_r[R], yt_i[R], yn_r[R], yn_i[R];
-        // Stages 2..7 share one RHS site (a rolled loop keeps the step's code
-        // small enough for the instruction cache); stage 7 is the solution,
-        // whose RHS is the FSAL derivative.
-#pragma unroll 1
+        // Stage 7 is the solution, whose RHS is the FSAL derivative.  With
+        // many slots a lane the stages share one RHS site (a rolled loop keeps
+        // the step's code small enough for the instruction cache); unrolled,
+        // the stage vectors need no copies and no zeros.
+#pragma unroll(LEAN && R <= 2 ? 6 : 1)
         for (int s = 2; s <= 7; ++s) {
           switch (s) {
             case 2: stage_combo<R, SOLVER, 2>(h, y_r, y_i, k_r, k_i, yt_r, yt_i); break;
@@ -1422,10 +1469,13 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           }
         }
         __syncthreads();
-        const StepControl ctl(C.replay_h ? 0.0 : block_total(P, L.red, 0) * inv_dim, lfo);
+        const StepControl ctl(replay ? 0.0 : block_total(P, L.red, 0) * inv_dim, lfo);
         const double err = ctl.err;
         double hn = h * ctl.factor();
-        if (C.tape_h && !C.replay_h) {
+        if (tape && !replay) {
+          const KernelArgs& A = fresh_args();
+          const DevPlan& P = A.P;
+          const DevCall& C = A.C;
           // attempt tape: what the adjoint needs to differentiate this attempt
           // and the controller's decision (one record per attempt)
           const int64_t a = ns - 1;
@@ -1489,6 +1539,9 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           double te = x;
           if constexpr (EV) {
             if (C.event_kind) {
+              const KernelArgs& A = fresh_args();
+              const DevPlan& P = A.P;
+              const DevCall& C = A.C;
               bool cpx = false;
               const double g1 = event_value<R>(P, C, L, S, tid, W, x, L.slots + 7 * P.v_slots, yn_r, cpx);
               if (cpx) { status = LB_TRAJ_EVENT_COMPLEX; fail_x = x; break; }
@@ -1536,9 +1589,12 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
                 last_v = v;
               }
               if constexpr (EV) last_pt = x;
-              if (C.trace) push(x, yn_r, yn_i, rate);
+              if (trace) push(x, yn_r, yn_i, rate);
             }
           } else {
+            const KernelArgs& A = fresh_args();
+            const DevPlan& P = A.P;
+            const DevCall& C = A.C;
             // save plan points inside (xo, x], or up to the root (dopri5.rs:318-344)
             const double tb = ev_hit ? te : x;
             while (si < C.n_saveat && C.saveat[si] <= tb + time_tol(tb)) {
@@ -1603,23 +1659,73 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
 #undef PUB
 
     // ---- outputs
-    if constexpr (EV) {
-      if (C.out_event_t && tid == 0) C.out_event_t[traj] = ev_t;
-    }
-    if (status == 0 && !step_push && si != C.n_saveat && (!EV || !ev_fired)) {
-      status = LB_TRAJ_SAVEAT;
-      fail_x = (double)si;  // plan points reached
-    }
-    if (status == 0 && C.trace && n_pushed > C.capacity) status = LB_TRAJ_CAPACITY;
-    if (status == 0 && C.tape_h && !C.replay_h && attempts > C.tape_cap) status = LB_TRAJ_CAPACITY;
-    if (C.tape_n && tid == 0) C.tape_n[traj] = (int32_t)attempts;
-    const bool ok = status == 0;
-    const double nanv = __builtin_nan("");
-    if (C.trace) {
-      // rows were written as the points were pushed; dropped elements stay
-      // at the zeros the caller provides
+    {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
+      if constexpr (EV) {
+        if (C.out_event_t && tid == 0) C.out_event_t[traj] = ev_t;
+      }
+      if (status == 0 && !step_push && si != C.n_saveat && (!EV || !ev_fired)) {
+        status = LB_TRAJ_SAVEAT;
+        fail_x = (double)si;  // plan points reached
+      }
+      if (status == 0 && C.trace && n_pushed > C.capacity) status = LB_TRAJ_CAPACITY;
+      if (status == 0 && C.tape_h && !C.replay_h && attempts > C.tape_cap) status = LB_TRAJ_CAPACITY;
+      if (C.tape_n && tid == 0) C.tape_n[traj] = (int32_t)attempts;
+      const bool ok = status == 0;
+      const double nanv = __builtin_nan("");
+      if (C.trace) {
+        // rows were written as the points were pushed; dropped elements stay
+        // at the zeros the caller provides
+        if (tid == 0) {
+          C.out_counts[traj] = (int32_t)n_pushed;
+          if (C.out_integral) C.out_integral[traj] = ok ? integral : nanv;
+          C.out_stats[4 * traj + 0] = accepted;
+          C.out_stats[4 * traj + 1] = rejected;
+          C.out_stats[4 * traj + 2] = rhs_calls;
+          C.out_stats[4 * traj + 3] = status;
+          C.out_fail_t[traj] = fail_x;
+        }
+        continue;
+      }
+      if (P.restricted) {
+        // elements outside the restricted plan are exactly zero
+        if (C.output_kind == LB_OUT_POPULATIONS) {
+          for (int i = tid; i < P.n; i += W)
+            if (!P.upper_active[P.packed_upper[i]]) C.out_values[traj * P.n + i] = ok ? 0.0 : nanv;
+        } else if (C.output_kind == LB_OUT_FULL) {
+          for (int k = tid; k < P.dim; k += W)
+            if (!P.upper_active[P.packed_upper[k]]) C.out_values[traj * P.dim + k] = ok ? 0.0 : nanv;
+        } else if (C.output_kind == LB_OUT_SELECTED) {
+          for (int q = tid; q < C.n_selected; q += W)
+            if (!P.upper_active[C.sel_upper[q]]) {
+              C.out_values[2 * (traj * C.n_selected + q)] = ok ? 0.0 : nanv;
+              C.out_values[2 * (traj * C.n_selected + q) + 1] = ok ? 0.0 : nanv;
+            }
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if (!S.valid(r)) continue;
+        const int s = tid + W * r;
+        if (C.output_kind == LB_OUT_POPULATIONS) {
+          if (S.diag(r)) C.out_values[traj * P.n + S.state(r)] = ok ? y_r[r] : nanv;
+        } else if (C.output_kind == LB_OUT_FULL) {
+          C.out_values[traj * P.dim + P.slot_re[s]] = ok ? y_r[r] : nanv;
+          if (!S.diag(r)) C.out_values[traj * P.dim + P.slot_im[s]] = ok ? y_i[r] : nanv;
+        } else if (C.output_kind == LB_OUT_SELECTED) {
+          const int up = P.slot_up[s];
+          for (int q = 0; q < C.n_selected; ++q) {
+            if (C.sel_upper[q] != up) continue;
+            const double im = (C.sel_flags[q] & 1) ? 0.0 : ((C.sel_flags[q] & 2) ? -y_i[r] : y_i[r]);
+            C.out_values[2 * (traj * C.n_selected + q)] = ok ? y_r[r] : nanv;
+            C.out_values[2 * (traj * C.n_selected + q) + 1] = ok ? im : nanv;
+          }
+        }
+      }
       if (tid == 0) {
-        C.out_counts[traj] = (int32_t)n_pushed;
+        if (C.output_kind == LB_OUT_INTEGRAL) C.out_values[traj] = ok ? integral : nanv;
         if (C.out_integral) C.out_integral[traj] = ok ? integral : nanv;
         C.out_stats[4 * traj + 0] = accepted;
         C.out_stats[4 * traj + 1] = rejected;
@@ -1627,51 +1733,6 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         C.out_stats[4 * traj + 3] = status;
         C.out_fail_t[traj] = fail_x;
       }
-      continue;
-    }
-    if (P.restricted) {
-      // elements outside the restricted plan are exactly zero
-      if (C.output_kind == LB_OUT_POPULATIONS) {
-        for (int i = tid; i < P.n; i += W)
-          if (!P.upper_active[P.packed_upper[i]]) C.out_values[traj * P.n + i] = ok ? 0.0 : nanv;
-      } else if (C.output_kind == LB_OUT_FULL) {
-        for (int k = tid; k < P.dim; k += W)
-          if (!P.upper_active[P.packed_upper[k]]) C.out_values[traj * P.dim + k] = ok ? 0.0 : nanv;
-      } else if (C.output_kind == LB_OUT_SELECTED) {
-        for (int q = tid; q < C.n_selected; q += W)
-          if (!P.upper_active[C.sel_upper[q]]) {
-            C.out_values[2 * (traj * C.n_selected + q)] = ok ? 0.0 : nanv;
-            C.out_values[2 * (traj * C.n_selected + q) + 1] = ok ? 0.0 : nanv;
-          }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if (!S.valid(r)) continue;
-      const int s = tid + W * r;
-      if (C.output_kind == LB_OUT_POPULATIONS) {
-        if (S.diag(r)) C.out_values[traj * P.n + S.state(r)] = ok ? y_r[r] : nanv;
-      } else if (C.output_kind == LB_OUT_FULL) {
-        C.out_values[traj * P.dim + P.slot_re[s]] = ok ? y_r[r] : nanv;
-        if (!S.diag(r)) C.out_values[traj * P.dim + P.slot_im[s]] = ok ? y_i[r] : nanv;
-      } else if (C.output_kind == LB_OUT_SELECTED) {
-        const int up = P.slot_up[s];
-        for (int q = 0; q < C.n_selected; ++q) {
-          if (C.sel_upper[q] != up) continue;
-          const double im = (C.sel_flags[q] & 1) ? 0.0 : ((C.sel_flags[q] & 2) ? -y_i[r] : y_i[r]);
-          C.out_values[2 * (traj * C.n_selected + q)] = ok ? y_r[r] : nanv;
-          C.out_values[2 * (traj * C.n_selected + q) + 1] = ok ? im : nanv;
-        }
-      }
-    }
-    if (tid == 0) {
-      if (C.output_kind == LB_OUT_INTEGRAL) C.out_values[traj] = ok ? integral : nanv;
-      if (C.out_integral) C.out_integral[traj] = ok ? integral : nanv;
-      C.out_stats[4 * traj + 0] = accepted;
-      C.out_stats[4 * traj + 1] = rejected;
-      C.out_stats[4 * traj + 2] = rhs_calls;
-      C.out_stats[4 * traj + 3] = status;
-      C.out_fail_t[traj] = fail_x;
     }
   }
 }
@@ -1869,45 +1930,51 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
     if (local >= C.n_traj) break;
     const int64_t traj = C.queue_order ? (int64_t)C.queue_order[local + C.traj_offset] : local + C.traj_offset;
     if (traj < 0 || traj >= C.n_total) continue;
-    const double t0 = C.t0;
-    const double t1 = C.t1_per_traj ? C.t1_per_traj[traj] : C.t1;
-
-    // ---- parameters and coefficients at t0, self-term folds, weights
-    init_slots(P, L.slots, tid, W);
-    if (tid == 0) {
-      apply_overrides(C, traj, L.slots);
-      eval_coefficients(P, L.slots, L.coef, t0, false, L.vm);
-    }
-    for (int i = tid; i < P.n; i += W) {
-      double w = 0.0;
-      for (int q = 0; q < C.n_weights; ++q)
-        if (C.weight_index[q] == i) w += C.weight_value[q];
-      L.wts[i] = w;
-      if constexpr (EV) L.evv[i] = 0.0;
-    }
-    __syncthreads();
-    for (int i = tid; i < 7 * P.v_slots; i += W) L.slots[P.v_slots + i] = L.slots[i % P.v_slots];
-    for (int i = tid; i < 7 * KK; i += W) L.coef[KK + i] = L.coef[i % KK];
-    fold_self(P, tid, W, L.coef, L.selfc);
-    if (P.couplings) fill_static_entries(P, L.coef, L.ent, tid, W);
-
-    double y_r[R], y_i[R];
-    const double* y0 = C.y0 + (C.y0_shared ? 0 : traj * (int64_t)P.dim);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int s = tid + W * r;
-      y_r[r] = S.valid(r) ? y0[P.slot_re[s]] : 0.0;
-      y_i[r] = (S.valid(r) && !S.diag(r)) ? y0[P.slot_im[s]] : 0.0;
-    }
+    double t1, y_r[R], y_i[R];
     bool bad_support = false;
-    if (P.restricted) {
-      if (tid == 0) L.misc[1] = 0;
+    {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
+      const double t0 = C.t0;
+      t1 = C.t1_per_traj ? C.t1_per_traj[traj] : C.t1;
+
+      // ---- parameters and coefficients at t0, self-term folds, weights
+      init_slots(P, L.slots, tid, W);
+      if (tid == 0) {
+        apply_overrides(C, traj, L.slots);
+        eval_coefficients(P, L.slots, L.coef, t0, false, L.vm);
+      }
+      for (int i = tid; i < P.n; i += W) {
+        double w = 0.0;
+        for (int q = 0; q < C.n_weights; ++q)
+          if (C.weight_index[q] == i) w += C.weight_value[q];
+        L.wts[i] = w;
+        if constexpr (EV) L.evv[i] = 0.0;
+      }
       __syncthreads();
-      for (int k = tid; k < P.dim; k += W)
-        if (!P.upper_active[P.packed_upper[k]] && y0[k] != 0.0) L.misc[1] = 1;
-      __syncthreads();
-      bad_support = L.misc[1] != 0;
+      for (int i = tid; i < 7 * P.v_slots; i += W) L.slots[P.v_slots + i] = L.slots[i % P.v_slots];
+      for (int i = tid; i < 7 * KK; i += W) L.coef[KK + i] = L.coef[i % KK];
+      fold_self(P, tid, W, L.coef, L.selfc);
+      if (P.couplings) fill_static_entries(P, L.coef, L.ent, tid, W);
+
+      const double* y0 = C.y0 + (C.y0_shared ? 0 : traj * (int64_t)P.dim);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int s = tid + W * r;
+        y_r[r] = S.valid(r) ? y0[P.slot_re[s]] : 0.0;
+        y_i[r] = (S.valid(r) && !S.diag(r)) ? y0[P.slot_im[s]] : 0.0;
+      }
+      if (P.restricted) {
+        if (tid == 0) L.misc[1] = 0;
+        __syncthreads();
+        for (int k = tid; k < P.dim; k += W)
+          if (!P.upper_active[P.packed_upper[k]] && y0[k] != 0.0) L.misc[1] = 1;
+        __syncthreads();
+        bad_support = L.misc[1] != 0;
+      }
     }
+    const double t0 = C.t0;
 
     int64_t accepted = 0, rhs_calls = 0, n_pushed = 0, si = 0;
     int status = 0;
@@ -1915,7 +1982,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
     double ev_old = 0.0, ev_t = __builtin_nan("");  // stop event: g at the last step end, root time
     bool ev_fired = false;
     const bool step_push = C.n_saveat == 0;
-    const bool rate = C.output_kind == LB_OUT_RATE;
+    const bool rate = C.output_kind == LB_OUT_RATE, trace = C.trace != 0;
     auto push = [&](double tp, const double (&vr)[R], const double (&vi)[R]) {
       double v = last_v;
       if (C.want_integral || rate) {
@@ -1931,7 +1998,10 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
           last_v = v;
         }
       }
-      if (C.trace) {
+      if (trace) {
+        const KernelArgs& A = fresh_args();
+        const DevPlan& P = A.P;
+        const DevCall& C = A.C;
         if (n_pushed < C.capacity) {
           const int64_t row = traj * C.capacity + n_pushed;
           if (C.output_kind == LB_OUT_INTEGRAL) {
@@ -2016,6 +2086,9 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
         // (its start when g was zero there), with the end state
         bool ev_hit = false;
         if constexpr (EV) {
+          const KernelArgs& A = fresh_args();
+          const DevPlan& P = A.P;
+          const DevCall& C = A.C;
           // slot copy 0 is free after the trajectory's start
           if (C.event_kind == LB_EVENT_EXPRESSION && tid == 0) eval_compounds(P, L.slots, x, L.vm);
           bool cpx = false;
@@ -2057,11 +2130,16 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_fixed_kernel(const DevPlan P, 
         fail_x = (double)si;
       }
     }
-    if (status == 0 && C.trace && n_pushed > C.capacity) status = LB_TRAJ_CAPACITY;
-    if constexpr (EV) {
-      if (C.out_event_t && tid == 0) C.out_event_t[traj] = ev_t;
+    {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
+      if (status == 0 && C.trace && n_pushed > C.capacity) status = LB_TRAJ_CAPACITY;
+      if constexpr (EV) {
+        if (C.out_event_t && tid == 0) C.out_event_t[traj] = ev_t;
+      }
+      write_final<R>(P, C, S, tid, W, traj, y_r, y_i, status, fail_x, integral, accepted, rhs_calls, n_pushed);
     }
-    write_final<R>(P, C, S, tid, W, traj, y_r, y_i, status, fail_x, integral, accepted, rhs_calls, n_pushed);
   }
 }
 
@@ -2452,7 +2530,7 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
   int status = 0, si = 0;
   bool reject = false, last = false, ev_fired = false;
   double ev_old = 0.0, ev_t = __builtin_nan("");
-  const bool step_push = !SAVE || C.n_saveat == 0;
+  const bool step_push = !SAVE || C.n_saveat == 0, tape = C.tape_h != nullptr;
   double2 selfv = double2{0.0, 0.0};
   double y_r[1] = {0.0}, y_i[1] = {0.0};
   double k_r[8][1], k_i[8][1];
@@ -2472,6 +2550,9 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
     if (__all(done)) break;
     // ---- initialise a new trajectory (rust/src/ode/dopri5.rs:160-220)
     if (starting) {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
       t1 = C.t1_per_traj ? C.t1_per_traj[traj] : C.t1;
       // entry row 5 holds t0 (the steps use rows 0..4)
       const bool bad_support = lane_start<LPT>(P, C, L, S, half, sl, traj, 5, selfv, y_r, y_i);
@@ -2620,7 +2701,10 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
       const StepControl ctl(e2 * inv_dim, lfo);
       const double err = ctl.err;
       double hn = h * ctl.factor();
-      if (C.tape_h) {
+      if (tape) {
+        const KernelArgs& A = fresh_args();
+        const DevPlan& P = A.P;
+        const DevCall& C = A.C;
         // attempt tape, as the multi-wave form records it: one record per
         // attempt by lane 0, the state every ckpt_every-th attempt
         if (ns - 1 < C.tape_cap) {
@@ -2802,6 +2886,9 @@ __global__ __launch_bounds__(64, WAVES) void lb_solve_pair_kernel(const DevPlan 
     }
     // ---- a finished trajectory writes its outputs
     if (active && last) {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
       if constexpr (EV) {
         if (C.out_event_t && sl == 0) C.out_event_t[traj] = ev_t;
       }
@@ -2858,6 +2945,9 @@ __global__ __launch_bounds__(64, WAVES) void lb_fixed_pair_kernel(const DevPlan 
     if (need) active = starting;
     if (__all(done)) break;
     if (starting) {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
       t1 = C.t1_per_traj ? C.t1_per_traj[traj] : C.t1;
       const bool bad_support = lane_start<LPT>(P, C, L, S, half, sl, traj, 0, selfv, y_r, y_i);
       steps = 0;
@@ -2933,6 +3023,9 @@ __global__ __launch_bounds__(64, WAVES) void lb_fixed_pair_kernel(const DevPlan 
       y_i[0] = yn_i[0];
     }
     if (active && last) {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
       if (status == 0 && C.trace && pts.n > C.capacity) status = LB_TRAJ_CAPACITY;
       lane_finish<LPT>(P, C, S, sl, traj, y_r, y_i, status, fail_x, pts.integral, pts.n, steps, 0, steps * NS);
       active = false;
@@ -4775,6 +4868,14 @@ void* solve_ptr(int solver) {
     return nullptr;
 }
 template <int I, int RR, int WW, int VV>
+void* lean_ptr(int solver) {
+  if constexpr (I % LB_NPART == LB_PART)
+    return solver == 1 ? (void*)&lb_solve_kernel<RR, 1, WW, VV, 0, false, true>
+                       : (void*)&lb_solve_kernel<RR, 0, WW, VV, 0, false, true>;
+  else
+    return nullptr;
+}
+template <int I, int RR, int WW, int VV>
 void* adjoint_ptr(int solver) {
   if constexpr (I % LB_NPART == LB_PART)
     return solver == 1 ? (void*)&lb_adjoint_kernel<RR, 1, WW, VV> : (void*)&lb_adjoint_kernel<RR, 0, WW, VV>;
@@ -4852,6 +4953,14 @@ extern "C" void* LB_PART_FN(lb_dev_solve_kernel)(int id, int solver) {
   if (id == i) return pair_solve_ptr<i, g, v>(solver);
   LB_PAIR_CONFIGS(Q)
 #undef Q
+  return nullptr;
+}
+
+extern "C" void* LB_PART_FN(lb_dev_lean_kernel)(int id, int solver) {
+#define X(i, r, w, v) \
+  if (id == i) return lean_ptr<i, r, w, v>(solver);
+  LB_CONFIGS(X)
+#undef X
   return nullptr;
 }
 

@@ -10,6 +10,14 @@ extern "C" void* lb_dev_solve_kernel_p4(int, int);
 extern "C" void* lb_dev_solve_kernel_p5(int, int);
 extern "C" void* lb_dev_solve_kernel_p6(int, int);
 extern "C" void* lb_dev_solve_kernel_p7(int, int);
+extern "C" void* lb_dev_lean_kernel_p0(int, int);
+extern "C" void* lb_dev_lean_kernel_p1(int, int);
+extern "C" void* lb_dev_lean_kernel_p2(int, int);
+extern "C" void* lb_dev_lean_kernel_p3(int, int);
+extern "C" void* lb_dev_lean_kernel_p4(int, int);
+extern "C" void* lb_dev_lean_kernel_p5(int, int);
+extern "C" void* lb_dev_lean_kernel_p6(int, int);
+extern "C" void* lb_dev_lean_kernel_p7(int, int);
 extern "C" void* lb_dev_fixed_kernel_p0(int, int);
 extern "C" void* lb_dev_fixed_kernel_p1(int, int);
 extern "C" void* lb_dev_fixed_kernel_p2(int, int);
@@ -99,6 +107,12 @@ extern "C" int lb_dev_variant_rows(int id) {
 
 extern "C" void* lb_dev_solve_kernel(int id, int solver) {
   void* (*parts[])(int, int) = {lb_dev_solve_kernel_p0, lb_dev_solve_kernel_p1, lb_dev_solve_kernel_p2, lb_dev_solve_kernel_p3, lb_dev_solve_kernel_p4, lb_dev_solve_kernel_p5, lb_dev_solve_kernel_p6, lb_dev_solve_kernel_p7};
+  return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);
+}
+
+// The lean form of a multi-wave variant (lb_solve_kernel); null for the others.
+extern "C" void* lb_dev_lean_kernel(int id, int solver) {
+  void* (*parts[])(int, int) = {lb_dev_lean_kernel_p0, lb_dev_lean_kernel_p1, lb_dev_lean_kernel_p2, lb_dev_lean_kernel_p3, lb_dev_lean_kernel_p4, lb_dev_lean_kernel_p5, lb_dev_lean_kernel_p6, lb_dev_lean_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);
 }
 

@@ -14,11 +14,13 @@ import pytest
 import sympy as smp
 
 from centrex_tlf_amd.lindblad import prepare_lindblad_problem
+from centrex_tlf_amd.lindblad.native import DevicePlan
 from centrex_tlf_amd.lindblad.systems import OBESystem
 from oracle.lb_oracle import Oracle
 
 from ._dense import CHAIN_PARAMETERS, chain_system, random_density
 from ._gpu import require_gpu
+from .systems import tlf_n39
 
 pytestmark = pytest.mark.gpu
 
@@ -74,3 +76,24 @@ def test_more_entries_than_fit_take_the_gather_tables():
     got = plan.rhs(torch.as_tensor(y, device="cuda"), torch.as_tensor(np.asarray([0.41]), device="cuda")).cpu().numpy()[0]
     want = oracle.rhs(y, 0.41)
     np.testing.assert_allclose(got, want, rtol=0, atol=1e-12 * np.abs(want).max())
+
+
+@pytest.mark.parametrize("solver", ["dopri5", "tsit5"])
+@pytest.mark.parametrize("variant", [1, 2, 3, 4])
+def test_lean_form_is_bitwise_the_general_form(solver, variant):
+    """Final outputs and the step integral (lean multi-wave form) against the
+    last row and the integral of a trace of the accepted steps (general form),
+    one, two and three slots a lane."""
+    require_gpu()
+    system, params, rho0, t_span, weights = tlf_n39()
+    prepared = prepare_lindblad_problem(system, params, backend="host")
+    plan, y0 = DevicePlan(prepared.flat_plan), prepared.layout.pack(rho0)
+    t1 = np.asarray([0.02, 0.3, 0.11]) * t_span[1]
+    kw = dict(abstol=1e-9, reltol=1e-7, dt=1e-8, solver=solver, variant=variant, restrict_support=False,
+              weights=weights, with_integral=True, output_kind="full", n_traj=3)
+    rows, stats, _, integral, counts, _ = plan.solve(y0, t_span[0], t1, trace=True, capacity=400, **kw)
+    final, lean_stats, *_, lean_integral = plan.solve(y0, t_span[0], t1, **kw)
+    assert bool((stats == lean_stats).all()) and int(stats[:, 3].max()) == 0
+    for b, n in enumerate(counts.cpu().numpy()):
+        assert n == int(stats[b, 0]) + 1 and bool((rows[b, n - 1] == final[b]).all())
+    assert bool((integral == lean_integral).all())

@@ -64,6 +64,7 @@ __host__ __device__ inline uint32_t lb_gword(uint32_t pub, bool real_in, bool co
 // buffer (16 x its publication index).
 #define LB_MAX_ENTRIES 4095
 #define LB_MAX_COUPLED 4096
+#define LB_Q_CHUNK 8   // couplings of one contraction of the adjoint
 #define LB_ENT_ROWS 6  // rows of time-dependent entry values: one per stage time of a step
 __host__ __device__ inline uint32_t lb_cword(uint32_t pub, bool conj_in, bool dyn, uint32_t entry) {
   return (pub << 20) | (entry << 4) | (conj_in ? 2u : 0u) | (dyn ? 1u : 0u);
@@ -139,6 +140,19 @@ struct DevPlan {
   const int32_t* ent_ptr;    // nv_dyn + nv_stat + 1, the time-dependent entries first
   const uint32_t* ent_coef;  // coefficient row index (K: the constant 1), bit 31 conjugated
   const double* ent_f;       // factors
+  // the adjoint over couplings: for each input slot the couplings that read
+  // it (a coupling word with 16 x the output slot in place of the input), and
+  // the contractions with the coefficient derivatives: chunks of LB_Q_CHUNK
+  // couplings of one entry (bits 16..31 of a word 16 x the output slot, S the
+  // padding; bits 4..15 16 x the publication index / 16, bit 1 conjugated)
+  int32_t nv_def, nv_def_terms;  // entries with derivatives or time dependence, the first of the list
+  int32_t tc_rows_total, q_chunks;
+  const int32_t* tc_row0;
+  const int32_t* tc_rows;
+  const uint32_t* tc_word;
+  const uint32_t* q_word;    // LB_Q_CHUNK x q_chunks
+  const uint32_t* q_ent;     // q_chunks: entry, or all ones on padding
+  int32_t adj_lds;           // tables in LDS: 1 coupling words, 2 transposed, 4 contractions
   // gather ELL, rows grouped per block (plans without couplings, and the
   // adjoint, which needs every term's own coefficient)
   const int32_t* blk_row0;   // nblk
@@ -180,7 +194,10 @@ struct DevPlan {
   const int32_t* v_const_slot;
   const double* v_const;        // v_n_const*2
   const DevVOp* v_ops;          // v_steps * LB_VOP_LANES
-  const DevVOp* v_ops_all;      // v_steps_all * LB_VOP_LANES
+  const DevVOp* v_ops_all;      // v_steps_all * LB_VOP_LANES, with slots and constants of their own:
+  int32_t va_slots, va_time, va_n_const;
+  const int32_t* va_const_slot;
+  const double* va_const;
 };
 
 // LDS of the multi-wave kernels, in bytes from the start: one layout for the
@@ -238,6 +255,35 @@ __host__ __device__ inline LbLdsPair lb_lds_pair(const DevPlan& P, uint32_t nh) 
   l.wts = q; q += 8u * (uint32_t)((P.n + 1) & ~1);
   l.ecoef = q; q += 4u * (uint32_t)P.nv_terms;
   l.eptr = q; q += 4u * (uint32_t)(P.nv_dyn + 1);
+  q = (q + 15u) & ~15u;
+  l.misc = q; q += 16u;
+  l.total = q;
+  return l;
+}
+
+// LDS of the multi-wave adjoint over couplings.
+struct LbLdsAdj {
+  uint32_t pub, kap, ent, coef, slots, vm, vops, ef, wts, red, cw, tw, qw, qe, ecoef, eptr, misc, total;
+};
+__host__ __device__ inline LbLdsAdj lb_lds_adj(const DevPlan& P) {
+  LbLdsAdj l;
+  uint32_t q = 0;
+  l.pub = q; q += 16u * (uint32_t)P.n_pub;
+  l.kap = q; q += 16u * (uint32_t)(P.S + 1);
+  l.ent = q; q += 16u * (uint32_t)(P.nv_stat + 7 * P.nv_dyn);
+  l.coef = q; q += 7u * 16u * (uint32_t)(P.KD + 1);
+  l.slots = q; q += 7u * 16u * (uint32_t)P.va_slots;
+  l.vm = q; q += 16u * (uint32_t)P.vm_depth;
+  l.vops = q; q += 16u * LB_VOP_LANES * (uint32_t)P.v_steps_all;
+  l.ef = q; q += 16u * (uint32_t)P.nv_def_terms;
+  l.wts = q; q += 8u * (uint32_t)((P.n + 1) & ~1);
+  l.red = q; q += 8u * 16u * LB_MAX_DIFF;
+  l.cw = q; q += (P.adj_lds & 1) ? 4u * 64u * (uint32_t)P.c_rows_total : 0u;
+  l.tw = q; q += (P.adj_lds & 2) ? 4u * 64u * (uint32_t)P.tc_rows_total : 0u;
+  l.qw = q; q += (P.adj_lds & 4) ? 4u * LB_Q_CHUNK * (uint32_t)P.q_chunks : 0u;
+  l.qe = q; q += (P.adj_lds & 4) ? 4u * (uint32_t)P.q_chunks : 0u;
+  l.ecoef = q; q += 4u * (uint32_t)P.nv_def_terms;
+  l.eptr = q; q += 4u * (uint32_t)(P.nv_def + 1);
   q = (q + 15u) & ~15u;
   l.misc = q; q += 16u;
   l.total = q;

@@ -55,6 +55,14 @@ __device__ __forceinline__ const KernelArgs& fresh_args() {
   return *(const KernelArgs*)p;
 }
 
+// A lane index that the compiler takes as new: addresses formed from it stay
+// inside the loop body that they are used in, instead of in (spilled) registers
+// outside.
+__device__ __forceinline__ int fresh_lane(int i) {
+  asm volatile("" : "+v"(i));
+  return i;
+}
+
 __device__ __forceinline__ dcpx mk(double r, double i) { return dcpx{r, i}; }
 __device__ __forceinline__ dcpx cadd(dcpx a, dcpx b) { return mk(a.re + b.re, a.im + b.im); }
 __device__ __forceinline__ dcpx csub(dcpx a, dcpx b) { return mk(a.re - b.re, a.im - b.im); }
@@ -420,12 +428,11 @@ struct Tab<1> {
   }
 };
 
-// Stage input y + h * sum_j a_sj k_j (dopri5.rs:45-86) for stage S; S = 7 is
-// the solution.  Zero tableau entries are skipped at compile time.
+// sum_j a_sj k_j of stage S (dopri5.rs:45-86); zero tableau entries are
+// skipped at compile time.
 template <int R, int SOLVER, int S>
-__device__ __forceinline__ void stage_combo(double h, const double (&y_r)[R], const double (&y_i)[R],
-                                            const double (&k_r)[8][R], const double (&k_i)[8][R],
-                                            double (&o_r)[R], double (&o_i)[R]) {
+__device__ __forceinline__ void stage_sum(const double (&k_r)[8][R], const double (&k_i)[8][R], double (&s_r)[R],
+                                          double (&s_i)[R]) {
   using T = Tab<SOLVER>;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -437,8 +444,22 @@ __device__ __forceinline__ void stage_combo(double h, const double (&y_r)[R], co
         si = fma(T::a(S, j), k_i[j][r], si);
       }
     }
-    o_r[r] = fma(h, sr, y_r[r]);
-    o_i[r] = fma(h, si, y_i[r]);
+    s_r[r] = sr;
+    s_i[r] = si;
+  }
+}
+
+// Stage input y + h * sum_j a_sj k_j for stage S; S = 7 is the solution.
+template <int R, int SOLVER, int S>
+__device__ __forceinline__ void stage_combo(double h, const double (&y_r)[R], const double (&y_i)[R],
+                                            const double (&k_r)[8][R], const double (&k_i)[8][R],
+                                            double (&o_r)[R], double (&o_i)[R]) {
+  double s_r[R], s_i[R];
+  stage_sum<R, SOLVER, S>(k_r, k_i, s_r, s_i);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    o_r[r] = fma(h, s_r[r], y_r[r]);
+    o_i[r] = fma(h, s_i[r], y_i[r]);
   }
 }
 
@@ -1343,9 +1364,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         if (ns > C.maxiters) { status = LB_TRAJ_MAXITERS; fail_x = x; break; }
         bool clipped = false;
         if (replay) {
-          const KernelArgs& A = fresh_args();
-          const DevPlan& P = A.P;
-          const DevCall& C = A.C;
+          const DevCall& C = fresh_args().C;
           // recorded schedule: step sizes of a tape, every step accepted
           const int64_t nrep = C.replay_n[traj];
           if (accepted >= nrep || accepted >= C.tape_cap) { status = LB_TRAJ_CAPACITY; fail_x = x; break; }
@@ -1592,9 +1611,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
               if (trace) push(x, yn_r, yn_i, rate);
             }
           } else {
-            const KernelArgs& A = fresh_args();
-            const DevPlan& P = A.P;
-            const DevCall& C = A.C;
+            const DevCall& C = fresh_args().C;
             // save plan points inside (xo, x], or up to the root (dopri5.rs:318-344)
             const double tb = ev_hit ? te : x;
             while (si < C.n_saveat && C.saveat[si] <= tb + time_tol(tb)) {
@@ -3670,6 +3687,676 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_adjoint_kernel(const DevPlan P
 }
 
 // ---------------------------------------------------------------------------
+// Discrete adjoint over couplings, any plan size (lb_adjoint_kernel's sweep).
+//
+// The same derivative with the terms arranged as the solve has them.  A
+// reverse stage publishes kappa and the stage input once; mu = A^T kappa of an
+// element is its transposed couplings (4 FMAs each, lb_device.h), and the
+// parameter and time contractions sum conj(kappa) x over the couplings of one
+// entry first -- chunks of at most LB_Q_CHUNK couplings, one lane each -- and
+// meet the entry's derivatives once per chunk, not once per term.  The self
+// terms' coefficients do not depend on time, so their contraction is summed
+// over the whole trajectory and meets the derivatives at its end.  The
+// recomputation takes k1 of an attempt from the attempt before it (FSAL; a
+// rejected attempt leaves it), and alternates the kappa and input buffers, so
+// a stage has one barrier.  What the sweep needs of an attempt are its start,
+// the stages' sums sum_j a_sj k_j (inputs and inner products) and the error
+// sum, so the workspace holds these in place of k1..k7 and a reverse stage
+// reads one of them, fetched while the stage after it runs.
+// Bound by the latency of a stage (publish, barrier, rows, barrier), seven of
+// them and a step of recomputation an attempt.  The reverse stages share one
+// site: unrolled, with the parameter loop inside, 575 registers spilled.
+// 64 gradients at 72 levels (one slot a lane, 8 waves): 282 -> 72 ms.
+// ---------------------------------------------------------------------------
+namespace {
+
+// a(i, i - l) of stages 1..6, the columns in which a reverse stage hands its mu
+// on; read with a uniform index.
+#define LB_LAG(n, i, l) ((i) > (l) ? Tab<n>::a(i, (i) > (l) ? (i) - (l) : 1) : 0.0)
+#define LB_LAGS(n, i) {LB_LAG(n, i, 1), LB_LAG(n, i, 2), LB_LAG(n, i, 3), LB_LAG(n, i, 4), LB_LAG(n, i, 5), 0.0}
+__constant__ double kLag[2][6][6] = {
+    {LB_LAGS(0, 1), LB_LAGS(0, 2), LB_LAGS(0, 3), LB_LAGS(0, 4), LB_LAGS(0, 5), LB_LAGS(0, 6)},
+    {LB_LAGS(1, 1), LB_LAGS(1, 2), LB_LAGS(1, 3), LB_LAGS(1, 4), LB_LAGS(1, 5), LB_LAGS(1, 6)}};
+#undef LB_LAGS
+#undef LB_LAG
+
+struct LdsAdjB {
+  char* pub;      // n_pub published stage inputs
+  char* kap;      // S + 1 published kappa by slot, the last one zero
+  dcpx* ent;      // nv_stat, then 7 x nv_dyn entry values (stages 1..7)
+  dcpx* coef;     // 7 rows x (KD + 1), stage s at row s - 1; row 0 also t0
+  dcpx* slots;    // 7 x va_slots
+  dcpx* vm;       // vm_depth
+  DevVOp* vops;   // v_steps_all x LB_VOP_LANES
+  double2* ef;    // definitions of the first nv_def entries
+  uint32_t* ecoef;
+  int* eptr;
+  double* wts;
+  double* red;    // LB_MAX_DIFF x 16
+  uint32_t *cw, *tw, *qw, *qe;  // coupling words, transposed, contractions and their entries
+  int* misc;
+};
+
+__device__ __forceinline__ LdsAdjB carve_adj_block(const DevPlan& P) {
+  extern __shared__ double smem[];
+  char* const base = reinterpret_cast<char*>(smem);
+  const LbLdsAdj l = lb_lds_adj(P);
+  LdsAdjB L;
+  L.pub = base + l.pub;
+  L.kap = base + l.kap;
+  L.ent = reinterpret_cast<dcpx*>(base + l.ent);
+  L.coef = reinterpret_cast<dcpx*>(base + l.coef);
+  L.slots = reinterpret_cast<dcpx*>(base + l.slots);
+  L.vm = reinterpret_cast<dcpx*>(base + l.vm);
+  L.vops = reinterpret_cast<DevVOp*>(base + l.vops);
+  L.ef = reinterpret_cast<double2*>(base + l.ef);
+  L.ecoef = reinterpret_cast<uint32_t*>(base + l.ecoef);
+  L.eptr = reinterpret_cast<int*>(base + l.eptr);
+  L.wts = reinterpret_cast<double*>(base + l.wts);
+  L.red = reinterpret_cast<double*>(base + l.red);
+  L.cw = reinterpret_cast<uint32_t*>(base + l.cw);
+  L.tw = reinterpret_cast<uint32_t*>(base + l.tw);
+  L.qw = reinterpret_cast<uint32_t*>(base + l.qw);
+  L.qe = reinterpret_cast<uint32_t*>(base + l.qe);
+  L.misc = reinterpret_cast<int*>(base + l.misc);
+  return L;
+}
+
+// One transposed coupling: mu += the pullback of kappa_o = v x (or v conj(x)).
+__device__ __forceinline__ void couple_back(uint32_t sign, double2 v, double2 k, double& mr, double& mi) {
+  mr = fma(k.y, v.y, fma(k.x, v.x, mr));
+  const double t = fma(k.y, v.x, -(k.x * v.y));  // d/d Im x of a plain input
+  mi += __hiloint2double(__double2hiint(t) ^ (int)sign, __double2loint(t));
+}
+
+template <int N, typename WordPtr>
+__device__ __forceinline__ void couple_back_rows(WordPtr tw, const char* kap, const char* ent, uint32_t dyn,
+                                                 double& mr, double& mi) {
+  uint32_t w[N];
+  double2 k[N], v[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) w[j] = tw[64 * j];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    k[j] = *reinterpret_cast<const double2*>(kap + (w[j] >> 16));
+    v[j] = *reinterpret_cast<const double2*>(ent + ((w[j] & 0xFFF0u) + (w[j] & 1u) * dyn));
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) couple_back((w[j] << 30) & 0x80000000u, v[j], k[j], mr, mi);
+}
+
+template <typename WordPtr>
+__device__ __forceinline__ void couple_back_block(WordPtr tw, int rows, const char* kap, const char* ent, uint32_t dyn,
+                                                  double& mr, double& mi) {
+  int j = 0;
+  for (; j + 4 <= rows; j += 4) couple_back_rows<4>(tw + 64 * j, kap, ent, dyn, mr, mi);
+  if (rows & 2) {
+    couple_back_rows<2>(tw + 64 * j, kap, ent, dyn, mr, mi);
+    j += 2;
+  }
+  if (rows & 1) couple_back_rows<1>(tw + 64 * j, kap, ent, dyn, mr, mi);
+}
+
+// The contractions of one stage: chunk `ch` of entry e sums conj(kappa) x over
+// its couplings and adds Re(q f d') of every term of the entry, d' the
+// derivatives of its coefficient (row `cf`: the values, the constant 1, then
+// d c_k / d p_m at K + 1 + k nd + m, the time column last).
+template <typename WordPtr>
+__device__ __forceinline__ void contract_entries(const DevPlan& P, const LdsAdjB& L, WordPtr qw, WordPtr qe, const dcpx* cf,
+                                                 int tid, int W, double (&g)[LB_MAX_DIFF], double& tc) {
+  const int nd = P.n_diff, np = P.n_diff - P.diff_time;
+  const dcpx* dc = cf + P.K + 1;
+  for (int ch = tid; ch < P.q_chunks; ch += W) {
+    const uint32_t e = qe[ch];
+    if (e == 0xFFFFFFFFu) continue;
+    double qr = 0.0, qi = 0.0;
+    for (int j0 = 0; j0 < LB_Q_CHUNK; j0 += 4) {
+      uint32_t w[4];
+      double2 k[4], x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = qw[(j0 + j) * P.q_chunks + ch];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        k[j] = *reinterpret_cast<const double2*>(L.kap + (w[j] >> 16));
+        x[j] = *reinterpret_cast<const double2*>(L.pub + (w[j] & 0xFFF0u));
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {  // conj(kappa) x, x conjugated by its sign bit
+        const double xi = __hiloint2double(__double2hiint(x[j].y) ^ (int)((w[j] << 30) & 0x80000000u),
+                                           __double2loint(x[j].y));
+        qr = fma(k[j].y, xi, fma(k[j].x, x[j].x, qr));
+        qi = fma(-k[j].y, x[j].x, fma(k[j].x, xi, qi));
+      }
+    }
+    const int t1 = L.eptr[e + 1];
+    for (int t = L.eptr[e]; t < t1; ++t) {
+      const uint32_t id = L.ecoef[t], k = id & 0x7FFFFFFFu;
+      if (k == (uint32_t)P.K) continue;
+      const double2 f = L.ef[t];
+      const double zr = fma(qr, f.x, -(qi * f.y));
+      double zi = fma(qr, f.y, qi * f.x);
+      zi = (id & 0x80000000u) ? -zi : zi;  // Re(z conj(d)) = Re(conj(z) d)
+      const dcpx* dk = dc + k * nd;
+#pragma unroll
+      for (int m = 0; m < LB_MAX_DIFF; ++m) {
+        if (m >= np) break;
+        const dcpx d = dk[m];
+        g[m] = fma(-zi, d.im, fma(zr, d.re, g[m]));
+      }
+      if (P.diff_time) {
+        const dcpx d = dk[np];
+        tc = fma(-zi, d.im, fma(zr, d.re, tc));
+      }
+    }
+  }
+}
+
+}  // namespace
+
+template <int R, int SOLVER, int MAXW, int WAVES>
+__global__ __launch_bounds__(MAXW, WAVES) void lb_adjoint_block_kernel(const DevPlan P, const DevCall C) {
+  using T = Tab<SOLVER>;
+  const int thread = threadIdx.x, W = blockDim.x;
+  const int wave = __builtin_amdgcn_readfirstlane(thread >> 6);
+  const LdsAdjB L = carve_adj_block(P);
+  const int KC = P.KD + 1, nd = P.n_diff, np = P.n_diff - P.diff_time;
+  const bool adaptive = C.adj_mode == LB_ADJOINT_ADAPTIVE;
+  const double dimf = (double)P.dim;
+  Slots<R> S;
+  load_slots<R>(P, S, thread, W);
+  {
+  const int tid = thread;
+  for (int i = tid; i < P.v_steps_all * LB_VOP_LANES; i += W) L.vops[i] = P.v_ops_all[i];
+  for (int i = tid; i < P.nv_def_terms; i += W) {
+    L.ef[i] = reinterpret_cast<const double2*>(P.ent_f)[i];
+    L.ecoef[i] = P.ent_coef[i];
+  }
+  for (int i = tid; i <= P.nv_def; i += W) L.eptr[i] = P.ent_ptr[i];
+  if (P.adj_lds & 1)
+    for (int i = tid; i < P.c_rows_total * 64; i += W) L.cw[i] = P.c_word[i];
+  if (P.adj_lds & 2)
+    for (int i = tid; i < P.tc_rows_total * 64; i += W) L.tw[i] = P.tc_word[i];
+  if (P.adj_lds & 4) {
+    for (int i = tid; i < P.q_chunks * LB_Q_CHUNK; i += W) L.qw[i] = P.q_word[i];
+    for (int i = tid; i < P.q_chunks; i += W) L.qe[i] = P.q_ent[i];
+  }
+  if (tid == 0) reinterpret_cast<double2*>(L.kap)[P.S] = double2{0.0, 0.0};
+  }
+  const int every = C.ckpt_every;
+  // workspace per attempt: [0] y, [1] sum e_j k_j, [s] the sum of stage s =
+  // 2..7 (8 x S complex), 7 coefficient rows
+  double2* const segY = reinterpret_cast<double2*>(C.seg_y) + (size_t)blockIdx.x * every * 8 * P.S;
+  dcpx* const segC = reinterpret_cast<dcpx*>(C.seg_c) + (size_t)blockIdx.x * every * 7 * KC;
+  const int64_t ncap = (C.tape_cap + every - 1) / every;
+
+  for (;;) {
+    __syncthreads();
+    if (thread == 0) L.misc[0] = atomicAdd(C.queue, 1);
+    __syncthreads();
+    const int64_t local = L.misc[0];
+    if (local >= C.n_traj) break;
+    // queue position -> trajectory (longest-first orders); entries outside
+    // the batch are skipped, so a bad order cannot address past the arrays
+    const int64_t traj = C.queue_order ? (int64_t)C.queue_order[local + C.traj_offset] : local + C.traj_offset;
+    if (traj < 0 || traj >= C.n_total) continue;
+
+    double2 sv[R];
+    {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
+      const LdsAdjB L = carve_adj_block(P);
+      const int tid = fresh_lane(thread);
+      // ---- parameters, coefficients at t0, entries and self folds, weights
+      for (int i = tid; i < P.n_slots; i += W)
+        L.slots[i] = i < P.n_base ? mk(P.base[2 * i], P.base[2 * i + 1]) : mk(0.0, 0.0);
+      for (int i = tid; i < P.va_n_const; i += W)
+        L.slots[P.va_const_slot[i]] = mk(P.va_const[2 * i], P.va_const[2 * i + 1]);
+      __syncthreads();
+      if (tid == 0) {
+        apply_overrides(C, traj, L.slots);
+        eval_coefficients(P, L.slots, L.coef, C.t0, false, L.vm, P.KD);
+      }
+      for (int i = tid; i < P.n; i += W) {
+        double w = 0.0;
+        for (int q = 0; q < C.n_weights; ++q)
+          if (C.weight_index[q] == i) w += C.weight_value[q];
+        L.wts[i] = w;
+      }
+      __syncthreads();
+      // the other stage rows start as the t0 row: each step rewrites only the
+      // time-dependent entries
+      for (int i = tid; i < 6 * P.va_slots; i += W) L.slots[P.va_slots + i] = L.slots[i % P.va_slots];
+      for (int i = tid; i < 6 * KC; i += W) L.coef[KC + i] = L.coef[i % KC];
+      fill_static_entries(P, L.coef, L.ent, tid, W);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int s = tid + W * r;
+        dcpx acc = mk(0.0, 0.0);
+        for (int j = 0; s < P.S && j < P.max_self; ++j) {
+          const size_t e = (size_t)s * P.max_self + j;
+          const int id = P.self_coef[e];
+          if (id == -2) break;
+          dcpx c = id < 0 ? mk(1.0, 0.0) : L.coef[id];
+          if (P.self_conj[e]) c.im = -c.im;
+          acc = cadd(acc, cmul(mk(P.self_f[2 * e], P.self_f[2 * e + 1]), c));
+        }
+        sv[r] = double2{acc.re, acc.im};
+      }
+      __syncthreads();
+    }
+
+    double g[LB_MAX_DIFF];
+#pragma unroll
+    for (int m = 0; m < LB_MAX_DIFF; ++m) g[m] = 0.0;
+    // conj(kappa) x of the self terms, over the trajectory
+    double sq_r[R], sq_i[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) sq_r[r] = sq_i[r] = 0.0;
+    const int N = C.tape_n[traj];
+    const bool ok = N > 0 && N <= C.tape_cap;
+    if (ok) {
+      const double* tt = C.tape_t + traj * C.tape_cap;
+      const double* th = C.tape_h + traj * C.tape_cap;
+      const double* tcr = C.tape_c + traj * C.tape_cap * 3;
+      const int32_t* tfl = C.tape_f + traj * C.tape_cap;
+      double wme[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) wme[r] = (S.valid(r) && S.diag(r)) ? L.wts[S.state(r)] : 0.0;
+      // cotangents: lam of the state at the start of the current step; Tb of
+      // its start time; Hb of the step size proposed into the attempt after
+      // the current one (before its clip); Qb of fac_old after the current
+      // step
+      double lam_r[R], lam_i[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) { lam_r[r] = 0.0; lam_i[r] = 0.0; }
+      double Tb = 0.0, Hb = 0.0, Qb = 0.0;
+      const int nseg = (N + every - 1) / every;
+      for (int sg = nseg - 1; sg >= 0; --sg) {
+        const int a0 = sg * every, a1 = min(a0 + every, N);
+        // ---- recompute the segment from its checkpoint
+        {
+        double y_r[R], y_i[R], k_r[8][R], k_i[8][R];
+        {
+          const double2* ck = reinterpret_cast<const double2*>(C.tape_y) + (traj * ncap + sg) * P.S;
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            const int s = thread + W * r;
+            const double2 v = s < P.S ? ck[s] : double2{0.0, 0.0};
+            y_r[r] = v.x;
+            y_i[r] = v.y;
+          }
+        }
+        bool flip = false;  // publication buffer of the next stage
+        for (int a = a0; a < a1; ++a) {
+          const KernelArgs& A = fresh_args();
+          const DevPlan& P = A.P;
+          const LdsAdjB L = carve_adj_block(P);
+          const int tid = fresh_lane(thread), lane = tid & 63;
+          const char* const ent = reinterpret_cast<const char*>(L.ent);
+            auto forward = [&](const char* pb, int vrow, const double2 (&sv)[R], const double (&xr)[R], const double (&xi)[R],
+                               double (&kr)[R], double (&ki)[R]) {
+              const uint32_t dyn = 16u * (uint32_t)(vrow * P.nv_dyn);
+#pragma unroll
+              for (int r = 0; r < R; ++r) {
+                const int blk = wave + (W >> 6) * r;
+                kr[r] = ki[r] = 0.0;
+                if (blk >= P.nblk) continue;
+                double ar = fma(sv[r].x, xr[r], -(sv[r].y * xi[r])), ai = fma(sv[r].x, xi[r], sv[r].y * xr[r]);
+                const int row0 = cst(P.c_row0)[blk], rows = cst(P.c_rows)[blk];
+                if (P.adj_lds & 1)
+                  couple_block(static_cast<const uint32_t*>(L.cw) + (row0 * 64 + lane), rows, pb, ent, dyn, ar, ai);
+                else
+                  couple_block(P.c_word + ((size_t)row0 * 64 + lane), rows, pb, ent, dyn, ar, ai);
+                kr[r] = ar;
+                ki[r] = S.diag(r) ? 0.0 : ai;
+              }
+            };
+            auto publish = [&](char* buf, const double (&xr)[R], const double (&xi)[R]) {
+#pragma unroll
+              for (int r = 0; r < R; ++r)
+                if (S.pub[r] >= 0) reinterpret_cast<double2*>(buf)[S.pub[r]] = double2{xr[r], xi[r]};
+            };
+          const double h = th[a];
+          __syncthreads();  // the previous attempt's coefficient and entry rows are read
+          if (tid < 64 && P.time_dependent) {
+            const int row = min(lane & 7, 6);
+            vector_eval(L.vops, P.v_steps_all, L.slots + row * P.va_slots, L.coef + row * KC, P.va_time,
+                        row == 0 ? tt[a] : tt[a] + h * T::c(row + 1), lane, (lane & 7) < 7);
+          }
+          double2* const wk = segY + (size_t)(a - a0) * 8 * P.S;
+          auto keep = [&](int j, const double (&vr)[R], const double (&vi)[R]) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              const int s = tid + W * r;
+              if (s < P.S) wk[(size_t)j * P.S + s] = double2{vr[r], vi[r]};
+            }
+          };
+          keep(0, y_r, y_i);
+          __syncthreads();
+          for (int q = tid; q < 7 * KC; q += W) segC[(size_t)(a - a0) * 7 * KC + q] = L.coef[q];
+          fill_entries<7>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef, KC, L.ent + P.nv_stat, tid, W);
+          double yt_r[R], yt_i[R];
+          if (a == a0) {
+            char* const b = flip ? L.kap : L.pub;
+            flip = !flip;
+            publish(b, y_r, y_i);
+            __syncthreads();
+            forward(b, 0, sv, y_r, y_i, k_r[1], k_i[1]);
+          }
+#define LB_ADJ_FWD(st)                                                     \
+  {                                                                        \
+    stage_sum<R, SOLVER, st>(k_r, k_i, yt_r, yt_i);                        \
+    keep(st, yt_r, yt_i);                                                  \
+    _Pragma("unroll") for (int r = 0; r < R; ++r) {                        \
+      yt_r[r] = fma(h, yt_r[r], y_r[r]);                                   \
+      yt_i[r] = fma(h, yt_i[r], y_i[r]);                                   \
+    }                                                                      \
+    char* const b = flip ? L.kap : L.pub;                                  \
+    flip = !flip;                                                          \
+    publish(b, yt_r, yt_i);                                                \
+    __syncthreads();                                                       \
+    forward(b, (st) - 1, sv, yt_r, yt_i, k_r[st], k_i[st]);                \
+  }
+          LB_ADJ_FWD(2)
+          LB_ADJ_FWD(3)
+          LB_ADJ_FWD(4)
+          LB_ADJ_FWD(5)
+          LB_ADJ_FWD(6)
+          LB_ADJ_FWD(7)
+#undef LB_ADJ_FWD
+          {
+            double se_r[R], se_i[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              se_r[r] = T::e(1) * k_r[1][r];
+              se_i[r] = T::e(1) * k_i[1][r];
+#pragma unroll
+              for (int j = 2; j <= 7; ++j) {
+                if (T::e(j) != 0.0) {
+                  se_r[r] = fma(T::e(j), k_r[j][r], se_r[r]);
+                  se_i[r] = fma(T::e(j), k_i[j][r], se_i[r]);
+                }
+              }
+            }
+            keep(1, se_r, se_i);
+          }
+          if (tfl[a] & LB_TAPE_ACCEPTED) {
+            // stage_combo<7> left the candidate solution in yt, k7 is its derivative
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              y_r[r] = yt_r[r];
+              y_i[r] = yt_i[r];
+              k_r[1][r] = k_r[7][r];
+              k_i[1][r] = k_i[7][r];
+            }
+          }
+        }
+        }
+        // ---- reverse sweep over the segment's attempts, last first
+        for (int a = a1 - 1; a >= a0; --a) {
+          const int fl = tfl[a];
+          const bool acc = (fl & LB_TAPE_ACCEPTED) != 0;
+          if (!adaptive && !acc) continue;
+          const double h = th[a];
+          double hb = 0.0, errb = 0.0, qnew = Qb;
+          if (adaptive) {
+            double dh, de, dq;
+            ctrl_partials(fl, h, tcr[3 * a], tcr[3 * a + 1], tcr[3 * a + 2], dh, de, dq);
+            if (acc) {
+              errb = Hb * de + ((fl & LB_TAPE_ERRQ) ? Qb : 0.0);
+              hb = Hb * dh + Tb;
+              qnew = Hb * dq;
+            } else {
+              errb = Hb * de;
+              hb = Hb * dh;
+            }
+            // a rejected attempt whose proposal nothing downstream depends on
+            if (!acc && errb == 0.0 && hb == 0.0) {
+              if (fl & LB_TAPE_CLIPPED) Hb = 0.0;
+              continue;
+            }
+          }
+          const KernelArgs& A = fresh_args();
+          const DevPlan& P = A.P;
+          const DevCall& C = A.C;
+          const LdsAdjB L = carve_adj_block(P);
+          const int tid = fresh_lane(thread), lane = tid & 63;
+          const char* const ent = reinterpret_cast<const char*>(L.ent);
+            auto back = [&](int vrow, const double2 (&sv)[R], const double (&kr)[R], const double (&ki)[R], double (&mr)[R],
+                            double (&mi)[R]) {
+              const uint32_t dyn = 16u * (uint32_t)(vrow * P.nv_dyn);
+#pragma unroll
+              for (int r = 0; r < R; ++r) {
+                const int blk = wave + (W >> 6) * r;
+                mr[r] = mi[r] = 0.0;
+                if (blk >= P.nblk) continue;
+                // self: conj(kappa) a
+                double ar = fma(kr[r], sv[r].x, ki[r] * sv[r].y), ai = fma(ki[r], sv[r].x, -(kr[r] * sv[r].y));
+                const int row0 = cst(P.tc_row0)[blk], rows = cst(P.tc_rows)[blk];
+                if (P.adj_lds & 2)
+                  couple_back_block(static_cast<const uint32_t*>(L.tw) + (row0 * 64 + lane), rows, L.kap, ent, dyn, ar, ai);
+                else
+                  couple_back_block(P.tc_word + ((size_t)row0 * 64 + lane), rows, L.kap, ent, dyn, ar, ai);
+                mr[r] = ar;
+                mi[r] = S.diag(r) ? 0.0 : ai;
+              }
+            };
+            auto publish = [&](char* buf, const double (&xr)[R], const double (&xi)[R]) {
+#pragma unroll
+              for (int r = 0; r < R; ++r)
+                if (S.pub[r] >= 0) reinterpret_cast<double2*>(buf)[S.pub[r]] = double2{xr[r], xi[r]};
+            };
+          const double2* const wk = segY + (size_t)(a - a0) * 8 * P.S;
+          double y_r[R], y_i[R], sb_r[R], sb_i[R], se_r[R], se_i[R], pn_r[R], pn_i[R];
+          auto fetch = [&](int j, double (&vr)[R], double (&vi)[R]) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              const int s = tid + W * r;
+              const double2 v = s < P.S ? wk[(size_t)j * P.S + s] : double2{0.0, 0.0};
+              vr[r] = v.x;
+              vi[r] = v.y;
+            }
+          };
+          fetch(0, y_r, y_i);
+          fetch(1, se_r, se_i);
+          fetch(7, sb_r, sb_i);
+          fetch(6, pn_r, pn_i);
+          __syncthreads();
+          for (int q = tid; q < 7 * KC; q += W) L.coef[q] = segC[(size_t)(a - a0) * 7 * KC + q];
+          __syncthreads();
+          fill_entries<7>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef, KC, L.ent + P.nv_stat, tid, W);
+          // lambda (cotangent of the candidate), ybar (of the start state),
+          // nu (of the error estimate), per-lane h and t cotangent pieces;
+          // sb = sum b_j k_j, se = sum e_j k_j
+          double yn_r[R], yn_i[R], lr[R], li[R], ybr[R], ybi[R], nur[R], nui[R];
+          double hbl = 0.0, tbl = 0.0;
+          const bool trap = acc && (!(fl & LB_TAPE_FIRST) || C.save_start);
+          const double err = tcr[3 * a];
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            yn_r[r] = fma(h, sb_r[r], y_r[r]);
+            yn_i[r] = fma(h, sb_i[r], y_i[r]);
+            lr[r] = acc ? lam_r[r] : 0.0;
+            li[r] = acc ? lam_i[r] : 0.0;
+            ybr[r] = ybi[r] = nur[r] = nui[r] = 0.0;
+            if (trap) {
+              // 0.5 (v_n + v_{n+1}) h with v = w . y
+              lr[r] += 0.5 * h * wme[r];
+              ybr[r] += 0.5 * h * wme[r];
+              hbl += 0.5 * wme[r] * (y_r[r] + yn_r[r]);
+            }
+            if (errb != 0.0 && S.valid(r)) {
+              err_component(errb, err, dimf, C.abstol, C.reltol, se_r[r] * h, y_r[r], yn_r[r], nur[r], ybr[r], lr[r]);
+              if (!S.diag(r))
+                err_component(errb, err, dimf, C.abstol, C.reltol, se_i[r] * h, y_i[r], yn_i[r], nui[r], ybi[r], li[r]);
+            }
+          }
+          // Stages 7 (k7 = f(x + h, yn), which enters the error estimate only),
+          // 6 .. 1 at one site.  ka[5] collects the next stage's kappa / h, the
+          // ones below it those of the stages after; a stage adds its mu to
+          // each with the tableau's column.  sr becomes the start's cotangent:
+          // ybar + lambda' + sum mu, lambda' = lambda + mu_7.
+          // dI/dh through the explicit h: lambda' . sum b_j k_j + nu . sum e_j
+          // k_j, and mu_i . sum_{j<i} a_ij k_j of each stage.
+          double ka_r[6][R], ka_i[6][R], sr[R], si[R];
+          auto start_stages = [&]() {  // from stage 7: lr, li hold lambda'
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              hbl += lr[r] * sb_r[r] + li[r] * sb_i[r] + nur[r] * se_r[r] + nui[r] * se_i[r];
+              sr[r] = ybr[r] + lr[r];
+              si[r] = ybi[r] + li[r];
+#pragma unroll
+              for (int j = 1; j <= 6; ++j) {
+                ka_r[j - 1][r] = T::a(7, j) * lr[r] + T::e(j) * nur[r];
+                ka_i[j - 1][r] = T::a(7, j) * li[r] + T::e(j) * nui[r];
+              }
+            }
+          };
+#pragma unroll 1
+          for (int i = 7; i >= 1; --i) {
+            double kr[R], ki[R], yr[R], yi[R], pr[R], pi[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              pr[r] = pi[r] = 0.0;
+              if (i == 7) {
+                kr[r] = T::e(7) * nur[r];
+                ki[r] = T::e(7) * nui[r];
+                yr[r] = yn_r[r];
+                yi[r] = yn_i[r];
+              } else {
+                if (i > 1) {
+                  pr[r] = pn_r[r];
+                  pi[r] = pn_i[r];
+                }
+                kr[r] = ka_r[5][r];
+                ki[r] = ka_i[5][r];
+                yr[r] = fma(h, pr[r], y_r[r]);
+                yi[r] = fma(h, pi[r], y_i[r]);
+              }
+              kr[r] *= h;
+              ki[r] = S.diag(r) ? 0.0 : h * ki[r];
+            }
+            if (i > 2 && i < 7) fetch(i - 1, pn_r, pn_i);
+            double mr[R], mi[R], tci = 0.0;
+#pragma unroll
+            for (int r = 0; r < R; ++r) mr[r] = mi[r] = 0.0;
+            if (i < 7 || errb != 0.0) {
+              // publish kappa and the stage input, mu = A^T kappa
+              publish(L.pub, yr, yi);
+#pragma unroll
+              for (int r = 0; r < R; ++r) {
+                const int s = tid + W * r;
+                if (s < P.S) reinterpret_cast<double2*>(L.kap)[s] = double2{kr[r], ki[r]};
+                sq_r[r] = fma(ki[r], yi[r], fma(kr[r], yr[r], sq_r[r]));
+                sq_i[r] = fma(-ki[r], yr[r], fma(kr[r], yi[r], sq_i[r]));
+              }
+              __syncthreads();
+              back(i - 1, sv, kr, ki, mr, mi);
+              if (P.adj_lds & 4)
+                contract_entries(P, L, static_cast<const uint32_t*>(L.qw), static_cast<const uint32_t*>(L.qe),
+                                 L.coef + (i - 1) * KC, tid, W, g, tci);
+              else
+                contract_entries(P, L, P.q_word, P.q_ent, L.coef + (i - 1) * KC, tid, W, g, tci);
+              __syncthreads();
+            }
+            tbl += tci;
+            if (i == 7) {
+              hbl += tci;  // c_7 = 1
+#pragma unroll
+              for (int r = 0; r < R; ++r) {
+                lr[r] += mr[r];
+                li[r] = S.diag(r) ? 0.0 : li[r] + mi[r];
+              }
+              start_stages();
+              continue;
+            }
+            hbl += T::c(i) * tci;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              hbl += mr[r] * pr[r] + mi[r] * pi[r];
+              sr[r] += mr[r];
+              si[r] += mi[r];
+#pragma unroll
+              for (int j = 5; j >= 1; --j) {  // the stage j - 5 + i - 1
+                const double c = kLag[SOLVER][i - 1][5 - j];
+                ka_r[j][r] = fma(c, mr[r], ka_r[j - 1][r]);
+                ka_i[j][r] = fma(c, mi[r], ka_i[j - 1][r]);
+              }
+            }
+          }
+          if (adaptive) {
+            hb += group_sum(hbl, L.red, tid, W);
+            Tb += group_sum(tbl, L.red, tid, W);
+            if (fl & LB_TAPE_CLIPPED) {
+              Tb -= hb;
+              Hb = 0.0;
+            } else {
+              Hb = hb;
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            lam_r[r] = acc ? sr[r] : lam_r[r] + sr[r];
+            lam_i[r] = S.diag(r) ? 0.0 : (acc ? si[r] : lam_i[r] + si[r]);
+          }
+          if (acc) Qb = qnew;
+        }
+      }
+      {
+        const KernelArgs& A = fresh_args();
+        const DevPlan& P = A.P;
+        const LdsAdjB L = carve_adj_block(P);
+        const int tid = fresh_lane(thread);
+        // the self terms: conj(kappa) x over the trajectory meets the
+        // derivatives of the folded coefficients
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int s = tid + W * r;
+          for (int j = 0; s < P.S && j < P.max_self; ++j) {
+            const size_t e = (size_t)s * P.max_self + j;
+            const int id = P.self_coef[e];
+            if (id == -2) break;
+            if (id < 0) continue;
+            const dcpx z = cmul(mk(sq_r[r], sq_i[r]), mk(P.self_f[2 * e], P.self_f[2 * e + 1]));
+            const double zi = P.self_conj[e] ? -z.im : z.im;
+            for (int m = 0; m < LB_MAX_DIFF; ++m) {
+              if (m >= np) break;
+              const dcpx d = L.coef[P.K + 1 + id * nd + m];
+              g[m] += z.re * d.re - zi * d.im;
+            }
+          }
+        }
+      }
+    }
+    {
+      const KernelArgs& A = fresh_args();
+      const DevPlan& P = A.P;
+      const DevCall& C = A.C;
+      const LdsAdjB L = carve_adj_block(P);
+      const int tid = fresh_lane(thread);
+      // ---- dI/dp: one block reduction per parameter
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < LB_MAX_DIFF; ++m) {
+        if (m >= np) break;
+        const double v = wave_sum(g[m]);
+        if ((tid & 63) == 0) L.red[m * 16 + (tid >> 6)] = v;
+      }
+      __syncthreads();
+      if (tid == 0) {
+        const int nw = W >> 6;
+        for (int m = 0; m < np; ++m) {
+          double tot = 0.0;
+          for (int b = 0; b < nw; ++b) tot += L.red[m * 16 + b];
+          C.out_grad[traj * np + m] = ok ? tot : __builtin_nan("");
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Adjoint for plans of one 64-slot block (lane = slot), several waves per
 // trajectory.
 //
@@ -4883,6 +5570,14 @@ void* adjoint_ptr(int solver) {
     return nullptr;
 }
 template <int I, int RR, int WW, int VV>
+void* adjoint_block_ptr(int solver) {
+  if constexpr (I % LB_NPART == LB_PART)
+    return solver == 1 ? (void*)&lb_adjoint_block_kernel<RR, 1, WW, VV>
+                       : (void*)&lb_adjoint_block_kernel<RR, 0, WW, VV>;
+  else
+    return nullptr;
+}
+template <int I, int RR, int WW, int VV>
 void* fixed_ptr(int solver) {
   if constexpr (I % LB_NPART == LB_PART)
     return solver == 2 ? (void*)&lb_fixed_kernel<RR, 0, WW, VV>
@@ -4989,6 +5684,14 @@ extern "C" void* LB_PART_FN(lb_dev_adjoint_kernel)(int id, int solver) {
   if (id == i) return adjoint_wave_ptr<i, g, v>(solver);
   LB_ADJ_WAVE_CONFIGS(V)
 #undef V
+  return nullptr;
+}
+
+extern "C" void* LB_PART_FN(lb_dev_adjoint_block_kernel)(int id, int solver) {
+#define B(i, r, w, v) \
+  if (id == i) return adjoint_block_ptr<i, r, w, v>(solver);
+  LB_ADJ_BLOCK_CONFIGS(B)
+#undef B
   return nullptr;
 }
 

@@ -42,6 +42,14 @@ extern "C" void* lb_dev_adjoint_kernel_p4(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p5(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p6(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p7(int, int);
+extern "C" void* lb_dev_adjoint_block_kernel_p0(int, int);
+extern "C" void* lb_dev_adjoint_block_kernel_p1(int, int);
+extern "C" void* lb_dev_adjoint_block_kernel_p2(int, int);
+extern "C" void* lb_dev_adjoint_block_kernel_p3(int, int);
+extern "C" void* lb_dev_adjoint_block_kernel_p4(int, int);
+extern "C" void* lb_dev_adjoint_block_kernel_p5(int, int);
+extern "C" void* lb_dev_adjoint_block_kernel_p6(int, int);
+extern "C" void* lb_dev_adjoint_block_kernel_p7(int, int);
 extern "C" void* lb_dev_rhs_kernel_p0(int);
 extern "C" void* lb_dev_rhs_kernel_p1(int);
 extern "C" void* lb_dev_rhs_kernel_p2(int);
@@ -174,4 +182,18 @@ extern "C" void* lb_dev_event_kernel(int id, int solver) {
 extern "C" void* lb_dev_fixed_kernel(int id, int solver) {
   void* (*parts[])(int, int) = {lb_dev_fixed_kernel_p0, lb_dev_fixed_kernel_p1, lb_dev_fixed_kernel_p2, lb_dev_fixed_kernel_p3, lb_dev_fixed_kernel_p4, lb_dev_fixed_kernel_p5, lb_dev_fixed_kernel_p6, lb_dev_fixed_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);
+}
+
+// The block adjoint's shape of the fewest slots per lane that covers S slots
+// (and its workgroup size); null where none does.
+extern "C" void* lb_dev_adjoint_block_kernel(int S, int solver, int* W) {
+  void* (*parts[])(int, int) = {lb_dev_adjoint_block_kernel_p0, lb_dev_adjoint_block_kernel_p1, lb_dev_adjoint_block_kernel_p2, lb_dev_adjoint_block_kernel_p3, lb_dev_adjoint_block_kernel_p4, lb_dev_adjoint_block_kernel_p5, lb_dev_adjoint_block_kernel_p6, lb_dev_adjoint_block_kernel_p7};
+#define B(i, r, w, v)                              \
+  if (S <= (r) * (w)) {                            \
+    *W = ((S + (r) - 1) / (r) + 63) / 64 * 64;     \
+    return parts[(i) % LB_NPARTS_BUILT](i, solver); \
+  }
+  LB_ADJ_BLOCK_CONFIGS(B)
+#undef B
+  return nullptr;
 }

@@ -37,6 +37,11 @@
 // Adjoint kernel variants: Z(id, slots per thread R, largest workgroup, waves-per-SIMD hint).
 #define LB_ADJ_CONFIGS(Z) Z(0, 1, 1024, 2) Z(1, 2, 512, 2) Z(2, 4, 256, 2) Z(3, 8, 256, 2)
 
+// Multi-wave adjoint over couplings: B(id, slots per thread R, largest
+// workgroup, waves-per-SIMD hint).  Two waves a SIMD: with 128 registers (one
+// slot a lane, 1024 threads) three times as many values spilled.
+#define LB_ADJ_BLOCK_CONFIGS(B) B(4, 1, 512, 2) B(5, 2, 512, 2) B(6, 4, 512, 2)
+
 // Single-block adjoint variants for plans of one 64-slot block (lane = slot,
 // several waves per trajectory): V(id, gather rows held in registers by
 // the recomputation, waves-per-SIMD hint), in increasing rows (the host takes

@@ -372,15 +372,18 @@ struct DevEffPlan {
   int32_t S;                // D padded to a multiple of 64
   int32_t nblk;             // S / 64
   const double* grid;       // G
-  // Each operator in sliced form: the 64 rows of a wave are one slice, and
-  // entry j of a slice's rows lies at cell slice_ptr + 64 j + (row mod 64),
-  // so a wave's lanes read consecutive cells; rows keep their CSR order.
-  const int32_t* row_len[3];    // S (0 on padding rows)
-  const int64_t* slice_ptr[3];  // nblk
-  const int32_t* col[3];        // cells
-  const double2* coef_lo[3];    // (G - 1) x cells: (c0, c1) of the cubic
-  const double2* coef_hi[3];    // (G - 1) x cells: (c2, c3)
-  int64_t cells[3];
+  // The three operators in sliced form: 64 rows are one slice, position s
+  // holds row row[s] (rows in decreasing number of entries, so a slice's rows
+  // are of like length), and entry j of its operator o lies at cell
+  // slice_ptr[3 slice + o] + 64 j + (s mod 64), so a wave's lanes read
+  // consecutive cells; rows keep their CSR order.
+  const int32_t* row;        // S (-1 on padding)
+  const int32_t* row_len;    // 3 x S (0 on padding)
+  const int64_t* slice_ptr;  // 3 nblk + 1, operator after operator in a slice
+  const uint32_t* col;       // cells (0 on padding)
+  const double2* coef_lo;    // (G - 1) x cells: (c0, c1) of the cubic
+  const double2* coef_hi;    // (G - 1) x cells: (c2, c3)
+  int64_t cells;
   int32_t field_slot, rabi_slot, det_slot;
   int32_t n_slots, n_base, n_comp, vm_depth;
   const double* base;       // n_base x 2

@@ -2027,7 +2027,7 @@ extern "C" int lb_variant_info(int32_t id, int32_t* slots_per_thread, int32_t* m
 // solver.rs:78-281).
 // ===========================================================================
 
-extern "C" int lb_dev_eff_variant(int id, int* R, int* maxw);
+extern "C" int lb_dev_eff_variant(int id, int* R, int* maxw, int* seats);
 extern "C" void* lb_dev_eff_kernel(int id, int solver);
 extern "C" void* lb_dev_eff_rhs_kernel(int id);
 
@@ -2044,7 +2044,13 @@ struct lb_eff_plan {
 namespace {
 
 // Must match carve_eff() in lb_kernels.hip.
-int64_t lds_bytes_eff(const DevEffPlan& P) {
+int64_t lds_bytes_eff(const DevEffPlan& P, int64_t seats, int64_t stride) {
+  return seats * (8 * 2 * (seats > 1 ? stride : P.S) + 16 * 6 * (int64_t)P.n_slots + 16 * 6 * (int64_t)P.vm_depth +
+                  8 * 3 * (int64_t)P.nblk + 8 * 32 + 8 * 5 + 4 * 2);
+}
+
+// What a plan may ask of a workgroup's LDS.
+int64_t lds_bytes_eff_limit(const DevEffPlan& P) {
   return 8 * 2 * (int64_t)P.S + 16 * 8 * (int64_t)P.n_slots + 16 * 8 * (int64_t)P.vm_depth +
          8 * 4 * (int64_t)P.nblk + 8 * 32 + 8 * 2 + 4 * 4;
 }
@@ -2059,14 +2065,18 @@ int eff_upload(lb_eff_plan* p, const std::vector<T>& host, const T** out) {
   return LB_OK;
 }
 
-// The multi-wave variant with the fewest rows per lane that covers D rows.
-int eff_config(const DevEffPlan& P, int* id, int* W) {
-  int R = 0, maxw = 0;
-  for (int v = 0; lb_dev_eff_variant(v, &R, &maxw); ++v) {
+// The variant of at most `seats` seats with the most seats, then the fewest
+// rows per lane, that covers D rows.
+int eff_config(const DevEffPlan& P, int seats, int* id, int* W, int* T, size_t* lds) {
+  int R = 0, maxw = 0, t = 0;
+  for (int v = 0; lb_dev_eff_variant(v, &R, &maxw, &t); ++v) {
     const int w = std::max(64, ((P.D + R - 1) / R + 63) / 64 * 64);
-    if (w <= maxw && (int64_t)R * w >= P.D) {
+    const int64_t need = lds_bytes_eff(P, t, (int64_t)R * maxw);
+    if (t <= seats && w <= maxw && (int64_t)R * w >= P.D && (t == 1 || need <= kMaxLdsBytes)) {
+      *lds = (size_t)need;
       *id = v;
       *W = w;
+      *T = t;
       return LB_OK;
     }
   }
@@ -2099,60 +2109,75 @@ extern "C" int lb_eff_plan_create(const lb_eff_plan_desc* d, lb_eff_plan** out_p
   P.n_base = d->n_base;
   int rc;
   if ((rc = eff_upload(p.get(), std::vector<double>(d->field_grid, d->field_grid + d->n_grid), &P.grid))) return rc;
+  std::vector<int32_t> rp[3];
+  int64_t apart = 0;  // cells of the operators sliced one by one, by which a plan's size is judged
   for (int o = 0; o < 3; ++o) {
     const int64_t nnz = d->nnz[o];
     if (nnz < 0 || nnz > INT32_MAX / 4) return fail(LB_ERR_UNSUPPORTED, "operator has too many stored entries");
     if (!d->row_ptrs[o] || (nnz > 0 && (!d->col_indices[o] || !d->coeffs[o])))
       return fail(LB_ERR_INVALID, "operator tables are required");
-    std::vector<int32_t> rp(D + 1), col(nnz);
     if (d->row_ptrs[o][0] != 0 || d->row_ptrs[o][D] != nnz)
       return fail(LB_ERR_INVALID, "operator row_ptrs must start at 0 and end at nnz");
+    rp[o].resize(D + 1);
     for (int i = 0; i <= D; ++i) {
       if (i < D && d->row_ptrs[o][i] > d->row_ptrs[o][i + 1])
         return fail(LB_ERR_INVALID, "operator row_ptrs must be monotonic");
-      rp[i] = (int32_t)d->row_ptrs[o][i];
+      rp[o][i] = (int32_t)d->row_ptrs[o][i];
     }
-    for (int64_t q = 0; q < nnz; ++q) {
+    for (int64_t q = 0; q < nnz; ++q)
       if (d->col_indices[o][q] < 0 || d->col_indices[o][q] >= D)
         return fail(LB_ERR_INVALID, "operator column index out of range");
-      col[q] = (int32_t)d->col_indices[o][q];
-    }
-    // sliced layout (lb_device.h): per 64-row slice, its longest row's
-    // entries x 64 cells; padding cells are never read
-    const int S = P.S, nblk = P.nblk, GI = d->n_grid - 1;
-    std::vector<int32_t> len(S, 0);
-    std::vector<int64_t> sp(nblk);
-    int64_t cells = 0;
-    for (int b = 0; b < nblk; ++b) {
+    apart = 0;
+    for (int b = 0; b < P.nblk; ++b) {
       int longest = 0;
-      for (int r = 64 * b; r < std::min(D, 64 * b + 64); ++r) {
-        len[r] = rp[r + 1] - rp[r];
-        longest = std::max(longest, len[r]);
-      }
-      sp[b] = cells;
-      cells += 64 * (int64_t)longest;
+      for (int r = 64 * b; r < std::min(D, 64 * b + 64); ++r) longest = std::max(longest, rp[o][r + 1] - rp[o][r]);
+      apart += 64 * (int64_t)longest;
     }
-    if (cells * (int64_t)std::max(GI, 1) > ((int64_t)1 << 31))
+    if (apart * (int64_t)std::max(d->n_grid - 1, 1) > ((int64_t)1 << 31))
       return fail(LB_ERR_UNSUPPORTED, "operator tables too large in sliced form");
-    std::vector<int32_t> scol(std::max<int64_t>(cells, 1), 0);
+  }
+  {
+    // the sliced form (lb_device.h); padding cells are zero
+    const int S = P.S, nblk = P.nblk, GI = d->n_grid - 1;
+    std::vector<int32_t> len(3 * (size_t)S, 0), row(S, -1);
+    auto entries = [&](int o, int r) { return rp[o][r + 1] - rp[o][r]; };
+    auto all = [&](int r) { return entries(0, r) + entries(1, r) + entries(2, r); };
+    std::iota(row.begin(), row.begin() + D, 0);
+    std::stable_sort(row.begin(), row.begin() + D, [&](int a, int b) { return all(a) > all(b); });
+    std::vector<int64_t> sp;
+    int64_t cells = 0;
+    for (int b = 0; b < nblk; ++b)
+      for (int o = 0; o < 3; ++o) {
+        int longest = 0;
+        for (int s = 64 * b; s < std::min(D, 64 * b + 64); ++s) {
+          len[(size_t)o * S + s] = entries(o, row[s]);
+          longest = std::max(longest, entries(o, row[s]));
+        }
+        sp.push_back(cells);
+        cells += 64 * (int64_t)longest;
+      }
+    sp.push_back(cells);
+    std::vector<uint32_t> scol(std::max<int64_t>(cells, 1), 0);
     std::vector<double2> lo((size_t)std::max<int64_t>(cells * GI, 1), double2{0.0, 0.0}), hi(lo);
-    for (int r = 0; r < D; ++r) {
-      for (int j = 0; j < len[r]; ++j) {
-        const int64_t q = rp[r] + j, c = sp[r / 64] + 64 * (int64_t)j + r % 64;
-        scol[c] = col[q];
-        for (int k = 0; k < GI; ++k) {
-          const double* e = d->coeffs[o] + ((size_t)k * nnz + q) * 4;
-          lo[(size_t)k * cells + c] = double2{e[0], e[1]};
-          hi[(size_t)k * cells + c] = double2{e[2], e[3]};
+    for (int s = 0; s < D; ++s)
+      for (int o = 0; o < 3; ++o) {
+        int64_t c = sp[3 * (s / 64) + o] + s % 64;
+        for (int q = rp[o][row[s]]; q < rp[o][row[s] + 1]; ++q, c += 64) {
+          scol[c] = (uint32_t)d->col_indices[o][q];
+          for (int k = 0; k < GI; ++k) {
+            const double* e = d->coeffs[o] + ((size_t)k * d->nnz[o] + q) * 4;
+            lo[(size_t)k * cells + c] = double2{e[0], e[1]};
+            hi[(size_t)k * cells + c] = double2{e[2], e[3]};
+          }
         }
       }
-    }
-    P.cells[o] = cells;
-    if ((rc = eff_upload(p.get(), len, &P.row_len[o]))) return rc;
-    if ((rc = eff_upload(p.get(), sp, &P.slice_ptr[o]))) return rc;
-    if ((rc = eff_upload(p.get(), scol, &P.col[o]))) return rc;
-    if ((rc = eff_upload(p.get(), lo, &P.coef_lo[o]))) return rc;
-    if ((rc = eff_upload(p.get(), hi, &P.coef_hi[o]))) return rc;
+    P.cells = cells;
+    if ((rc = eff_upload(p.get(), row, &P.row))) return rc;
+    if ((rc = eff_upload(p.get(), len, &P.row_len))) return rc;
+    if ((rc = eff_upload(p.get(), sp, &P.slice_ptr))) return rc;
+    if ((rc = eff_upload(p.get(), scol, &P.col))) return rc;
+    if ((rc = eff_upload(p.get(), lo, &P.coef_lo))) return rc;
+    if ((rc = eff_upload(p.get(), hi, &P.coef_hi))) return rc;
   }
   // parameter graph: base values and compounds (checked as plan expressions)
   std::vector<double> base(2 * (size_t)std::max(d->n_base, 0));
@@ -2203,9 +2228,10 @@ extern "C" int lb_eff_plan_create(const lb_eff_plan_desc* d, lb_eff_plan** out_p
   HIP_TRY(hipGetDevice(&p->device));
   HIP_TRY(hipDeviceGetAttribute(&p->cus, hipDeviceAttributeMultiprocessorCount, p->device));
   if ((rc = p->queues.init())) return rc;
-  int id, W;
-  if ((rc = eff_config(P, &id, &W))) return rc;
-  if (lds_bytes_eff(P) > kMaxLdsBytes) return fail(LB_ERR_UNSUPPORTED, "effective plan needs more LDS than a workgroup has");
+  int id, W, T;
+  size_t lds;
+  if ((rc = eff_config(P, 1, &id, &W, &T, &lds))) return rc;
+  if (lds_bytes_eff_limit(P) > kMaxLdsBytes) return fail(LB_ERR_UNSUPPORTED, "effective plan needs more LDS than a workgroup has");
   *out_plan = p.release();
   return LB_OK;
 }
@@ -2285,11 +2311,15 @@ extern "C" int lb_eff_solve(const lb_eff_plan* p, const lb_eff_solve_args* a, vo
   c.out_counts = a->out_counts;
   c.out_stats = a->out_stats;
   c.out_fail_t = a->out_fail_t;
-  int id, W, rc;
-  if ((rc = eff_config(P, &id, &W))) return rc;
+  // Seats share the loads of the operators; a workgroup of one has the shorter
+  // step.  16 levels, 256 CUs: 256 trajectories 2.3 ms with one seat, 512 in
+  // 2.8 ms with two, 768 in 3.9 ms with four (with one seat a round of 256 each).
+  const int64_t per_cu_traj = (a->n_traj + std::max(1, p->cus) - 1) / std::max(1, p->cus);
+  int id, W, T, rc;
+  size_t lds;
+  if ((rc = eff_config(P, (int)std::min<int64_t>(per_cu_traj >= 3 ? 4 : per_cu_traj, 4), &id, &W, &T, &lds))) return rc;
   void* fn = lb_dev_eff_kernel(id, a->solver);
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "effective kernel variant is not built");
-  const size_t lds = (size_t)lds_bytes_eff(P);
   if ((rc = set_lds_limit(fn, lds))) return rc;
   hipStream_t s = (hipStream_t)stream;
   int grid = a->workgroups;
@@ -2298,7 +2328,7 @@ extern "C" int lb_eff_solve(const lb_eff_plan* p, const lb_eff_solve_args* a, vo
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, W, lds));
     grid = std::max(1, per_cu) * std::max(1, p->cus);
   }
-  grid = (int)std::min<int64_t>(grid, a->n_traj);
+  grid = (int)std::min<int64_t>(grid, (a->n_traj + T - 1) / T);
   void* reset = lb_dev_queue_reset_kernel();
   int slot = 0;
   if ((rc = const_cast<lb_eff_plan*>(p)->queues.acquire(s, &c.queue, &slot))) return rc;
@@ -2316,11 +2346,11 @@ extern "C" int lb_eff_rhs_eval(const lb_eff_plan* p, int64_t batch, const double
   if (!p || !y || !t || !out || !out_status) return fail(LB_ERR_INVALID, "null argument");
   if (batch <= 0) return LB_OK;
   const DevEffPlan& P = p->dev;
-  int id, W, rc;
-  if ((rc = eff_config(P, &id, &W))) return rc;
+  int id, W, T, rc;
+  size_t lds;
+  if ((rc = eff_config(P, 1, &id, &W, &T, &lds))) return rc;
   void* fn = lb_dev_eff_rhs_kernel(id);
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "effective kernel variant is not built");
-  const size_t lds = (size_t)lds_bytes_eff(P);
   if ((rc = set_lds_limit(fn, lds))) return rc;
   DevEffCall c{};
   DevEffRhsCall Q{batch, y, t, out, out_status};

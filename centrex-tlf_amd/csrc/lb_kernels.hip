@@ -44,16 +44,20 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T* cst(const 
 // stay in scalar registers for the whole launch (and most of them spill);
 // code outside the step reads the arguments through fresh_args() instead,
 // whose result the compiler cannot merge with earlier loads.
-struct KernelArgs {
-  DevPlan P;
-  DevCall C;
+template <typename Plan, typename Call>
+struct ArgsOf {
+  Plan P;
+  Call C;
 };
-__device__ __forceinline__ const KernelArgs& fresh_args() {
-  typedef const __attribute__((address_space(4))) KernelArgs* Ptr;
+template <typename Args = ArgsOf<DevPlan, DevCall>>
+__device__ __forceinline__ const Args& fresh_args() {
+  typedef const __attribute__((address_space(4))) Args* Ptr;
   Ptr p = (Ptr)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(p));
-  return *(const KernelArgs*)p;
+  return *(const Args*)p;
 }
+using KernelArgs = ArgsOf<DevPlan, DevCall>;
+using EffArgs = ArgsOf<DevEffPlan, DevEffCall>;
 
 // A lane index that the compiler takes as new: addresses formed from it stay
 // inside the loop body that they are used in, instead of in (spilled) registers
@@ -1423,7 +1427,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         // many slots a lane the stages share one RHS site (a rolled loop keeps
         // the step's code small enough for the instruction cache); unrolled,
         // the stage vectors need no copies and no zeros.
-#pragma unroll(LEAN && R <= 2 ? 6 : 1)
+#pragma unroll LEAN && R <= 2 ? 6 : 1
         for (int s = 2; s <= 7; ++s) {
           switch (s) {
             case 2: stage_combo<R, SOLVER, 2>(h, y_r, y_i, k_r, k_i, yt_r, yt_i); break;
@@ -4959,60 +4963,67 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_rhs_kernel(const DevPlan P, co
 //   dy = A_comb(x) y + (Omega / 2) A_opt(x) y + delta A_det(x) y
 // (rhs.rs:86-138): three CSR operators whose stored entries are cubics in
 // dx = x - grid[k] on grid interval k, with x, Omega, delta the parameter
-// slots at t.  One workgroup per trajectory from the work queue, R rows per
-// lane, the stage input published to LDS (double-buffered) for the column
-// gathers.  The parameter graph runs in six lanes per step, one per stage
-// time; lane 0 then finds the grid intervals in the order the reference's
-// RHS calls would, carrying its cached interval hint (rhs.rs:47-84).  The
-// integrator is the expanded-sparse one: Dopri5 / Tsit5 tableaus,
-// controller, stiffness test, save plan and dense output.
+// slots at t.  A workgroup holds T seats, each integrating a trajectory of its
+// own from the work queue, R rows per lane; the seats' stages run together,
+// the stage inputs published to LDS (double-buffered) for the column gathers.
+// Lane t holds the controller of seat t.  The parameter graph runs in six
+// lanes per seat and step, one per stage time; lane t then finds the grid
+// intervals in the order the reference's RHS calls would, carrying its cached
+// interval hint (rhs.rs:47-84).  The integrator is the expanded-sparse one:
+// Dopri5 / Tsit5 tableaus, controller, stiffness test, save plan and dense
+// output.
+//
+// One trajectory per workgroup read every cubic of its interval from L2 for
+// every stage (10.7 TB/s at 512 reals and 32 entries a row, 2048
+// trajectories: 52.4 ms).  With four seats that share the loads 19.2 ms; rows
+// ordered by length serve every batch (256 trajectories, one seat: 3.7 ->
+// 2.3 ms at 16 levels, 21.7 -> 11.6 ms at 45).  A stage of four seats is bound
+// about equally by the CU's load path (64 B a cycle), FP64 issue and the LDS
+// gathers' bank conflicts, 39k cycles together.
 // ---------------------------------------------------------------------------
 #if LB_PART == 7
 namespace {
 
+// LDS of one workgroup with T seats.
 struct LdsEff {
-  double* ybuf;  // 2 x S stage inputs
-  dcpx* slots;   // 8 x n_slots: t0 / hinit copy and the six stage times
-  dcpx* vm;      // 8 x vm_depth
-  double* red;   // 4 x nblk block sums
-  double* sp;    // 8 x 4 per RHS site: Omega/2, delta, dx, interval; [4 s + 2] field value before lookup
-  double* ev;    // [0] field value of a failed lookup
-  int* misc;     // [0] queue value, [1] status, [2] interval hint
+  double* ybuf;  // 2 x T x stride stage inputs, by row
+  dcpx* slots;   // T x 6 x n_slots: the six stage times (copy 0: t0 and hinit)
+  dcpx* vm;      // T x 6 x vm_depth
+  double* red;   // 3 x T x nblk block sums: error norm and the two stiffness sums
+  double* sp;    // T x 8 x 4 per RHS site: Omega/2, delta, dx, interval; [2] field value before lookup
+  double* x;     // T: time at the start of the step
+  double* h;     // T: step size
+  double* pt;    // T: last pushed time
+  double* pv;    // T: its weighted sum
+  double* pi;    // T: the integral so far
+  int* traj;     // T
+  int* flag;     // T
 };
 
 // Must match lds_bytes_eff() in lb_host.cpp.
-__device__ __forceinline__ LdsEff carve_eff(const DevEffPlan& P) {
+__device__ __forceinline__ LdsEff carve_eff(const DevEffPlan& P, int T, int stride) {
   extern __shared__ double smem[];
   LdsEff L;
   L.ybuf = smem;
-  L.slots = reinterpret_cast<dcpx*>(L.ybuf + 2 * (size_t)P.S);
-  L.vm = L.slots + 8 * (size_t)P.n_slots;
-  L.red = reinterpret_cast<double*>(L.vm + 8 * (size_t)P.vm_depth);
-  L.sp = L.red + 4 * (size_t)P.nblk;
-  L.ev = L.sp + 32;
-  L.misc = reinterpret_cast<int*>(L.ev + 2);
+  L.slots = reinterpret_cast<dcpx*>(L.ybuf + 2 * (size_t)T * stride);
+  L.vm = L.slots + 6 * (size_t)T * P.n_slots;
+  L.red = reinterpret_cast<double*>(L.vm + 6 * (size_t)T * P.vm_depth);
+  L.sp = L.red + 3 * (size_t)T * P.nblk;
+  L.x = L.sp + 32 * (size_t)T;
+  L.h = L.x + T;
+  L.pt = L.h + T;
+  L.pv = L.pt + T;
+  L.pi = L.pv + T;
+  L.traj = reinterpret_cast<int*>(L.pi + T);
+  L.flag = L.traj + T;
   return L;
 }
 
-__device__ __forceinline__ void eff_block_store(const DevEffPlan& P, int tid, int W, int r, double* red, int q,
-                                                double value) {
-  const int s = tid + W * r;
-  const double sum = wave_sum(value);
-  if ((tid & 63) == 0 && s < P.S) red[q * P.nblk + (s >> 6)] = sum;
-}
-
-__device__ __forceinline__ double eff_block_total(const DevEffPlan& P, const double* red, int q) {
-  const int lane = threadIdx.x & 63;
-  double v = 0.0;
-  for (int b = lane; b < P.nblk; b += 64) v += red[q * P.nblk + b];
-  return wave_sum(v);
-}
-
 // Parameter graph at t with the trajectory's (real) overrides, into slot copy
-// `sl` (evaluate_with_overrides_into); returns the field value and stores
-// Omega/2 and delta in sp[0], sp[1].  One lane.
-__device__ __forceinline__ double eff_params(const DevEffPlan& P, const DevEffCall& C, int64_t traj, dcpx* sl,
-                                             double t, dcpx* stk, double* sp) {
+// `sl` (evaluate_with_overrides_into); stores Omega/2, delta and the field
+// value in sp[0..2].  One lane.
+__device__ __forceinline__ void eff_params(const DevEffPlan& P, const DevEffCall& C, int64_t traj, dcpx* sl, double t,
+                                           dcpx* stk, double* sp) {
   for (int i = 0; i < P.n_slots; ++i) sl[i] = i < P.n_base ? mk(P.base[2 * i], P.base[2 * i + 1]) : mk(0.0, 0.0);
   for (int j = 0; j < C.n_override; ++j)
     sl[C.override_slot[j]] = mk(C.override_values ? C.override_values[traj * C.n_override + j] : 0.0, 0.0);
@@ -5023,7 +5034,7 @@ __device__ __forceinline__ double eff_params(const DevEffPlan& P, const DevEffCa
   }
   sp[0] = 0.5 * sl[P.rabi_slot].re;
   sp[1] = sl[P.det_slot].re;
-  return sl[P.field_slot].re;
+  sp[2] = sl[P.field_slot].re;
 }
 
 // find_interval_cached (rhs.rs:47-84): the interval of field value x and
@@ -5060,60 +5071,170 @@ __device__ __forceinline__ int eff_interval(const DevEffPlan& P, double x, int& 
   return idx;
 }
 
-// Interval lookup for RHS site s (field value in sp[4 s + 2]); lane 0, in
-// call order.  A failed lookup records the first failure and leaves interval
-// 0 so the RHS still reads inside the tables.
-__device__ __forceinline__ void eff_lookup(const DevEffPlan& P, const LdsEff& L, int s) {
-  const double x = L.sp[4 * s + 2];
-  int hint = L.misc[2];
+// Interval lookup of one RHS site (field value in sp[2]), in call order.  A
+// failed lookup records the first failure and leaves interval 0 so the RHS
+// still reads inside the tables.
+__device__ __forceinline__ void eff_lookup(const DevEffPlan& P, double* sp, int& hint, int& status, double& fail_x) {
+  const double x = sp[2];
   double dx = 0.0;
   const int idx = eff_interval(P, x, hint, dx);
-  L.misc[2] = hint;
-  if (idx < 0 && L.misc[1] == 0) {
-    L.misc[1] = idx == -1 ? LB_TRAJ_FIELD_BELOW : LB_TRAJ_FIELD_ABOVE;
-    L.ev[0] = x;
+  if (idx < 0 && status == 0) {
+    status = idx == -1 ? LB_TRAJ_FIELD_BELOW : LB_TRAJ_FIELD_ABOVE;
+    fail_x = x;
   }
-  L.sp[4 * s + 2] = idx < 0 ? 0.0 : dx;
-  L.sp[4 * s + 3] = (double)(idx < 0 ? 0 : idx);
+  sp[2] = idx < 0 ? 0.0 : dx;
+  sp[3] = (double)(idx < 0 ? 0 : idx);
 }
+
+// U entries of a row of one operator.
+template <int U>
+struct EffChunk {
+  double2 a[U], b[U];
+  uint32_t c[U];
+  // entries j .. of a lane whose row holds `len`; lo, hi and col are the
+  // slice's (uniform), so a load has no address arithmetic of its own
+  __device__ __forceinline__ void load(const double2* lo, const double2* hi, const uint32_t* col, int j, int len,
+                                       uint32_t lane) {
+    lo += 64 * j;
+    hi += 64 * j;
+    col += 64 * j;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (j + u < len) {
+        a[u] = lo[64 * u + lane];
+        b[u] = hi[64 * u + lane];
+        c[u] = col[64 * u + lane];
+      }
+    }
+  }
+};
 
 // dy = sum_o scale_o * sum_p cubic_p(dx) * y[col_p] row by row, each operator
 // summed in CSR order and added in the reference's order (rhs.rs:123-135,
-// plan.rs:18-40).  Publishes y to LDS buffer `yb` first (one barrier).
-template <int R>
-__device__ __forceinline__ void eff_rhs(const DevEffPlan& P, double* yb, const double (&y)[R], double (&k)[R],
-                                        const double* sp, int tid, int W) {
+// plan.rs:18-40), for the seats in `mask`.  Publishes y to LDS buffer `yb`
+// first (one barrier).
+//
+// The seats whose field lies in one grid interval share the loads of its
+// cubics, which bound this kernel: 36 bytes an entry against 8 FP64 operations
+// and one LDS read a seat.  Rows of like length share a wave, the next chunk's
+// loads are in flight while a chunk is applied, also into the next operator,
+// and a chunk's LDS reads are issued together: every seat is computed and the
+// ones outside the group dropped, as a branch per seat would wait for its own
+// read each time.
+template <int R, int T, int Y, bool NARROW>
+__device__ __forceinline__ void eff_rhs(const DevEffPlan& P, double* yb, const double (&y)[T][R], double (&k)[T][R],
+                                        const double* sp, uint32_t mask, const int (&row)[R], int tid, int W) {
+  // chunks of U entries, N of them in flight (registers allow no more)
+  constexpr int U = T == 1 && R == 1 && !NARROW ? 4 : 2, N = NARROW ? 2 : 4;
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int row = tid + W * r;
-    if (row < P.D) yb[row] = y[r];
-  }
-  __syncthreads();
-  const double half_rabi = sp[0], det = sp[1], dx = sp[2];
-  const int idx = (int)sp[3];
+  for (int r = 0; r < R; ++r)
+    if (row[r] >= 0) {
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int row = tid + W * r;
-    double acc = 0.0;
-    if (row < P.D) {
-#pragma unroll
-      for (int o = 0; o < 3; ++o) {
-        const double2* lo = P.coef_lo[o] + (size_t)idx * P.cells[o];
-        const double2* hi = P.coef_hi[o] + (size_t)idx * P.cells[o];
-        const int* col = P.col[o];
-        const int len = P.row_len[o][row];
-        const int64_t c0 = P.slice_ptr[o][row >> 6] + (row & 63);
-        double sum = 0.0;
-        for (int j = 0; j < len; ++j) {  // the row's entries in CSR order
-          const int64_t c = c0 + 64 * (int64_t)j;
-          const double2 a = lo[c], b = hi[c];
-          const double val = a.x + dx * (a.y + dx * (b.x + dx * b.y));
-          sum += val * yb[col[c]];
-        }
-        acc += (o == 0 ? 1.0 : o == 1 ? half_rabi : det) * sum;
-      }
+      for (int t = 0; t < T; ++t) yb[t * Y + row[r]] = y[t][r];
     }
-    k[r] = acc;
+  __syncthreads();
+  const uint32_t lane = tid & 63;
+  while (mask) {
+    const int idx = __builtin_amdgcn_readfirstlane((int)sp[32 * (__ffs((int)mask) - 1) + 3]);
+    uint32_t group = 0;
+    double half_rabi[T], det[T], dx[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      if ((mask >> t & 1u) && __builtin_amdgcn_readfirstlane((int)sp[32 * t + 3]) == idx) group |= 1u << t;
+      half_rabi[t] = lane_d(sp[32 * t], 0);
+      det[t] = lane_d(sp[32 * t + 1], 0);
+      dx[t] = lane_d(sp[32 * t + 2], 0);
+    }
+    mask &= ~group;
+    const double2* lo = P.coef_lo + (size_t)idx * P.cells;
+    const double2* hi = P.coef_hi + (size_t)idx * P.cells;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int s = tid + W * r;
+      if (s >= P.S) continue;
+      const int b = __builtin_amdgcn_readfirstlane(s >> 6);
+      const int64_t c0 = cst(P.slice_ptr)[3 * b];
+      // first entries of the operators in the slice, and the row's own counts
+      const int e1 = (int)(cst(P.slice_ptr)[3 * b + 1] - cst(P.slice_ptr)[3 * b]) >> 6,
+                e2 = (int)(cst(P.slice_ptr)[3 * b + 2] - cst(P.slice_ptr)[3 * b]) >> 6,
+                e3 = (int)(cst(P.slice_ptr)[3 * b + 3] - cst(P.slice_ptr)[3 * b]) >> 6;
+      const int l0 = P.row_len[s], l1 = e1 + P.row_len[P.S + s], l2 = e2 + P.row_len[2 * P.S + s];
+      double acc[T], sum[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t) acc[t] = sum[t] = 0.0;
+      // entry j of operator o, whose entries in the slice end at `end`, the
+      // row's own at `len`
+      struct Cursor {
+        int o, j, end, len;
+      };
+      auto settle = [&](Cursor& q) {  // past the end of an operator: to the next that has entries
+        while (q.o < 3 && q.j >= q.end) {
+          ++q.o;
+          q.j = q.end;
+          q.end = q.o == 1 ? e2 : e3;
+          q.len = q.o == 1 ? l1 : l2;
+        }
+      };
+      auto close = [&](int op) {  // the sums of operator op are complete
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          acc[t] += (op == 0 ? 1.0 : op == 1 ? half_rabi[t] : det[t]) * sum[t];
+          sum[t] = 0.0;
+        }
+      };
+      Cursor use{0, 0, e1, l0};
+      settle(use);
+      for (int op = 0; op < use.o; ++op) close(op);
+      Cursor get = use;
+      EffChunk<U> ring[N];
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          ring[n].a[u] = ring[n].b[u] = double2{0.0, 0.0};
+          ring[n].c[u] = 0;
+        }
+        if (get.o < 3) {
+          ring[n].load(lo + c0, hi + c0, P.col + c0, get.j, get.len, lane);
+          get.j += U;
+          settle(get);
+        }
+      }
+      while (use.o < 3) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+          if (use.o < 3) {
+            double yv[U][T];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+              for (int t = 0; t < T; ++t) yv[u][t] = yb[t * Y + ring[n].c[u]];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (use.j + u < use.len) {
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                  const double val = ring[n].a[u].x +
+                                     dx[t] * (ring[n].a[u].y + dx[t] * (ring[n].b[u].x + dx[t] * ring[n].b[u].y));
+                  sum[t] += val * yv[u][t];
+                }
+              }
+            const int op0 = use.o;
+            use.j += U;
+            settle(use);
+            if (get.o < 3) {
+              ring[n].load(lo + c0, hi + c0, P.col + c0, get.j, get.len, lane);
+              get.j += U;
+              settle(get);
+            }
+            for (int op = op0; op < use.o; ++op) close(op);
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        if (group >> t & 1u) k[t][r] = acc[t];
+    }
   }
 }
 
@@ -5162,243 +5283,374 @@ __device__ __forceinline__ void eff_dense(double th, double h, const double (&y)
   }
 }
 
+// What a seat does in this pass of the kernel's loop.
+#define LB_SEAT_ON 1      // holds a trajectory
+#define LB_SEAT_START 2   // took it in this pass
+#define LB_SEAT_STEP 4    // attempts a step
+#define LB_SEAT_STIFF 8   // with the stiffness sums
+#define LB_SEAT_ACCEPT 16 // and accepts it
+#define LB_SEAT_DONE 32   // ends
+
 }  // namespace
 
-template <int R, int SOLVER, int MAXW, int WAVES>
+template <int R, int SOLVER, int MAXW, int WAVES, int T>
 __global__ __launch_bounds__(MAXW, WAVES) void lb_eff_kernel(const DevEffPlan P, const DevEffCall C) {
-  using T = Tab<SOLVER>;
+  using TB = Tab<SOLVER>;
+  static_assert(T <= 8, "a wave evaluates the parameters of every seat");
   const int tid = threadIdx.x, W = blockDim.x;
-  const LdsEff L = carve_eff(P);
-  for (;;) {
-    __syncthreads();
-    if (tid == 0) L.misc[0] = atomicAdd(C.queue, 1);
-    __syncthreads();
-    const int64_t traj = L.misc[0];
-    if (traj >= C.n_traj) break;
-    const double t0 = C.t0, t1 = C.t1;
-    if (tid == 0) {
-      L.misc[1] = 0;
-      L.misc[2] = 0;
-    }
-    double y[R];
+  // a seat's stage inputs lie Y apart, a constant, so that a gather's address
+  // serves all seats
+  constexpr int Y = R * MAXW;
+  const LdsEff L = carve_eff(P, T, T > 1 ? Y : P.S);
+  int row[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) row[r] = tid + W * r < P.S ? P.row[tid + W * r] : -1;
+  const double t0 = C.t0, t1 = C.t1, hmax = fabs(t1 - t0), inv_dim = 1.0 / (double)P.D;
+  const bool step_push = C.n_saveat == 0, want_int = C.output_kind == LB_EFF_OUT_INTEGRAL;
+  const bool given = isfinite(C.dt) && C.dt > 0.0;
+  // the state of seat t in lane t: flags, and the controller of its trajectory
+  int flag = 0, status = 0, hint = 0;
+  bool dry = false, reject = false, last = false;
+  int64_t accepted = 0, rejected = 0, rhs_calls = 0, ns = 0, nst = 0, ia = 0, traj = 0;
+  double x = 0.0, h = 0.0, lfo = LB_LOG_FAC_MIN, fail_x = 0.0;
+  // rows, and what every lane follows: save points reached and rows pushed
+  double y[T][R], k[8][T][R];
+  int64_t si[T], n_pushed[T];
+  int buf = 0;
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    si[t] = n_pushed[t] = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int row = tid + W * r;
-      y[r] = row < P.D ? C.y0[row] : 0.0;
+      y[t][r] = 0.0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) k[j][t][r] = 0.0;
     }
-    int64_t accepted = 0, rejected = 0, rhs_calls = 0, n_pushed = 0, si = 0;
-    int status = 0, buf = 0;
-    double fail_x = 0.0, integral = 0.0, last_t = __builtin_nan(""), last_v = 0.0;
-    const bool step_push = C.n_saveat == 0;
-    const bool want_int = C.output_kind == LB_EFF_OUT_INTEGRAL;
-    // a pushed point: the weighted sum for the integral (in weight order,
-    // output.rs:315-330), or an output row
-    auto push = [&](double tp, const double (&v)[R]) {
-      if (want_int) {
-        double* yb = L.ybuf + buf * P.S;
-        buf ^= 1;
+  }
+  auto seats = [&](int bits) {  // seats whose flags have one of `bits`
+    uint32_t m = 0;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int row = tid + W * r;
-          if (row < P.D) yb[row] = v[r];
-        }
-        __syncthreads();
-        if (tid == 0) {
-          double w = 0.0;
-          for (int q = 0; q < C.n_weights; ++q) w += C.weight_value[q] * yb[C.weight_index[q]];
-          if (isfinite(last_t)) integral += 0.5 * (last_v + w) * (tp - last_t);
-          last_v = w;
-        }
-        last_t = tp;
-        ++n_pushed;
-        return;
-      }
-      if (n_pushed < C.capacity) {
-        const int64_t base = (traj * C.capacity + n_pushed) * C.width;
+    for (int t = 0; t < T; ++t)
+      if (__builtin_amdgcn_readfirstlane(L.flag[t]) & bits) m |= 1u << t;
+    return m;
+  };
+  // a pushed point: the weighted sum for the integral (in weight order,
+  // output.rs:315-330), or an output row
+  auto push = [&](int t, double tp, const double (&v)[R]) {
+    const EffArgs& A = fresh_args<EffArgs>();
+    const DevEffPlan& P = A.P;
+    const DevEffCall& C = A.C;
+    if (want_int) {
+      double* yb = L.ybuf + t * (T > 1 ? Y : P.S);
+      __syncthreads();
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int row = tid + W * r;
-          if (row >= P.D) continue;
-          if (C.output_kind == LB_EFF_OUT_FULL) {
-            C.out_values[base + row] = v[r];
-          } else if (C.output_kind == LB_EFF_OUT_POPULATIONS) {
-            if (row < P.n * P.n && row % (P.n + 1) == 0) C.out_values[base + row / (P.n + 1)] = v[r];
-          } else {
-            for (int q = 0; q < C.n_selected; ++q) {
-              if (C.sel_re[q] == row) {
-                C.out_values[base + 2 * q] = v[r];
-                if (C.sel_im[q] < 0) C.out_values[base + 2 * q + 1] = 0.0;
-              }
-              if (C.sel_im[q] == row) C.out_values[base + 2 * q + 1] = v[r];
-            }
-          }
-        }
-        if (tid == 0 && C.out_times) C.out_times[traj * C.capacity + n_pushed] = tp;
-      }
-      last_t = tp;
-      ++n_pushed;
-    };
-    // field, Omega/2, delta at t for RHS site s (lane 0), then the lookup
-    auto site = [&](int s, double t) {
+      for (int r = 0; r < R; ++r)
+        if (row[r] >= 0) yb[row[r]] = v[r];
+      __syncthreads();
       if (tid == 0) {
-        L.sp[4 * s + 2] = eff_params(P, C, traj, L.slots + s * P.n_slots, t, L.vm, L.sp + 4 * s);
-        eff_lookup(P, L, s);
+        double w = 0.0;
+        for (int q = 0; q < C.n_weights; ++q) w += C.weight_value[q] * yb[C.weight_index[q]];
+        if (isfinite(L.pt[t])) L.pi[t] += 0.5 * (L.pv[t] + w) * (tp - L.pt[t]);
+        L.pv[t] = w;
+        L.pt[t] = tp;
       }
       __syncthreads();
-      if (L.misc[1] != 0) {
-        status = L.misc[1];
-        fail_x = L.ev[0];
+      ++n_pushed[t];
+      return;
+    }
+    if (n_pushed[t] < C.capacity) {
+      const int64_t tr = L.traj[t], base = (tr * C.capacity + n_pushed[t]) * C.width;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int w = row[r];
+        if (w < 0) continue;
+        if (C.output_kind == LB_EFF_OUT_FULL) {
+          C.out_values[base + w] = v[r];
+        } else if (C.output_kind == LB_EFF_OUT_POPULATIONS) {
+          if (w < P.n * P.n && w % (P.n + 1) == 0) C.out_values[base + w / (P.n + 1)] = v[r];
+        } else {
+          for (int q = 0; q < C.n_selected; ++q) {
+            if (C.sel_re[q] == w) {
+              C.out_values[base + 2 * q] = v[r];
+              if (C.sel_im[q] < 0) C.out_values[base + 2 * q + 1] = 0.0;
+            }
+            if (C.sel_im[q] == w) C.out_values[base + 2 * q + 1] = v[r];
+          }
+        }
       }
-    };
-#define LB_EFF_RHS(yy, kk, s)                              \
-  do {                                                     \
-    eff_rhs<R>(P, L.ybuf + buf * P.S, yy, kk, L.sp + 4 * (s), tid, W); \
-    buf ^= 1;                                              \
+      if (tid == 0 && C.out_times) C.out_times[tr * C.capacity + n_pushed[t]] = tp;
+    }
+    ++n_pushed[t];
+  };
+  // field, Omega/2, delta of a starting seat at t (lane = seat), then the lookup
+  auto site = [&](double t) {
+    const EffArgs& A = fresh_args<EffArgs>();
+    const DevEffPlan& P = A.P;
+    const DevEffCall& C = A.C;
+    double* sp = L.sp + 32 * tid;
+    eff_params(P, C, traj, L.slots + (size_t)tid * 6 * P.n_slots, t, L.vm + (size_t)tid * 6 * P.vm_depth, sp);
+    eff_lookup(P, sp, hint, status, fail_x);
+  };
+  // sums over the rows of a seat as red[q][t][block], and their total by one lane
+  auto store_sum = [&](int q, int t, int r, double v) {
+    const int s = tid + W * r;
+    const double sum = wave_sum(v);
+    if ((tid & 63) == 0 && s < P.S) L.red[(q * T + t) * P.nblk + (s >> 6)] = sum;
+  };
+  auto total = [&](int q) {
+    double v = 0.0;
+    for (int b = 0; b < P.nblk; ++b) v += L.red[(q * T + tid) * P.nblk + b];
+    return v;
+  };
+#define LB_EFF_RHS(yy, kk, site_, mask)                                                                   \
+  do {                                                                                                    \
+    eff_rhs<R, T, Y, (WAVES > 2 || R > 1)>(P, L.ybuf + buf * (T > 1 ? T * Y : P.S), yy, kk, L.sp + 4 * (site_), \
+                                           mask, row, tid, W);                                          \
+    buf ^= 1;                                                                                             \
   } while (0)
 
-    double k[8][R];
-    if (t1 < t0) {
-      status = LB_TRAJ_BAD_SPAN;
-      fail_x = t0;
-    } else if (t1 == t0) {
-      if (C.save_start) push(t0, y);
-    } else {
-      double x = t0, h = 0.0;
-      if (isfinite(C.dt) && C.dt > 0.0) {
-        h = fmin(C.dt, t1 - t0);
-      } else {
-        // hinit (rust/src/ode/common.rs:72-118): f0 at t0, f1 at t0 + h0
-        double f0[R], yt[R], f1[R];
-        site(0, t0);
-        if (status == 0) {
-          LB_EFF_RHS(y, f0, 0);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const int row = tid + W * r;
-            const double sc = C.abstol + fabs(y[r]) * C.reltol;
-            const double a0 = y[r] / sc, b0 = f0[r] / sc;
-            eff_block_store(P, tid, W, r, L.red, 0, row < P.D ? a0 * a0 : 0.0);
-            eff_block_store(P, tid, W, r, L.red, 1, row < P.D ? b0 * b0 : 0.0);
+  for (;;) {
+    // ---- free seats take trajectories
+    __syncthreads();
+    if (tid < T) {
+      flag &= LB_SEAT_ON;
+      if (!flag && !dry) {
+        const int64_t q = atomicAdd(C.queue, 1);
+        if (q < C.n_traj) {
+          flag = LB_SEAT_ON | LB_SEAT_START;
+          traj = q;
+          status = hint = 0;
+          reject = last = false;
+          accepted = rejected = rhs_calls = ns = nst = ia = 0;
+          x = t0;
+          h = given ? fmin(C.dt, t1 - t0) : 0.0;
+          lfo = LB_LOG_FAC_MIN;
+          fail_x = 0.0;
+          L.traj[tid] = (int)q;
+          L.pt[tid] = __builtin_nan("");
+          L.pv[tid] = L.pi[tid] = 0.0;
+          if (t1 < t0) {
+            status = LB_TRAJ_BAD_SPAN;
+            fail_x = t0;
           }
-          __syncthreads();
-          const double d0 = eff_block_total(P, L.red, 0), d1 = eff_block_total(P, L.red, 1), hmax = fabs(t1 - x);
-          double h0 = (d0 < 1.0e-10 || d1 < 1.0e-10) ? 1.0e-6 : 0.01 * sqrt(d0 / d1);
-          h0 = fmin(h0, hmax);
+          if (!(t1 > t0)) flag |= LB_SEAT_DONE;
+        } else {
+          dry = true;
+        }
+      }
+      L.flag[tid] = flag;
+    }
+    __syncthreads();
+    if (!seats(LB_SEAT_ON)) break;
+    uint32_t fresh = seats(LB_SEAT_START);
+    if (fresh) {
+      const EffArgs& A = fresh_args<EffArgs>();
+      const DevEffPlan& P = A.P;
+      const DevEffCall& C = A.C;
 #pragma unroll
-          for (int r = 0; r < R; ++r) yt[r] = y[r] + f0[r] * h0;
-          site(1, x + h0);
-          if (status == 0) {
-            LB_EFF_RHS(yt, f1, 1);
+      for (int t = 0; t < T; ++t)
+        if (fresh >> t & 1u) {
+          si[t] = n_pushed[t] = 0;
+#pragma unroll
+          for (int r = 0; r < R; ++r) y[t][r] = row[r] >= 0 ? C.y0[row[r]] : 0.0;
+        }
+      const bool start = (flag & LB_SEAT_START) && tid < T;
+      if (t1 == t0 && C.save_start) {
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+          if (fresh >> t & 1u) push(t, t0, y[t]);
+      }
+      if (t1 > t0) {
+        if (!given) {
+          // hinit (rust/src/ode/common.rs:72-118): f0 at t0 (k1), f1 at t0 + h0 (k2)
+          double h0 = 0.0, d1 = 0.0;
+          if (start) site(t0);
+          __syncthreads();
+          LB_EFF_RHS(y, k[1], 0, fresh);
+#pragma unroll
+          for (int t = 0; t < T; ++t)
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-              const int row = tid + W * r;
-              const double sc = C.abstol + fabs(y[r]) * C.reltol;
-              const double a0 = (f1[r] - f0[r]) / sc;
-              eff_block_store(P, tid, W, r, L.red, 2, row < P.D ? a0 * a0 : 0.0);
+              const double sc = C.abstol + fabs(y[t][r]) * C.reltol;
+              const double a0 = y[t][r] / sc, b0 = k[1][t][r] / sc;
+              store_sum(0, t, r, row[r] >= 0 ? a0 * a0 : 0.0);
+              store_sum(1, t, r, row[r] >= 0 ? b0 * b0 : 0.0);
             }
-            __syncthreads();
-            const double d2 = sqrt(eff_block_total(P, L.red, 2)) / h0;
+          __syncthreads();
+          if (start) {
+            const double d0 = total(0);
+            d1 = total(1);
+            h0 = (d0 < 1.0e-10 || d1 < 1.0e-10) ? 1.0e-6 : 0.01 * sqrt(d0 / d1);
+            h0 = fmin(h0, hmax);
+            L.h[tid] = h0;
+            if (status == 0) site(x + h0);
+          }
+          __syncthreads();
+          double yt[T][R];
+#pragma unroll
+          for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int r = 0; r < R; ++r) yt[t][r] = fresh >> t & 1u ? y[t][r] + k[1][t][r] * L.h[t] : 0.0;
+          LB_EFF_RHS(yt, k[2], 0, fresh);
+#pragma unroll
+          for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              const double sc = C.abstol + fabs(y[t][r]) * C.reltol;
+              const double a0 = (k[2][t][r] - k[1][t][r]) / sc;
+              store_sum(2, t, r, row[r] >= 0 ? a0 * a0 : 0.0);
+            }
+          __syncthreads();
+          if (start) {
+            const double d2 = sqrt(total(2)) / h0;
             const double h1 = fmax(sqrt(d1), fabs(d2)) <= 1.0e-15 ? fmax(1.0e-6, fabs(h0) * 1.0e-3)
                                                                   : pow(0.01 / fmax(sqrt(d1), d2), 1.0 / 5.0);
             h = fmin(100.0 * fabs(h0), fmin(h1, hmax));
           }
         }
-      }
-      // k1 = f(t0, y0)
-      if (status == 0) site(0, t0);
-      if (status == 0) {
-        LB_EFF_RHS(y, k[1], 0);
-        rhs_calls = 1;
-        if (!step_push) {
-          while (si < C.n_saveat && fabs(C.saveat[si] - t0) <= time_tol(t0)) {
-            push(C.saveat[si], y);
-            ++si;
-          }
-        } else if (C.save_start) {
-          push(t0, y);
+        // k1 = f(t0, y0)
+        if (start) {
+          if (status == 0) site(t0);
+          if (status != 0) flag |= LB_SEAT_DONE;
+          else rhs_calls = 1;
+          L.flag[tid] = flag;
         }
+        __syncthreads();
+        fresh &= ~seats(LB_SEAT_DONE);
+        LB_EFF_RHS(y, k[1], 0, fresh);
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+          if (fresh >> t & 1u) {
+            if (!step_push) {
+              while (si[t] < C.n_saveat && fabs(C.saveat[si[t]] - t0) <= time_tol(t0)) {
+                push(t, C.saveat[si[t]], y[t]);
+                ++si[t];
+              }
+            } else if (C.save_start) {
+              push(t, t0, y[t]);
+            }
+          }
       }
-      const double hmax = fabs(t1 - t0), inv_dim = 1.0 / (double)P.D;
-      double lfo = LB_LOG_FAC_MIN;
-      bool reject = false, last = false;
-      int64_t ns = 0, nst = 0, ia = 0;
-      while (!last && status == 0) {
-        if (ns > C.maxiters) { status = LB_TRAJ_MAXITERS; fail_x = x; break; }
-        if (0.1 * fabs(h) <= DBL_EPSILON * fabs(x)) { status = LB_TRAJ_UNDERFLOW; fail_x = x; break; }
+    }
+    // ---- the next step of every seat
+    if (tid < T && (flag & LB_SEAT_ON) && !(flag & LB_SEAT_DONE)) {
+      if (ns > C.maxiters) status = LB_TRAJ_MAXITERS;
+      else if (0.1 * fabs(h) <= DBL_EPSILON * fabs(x)) status = LB_TRAJ_UNDERFLOW;
+      if (status != 0) {
+        fail_x = x;
+        flag |= LB_SEAT_DONE;
+      } else {
         if (x + 1.01 * h - t1 > 0.0) { h = t1 - x; last = true; }
         ++ns;
-        // parameters at the six stage times (lanes 0-5), then the interval
-        // lookups in call order (lane 0)
-        if (tid < 6) {
-          const int s = tid + 2;
-          L.sp[4 * s + 2] = eff_params(P, C, traj, L.slots + s * P.n_slots, x + h * T::c(s), L.vm + tid * P.vm_depth,
-                                       L.sp + 4 * s);
+        flag |= LB_SEAT_STEP;
+        if ((accepted + 1) % 1000 == 0 || ia > 0) flag |= LB_SEAT_STIFF;
+      }
+      L.x[tid] = x;
+      L.h[tid] = h;
+    }
+    if (tid < T) L.flag[tid] = flag;
+    if (tid < 64) {
+      // parameters at the six stage times (lanes 8 t .. 8 t + 5 of seat t),
+      // then the interval lookups in call order (lane t)
+      wave_sync();
+      const EffArgs& A = fresh_args<EffArgs>();
+      const DevEffPlan& P = A.P;
+      const DevEffCall& C = A.C;
+      const int t = tid >> 3, q = tid & 7;
+      if (t < T && q < 6 && (L.flag[t] & LB_SEAT_STEP))
+        eff_params(P, C, L.traj[t], L.slots + (size_t)(6 * t + q) * P.n_slots, L.x[t] + L.h[t] * TB::c(q + 2),
+                   L.vm + (size_t)(6 * t + q) * P.vm_depth, L.sp + 32 * t + 4 * (q + 2));
+      wave_sync();
+      if (tid < T && (flag & LB_SEAT_STEP)) {
+        for (int s = 2; s <= 7; ++s) eff_lookup(P, L.sp + 32 * tid + 4 * s, hint, status, fail_x);
+        if (status != 0) {
+          flag = (flag & ~LB_SEAT_STEP) | LB_SEAT_DONE;
+          L.flag[tid] = flag;
         }
-        __syncthreads();
-        if (tid == 0)
-          for (int s = 2; s <= 7; ++s) eff_lookup(P, L, s);
-        __syncthreads();
-        if (L.misc[1] != 0) {
-          status = L.misc[1];
-          fail_x = L.ev[0];
-          break;
-        }
-        const bool need_stiff = ((accepted + 1) % 1000 == 0) || ia > 0;
-        double yt[R], yn[R];
+      }
+    }
+    __syncthreads();
+    const uint32_t step = seats(LB_SEAT_STEP), stiff = seats(LB_SEAT_STIFF) & step;
+    if (step) {
+      double hs[T], yt[T][R], yn[T][R];
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        hs[t] = lane_d(L.h[t], 0);
+#pragma unroll
+        for (int r = 0; r < R; ++r) yt[t][r] = yn[t][r] = 0.0;
+      }
 #pragma unroll 1
-        for (int s = 2; s <= 7; ++s) {
+      for (int s = 2; s <= 7; ++s) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          double kt[8][R];
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int r = 0; r < R; ++r) kt[j][r] = k[j][t][r];
           switch (s) {
-            case 2: eff_stage<R, SOLVER, 2>(h, y, k, yt); break;
-            case 3: eff_stage<R, SOLVER, 3>(h, y, k, yt); break;
-            case 4: eff_stage<R, SOLVER, 4>(h, y, k, yt); break;
-            case 5: eff_stage<R, SOLVER, 5>(h, y, k, yt); break;
-            case 6: eff_stage<R, SOLVER, 6>(h, y, k, yt); break;
+            case 2: eff_stage<R, SOLVER, 2>(hs[t], y[t], kt, yt[t]); break;
+            case 3: eff_stage<R, SOLVER, 3>(hs[t], y[t], kt, yt[t]); break;
+            case 4: eff_stage<R, SOLVER, 4>(hs[t], y[t], kt, yt[t]); break;
+            case 5: eff_stage<R, SOLVER, 5>(hs[t], y[t], kt, yt[t]); break;
+            case 6: eff_stage<R, SOLVER, 6>(hs[t], y[t], kt, yt[t]); break;
             default:
-              eff_stage<R, SOLVER, 7>(h, y, k, yn);
-              if (need_stiff) {
+              eff_stage<R, SOLVER, 7>(hs[t], y[t], kt, yn[t]);
+              if (stiff >> t & 1u) {
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
-                  const double a0 = yn[r] - yt[r];
-                  eff_block_store(P, tid, W, r, L.red, 3, a0 * a0);
+                  const double a0 = yn[t][r] - yt[t][r];
+                  store_sum(2, t, r, a0 * a0);
                 }
               }
 #pragma unroll
-              for (int r = 0; r < R; ++r) yt[r] = yn[r];
+              for (int r = 0; r < R; ++r) yt[t][r] = yn[t][r];
               break;
           }
-          double ko[R];
-          LB_EFF_RHS(yt, ko, s);
+        }
+        double ko[T][R];
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+          for (int r = 0; r < R; ++r) ko[t][r] = 0.0;
+        LB_EFF_RHS(yt, ko, s, step);
+#pragma unroll
+        for (int t = 0; t < T; ++t)
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             switch (s) {
-              case 2: k[2][r] = ko[r]; break;
-              case 3: k[3][r] = ko[r]; break;
-              case 4: k[4][r] = ko[r]; break;
-              case 5: k[5][r] = ko[r]; break;
-              case 6: k[6][r] = ko[r]; break;
-              default: k[7][r] = ko[r]; break;
+              case 2: k[2][t][r] = ko[t][r]; break;
+              case 3: k[3][t][r] = ko[t][r]; break;
+              case 4: k[4][t][r] = ko[t][r]; break;
+              case 5: k[5][t][r] = ko[t][r]; break;
+              case 6: k[6][t][r] = ko[t][r]; break;
+              default: k[7][t][r] = ko[t][r]; break;
             }
           }
-        }
-        rhs_calls += 6;
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        if (!(step >> t & 1u)) continue;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-          const int row = tid + W * r;
-          double er = T::e(1) * k[1][r];
+          double er = TB::e(1) * k[1][t][r];
 #pragma unroll
           for (int j = 2; j <= 7; ++j)
-            if (T::e(j) != 0.0) er = fma(T::e(j), k[j][r], er);
-          er *= h;
-          const double sc = C.abstol + fmax(fabs(y[r]), fabs(yn[r])) * C.reltol;
+            if (TB::e(j) != 0.0) er = fma(TB::e(j), k[j][t][r], er);
+          er *= hs[t];
+          const double sc = C.abstol + fmax(fabs(y[t][r]), fabs(yn[t][r])) * C.reltol;
           const double q = er / sc;
-          eff_block_store(P, tid, W, r, L.red, 0, row < P.D ? q * q : 0.0);
-          if (need_stiff) {
-            const double a0 = k[7][r] - k[6][r];
-            eff_block_store(P, tid, W, r, L.red, 2, a0 * a0);
+          store_sum(0, t, r, row[r] >= 0 ? q * q : 0.0);
+          if (stiff >> t & 1u) {
+            const double a0 = k[7][t][r] - k[6][t][r];
+            store_sum(1, t, r, a0 * a0);
           }
         }
-        __syncthreads();
-        const StepControl ctl(eff_block_total(P, L.red, 0) * inv_dim, lfo);
+      }
+      __syncthreads();
+      if (tid < T && (flag & LB_SEAT_STEP)) {
+        rhs_calls += 6;
+        const StepControl ctl(total(0) * inv_dim, lfo);
         double hn = h * ctl.factor();
         if (ctl.accept) {
           lfo = fmax(ctl.lerr, LB_LOG_FAC_MIN);
@@ -5406,74 +5658,99 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_eff_kernel(const DevEffPlan P,
           if (reject) hn = fmin(fabs(hn), fabs(h));
           reject = false;
           ++accepted;
-          if (accepted % 1000 == 0 || ia > 0) {
-            const double n2 = eff_block_total(P, L.red, 2), dd2 = eff_block_total(P, L.red, 3);
+          if (flag & LB_SEAT_STIFF) {
+            const double n2 = total(1), dd2 = total(2);
             const double hl = dd2 > 0.0 ? h * sqrt(n2 / dd2) : 0.0;
             if (hl > 3.25) {
               ++ia;
               nst = 0;
-              if (ia == 15) { status = LB_TRAJ_STIFF; fail_x = x; break; }
+              if (ia == 15) { status = LB_TRAJ_STIFF; fail_x = x; }
             } else {
               ++nst;
               if (nst == 6) ia = 0;
             }
           }
-          const double xo = x;
-          x += h;
-          if (step_push) {
-            push(x, yn);
-          } else {
-            while (si < C.n_saveat && C.saveat[si] <= x + time_tol(x)) {
-              const double ts = C.saveat[si];
-              if (ts >= xo - time_tol(xo)) {
-                if (fabs(ts - xo) <= time_tol(xo)) {
-                  push(ts, y);
-                } else if (fabs(ts - x) <= time_tol(x)) {
-                  push(ts, yn);
-                } else {
-                  double ds[R];
-                  eff_dense<R, SOLVER>((ts - xo) / h, h, y, yn, k, ds);
-                  push(ts, ds);
-                }
-              }
-              ++si;
-            }
+          if (status == 0) {
+            flag |= LB_SEAT_ACCEPT;
+            x += h;
           }
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            y[r] = yn[r];
-            k[1][r] = k[7][r];
-          }
-          if (last) break;
+          if (status != 0 || last) flag |= LB_SEAT_DONE;
         } else {
           reject = true;
           last = false;
           if (accepted >= 1) ++rejected;
         }
         h = hn;
+        L.flag[tid] = flag;
+      }
+      __syncthreads();
+      const uint32_t took = seats(LB_SEAT_ACCEPT);
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        if (!(took >> t & 1u)) continue;
+        const double xo = L.x[t], xn = xo + hs[t];
+        if (step_push) {
+          push(t, xn, yn[t]);
+        } else {
+          const DevEffCall& C = fresh_args<EffArgs>().C;
+          while (si[t] < C.n_saveat && C.saveat[si[t]] <= xn + time_tol(xn)) {
+            const double ts = C.saveat[si[t]];
+            if (ts >= xo - time_tol(xo)) {
+              if (fabs(ts - xo) <= time_tol(xo)) {
+                push(t, ts, y[t]);
+              } else if (fabs(ts - xn) <= time_tol(xn)) {
+                push(t, ts, yn[t]);
+              } else {
+                double ds[R], kt[8][R];
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+#pragma unroll
+                  for (int r = 0; r < R; ++r) kt[j][r] = k[j][t][r];
+                eff_dense<R, SOLVER>((ts - xo) / hs[t], hs[t], y[t], yn[t], kt, ds);
+                push(t, ts, ds);
+              }
+            }
+            ++si[t];
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          y[t][r] = yn[t][r];
+          k[1][t][r] = k[7][t][r];
+        }
       }
     }
-#undef LB_EFF_RHS
-    if (status == 0 && !step_push && si != C.n_saveat) {
-      status = LB_TRAJ_SAVEAT;
-      fail_x = (double)si;
-    }
-    if (status == 0 && !want_int && n_pushed > C.capacity) status = LB_TRAJ_CAPACITY;
-    if (tid == 0) {
+    // ---- finished trajectories
+    if (tid < T && (flag & LB_SEAT_DONE)) {
+      const DevEffCall& C = fresh_args<EffArgs>().C;
+      int64_t np = 0, sv = 0;
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        if (tid == t) {
+          np = n_pushed[t];
+          sv = si[t];
+        }
+      if (status == 0 && !step_push && sv != C.n_saveat) {
+        status = LB_TRAJ_SAVEAT;
+        fail_x = (double)sv;
+      }
+      if (status == 0 && !want_int && np > C.capacity) status = LB_TRAJ_CAPACITY;
       if (want_int) {
-        C.out_values[traj * C.capacity] = status == 0 ? integral : __builtin_nan("");
-        if (C.out_times) C.out_times[traj * C.capacity] = last_t;
-        C.out_counts[traj] = n_pushed > 0 ? 1 : 0;
+        C.out_values[traj * C.capacity] = status == 0 ? L.pi[tid] : __builtin_nan("");
+        if (C.out_times) C.out_times[traj * C.capacity] = L.pt[tid];
+        C.out_counts[traj] = np > 0 ? 1 : 0;
       } else {
-        C.out_counts[traj] = (int32_t)n_pushed;
+        C.out_counts[traj] = (int32_t)np;
       }
       C.out_stats[4 * traj + 0] = accepted;
       C.out_stats[4 * traj + 1] = rejected;
       C.out_stats[4 * traj + 2] = rhs_calls;
       C.out_stats[4 * traj + 3] = status;
       C.out_fail_t[traj] = fail_x;
+      flag = 0;
     }
   }
+#undef LB_EFF_RHS
 }
 
 // One effective RHS per workgroup (debug_effective_lindblad_rhs_py): the
@@ -5482,42 +5759,43 @@ template <int R, int MAXW>
 __global__ __launch_bounds__(MAXW, 1) void lb_eff_rhs_kernel(const DevEffPlan P, const DevEffCall C,
                                                              const DevEffRhsCall Q) {
   const int tid = threadIdx.x, W = blockDim.x;
-  const LdsEff L = carve_eff(P);
+  const LdsEff L = carve_eff(P, 1, P.S);
+  int row[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) row[r] = tid + W * r < P.S ? P.row[tid + W * r] : -1;
   for (int64_t b = blockIdx.x; b < Q.batch; b += gridDim.x) {
     __syncthreads();
     if (tid == 0) {
-      L.misc[1] = 0;
-      L.misc[2] = 0;
-      L.sp[2] = eff_params(P, C, 0, L.slots, Q.t[b], L.vm, L.sp);
-      eff_lookup(P, L, 0);
+      int status = 0, hint = 0;
+      double fail_x;
+      eff_params(P, C, 0, L.slots, Q.t[b], L.vm, L.sp);
+      eff_lookup(P, L.sp, hint, status, fail_x);
+      Q.status[b] = status;
     }
     __syncthreads();
-    double y[R], k[R];
+    double y[1][R], k[1][R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int row = tid + W * r;
-      y[r] = row < P.D ? Q.y[b * (int64_t)P.D + row] : 0.0;
+      y[0][r] = row[r] >= 0 ? Q.y[b * (int64_t)P.D + row[r]] : 0.0;
+      k[0][r] = 0.0;
     }
-    eff_rhs<R>(P, L.ybuf, y, k, L.sp, tid, W);
+    eff_rhs<R, 1, 0, true>(P, L.ybuf, y, k, L.sp, 1u, row, tid, W);
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int row = tid + W * r;
-      if (row < P.D) Q.out[b * (int64_t)P.D + row] = k[r];
-    }
-    if (tid == 0) Q.status[b] = L.misc[1];
+    for (int r = 0; r < R; ++r)
+      if (row[r] >= 0) Q.out[b * (int64_t)P.D + row[r]] = k[0][r];
   }
 }
 
 extern "C" void* lb_dev_eff_kernel(int id, int solver) {
-#define E(i, r, w, v) \
-  if (id == i) return solver == 1 ? (void*)&lb_eff_kernel<r, 1, w, v> : (void*)&lb_eff_kernel<r, 0, w, v>;
+#define E(i, r, w, v, t) \
+  if (id == i) return solver == 1 ? (void*)&lb_eff_kernel<r, 1, w, v, t> : (void*)&lb_eff_kernel<r, 0, w, v, t>;
   LB_EFF_CONFIGS(E)
 #undef E
   return nullptr;
 }
 
 extern "C" void* lb_dev_eff_rhs_kernel(int id) {
-#define E(i, r, w, v) \
+#define E(i, r, w, v, t) \
   if (id == i) return (void*)&lb_eff_rhs_kernel<r, w>;
   LB_EFF_CONFIGS(E)
 #undef E

@@ -158,9 +158,9 @@ extern "C" int lb_dev_fixed_variant(int id, int* R, int* maxw) {
   return 0;
 }
 
-extern "C" int lb_dev_eff_variant(int id, int* R, int* maxw) {
-#define E(i, r, w, v)                                                                           \
-  if (id == i) { *R = r; *maxw = w; return 1; }
+extern "C" int lb_dev_eff_variant(int id, int* R, int* maxw, int* seats) {
+#define E(i, r, w, v, t)                                                                        \
+  if (id == i) { *R = r; *maxw = w; *seats = t; return 1; }
   LB_EFF_CONFIGS(E)
 #undef E
   return 0;

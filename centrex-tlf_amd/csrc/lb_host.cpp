@@ -16,6 +16,7 @@
 #include <memory>
 #include <mutex>
 #include <numeric>
+#include <unordered_map>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -196,16 +197,28 @@ struct lb_plan {
 
 namespace {
 
-template <typename T>
-int upload(DevImage* im, const std::vector<T>& host, const T** out) {
-  size_t bytes = std::max<size_t>(host.size(), 1) * sizeof(T);
-  void* d = nullptr;
-  HIP_TRY(hipMalloc(&d, bytes));
-  im->allocations.push_back(d);
-  if (!host.empty()) HIP_TRY(hipMemcpy(d, host.data(), host.size() * sizeof(T), hipMemcpyHostToDevice));
-  *out = static_cast<const T*>(d);
-  return LB_OK;
-}
+// The tables of one image, packed into one device allocation and one copy (an
+// allocation and a copy each were a third of a plan's creation).
+struct TablePack {
+  std::vector<char> bytes;
+  std::vector<std::pair<const void**, size_t>> at;  // device pointer to set, offset
+  template <typename T>
+  void add(const std::vector<T>& host, const T** out) {
+    const size_t off = (bytes.size() + 255) / 256 * 256;
+    bytes.resize(off + std::max<size_t>(host.size(), 1) * sizeof(T));
+    if (!host.empty()) std::memcpy(bytes.data() + off, host.data(), host.size() * sizeof(T));
+    at.push_back({reinterpret_cast<const void**>(out), off});
+  }
+  int upload(DevImage* im) {
+    bytes.resize(bytes.size() + 4096);  // program records are fetched one ahead
+    void* d = nullptr;
+    HIP_TRY(hipMalloc(&d, bytes.size()));
+    im->allocations.push_back(d);
+    HIP_TRY(hipMemcpy(d, bytes.data(), bytes.size(), hipMemcpyHostToDevice));
+    for (const auto& a : at) *a.first = static_cast<char*>(d) + a.second;
+    return LB_OK;
+  }
+};
 
 // Simulated stack depth of one expression; rejects what the device machine
 // does not evaluate (temps, tuple helpers, unknown ids).
@@ -363,7 +376,24 @@ Couplings merge_couplings(const PlanSource& src, const std::vector<uint8_t>& act
   };
   Couplings out;
   out.of.resize(src.U);
-  std::map<std::vector<EntryTerm>, int> dyn_id, stat_id;
+  struct Hash {
+    size_t operator()(const std::vector<EntryTerm>& v) const {
+      uint64_t h = v.size();
+      auto mix = [&](uint64_t x) { h = (h ^ x) * 0x9E3779B97F4A7C15ull; h ^= h >> 29; };
+      for (const EntryTerm& t : v) {
+        uint64_t re, im;
+        // -0.0 and 0.0 compare equal
+        const double fr = t.re + 0.0, fi = t.im + 0.0;
+        std::memcpy(&re, &fr, 8);
+        std::memcpy(&im, &fi, 8);
+        mix(t.coef);
+        mix(re);
+        mix(im);
+      }
+      return h;
+    }
+  };
+  std::unordered_map<std::vector<EntryTerm>, int, Hash> dyn_id, stat_id;
   auto is_dyn = [&](const std::vector<EntryTerm>& v) {
     for (const EntryTerm& t : v) {
       const uint32_t k = t.coef & 0x7FFFFFFFu;
@@ -839,10 +869,8 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   P.max_self = max_self;
   P.time_dependent = src.time_dependent ? 1 : 0;
   P.restricted = n_act < U ? 1 : 0;
-  int rc = LB_OK;
-  auto up = [&](auto& v, auto** dst) {
-    if (rc == LB_OK) rc = upload(im, v, dst);
-  };
+  TablePack tables;
+  auto up = [&](auto& v, auto** dst) { tables.add(v, dst); };
   up(slot_up, &P.slot_up);
   up(slot_re, &P.slot_re);
   up(slot_im, &P.slot_im);
@@ -897,6 +925,7 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   up(t_rows, &P.t_blk_rows);
   up(t_word, &P.t_word);
   up(t_f, &P.t_f);
+  const int rc = tables.upload(im);
   if (rc != LB_OK) return rc;
   const int solve_rows = P.couplings ? c_total : rows_total;
   pick_config(S, solve_rows, &im->default_variant, &im->default_W);
@@ -1864,7 +1893,7 @@ int lb_adjoint_launch(const lb_plan* p, const lb_solve_args* a, void* stream, vo
   }
   grid = (int)std::min<int64_t>(grid, a->n_traj);
   // workspace: ckpt_every recomputed attempts per resident workgroup (y and
-  // k1..k7, per segment buffer, and the seven coefficient rows of each), in
+  // k1..k7 (or the stages' sums), per segment buffer, and the seven coefficient rows of each), in
   // doubles
   const size_t per_y = (size_t)a->ckpt_every * 8 * S * 2 * (wave ? wave_bufs : 1);
   const size_t per_c = (size_t)a->ckpt_every * 7 * (im->dev.KD + 1) * 2;

@@ -207,9 +207,9 @@ class DevicePlan:
         self._spec_warned = False
 
     def specialize(self, enable: bool = True) -> "DevicePlan":
-        """``lb_plan_specialize``: run the paired kernels of this plan with its
+        """``lb_plan_specialize``: run the one-wave kernels of this plan with its
         time-dependent coefficient programs compiled in (bitwise the values of
-        the expression machine).  Each (variant, solver) compiles on its first
+        the expression machine).  Each (form, solver) compiles on its first
         solve, about 2 s; a plan without time dependence is unchanged."""
         _check(library().lb_plan_specialize(self._handle, 1 if enable else 0))
         self.specialized = bool(enable)

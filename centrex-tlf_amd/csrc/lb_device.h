@@ -350,7 +350,7 @@ struct DevCall {
                            // adjoint before the launch is marked broken (< 0: broken from the start)
   int32_t adj_row_batch;   // multi-wave adjoint: attempts whose coefficient rows one pass evaluates
   // adjoint workspace (per workgroup) and output
-  double* seg_y;           // workgroups x ckpt_every x 8 x S x 2: y and k1..k7 of each attempt
+  double* seg_y;           // workgroups x ckpt_every x 8 x S x 2: of each attempt y and k1..k7, or the stages' sums
   double* seg_c;           // workgroups x ckpt_every x 7 x (KD + 1) x 2: coefficient rows
   double* out_grad;        // n_traj x (n_diff - diff_time): d(integral)/d(parameter)
   // replay: take the accepted step sizes of a recorded tape (stride tape_cap)

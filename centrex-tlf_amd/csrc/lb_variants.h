@@ -20,7 +20,8 @@
 // Paired variants for plans of at most 32 elements: two trajectories per wave
 // (one per 32-lane half); Q(id, gather rows in registers, waves-per-SIMD
 // hint).  Only for persistent calls that push at every accepted step with a
-// given initial step (no trace, save plan or replay; a tape may be recorded).
+// given initial step (no trace, save plan or replay; a tape may be recorded);
+// the forms compiled per plan cover more (lb_host.cpp).
 #define LB_PAIR_CONFIGS(Q) Q(15, 4, 2) Q(16, 8, 2) Q(17, 12, 2)
 
 // Fixed-step kernel variants (fixed_dopri5 / fixed_rk2 / fixed_rk4):

@@ -140,18 +140,19 @@ int lb_plan_create(const lb_plan_desc* desc, lb_plan** out_plan);
 void lb_plan_destroy(lb_plan* plan);
 
 /*
- * Plan-specialised paired kernels (no counterpart in the reference, whose
+ * Plan-specialised one-wave kernels (no counterpart in the reference, whose
  * Rust RHS interprets the coefficient programs on every call,
  * rust/src/lindblad/eval.rs:791-911).  With enable != 0, the plan's
  * time-dependent compound and coefficient programs are emitted as
- * straight-line device code; the first lb_solve call that takes a paired
- * variant for a solver compiles that variant with the code at run time
- * (hiprtc, about 2 s) and later calls reuse it.  Values are bitwise those of
- * the expression machine.  A plan without time dependence is left as it is.
+ * straight-line device code; the first lb_solve call that takes a one-wave
+ * kernel of a form (plans of at most 64 elements, persistent mode with dt
+ * given: final outputs, tapes, traces, save plans, stop events, fixed steps)
+ * compiles that form with the code at run time (hiprtc, about 2 s) and later
+ * calls reuse it.  Values are bitwise those of the expression machine.  A plan without time dependence is left as it is.
  * Returns LB_ERR_UNSUPPORTED (with the reason) when an instruction has no
  * generated form.  When the run-time compilation or the module load of a
- * variant fails, lb_solve runs the precompiled kernel instead (bitwise the
- * same results), never tries that variant again for the plan, and records
+ * form fails, lb_solve runs the precompiled kernel instead (bitwise the
+ * same results), never tries that form again for the plan, and records
  * the reason for lb_plan_specialize_status.  The environment variable
  * CENTREX_LB_RTC_OPTIONS, when set, is appended to the compile options
  * (whitespace-separated; a diagnostic hook).
@@ -305,8 +306,9 @@ typedef struct lb_solve_args {
    * (dopri5.rs:280-317, tsit5.rs:274-309), the step end for the fixed-step ones
    * (fixed.rs:213-238).  The root is pushed once as the last point; save-plan
    * points past it are not pushed and are not an error.  Final outputs hold the
-   * state at the root.  Runs on the multi-wave kernels (the single-wave and
-   * paired forms are not used for such a call); no tapes or replays. */
+   * state at the root.  Runs on the plan-specialised one-wave kernels where
+   * they apply (adaptive solvers), else on the multi-wave ones; no tapes or
+   * replays. */
   int32_t event_kind;             /* LB_EVENT_* */
   int32_t n_event_indices;        /* population: diagonal indices summed in this order */
   const int32_t* event_indices;   /* host */

@@ -16,11 +16,14 @@
 // (computed once per trajectory), and the "gather" terms read other elements
 // that the owning threads publish to LDS.
 //
-// Couplings.  The gather terms of an output that read the same element (with
-// the same conjugation) are merged into one coupling v * x_in, v = sum f_g
-// c_g(t); on a diagonal output, whose imaginary part is zero, a term and its
-// conjugate merge into twice the one (their sum is twice its real part).  The
-// distinct values v of a plan are its entries.  They are evaluated once per
+// Couplings.  In plans of one block and differentiable ones the gather terms
+// of an output that read the same element (with the same conjugation) are
+// merged into one coupling v * x_in, v = sum f_g c_g(t); on a diagonal output,
+// whose imaginary part is zero, a term and its conjugate merge into twice the
+// one (their sum is twice its real part).  In the others each term is a
+// coupling of its own, with the value and the place in the sum that it has in
+// the gather form, so both forms round alike.  The distinct values v of a plan
+// are its entries.  They are evaluated once per
 // stage into LDS (the time-independent ones once per trajectory), so a
 // coupling is four FMAs on two 16-byte LDS reads, and its table is one word.
 #pragma once

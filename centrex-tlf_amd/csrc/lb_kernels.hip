@@ -468,12 +468,22 @@ __device__ __forceinline__ void stage_combo(double h, const double (&y_r)[R], co
 }
 
 // The step-size controller (common.rs:32-70): alpha = 0.2 - 0.75 beta, beta =
-// 0.04, safety 0.9, the step's factor within [1/5, 10].  The reference's h /
-// (err^alpha fac_old^-beta / 0.9) is h times 0.9 exp(beta ln fac_old - alpha
-// ln err): one log of the squared norm and one exp.  ln fac_old = max(ln err,
-// ln 1e-4) is carried from the last accepted step.  As two pow, a square root
-// and three divisions one after another the chain was 3.1k of a paired
-// attempt's 15k cycles.  A NaN error norm is a rejection with the largest cut.
+// 0.04, safety 0.9, the step's factor within [1/5, 10].  Two forms.
+//
+// StepPowers is the reference's h / (err^alpha fac_old^-beta / 0.9) operation
+// by operation, the two powers at once in the halves of every wave.  Plans of
+// several blocks take it: over the 10,000 steps and more of a 72-level flight,
+// whose drive jumps, a rounding of the step sizes grows 10,000-fold (an input
+// moved by one rounding moves the populations by 1e-12 to 5e-12 in norm), so
+// another form of the same controller gives other digits there.
+//
+// StepControl, for plans of one block and the effective Hamiltonian, is h times
+// 0.9 exp(beta ln fac_old - alpha ln err): one log of the squared norm and one
+// exp, ln fac_old = max(ln err, ln 1e-4) carried from the last accepted step.
+// The other form's chain of two pow, a square root and three divisions was 3.1k
+// of a paired attempt's 15k cycles (64 x 64 grid 1.73 against 1.61 ms; 318
+// against 312 ms in the 512 + 512 uneven batch); photon counts move by 1e-15.
+// A NaN error norm is a rejection with the largest cut in both.
 #define LB_LOG_FAC_MIN -9.210340371976182  // ln 1e-4
 struct StepControl {
   double err, lerr, raw;  // error norm, its log, the factor before its bounds
@@ -490,6 +500,27 @@ struct StepControl {
   }
   // the factor is one of its bounds (no dependence on err or fac_old)
   __device__ __forceinline__ bool clamped() const { return accept ? !(raw < 10.0 && raw > 0.2) : !(raw > 0.2); }
+};
+
+struct StepPowers {
+  double err, div;  // error norm, what the step is divided by before its bounds
+  bool accept;
+  // q = err^2; every lane of the wave calls
+  __device__ __forceinline__ StepPowers(double q, double fac_old, int tid) {
+    const double beta = 0.04, alpha = 0.2 - beta * 0.75, safety = 0.9;
+    err = sqrt(q);
+    accept = err <= 1.0;
+    const bool low = (tid & 63) < 32;
+    const double pw = pow(low ? err : fac_old, low ? alpha : -beta);
+    const double fac11 = __shfl(pw, 0, 64), fo = __shfl(pw, 32, 64);
+    div = (accept ? fac11 * fo : fac11) / safety;
+  }
+  __device__ __forceinline__ double next(double h) const {
+    return accept ? h / fmax(1.0 / 10.0, fmin(1.0 / 0.2, div)) : h / fmin(1.0 / 0.2, div);
+  }
+  __device__ __forceinline__ bool clamped() const {
+    return accept ? !(div > 1.0 / 10.0 && div < 1.0 / 0.2) : !(div < 1.0 / 0.2);
+  }
 };
 
 template <int R>
@@ -1359,7 +1390,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         push(t0, y_r, y_i, true);
       }
       // ---- controller state (common.rs:32-70)
-      const double hmax = fabs(t1 - t0), inv_dim = 1.0 / (double)P.dim;
+      const double hmax = fabs(t1 - t0);
       double fac_old = 1.0e-4, lfo = LB_LOG_FAC_MIN;
       bool reject = false, last = false;
       int64_t ns = 0, nst = 0, ia = 0;
@@ -1492,9 +1523,23 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           }
         }
         __syncthreads();
-        const StepControl ctl(replay ? 0.0 : block_total(P, L.red, 0) * inv_dim, lfo);
-        const double err = ctl.err;
-        double hn = h * ctl.factor();
+        double err, hn;
+        bool accept, clamped;
+        const double e2 = replay ? 0.0 : block_total(P, L.red, 0);
+        if (G == 0 && (LEAN || P.nblk > 1)) {
+          const StepPowers ctl(e2 / (double)P.dim, fac_old, tid);
+          err = ctl.err;
+          accept = ctl.accept;
+          clamped = ctl.clamped();
+          hn = ctl.next(h);
+        } else {
+          const StepControl ctl(e2 * (1.0 / (double)P.dim), lfo);
+          err = ctl.err;
+          accept = ctl.accept;
+          clamped = ctl.clamped();
+          hn = h * ctl.factor();
+          if (accept) lfo = fmax(ctl.lerr, LB_LOG_FAC_MIN);
+        }
         if (tape && !replay) {
           const KernelArgs& A = fresh_args();
           const DevPlan& P = A.P;
@@ -1505,8 +1550,8 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           if (a < C.tape_cap) {
             if (tid == 0) {
               int fl = clipped ? LB_TAPE_CLIPPED : 0;
-              if (ctl.clamped()) fl |= LB_TAPE_CLAMPED;
-              if (ctl.accept) {
+              if (clamped) fl |= LB_TAPE_CLAMPED;
+              if (accept) {
                 fl |= LB_TAPE_ACCEPTED | (accepted == 0 ? LB_TAPE_FIRST : 0) | (err > 1.0e-4 ? LB_TAPE_ERRQ : 0);
                 double hc = hn;
                 if (fabs(hc) > hmax) { hc = hmax; fl |= LB_TAPE_HMAX; }
@@ -1534,9 +1579,8 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
             }
           }
         }
-        if (ctl.accept) {
+        if (accept) {
           fac_old = fmax(err, 1.0e-4);
-          lfo = fmax(ctl.lerr, LB_LOG_FAC_MIN);
           if (fabs(hn) > hmax) hn = hmax;
           if (reject) hn = fmin(fabs(hn), fabs(h));
           reject = false;

@@ -5,7 +5,8 @@ coefficients on one coupling, a term and its conjugate on a diagonal output,
 conjugated inputs.  The sizes are the edges of the tables: one block with few
 rows, with as many as the paired forms hold, and several blocks.  A chain
 whose every term has a factor of its own has more entries than a workgroup
-holds, and takes the gather tables."""
+holds, and takes the gather tables.  Plans of several blocks give bitwise the
+right-hand side of the gather tables."""
 
 from __future__ import annotations
 
@@ -97,3 +98,35 @@ def test_lean_form_is_bitwise_the_general_form(solver, variant):
     for b, n in enumerate(counts.cpu().numpy()):
         assert n == int(stats[b, 0]) + 1 and bool((rows[b, n - 1] == final[b]).all())
     assert bool((integral == lean_integral).all())
+
+
+def in_gather_form(flat: dict) -> dict:
+    """The plan with further terms on every output, each of a value and an input
+    of its own: too many values for the coupling tables, and at 1e-300 too small
+    to change a rounded sum."""
+    ptrs = np.asarray(flat["output_ptrs"])
+    outputs = len(ptrs) - 1
+    each = -(-4200 // outputs)
+    at = np.repeat(ptrs[1:], each)
+    value = 1e-300 * (1.0 + np.arange(at.size) / at.size)
+    inputs = (np.repeat(np.arange(outputs), each) + np.tile(np.arange(each), outputs)) % outputs
+    extra = dict(input_indices=inputs, coeff_indices=-1, factors_re=value,
+                 factors_im=-value, input_conj=1, coeff_conj=0)
+    out = dict(flat, output_ptrs=ptrs + (each * np.arange(outputs + 1)).astype(ptrs.dtype))
+    for name, v in extra.items():
+        old = np.asarray(flat[name])
+        out[name] = np.ascontiguousarray(np.insert(old, at, np.asarray(v).astype(old.dtype)))
+    return out
+
+
+@pytest.mark.parametrize("case", ["n39", "dense 12"])
+def test_several_blocks_round_as_the_gather_tables(case):
+    torch = require_gpu()
+    system, params = tlf_n39()[:2] if case == "n39" else dense_system(12)
+    prepared = prepare_lindblad_problem(system, params, backend="host")
+    plans = [DevicePlan(prepared.flat_plan), DevicePlan(in_gather_form(prepared.flat_plan))]
+    n = 39 if case == "n39" else 12
+    ys = torch.as_tensor(np.stack([prepared.layout.pack(random_density(n, seed=s)) for s in range(3)]), device="cuda")
+    ts = torch.as_tensor(np.asarray([0.0, 0.3, 1.7]) * (1e-6 if case == "n39" else 1.0), device="cuda")
+    got, want = (plan.rhs(ys, ts) for plan in plans)
+    assert float(want.abs().max()) > 0.1 and int(((got - want).abs() >= 1e-290).sum()) == 0

@@ -147,6 +147,7 @@ struct DevImage {
   int64_t lds_bytes = 0;
   int64_t n_pub = 0, gather_terms = 0, self_terms = 0, rows_total = 0, flops = 0, active = 0;
   std::vector<uint8_t> active_mask;  // upper_len
+  std::unique_ptr<DevImage> gather;  // the same elements as gather tables (launch_table), built on first use
   std::map<std::pair<const void*, int>, int> per_cu;  // (kernel, W) -> resident workgroups per CU
   void* ws_y = nullptr;  // adjoint workspace (grow-only)
   void* ws_c = nullptr;
@@ -186,8 +187,12 @@ struct lb_plan {
       if (im->ws_c) (void)hipFree(im->ws_c);
       if (im->ws_done) (void)hipEventDestroy(im->ws_done);
     };
-    release(full.get());
-    for (auto& kv : restricted) release(kv.second.get());
+    auto release_all = [&](DevImage* im) {
+      if (im) release(im->gather.get());
+      release(im);
+    };
+    release_all(full.get());
+    for (auto& kv : restricted) release_all(kv.second.get());
     if (ev_copied) (void)hipEventSynchronize(ev_copied);
     if (ev_dev) (void)hipFree(ev_dev);
     if (ev_pinned) (void)hipHostFree(ev_pinned);
@@ -317,6 +322,12 @@ constexpr int64_t kMaxVectorBytes = 24 * 1024;
 constexpr int64_t kMaxLdsBytes = 160 * 1024;
 
 int64_t lds_bytes_for(const DevPlan& P) { return lb_lds_layout(P).total; }
+bool lds_fits(const DevPlan& P) { return lds_bytes_for(P) <= kMaxLdsBytes; }
+// The interpreted form of the time-dependent programs, which needs less LDS.
+void drop_steps(DevPlan& P) {
+  P.v_steps = P.v_n_const = 0;
+  P.v_slots = P.n_slots;
+}
 int64_t lds_bytes_pair(const DevPlan& P, int nh = 2) { return lb_lds_pair(P, (uint32_t)nh).total; }
 
 int set_lds_limit(const void* fn, size_t lds) {
@@ -487,8 +498,9 @@ Couplings merge_couplings(const PlanSource& src, const std::vector<uint8_t>& act
   return out;
 }
 
-// Lane layout and device tables for the active elements `act` (lb_device.h).
-int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage* im) {
+// Lane layout and device tables for the active elements `act` (lb_device.h);
+// `couplings`: as couplings where they fit, else as gather tables.
+int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage* im, bool couplings = true) {
   const int n = src.n, U = src.U;
   auto is_dyn = [&](int64_t k) { return src.coeff_indices[k] >= 0 && src.coef_dyn[src.coeff_indices[k]]; };
   // ---- split terms of active outputs into self (own element, time-independent
@@ -578,8 +590,9 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   P.v_slots = P.v_steps > 0 ? im->vec.n_slots : P.n_slots;
   P.v_time = im->vec.time_slot;
   P.n_pub = one_block ? n_act : (int)std::count(published.begin(), published.end(), (uint8_t)1);
-  // Couplings, when their entries (and the rest of a workgroup's LDS) fit;
-  // the gather tables otherwise.
+  // Couplings, when their entries (and the rest of a workgroup's LDS) fit,
+  // without the programs in steps where only that fits; the gather tables
+  // otherwise.
   // Merged, an output's sum is rounded otherwise than term by term.  Plans of
   // one block and differentiable ones merge: their results move by 1e-15
   // (gradients by 1e-13).  Larger plans keep a coupling per term, applied in the
@@ -596,13 +609,14 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   P.nv_terms = (int32_t)std::min<int64_t>(cpl.dyn_terms, 1 << 20);
   P.lds_tables = 0;
   P.c_rows_total = P.g_rows = 0;
-  if (P.v_steps > 0 && 16 * 8 * (int64_t)(P.v_slots + P.v_steps) > kMaxVectorBytes) {
-    P.v_steps = 0;  // a long program stays interpreted
-    P.v_slots = P.n_slots;
-  }
-  if (P.nv_dyn + P.nv_stat > LB_MAX_ENTRIES || P.n_pub > LB_MAX_COUPLED ||
-      16 * (int64_t)(P.nv_stat + LB_ENT_ROWS * P.nv_dyn) + 20 * (int64_t)P.nv_terms > kMaxLdsBytes ||
-      lds_bytes_for(P) > kMaxLdsBytes) {
+  P.v_n_const = (int32_t)im->vec.const_slot.size();
+  if (P.v_steps == 0 || 16 * 8 * (int64_t)(P.v_slots + P.v_steps) > kMaxVectorBytes)
+    drop_steps(P);  // a long program stays interpreted
+  const DevPlan with_steps = P;
+  if (!lds_fits(P)) drop_steps(P);
+  if (!couplings || P.nv_dyn + P.nv_stat > LB_MAX_ENTRIES || P.n_pub > LB_MAX_COUPLED ||
+      16 * (int64_t)(P.nv_stat + LB_ENT_ROWS * P.nv_dyn) + 20 * (int64_t)P.nv_terms > kMaxLdsBytes || !lds_fits(P)) {
+    P = with_steps;
     P.couplings = 0;
     P.nv_dyn = P.nv_stat = P.nv_terms = 0;
   }
@@ -749,7 +763,7 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
     add({EntryTerm{(uint32_t)src.K, 0.0, 0.0}});
     P.c_rows_total = c_total;
     P.lds_tables = 1;
-    if (4 * 64 * (int64_t)c_total > kLdsTableBytes || lds_bytes_for(P) > kMaxLdsBytes) P.lds_tables = 0;
+    if (4 * 64 * (int64_t)c_total > kLdsTableBytes || !lds_fits(P)) P.lds_tables = 0;
   }
   // transposed couplings and contractions of a differentiable plan
   std::vector<int32_t> tc_row0(nblk, 0), tc_rows(nblk, 0);
@@ -874,7 +888,10 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   P.n_base = src.n_base;
   P.n_compounds = src.prog.n_compounds;
   P.g_rows = rows_total;
-  if (!P.couplings) P.lds_tables = (int64_t)rows_total * 64 * 20 <= kLdsTableBytes ? 1 : 0;
+  if (!P.couplings) {
+    P.lds_tables = (int64_t)rows_total * 64 * 20 <= kLdsTableBytes ? 1 : 0;
+    if (!lds_fits(P)) drop_steps(P);
+  }
   P.max_self = max_self;
   P.time_dependent = src.time_dependent ? 1 : 0;
   P.restricted = n_act < U ? 1 : 0;
@@ -921,7 +938,6 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   up(src.expr_dyn, &P.expr_dyn);
   up(ex_all, &P.ex_all);
   up(ex_dyn, &P.ex_dyn);
-  P.v_n_const = P.v_steps > 0 ? (int32_t)im->vec.const_slot.size() : 0;
   up(im->vec.const_slot, &P.v_const_slot);
   up(im->vec.const_value, &P.v_const);
   up(im->vec.ops, &P.v_ops);
@@ -1299,6 +1315,24 @@ int select_image(lb_plan* p, const uint8_t* y0_support, const DevImage** out, bo
   return LB_OK;
 }
 
+// The elements of `im` in gather form, for a call whose LDS leaves no room for
+// the entries; built on first use and kept with the image.
+int gather_image(lb_plan* p, const DevImage* im, const DevImage** out) {
+  std::lock_guard<std::mutex> lock(p->mu);
+  std::unique_ptr<DevImage>& g = const_cast<DevImage*>(im)->gather;
+  if (!g) {
+    std::unique_ptr<DevImage> made(new DevImage());
+    const int rc = build_image(p->src, im->active_mask, made.get(), false);
+    if (rc != LB_OK) {
+      for (void* a : made->allocations) (void)hipFree(a);
+      return rc;
+    }
+    g = std::move(made);
+  }
+  *out = g.get();
+  return LB_OK;
+}
+
 }  // namespace
 
 extern "C" int lb_rhs_eval(const lb_plan* p, int64_t batch, const double* y, const double* t,
@@ -1548,12 +1582,23 @@ int launch_table(const lb_plan* p, const lb_solve_args* a, const DevImage* im, D
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "kernel variant is not built");
   void* reset = lb_dev_queue_reset_kernel();
   hipStream_t s = (hipStream_t)stream;
+  // The stop-event expression runs on lane 0's stack.  A deep one takes the
+  // place of the tables, of the programs in steps, and at last of the entries.
   DevPlan P = im->dev;
-  P.vm_depth = std::max(P.vm_depth, ev_depth);  // the stop-event expression runs on lane 0's stack
-  if (lds_bytes_for(P) > kMaxLdsBytes && P.couplings) P.lds_tables = 0;  // a deep expression's stack
+  auto fit = [&]() {
+    P.vm_depth = std::max(P.vm_depth, ev_depth);
+    if (!lds_fits(P)) P.lds_tables = 0;
+    if (!lds_fits(P)) drop_steps(P);
+    return lds_fits(P);
+  };
+  int rc = LB_OK;
+  if (!fit() && P.couplings) {
+    if ((rc = gather_image(const_cast<lb_plan*>(p), im, &im))) return rc;
+    P = im->dev;
+    fit();
+  }
   const size_t lds = (size_t)lds_bytes_for(P);
-  int rc = set_lds_limit(fn, lds);
-  if (rc) return rc;
+  if ((rc = set_lds_limit(fn, lds))) return rc;
   int slot = 0;
   if ((rc = const_cast<lb_plan*>(p)->queues.acquire(s, &c.queue, &slot))) return rc;
   if (a->mode == LB_MODE_PLAIN) {

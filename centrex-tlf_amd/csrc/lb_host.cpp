@@ -30,13 +30,12 @@ extern "C" int lb_dev_variant_count(void);
 extern "C" int lb_dev_variant(int id, int* R, int* maxw, int* waves);
 extern "C" int lb_dev_variant_rows(int id);
 extern "C" int lb_dev_variant_pair(int id);
-extern "C" int lb_dev_adjoint_variant(int id, int* R, int* maxw, int* rows);
+extern "C" int lb_dev_adjoint_variant(int id, int* R, int* maxw, int* rows, int* block);
 extern "C" int lb_dev_fixed_variant(int id, int* R, int* maxw);
 extern "C" void* lb_dev_fixed_kernel(int id, int solver);
 extern "C" int lb_dev_event_variant(int id, int* R, int* maxw);
 extern "C" void* lb_dev_event_kernel(int id, int solver);
 extern "C" void* lb_dev_adjoint_kernel(int id, int solver);
-extern "C" void* lb_dev_adjoint_block_kernel(int S, int solver, int* W);
 extern "C" void* lb_dev_solve_kernel(int id, int solver);
 extern "C" void* lb_dev_lean_kernel(int id, int solver);
 extern "C" void* lb_dev_rhs_kernel(int id);
@@ -1864,10 +1863,13 @@ int lb_adjoint_launch(const lb_plan* p, const lb_solve_args* a, void* stream, vo
                 "the adjoint of the adaptive solve needs the time derivative programs (lb_plan_desc.diff_time = 1)");
   c.adj_mode = a->adjoint_mode;
   // A plan of one 64-slot block whose gather rows and LDS fit takes the
-  // single-block adjoint (lane = slot, several waves per trajectory);
-  // otherwise the multi-wave variant with the fewest slots per thread that
-  // covers the plan.  args->variant = k + 1 forces adjoint variant k (both
-  // forms compute the same derivative).
+  // single-block adjoint (lane = slot, several waves per trajectory); others
+  // the multi-wave form over couplings where the plan has them (and its
+  // programs as steps) and it covers the plan: 64 gradients at 72 levels 72 ms
+  // against 282 ms in the form over gather tables, which takes the rest.  Of a
+  // form, the variant with the fewest slots per thread that covers the plan.
+  // args->variant = k + 1 names adjoint variant k; all compute the same
+  // derivative.
   const int S = im->dev.S;
   int wave_bufs =
       lds_bytes_adj_wave(im->dev, im->g_rows_host, im->t_rows_host, a->ckpt_every, 2) <= kMaxLdsBytes ? 2 : 1;
@@ -1887,37 +1889,39 @@ int lb_adjoint_launch(const lb_plan* p, const lb_solve_args* a, void* stream, vo
     return im->dev.nblk == 1 && !im->g_rows_host.empty() && im->g_rows_host[0] <= rows &&
            lds_wave <= kMaxLdsBytes;
   };
-  int id = -1, W = 0, R = 0, maxw = 0, rows = 0;
-  bool wave = false;
-  if (a->variant > 0) {
-    if (!lb_dev_adjoint_variant(a->variant - 1, &R, &maxw, &rows))
-      return fail(LB_ERR_INVALID, "no such adjoint variant");
+  const bool block_fits =
+      im->dev.couplings && im->dev.nv_def > 0 && (!im->dev.time_dependent || im->dev.v_steps_all > 0);
+  int id = -1, W = 0;
+  bool wave = false, block = false;
+  // whether variant v covers the plan; takes it if so
+  auto take = [&](int v, int R, int maxw, int rows, int is_block) {
+    const int w = rows > 0 ? wave_threads : std::max(64, ((S + R - 1) / R + 63) / 64 * 64);
+    if (rows > 0 ? !wave_fits(rows) : w > maxw || (is_block && !block_fits)) return false;
+    id = v;
+    W = w;
     wave = rows > 0;
-    W = wave ? wave_threads : std::max(64, ((S + R - 1) / R + 63) / 64 * 64);
-    if (wave ? !wave_fits(rows) : W > maxw)
+    block = is_block != 0;
+    return true;
+  };
+  int R = 0, maxw = 0, rows = 0, is_block = 0;
+  if (a->variant > 0) {
+    if (!lb_dev_adjoint_variant(a->variant - 1, &R, &maxw, &rows, &is_block))
+      return fail(LB_ERR_INVALID, "no such adjoint variant");
+    if (!take(a->variant - 1, R, maxw, rows, is_block))
       return fail(LB_ERR_INVALID, "the adjoint variant does not cover this plan");
-    id = a->variant - 1;
   } else {
-    for (int v = 0; lb_dev_adjoint_variant(v, &R, &maxw, &rows); ++v)
-      if (rows > 0 && wave_fits(rows)) { id = v; W = wave_threads; wave = true; break; }
-    for (int v = 0; id < 0 && lb_dev_adjoint_variant(v, &R, &maxw, &rows); ++v) {
-      if (rows > 0) continue;
-      const int w = std::max(64, ((S + R - 1) / R + 63) / 64 * 64);
-      if (w <= maxw) { id = v; W = w; }
-    }
+    auto first_of = [&](bool want_wave, bool want_block) {
+      for (int v = 0; id < 0 && lb_dev_adjoint_variant(v, &R, &maxw, &rows, &is_block); ++v)
+        if ((rows > 0) == want_wave && (is_block != 0) == want_block) take(v, R, maxw, rows, is_block);
+    };
+    first_of(true, false);
+    first_of(false, true);
+    first_of(false, false);
   }
   if (id < 0) return fail(LB_ERR_UNSUPPORTED, "plan is too large for the adjoint kernel variants");
-  // The multi-wave form over couplings, for plans that have them (and their
-  // programs as steps): 64 gradients at 72 levels 72 ms against 282 ms in the
-  // gather form.  It has shapes of its own and computes the same derivative as
-  // the variant named.
-  void* fn = nullptr;
-  if (!wave && im->dev.couplings && im->dev.nv_def > 0 && (!im->dev.time_dependent || im->dev.v_steps_all > 0))
-    fn = lb_dev_adjoint_block_kernel(S, a->solver, &W);
-  const bool block = fn != nullptr;
-  if (!block) fn = lb_dev_adjoint_kernel(id, a->solver);
+  void* fn = lb_dev_adjoint_kernel(id, a->solver);
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "adjoint kernel variant is not built");
-  // the multi-wave form evaluates the coefficient rows of E attempts per pass
+  // the form over gather tables evaluates the coefficient rows of E attempts per pass
   // (7E lanes): the largest E of 8, 4, 2 whose LDS keeps the workgroups per CU
   // that E = 1 has (the registers often allow one workgroup per CU anyway)
   int row_batch = 1;

@@ -6006,10 +6006,6 @@ extern "C" void* LB_PART_FN(lb_dev_adjoint_kernel)(int id, int solver) {
   if (id == i) return adjoint_wave_ptr<i, g, v>(solver);
   LB_ADJ_WAVE_CONFIGS(V)
 #undef V
-  return nullptr;
-}
-
-extern "C" void* LB_PART_FN(lb_dev_adjoint_block_kernel)(int id, int solver) {
 #define B(i, r, w, v) \
   if (id == i) return adjoint_block_ptr<i, r, w, v>(solver);
   LB_ADJ_BLOCK_CONFIGS(B)

@@ -42,14 +42,6 @@ extern "C" void* lb_dev_adjoint_kernel_p4(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p5(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p6(int, int);
 extern "C" void* lb_dev_adjoint_kernel_p7(int, int);
-extern "C" void* lb_dev_adjoint_block_kernel_p0(int, int);
-extern "C" void* lb_dev_adjoint_block_kernel_p1(int, int);
-extern "C" void* lb_dev_adjoint_block_kernel_p2(int, int);
-extern "C" void* lb_dev_adjoint_block_kernel_p3(int, int);
-extern "C" void* lb_dev_adjoint_block_kernel_p4(int, int);
-extern "C" void* lb_dev_adjoint_block_kernel_p5(int, int);
-extern "C" void* lb_dev_adjoint_block_kernel_p6(int, int);
-extern "C" void* lb_dev_adjoint_block_kernel_p7(int, int);
 extern "C" void* lb_dev_rhs_kernel_p0(int);
 extern "C" void* lb_dev_rhs_kernel_p1(int);
 extern "C" void* lb_dev_rhs_kernel_p2(int);
@@ -132,15 +124,20 @@ extern "C" void* lb_dev_rhs_kernel(int id) {
 // Adjoint variants: Z(id, R, largest workgroup, waves hint), then the
 // single-wave V(id, gather rows, waves hint) with *rows = gather rows (0 for
 // the multi-wave form).
-extern "C" int lb_dev_adjoint_variant(int id, int* R, int* maxw, int* rows) {
+// rows > 0: a single-block variant; block: a multi-wave one over couplings.
+extern "C" int lb_dev_adjoint_variant(int id, int* R, int* maxw, int* rows, int* block) {
 #define Z(i, r, w, v)                                                                           \
-  if (id == i) { *R = r; *maxw = w; *rows = 0; return 1; }
+  if (id == i) { *R = r; *maxw = w; *rows = 0; *block = 0; return 1; }
   LB_ADJ_CONFIGS(Z)
 #undef Z
 #define V(i, g, v)                                                                              \
-  if (id == i) { *R = 1; *maxw = 64; *rows = g; return 1; }
+  if (id == i) { *R = 1; *maxw = 64; *rows = g; *block = 0; return 1; }
   LB_ADJ_WAVE_CONFIGS(V)
 #undef V
+#define B(i, r, w, v)                                                                           \
+  if (id == i) { *R = r; *maxw = w; *rows = 0; *block = 1; return 1; }
+  LB_ADJ_BLOCK_CONFIGS(B)
+#undef B
   return 0;
 }
 
@@ -182,18 +179,4 @@ extern "C" void* lb_dev_event_kernel(int id, int solver) {
 extern "C" void* lb_dev_fixed_kernel(int id, int solver) {
   void* (*parts[])(int, int) = {lb_dev_fixed_kernel_p0, lb_dev_fixed_kernel_p1, lb_dev_fixed_kernel_p2, lb_dev_fixed_kernel_p3, lb_dev_fixed_kernel_p4, lb_dev_fixed_kernel_p5, lb_dev_fixed_kernel_p6, lb_dev_fixed_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);
-}
-
-// The block adjoint's shape of the fewest slots per lane that covers S slots
-// (and its workgroup size); null where none does.
-extern "C" void* lb_dev_adjoint_block_kernel(int S, int solver, int* W) {
-  void* (*parts[])(int, int) = {lb_dev_adjoint_block_kernel_p0, lb_dev_adjoint_block_kernel_p1, lb_dev_adjoint_block_kernel_p2, lb_dev_adjoint_block_kernel_p3, lb_dev_adjoint_block_kernel_p4, lb_dev_adjoint_block_kernel_p5, lb_dev_adjoint_block_kernel_p6, lb_dev_adjoint_block_kernel_p7};
-#define B(i, r, w, v)                              \
-  if (S <= (r) * (w)) {                            \
-    *W = ((S + (r) - 1) / (r) + 63) / 64 * 64;     \
-    return parts[(i) % LB_NPARTS_BUILT](i, solver); \
-  }
-  LB_ADJ_BLOCK_CONFIGS(B)
-#undef B
-  return nullptr;
 }

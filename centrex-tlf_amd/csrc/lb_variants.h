@@ -36,18 +36,20 @@
 #define LB_EFF_CONFIGS(E) \
   E(0, 1, 512, 2, 4) E(1, 1, 512, 2, 2) E(2, 1, 512, 2, 1) E(3, 1, 1024, 4, 1) E(4, 4, 512, 2, 1) E(5, 8, 512, 1, 1)
 
-// Adjoint kernel variants: Z(id, slots per thread R, largest workgroup, waves-per-SIMD hint).
+// Adjoint kernel variants over gather tables: Z(id, slots per thread R, largest
+// workgroup, waves-per-SIMD hint).
 #define LB_ADJ_CONFIGS(Z) Z(0, 1, 1024, 2) Z(1, 2, 512, 2) Z(2, 4, 256, 2) Z(3, 8, 256, 2)
-
-// Multi-wave adjoint over couplings: B(id, slots per thread R, largest
-// workgroup, waves-per-SIMD hint).  Two waves a SIMD: with 128 registers (one
-// slot a lane, 1024 threads) three times as many values spilled.
-#define LB_ADJ_BLOCK_CONFIGS(B) B(4, 1, 512, 2) B(5, 2, 512, 2) B(6, 4, 512, 2)
 
 // Single-block adjoint variants for plans of one 64-slot block (lane = slot,
 // several waves per trajectory): V(id, gather rows held in registers by
 // the recomputation, waves-per-SIMD hint), in increasing rows (the host takes
 // the first that covers the plan).
 #define LB_ADJ_WAVE_CONFIGS(V) V(4, 12, 2) V(5, 16, 2)
+
+// Multi-wave adjoint over couplings: B(id, slots per thread R, largest
+// workgroup, waves-per-SIMD hint), in increasing slots (the host takes the
+// first that covers the plan).  Two waves a SIMD: with 128 registers (one
+// slot a lane, 1024 threads) three times as many values spilled.
+#define LB_ADJ_BLOCK_CONFIGS(B) B(6, 1, 512, 2) B(7, 2, 512, 2) B(8, 4, 512, 2)
 
 #define LB_NPARTS_BUILT 8

@@ -255,7 +255,10 @@ typedef struct lb_solve_args {
                                      instead of the reference's two solves) */
   int32_t variant;                /* kernel variant: 0 = plan default, k = variant k-1
                                      (slots per thread / occupancy; results are
-                                     bitwise independent of it) */
+                                     bitwise independent of it).  lb_adjoint counts
+                                     variants of its own: 1..4 over gather tables,
+                                     5 and 6 for plans of 64 slots, 7..9 over
+                                     couplings (equal to rounding) */
   int32_t n_saveat;               /* > 0: push points at these times (dense output inside steps),
                                      otherwise at t0 (save_start) and every accepted step */
   const double* saveat;           /* device, ascending, within [t0, t1] (the save plan of

@@ -1,7 +1,8 @@
 """The multi-wave adjoint over couplings: dense systems with every kind of
 entry (time-independent and time-dependent parameters, complex factors, two
 coefficients on one coupling), one to four slots a lane, and a plan whose
-entries do not fit, which takes the gather form."""
+entries do not fit, which takes the gather form.  Every shape of both forms that
+covers a plan gives the same gradient of one tape."""
 
 from __future__ import annotations
 
@@ -11,6 +12,7 @@ import sympy as smp
 
 from centrex_tlf_amd.lindblad import prepare_lindblad_problem
 from centrex_tlf_amd.lindblad.adjoint import DifferentiablePhotonCount
+from centrex_tlf_amd.lindblad.native import NativeError
 from centrex_tlf_amd.lindblad.systems import OBESystem
 
 from ._dense import chain_system, random_density
@@ -57,6 +59,12 @@ def chain_problem(n: int, unique_factors: bool):
     return prepared, ["omega0", "delta", "frequency"], 0.6
 
 
+# the shapes (1-based variants) over couplings and over gather tables that cover
+# 64, 128, 832 and 1,856 slots
+SHAPES = {"dense 4": ((7, 8, 9), (1, 2, 3, 4)), "dense 12": ((7, 8, 9), (1, 2, 3, 4)),
+          "chain 40": ((8, 9), (1, 2, 3, 4)), "chain 60": ((9,), (4,)), "chain 60 unique": ((), (4,))}
+
+
 @pytest.mark.parametrize("solver", ["dopri5", "tsit5"])
 @pytest.mark.parametrize("case", ["dense 4", "dense 12", "chain 40", "chain 60", "chain 60 unique"])
 def test_matches_finite_differences_of_the_replayed_steps(case, solver):
@@ -69,8 +77,10 @@ def test_matches_finite_differences_of_the_replayed_steps(case, solver):
     base = np.asarray([complex(prepared.parameters.base_parameters[k]).real for k in names])
     p = base * (1.0 + np.asarray([[0.0], [0.1], [-0.2]]))
     counts, tape = engine.forward(p, y0)
-    frozen = engine.gradient(p, y0, tape, mode="frozen", variant=1 if n == 4 else 0).cpu().numpy()
-    adaptive = engine.gradient(p, y0, tape, variant=1 if n == 4 else 0).cpu().numpy()
+    block, gather = SHAPES[case]
+    variant = block[0] if n == 4 else 0  # a plan of one block takes the single-block form by itself
+    frozen = engine.gradient(p, y0, tape, mode="frozen", variant=variant).cpu().numpy()
+    adaptive = engine.gradient(p, y0, tape, variant=variant).cpu().numpy()
     fd, fd_adaptive, same = np.zeros_like(p), np.zeros_like(p), np.ones(len(p), dtype=bool)
     for m in range(p.shape[1]):
         hi, lo = p.copy(), p.copy()
@@ -88,7 +98,14 @@ def test_matches_finite_differences_of_the_replayed_steps(case, solver):
     # an attempt count that changes under +-D is a jump of the adaptive map
     assert same.any()
     np.testing.assert_allclose(adaptive[same], fd_adaptive[same], rtol=0, atol=bound + 2 * NOISE / D * share)
-    if n == 4:  # the single-block form, the default of a plan this small
+    # 0: the single-block form for n = 4, the form above for the others; 5 and 6
+    # are the single-block shapes of 12 and 16 gather rows
+    for v in (0, 1, 2, 3, 4, 7, 8, 9) if n == 4 else range(10):
+        if v not in (0,) + block + gather:
+            with pytest.raises(NativeError, match="does not cover"):
+                engine.gradient(p, y0, tape, variant=v)
+            continue
         for mode, got in (("frozen", frozen), ("adaptive", adaptive)):
-            other = engine.gradient(p, y0, tape, mode=mode).cpu().numpy()
-            np.testing.assert_allclose(got, other, rtol=0, atol=1e-12 * scale + 2 * NOISE * share)
+            other = engine.gradient(p, y0, tape, mode=mode, variant=v).cpu().numpy()
+            np.testing.assert_allclose(got, other, rtol=0, atol=1e-12 * scale + 2 * NOISE * share,
+                                       err_msg=f"{mode}, variant {v}")

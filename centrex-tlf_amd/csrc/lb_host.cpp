@@ -15,6 +15,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <numeric>
 #include <unordered_map>
 #include <string>
@@ -2174,7 +2175,7 @@ int eff_config(const DevEffPlan& P, int seats, int* id, int* W, int* T, size_t* 
 
 }  // namespace
 
-extern "C" int lb_eff_plan_create(const lb_eff_plan_desc* d, lb_eff_plan** out_plan) {
+extern "C" int lb_eff_plan_create(const lb_eff_plan_desc* d, lb_eff_plan** out_plan) try {
   if (!out_plan) return fail(LB_ERR_INVALID, "out_plan is null");
   *out_plan = nullptr;
   if (!d || d->n_states <= 0) return fail(LB_ERR_INVALID, "n_states must be positive");
@@ -2199,7 +2200,7 @@ extern "C" int lb_eff_plan_create(const lb_eff_plan_desc* d, lb_eff_plan** out_p
   int rc;
   if ((rc = eff_upload(p.get(), std::vector<double>(d->field_grid, d->field_grid + d->n_grid), &P.grid))) return rc;
   std::vector<int32_t> rp[3];
-  int64_t apart = 0;  // cells of the operators sliced one by one, by which a plan's size is judged
+  int64_t in_order = 0;  // cells with the rows in their own order
   for (int o = 0; o < 3; ++o) {
     const int64_t nnz = d->nnz[o];
     if (nnz < 0 || nnz > INT32_MAX / 4) return fail(LB_ERR_UNSUPPORTED, "operator has too many stored entries");
@@ -2216,36 +2217,49 @@ extern "C" int lb_eff_plan_create(const lb_eff_plan_desc* d, lb_eff_plan** out_p
     for (int64_t q = 0; q < nnz; ++q)
       if (d->col_indices[o][q] < 0 || d->col_indices[o][q] >= D)
         return fail(LB_ERR_INVALID, "operator column index out of range");
-    apart = 0;
+    int64_t cells = 0;
     for (int b = 0; b < P.nblk; ++b) {
       int longest = 0;
       for (int r = 64 * b; r < std::min(D, 64 * b + 64); ++r) longest = std::max(longest, rp[o][r + 1] - rp[o][r]);
-      apart += 64 * (int64_t)longest;
+      cells += 64 * (int64_t)longest;
     }
-    if (apart * (int64_t)std::max(d->n_grid - 1, 1) > ((int64_t)1 << 31))
+    if (cells * (int64_t)std::max(d->n_grid - 1, 1) > ((int64_t)1 << 31))
       return fail(LB_ERR_UNSUPPORTED, "operator tables too large in sliced form");
+    in_order += cells;
   }
   {
-    // the sliced form (lb_device.h); padding cells are zero
+    // the sliced form (lb_device.h); padding cells are zero.  Rows in
+    // decreasing number of entries, unless that pads more than their own order
+    // (rows of one length whose entries lie in different operators), so no plan
+    // takes more cells than the size check above allows.
     const int S = P.S, nblk = P.nblk, GI = d->n_grid - 1;
     std::vector<int32_t> len(3 * (size_t)S, 0), row(S, -1);
     auto entries = [&](int o, int r) { return rp[o][r + 1] - rp[o][r]; };
     auto all = [&](int r) { return entries(0, r) + entries(1, r) + entries(2, r); };
-    std::iota(row.begin(), row.begin() + D, 0);
-    std::stable_sort(row.begin(), row.begin() + D, [&](int a, int b) { return all(a) > all(b); });
     std::vector<int64_t> sp;
     int64_t cells = 0;
-    for (int b = 0; b < nblk; ++b)
-      for (int o = 0; o < 3; ++o) {
-        int longest = 0;
-        for (int s = 64 * b; s < std::min(D, 64 * b + 64); ++s) {
-          len[(size_t)o * S + s] = entries(o, row[s]);
-          longest = std::max(longest, entries(o, row[s]));
+    auto slice = [&]() {
+      sp.clear();
+      cells = 0;
+      for (int b = 0; b < nblk; ++b)
+        for (int o = 0; o < 3; ++o) {
+          int longest = 0;
+          for (int s = 64 * b; s < std::min(D, 64 * b + 64); ++s) {
+            len[(size_t)o * S + s] = entries(o, row[s]);
+            longest = std::max(longest, entries(o, row[s]));
+          }
+          sp.push_back(cells);
+          cells += 64 * (int64_t)longest;
         }
-        sp.push_back(cells);
-        cells += 64 * (int64_t)longest;
-      }
-    sp.push_back(cells);
+      sp.push_back(cells);
+    };
+    std::iota(row.begin(), row.begin() + D, 0);
+    std::stable_sort(row.begin(), row.begin() + D, [&](int a, int b) { return all(a) > all(b); });
+    slice();
+    if (cells > in_order) {
+      std::iota(row.begin(), row.begin() + D, 0);
+      slice();
+    }
     std::vector<uint32_t> scol(std::max<int64_t>(cells, 1), 0);
     std::vector<double2> lo((size_t)std::max<int64_t>(cells * GI, 1), double2{0.0, 0.0}), hi(lo);
     for (int s = 0; s < D; ++s)
@@ -2323,6 +2337,8 @@ extern "C" int lb_eff_plan_create(const lb_eff_plan_desc* d, lb_eff_plan** out_p
   if (lds_bytes_eff_limit(P) > kMaxLdsBytes) return fail(LB_ERR_UNSUPPORTED, "effective plan needs more LDS than a workgroup has");
   *out_plan = p.release();
   return LB_OK;
+} catch (const std::bad_alloc&) {
+  return fail(LB_ERR_UNSUPPORTED, "not enough host memory for the operator tables");
 }
 
 extern "C" void lb_eff_plan_destroy(lb_eff_plan* p) { delete p; }

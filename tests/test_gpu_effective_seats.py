@@ -1,14 +1,20 @@
 """Effective-Hamiltonian trajectories that share a workgroup give bitwise the
 results of a workgroup each: batches of one, two and four seats per workgroup
 (by the number of trajectories), fields in different grid intervals and off the
-grid, odd batches, every output kind and both ways to take the first step."""
+grid, odd batches, every output kind and both ways to take the first step.
+Rows are sorted by length only where that does not pad the tables more."""
 
 from __future__ import annotations
 
 import numpy as np
 import pytest
 
-from centrex_tlf_amd.lindblad.effective import prepare_effective_lindblad_plan, split_real_rho
+from centrex_tlf_amd.lindblad.effective import (
+    debug_effective_lindblad_rhs,
+    effective_operator_payload,
+    prepare_effective_lindblad_plan,
+    split_real_rho,
+)
 
 from ._effective import random_plan_dict
 from ._gpu import require_gpu
@@ -46,3 +52,29 @@ def test_seats_are_bitwise_a_workgroup_each(n, density, solver, dt):
                 assert bool((got[k].nan_to_num(7.0) == ref.nan_to_num(7.0)).all()), (call["output_kind"], rows, k)
     status = got[1][:, 3].cpu().numpy()
     assert 0 < (status != 0).sum() < len(status)  # a field above the grid ends its own trajectory only
+
+
+def test_rows_keep_their_order_where_sorting_pads_more():
+    """Rows 0..63 hold 1..64 entries of one operator, rows 64..127 of another:
+    in their own order 64 + 64 cells a lane, sorted by length 64 + 64 + 32 + 32."""
+    torch = require_gpu()
+    n, grid = 8, np.linspace(-1.0, 1.0, 400)
+    plan = random_plan_dict(n=n, n_grid=2, seed=1)
+    rng = np.random.default_rng(2)
+    first, second = np.zeros((128, 128)), np.zeros((128, 128))
+    for r in range(64):
+        first[r, : r + 1] = rng.normal(size=r + 1)
+        second[64 + r, 127 - r:] = rng.normal(size=r + 1)
+    for key, m in (("sparse_combined", first), ("sparse_opt", second), ("sparse_det", 0 * first)):
+        plan[key] = effective_operator_payload([m] * grid.size, grid)
+    plan.update(n_grid=grid.size, field_grid=grid)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    plan = prepare_effective_lindblad_plan(plan)
+    used = free - torch.cuda.mem_get_info()[0]
+    cells = 32 * 399 * 64 * 128  # 32 bytes a cell and grid interval
+    assert used < 1.25 * cells, (used, cells)
+    y = rng.normal(size=128)
+    got = np.asarray(debug_effective_lindblad_rhs(plan, y, 2.5)["dy"])
+    want = first @ y + 0.5 * second @ y  # the pulse's top, Omega = 1
+    np.testing.assert_allclose(got, want, rtol=0, atol=1e-13 * np.abs(want).max())

@@ -31,6 +31,7 @@ extern "C" int lb_dev_variant_count(void);
 extern "C" int lb_dev_variant(int id, int* R, int* maxw, int* waves);
 extern "C" int lb_dev_variant_rows(int id);
 extern "C" int lb_dev_variant_pair(int id);
+extern "C" int lb_dev_variant_shape(int id, int rows);
 extern "C" int lb_dev_adjoint_variant(int id, int* R, int* maxw, int* rows, int* block);
 extern "C" int lb_dev_fixed_variant(int id, int* R, int* maxw);
 extern "C" void* lb_dev_fixed_kernel(int id, int solver);
@@ -1753,7 +1754,7 @@ extern "C" int lb_solve(const lb_plan* p, const lb_solve_args* a, void* stream) 
   if (pair_ok && !lb_dev_variant_rows(id) && im->dev.nblk > 1 && im->dev.couplings &&
       (!im->dev.time_dependent || im->dev.v_steps > 0))
     fn = lb_dev_lean_kernel(id, a->solver);
-  if (!fn) fn = lb_dev_solve_kernel(id, a->solver);
+  if (!fn) fn = lb_dev_solve_kernel(lb_dev_variant_shape(id, (int)im->rows_total), a->solver);
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "kernel variant is not built");
   void* reset = lb_dev_queue_reset_kernel();
   hipStream_t s = (hipStream_t)stream;
@@ -2089,7 +2090,7 @@ extern "C" int lb_launch_info(const lb_plan* p, const uint8_t* y0_support, int32
   if (rc) return rc;
   int id, W;
   if ((rc = resolve_config(im, variant, threads_per_traj, true, &id, &W))) return rc;
-  void* fn = lb_dev_solve_kernel(id, LB_SOLVER_DOPRI5);
+  void* fn = lb_dev_solve_kernel(lb_dev_variant_shape(id, (int)im->rows_total), LB_SOLVER_DOPRI5);
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "kernel variant is not built");
   const size_t lds = (size_t)(lb_dev_variant_pair(id) ? lds_bytes_pair(im->dev) : im->lds_bytes);
   if ((rc = set_lds_limit(fn, lds))) return rc;

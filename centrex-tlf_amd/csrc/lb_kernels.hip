@@ -5969,6 +5969,7 @@ extern "C" void* LB_PART_FN(lb_dev_solve_kernel)(int id, int solver) {
 #define Q(i, g, v) \
   if (id == i) return pair_solve_ptr<i, g, v>(solver);
   LB_PAIR_CONFIGS(Q)
+  LB_PAIR_NARROW(Q)
 #undef Q
   return nullptr;
 }

@@ -105,6 +105,15 @@ extern "C" int lb_dev_variant_rows(int id) {
   return 0;
 }
 
+// The shape that runs variant `id` on a plan of `rows` coupling rows.
+extern "C" int lb_dev_variant_shape(int id, int rows) {
+#define Q(i, g, v) \
+  if (id == 15 && rows <= g) return i;
+  LB_PAIR_NARROW(Q)
+#undef Q
+  return id;
+}
+
 extern "C" void* lb_dev_solve_kernel(int id, int solver) {
   void* (*parts[])(int, int) = {lb_dev_solve_kernel_p0, lb_dev_solve_kernel_p1, lb_dev_solve_kernel_p2, lb_dev_solve_kernel_p3, lb_dev_solve_kernel_p4, lb_dev_solve_kernel_p5, lb_dev_solve_kernel_p6, lb_dev_solve_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);

@@ -18,11 +18,14 @@
 #define LB_WAVE_CONFIGS(Y) Y(11, 8, 4) Y(12, 8, 2) Y(13, 16, 2) Y(14, 12, 2)
 
 // Paired variants for plans of at most 32 elements: two trajectories per wave
-// (one per 32-lane half); Q(id, gather rows in registers, waves-per-SIMD
+// (one per 32-lane half); Q(id, coupling rows in registers, waves-per-SIMD
 // hint).  Only for persistent calls that push at every accepted step with a
 // given initial step (no trace, save plan or replay; a tape may be recorded);
-// the forms compiled per plan cover more (lb_host.cpp).
-#define LB_PAIR_CONFIGS(Q) Q(15, 4, 2) Q(16, 8, 2) Q(17, 12, 2)
+// the forms compiled per plan cover more (lb_host.cpp).  Variant 15 runs plans
+// of at most four rows in a shape of their own, which needs fewer registers
+// (two-level scan 2.37 against 3.04 ms, n=39 grid 2.70 against 2.96).
+#define LB_PAIR_CONFIGS(Q) Q(15, 8, 2) Q(16, 12, 2)
+#define LB_PAIR_NARROW(Q) Q(17, 4, 2)
 
 // Fixed-step kernel variants (fixed_dopri5 / fixed_rk2 / fixed_rk4):
 // F(id, slots per thread R, largest workgroup, waves-per-SIMD hint).

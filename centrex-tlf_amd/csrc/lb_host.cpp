@@ -30,7 +30,8 @@
 extern "C" int lb_dev_variant_count(void);
 extern "C" int lb_dev_variant(int id, int* R, int* maxw, int* waves);
 extern "C" int lb_dev_variant_rows(int id);
-extern "C" int lb_dev_variant_pair(int id);
+extern "C" int lb_dev_variant_wave(int id);
+extern "C" int lb_dev_variant_of(int id);
 extern "C" int lb_dev_variant_shape(int id, int rows);
 extern "C" int lb_dev_adjoint_variant(int id, int* R, int* maxw, int* rows, int* block);
 extern "C" int lb_dev_fixed_variant(int id, int* R, int* maxw);
@@ -278,12 +279,11 @@ int check_expression(const lb_plan_desc* d, int start, int end, int n_slots, std
   return 0;
 }
 
-// Smallest workgroup (multiple of 64) with which variant `id` covers S slots
-// and `rows` gather rows, or 0.
-int variant_threads(int id, int S, int rows) {
+// Smallest workgroup (multiple of 64) with which variant `id` covers S slots,
+// or 0.
+int variant_threads(int id, int S) {
   int R, maxw, waves;
   if (!lb_dev_variant(id, &R, &maxw, &waves)) return 0;
-  if (const int g = lb_dev_variant_rows(id)) return (S <= 64 && rows <= g) ? 64 : 0;
   int W = ((S + R - 1) / R + 63) / 64 * 64;
   if (W < 64) W = 64;
   return W <= maxw ? W : 0;
@@ -292,21 +292,20 @@ int variant_threads(int id, int S, int rows) {
 // Default variant: the most registers per lane that still keeps two
 // workgroups' worth of waves per SIMD pair, then the least padding.  The
 // autotuner (centrex_tlf_amd.lindblad.autotune) replaces this by measurement.
-void pick_config(int S, int rows, int* id_out, int* W_out) {
+void pick_config(int S, int* id_out, int* W_out) {
   int best = -1, bestW = 0;
   int64_t bestScore = INT64_MAX;
   for (int id = 0; id < lb_dev_variant_count(); ++id) {
     int R, maxw, waves;
     lb_dev_variant(id, &R, &maxw, &waves);
-    if (lb_dev_variant_pair(id)) continue;  // chosen per call (lb_solve)
-    int W = variant_threads(id, S, rows);
+    if (lb_dev_variant_rows(id)) continue;  // chosen per call (lb_solve)
+    int W = variant_threads(id, S);
     if (!W) continue;
     const int64_t waste = (int64_t)R * W - S;
-    const int g = lb_dev_variant_rows(id);
-    // single-wave variants first: the fewest register rows that hold the
-    // plan, at two waves per SIMD (256 registers per lane, no spills)
-    const int64_t score = g ? -1000 + g + (waves == 2 ? 0 : 1)
-                            : waste + (waves == 2 ? 0 : 256) + 8 * R;
+    // single-wave variants first, at two waves per SIMD (256 registers per
+    // lane, no spills)
+    const int64_t score = lb_dev_variant_wave(id) ? -1000 + (waves == 2 ? 0 : 1)
+                                                  : waste + (waves == 2 ? 0 : 256) + 8 * R;
     if (score < bestScore) { bestScore = score; best = id; bestW = W; }
   }
   *id_out = best;
@@ -636,16 +635,13 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   std::vector<int> slot_el(S, -1);  // slot -> element, or -1
   {
     std::vector<int> brows(nblk, 0);
-    int rows_sum = 0;
-    for (int b = 0; b < nblk; ++b) {
+    for (int b = 0; b < nblk; ++b)
       for (int l = 0; l < 64 && 64 * b + l < n_act; ++l) brows[b] = std::max(brows[b], n_rows[order[64 * b + l]]);
-      rows_sum += brows[b];
-    }
     std::vector<int> pos_of(nblk);
     std::iota(pos_of.begin(), pos_of.end(), 0);
     int id = -1, W = 0, R = 1, maxw = 0, waves = 0;
-    pick_config(S, rows_sum, &id, &W);
-    if (nblk > 1 && id >= 0 && lb_dev_variant(id, &R, &maxw, &waves) && !lb_dev_variant_rows(id) && R > 1) {
+    pick_config(S, &id, &W);
+    if (nblk > 1 && id >= 0 && lb_dev_variant(id, &R, &maxw, &waves) && R > 1) {
       const int nw = W / 64;
       std::vector<int> load(nw, 0), next_r(nw, 0), cap(nw, 0);
       for (int w = 0; w < nw; ++w)
@@ -954,14 +950,14 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   const int rc = tables.upload(im);
   if (rc != LB_OK) return rc;
   const int solve_rows = P.couplings ? c_total : rows_total;
-  pick_config(S, solve_rows, &im->default_variant, &im->default_W);
+  pick_config(S, &im->default_variant, &im->default_W);
   // paired variant: the fewest register rows holding a one-block plan of <= 32 elements
   im->pair_variant = -1;
   if (nblk == 1 && n_act <= 32 && P.couplings) {
     int best_g = 1 << 30;
     for (int id = 0; id < lb_dev_variant_count(); ++id) {
       const int g = lb_dev_variant_rows(id);
-      if (lb_dev_variant_pair(id) && solve_rows <= g && g < best_g) { best_g = g; im->pair_variant = id; }
+      if (g && solve_rows <= g && g < best_g) { best_g = g; im->pair_variant = id; }
     }
   }
   im->lds_bytes = lds_bytes_for(P);
@@ -1233,8 +1229,7 @@ int resolve_config(const DevImage* p, int variant, int threads, bool pair_ok, in
     *W = 64;
     return LB_OK;
   }
-  if (variant > 0 && lb_dev_variant_pair(variant - 1)) {
-    const int g = lb_dev_variant_rows(variant - 1);
+  if (const int g = variant > 0 ? lb_dev_variant_rows(variant - 1) : 0) {
     if (!pair_ok || p->pair_variant < 0 || p->rows_total > g)
       return fail(LB_ERR_UNSUPPORTED,
                   "a paired variant needs a plan of at most 32 elements (and its gather rows) and a persistent "
@@ -1251,10 +1246,10 @@ int resolve_config(const DevImage* p, int variant, int threads, bool pair_ok, in
   }
   int R, maxw, waves;
   if (variant > 0) {
-    *id = variant - 1;
+    *id = lb_dev_variant_of(variant - 1);
     if (!lb_dev_variant(*id, &R, &maxw, &waves)) return fail(LB_ERR_INVALID, "unknown kernel variant");
-    *W = threads ? threads : variant_threads(*id, p->dev.S, (int)p->rows_total);
-    if (lb_dev_variant_rows(*id) && (*W != 64 || !variant_threads(*id, p->dev.S, (int)p->rows_total)))
+    *W = threads ? threads : variant_threads(*id, p->dev.S);
+    if (lb_dev_variant_wave(*id) && (*W != 64 || p->dev.S > 64))
       return fail(LB_ERR_UNSUPPORTED, "single-wave variant needs a plan of at most 64 elements");
     if (!*W || *W > maxw || (int64_t)R * *W < p->dev.S)
       return fail(LB_ERR_UNSUPPORTED, "kernel variant does not cover the plan with this workgroup size");
@@ -1263,7 +1258,7 @@ int resolve_config(const DevImage* p, int variant, int threads, bool pair_ok, in
   // threads given: the variant with the fewest slots per thread that covers the plan
   for (int v = 0; v < lb_dev_variant_count(); ++v) {
     lb_dev_variant(v, &R, &maxw, &waves);
-    if (lb_dev_variant_rows(v)) continue;
+    if (lb_dev_variant_rows(v) || lb_dev_variant_wave(v)) continue;
     if (threads <= maxw && (int64_t)R * threads >= p->dev.S) {
       *id = v;
       *W = threads;
@@ -1271,6 +1266,18 @@ int resolve_config(const DevImage* p, int variant, int threads, bool pair_ok, in
     }
   }
   return fail(LB_ERR_UNSUPPORTED, "no kernel variant covers the plan with this workgroup size");
+}
+
+// The precompiled kernel of variant `id`.  pair_ok (but for the launch mode) is
+// what the lean form of a multi-wave kernel covers of a call; of a plan it needs
+// several blocks (it has their controller only), couplings and, where it is
+// time-dependent, its programs as steps: 512 + 512 trajectories, 72 levels,
+// 310 ms against 390 ms in the general form.
+void* solve_kernel(const DevImage* im, int id, int solver, bool pair_ok) {
+  const DevPlan& P = im->dev;
+  void* fn = nullptr;
+  if (pair_ok && P.nblk > 1 && P.couplings && (!P.time_dependent || P.v_steps > 0)) fn = lb_dev_lean_kernel(id, solver);
+  return fn ? fn : lb_dev_solve_kernel(lb_dev_variant_shape(id, (int)im->rows_total), solver);
 }
 
 int fill_overrides(const lb_plan* p, int32_t n, const int32_t* slots, int32_t* dst) {
@@ -1738,23 +1745,14 @@ extern "C" int lb_solve(const lb_plan* p, const lb_solve_args* a, void* stream) 
   const bool pair_ok = a->mode == LB_MODE_PERSISTENT && !a->trace && a->n_saveat == 0 &&
                        !a->replay_h && std::isfinite(a->dt) && a->dt > 0.0 && a->output_kind != LB_OUT_RATE;
   if ((rc = resolve_config(im, a->variant, a->threads_per_traj, pair_ok, &id, &W))) return rc;
-  const bool pair = lb_dev_variant_pair(id) != 0;
+  const bool pair = lb_dev_variant_rows(id) != 0;
   // a single-wave variant named for a plan that pairs is that variant
-  if (pair || (lb_dev_variant_rows(id) && (a->variant <= 0 || im->active > 32))) {
+  if (pair || (lb_dev_variant_wave(id) && (a->variant <= 0 || im->active > 32))) {
     bool launched = false;
     rc = launch_spec(const_cast<lb_plan*>(p), a, im, c, (hipStream_t)stream, false, 0, &launched);
     if (rc || launched) return rc;
   }
-  // pair_ok (but for the launch mode) is what the lean form of a multi-wave
-  // kernel covers of a call; of a plan it needs several blocks (it has their
-  // controller only), couplings and, where it is time-dependent, its programs
-  // as steps: 512 + 512 trajectories, 72 levels, 310 ms against 390 ms in the
-  // general form.
-  void* fn = nullptr;
-  if (pair_ok && !lb_dev_variant_rows(id) && im->dev.nblk > 1 && im->dev.couplings &&
-      (!im->dev.time_dependent || im->dev.v_steps > 0))
-    fn = lb_dev_lean_kernel(id, a->solver);
-  if (!fn) fn = lb_dev_solve_kernel(lb_dev_variant_shape(id, (int)im->rows_total), a->solver);
+  void* fn = solve_kernel(im, id, a->solver, pair_ok);
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "kernel variant is not built");
   void* reset = lb_dev_queue_reset_kernel();
   hipStream_t s = (hipStream_t)stream;
@@ -2090,9 +2088,9 @@ extern "C" int lb_launch_info(const lb_plan* p, const uint8_t* y0_support, int32
   if (rc) return rc;
   int id, W;
   if ((rc = resolve_config(im, variant, threads_per_traj, true, &id, &W))) return rc;
-  void* fn = lb_dev_solve_kernel(lb_dev_variant_shape(id, (int)im->rows_total), LB_SOLVER_DOPRI5);
+  void* fn = solve_kernel(im, id, LB_SOLVER_DOPRI5, true);
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "kernel variant is not built");
-  const size_t lds = (size_t)(lb_dev_variant_pair(id) ? lds_bytes_pair(im->dev) : im->lds_bytes);
+  const size_t lds = (size_t)(lb_dev_variant_rows(id) ? lds_bytes_pair(im->dev) : im->lds_bytes);
   if ((rc = set_lds_limit(fn, lds))) return rc;
   int per_cu = 0;
   HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, W, lds));

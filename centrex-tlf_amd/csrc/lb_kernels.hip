@@ -1173,8 +1173,8 @@ __device__ __forceinline__ void write_row(const DevPlan& P, const DevCall& C, co
 // ---------------------------------------------------------------------------
 // Persistent integrator.
 // ---------------------------------------------------------------------------
-// G > 0 selects the single-wave form (R = 1, 64 threads, G gather rows in
-// registers); G = 0 is the multi-wave form.  LEAN: the multi-wave form of a
+// ONE_WAVE: the single-wave form (R = 1, 64 threads), which parks the state in
+// LDS around the expression machine; otherwise the multi-wave form.  LEAN: the multi-wave form of a
 // plan with couplings (and step programs, where it is time-dependent) for a
 // call with a given initial step that pushes at accepted steps at most into
 // the weighted integral: no trace, save plan, replay or stop event.
@@ -1186,11 +1186,11 @@ __device__ __forceinline__ void write_row(const DevPlan& P, const DevCall& C, co
 // and what runs once a trajectory reads its arguments anew (fresh_args).
 // 512 + 512 uneven batch (72 levels) 390 -> 310 ms, 500 thermal atoms (780
 // elements, kernel) 1.3 -> 0.82 ms.
-template <int R, int SOLVER, int MAXW, int WAVES, int G, bool EV = false, bool LEAN = false>
+template <int R, int SOLVER, int MAXW, int WAVES, bool ONE_WAVE = false, bool EV = false, bool LEAN = false>
 __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, const DevCall C) {
-  static_assert(G == 0 || (R == 1 && MAXW == 64), "the single-wave form holds one slot per lane");
-  static_assert(!EV || G == 0, "stop events run in the multi-wave form");
-  static_assert(!LEAN || (G == 0 && !EV), "the lean form is a multi-wave form without stop events");
+  static_assert(!ONE_WAVE || (R == 1 && MAXW == 64), "the single-wave form holds one slot per lane");
+  static_assert(!EV || !ONE_WAVE, "stop events run in the multi-wave form");
+  static_assert(!LEAN || (!ONE_WAVE && !EV), "the lean form is a multi-wave form without stop events");
   using T = Tab<SOLVER>;
   const int tid = threadIdx.x, W = blockDim.x;
   const Lds L = carve(P);
@@ -1413,7 +1413,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         // The expression machine needs registers of its own: the single-wave
         // form parks its state in LDS meanwhile (the multi-wave form keeps
         // it in the other waves' registers).
-        if constexpr (G > 0) {
+        if constexpr (ONE_WAVE) {
           L.park[tid] = double2{y_r[0], y_i[0]};
           L.park[64 + tid] = double2{k_r[1][0], k_i[1][0]};
         }
@@ -1437,7 +1437,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           if (LEAN || P.couplings)
             fill_entries<5>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + 2 * KK, KK, L.ent + P.nv_stat, tid, W);
         }
-        if constexpr (G > 0) {
+        if constexpr (ONE_WAVE) {
           const double2 py = L.park[tid], pk = L.park[64 + tid];
           y_r[0] = py.x;
           y_i[0] = py.y;
@@ -1526,7 +1526,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         double err, hn;
         bool accept, clamped;
         const double e2 = replay ? 0.0 : block_total(P, L.red, 0);
-        if (G == 0 && (LEAN || P.nblk > 1)) {
+        if (!ONE_WAVE && (LEAN || P.nblk > 1)) {
           const StepPowers ctl(e2 / (double)P.dim, fac_old, tid);
           err = ctl.err;
           accept = ctl.accept;
@@ -5872,15 +5872,15 @@ namespace {
 template <int I, int RR, int WW, int VV>
 void* solve_ptr(int solver) {
   if constexpr (I % LB_NPART == LB_PART)
-    return solver == 1 ? (void*)&lb_solve_kernel<RR, 1, WW, VV, 0> : (void*)&lb_solve_kernel<RR, 0, WW, VV, 0>;
+    return solver == 1 ? (void*)&lb_solve_kernel<RR, 1, WW, VV> : (void*)&lb_solve_kernel<RR, 0, WW, VV>;
   else
     return nullptr;
 }
 template <int I, int RR, int WW, int VV>
 void* lean_ptr(int solver) {
   if constexpr (I % LB_NPART == LB_PART)
-    return solver == 1 ? (void*)&lb_solve_kernel<RR, 1, WW, VV, 0, false, true>
-                       : (void*)&lb_solve_kernel<RR, 0, WW, VV, 0, false, true>;
+    return solver == 1 ? (void*)&lb_solve_kernel<RR, 1, WW, VV, false, false, true>
+                       : (void*)&lb_solve_kernel<RR, 0, WW, VV, false, false, true>;
   else
     return nullptr;
 }
@@ -5912,8 +5912,8 @@ void* fixed_ptr(int solver) {
 template <int I, int RR, int WW, int VV>
 void* event_ptr(int solver) {
   if constexpr (I % LB_NPART == LB_PART)
-    return solver == 0   ? (void*)&lb_solve_kernel<RR, 0, WW, VV, 0, true>
-         : solver == 1 ? (void*)&lb_solve_kernel<RR, 1, WW, VV, 0, true>
+    return solver == 0   ? (void*)&lb_solve_kernel<RR, 0, WW, VV, false, true>
+         : solver == 1 ? (void*)&lb_solve_kernel<RR, 1, WW, VV, false, true>
          : solver == 2 ? (void*)&lb_fixed_kernel<RR, 0, WW, VV, true>
          : solver == 3 ? (void*)&lb_fixed_kernel<RR, 1, WW, VV, true>
                        : (void*)&lb_fixed_kernel<RR, 2, WW, VV, true>;
@@ -5934,10 +5934,10 @@ void* adjoint_wave_ptr(int solver) {
   else
     return nullptr;
 }
-template <int I, int GG, int VV>
+template <int I, int VV>
 void* wave_solve_ptr(int solver) {
   if constexpr (I % LB_NPART == LB_PART)
-    return solver == 1 ? (void*)&lb_solve_kernel<1, 1, 64, VV, GG> : (void*)&lb_solve_kernel<1, 0, 64, VV, GG>;
+    return solver == 1 ? (void*)&lb_solve_kernel<1, 1, 64, VV, true> : (void*)&lb_solve_kernel<1, 0, 64, VV, true>;
   else
     return nullptr;
 }
@@ -5962,8 +5962,8 @@ extern "C" void* LB_PART_FN(lb_dev_solve_kernel)(int id, int solver) {
   if (id == i) return solve_ptr<i, r, w, v>(solver);
   LB_CONFIGS(X)
 #undef X
-#define Y(i, g, v) \
-  if (id == i) return wave_solve_ptr<i, g, v>(solver);
+#define Y(i, v) \
+  if (id == i) return wave_solve_ptr<i, v>(solver);
   LB_WAVE_CONFIGS(Y)
 #undef Y
 #define Q(i, g, v) \
@@ -6019,7 +6019,7 @@ extern "C" void* LB_PART_FN(lb_dev_rhs_kernel)(int id) {
   if (id == i) return rhs_ptr<i, r, w, v>();
   LB_CONFIGS(X)
 #undef X
-#define Y(i, g, v) \
+#define Y(i, v) \
   if (id == i) return wave_rhs_ptr<i, v>();
   LB_WAVE_CONFIGS(Y)
 #undef Y

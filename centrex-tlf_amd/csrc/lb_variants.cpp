@@ -58,21 +58,34 @@ extern "C" int lb_dev_variant_count(void) {
 #define X(i, r, w, v) ++n;
   LB_CONFIGS(X)
 #undef X
-#define Y(i, g, v) ++n;
+#define Y(i, v) ++n;
   LB_WAVE_CONFIGS(Y)
 #undef Y
+#define A(i, of) ++n;
+  LB_WAVE_ALIASES(A)
+#undef A
 #define Q(i, g, v) ++n;
   LB_PAIR_CONFIGS(Q)
 #undef Q
   return n;
 }
 
+// The id that variant `id` is another name of, or itself.
+extern "C" int lb_dev_variant_of(int id) {
+#define A(i, of) \
+  if (id == i) return of;
+  LB_WAVE_ALIASES(A)
+#undef A
+  return id;
+}
+
 extern "C" int lb_dev_variant(int id, int* R, int* maxw, int* waves) {
+  id = lb_dev_variant_of(id);
 #define X(i, r, w, v)                                                                           \
   if (id == i) { *R = r; *maxw = w; *waves = v; return 1; }
   LB_CONFIGS(X)
 #undef X
-#define Y(i, g, v)                                                                              \
+#define Y(i, v)                                                                                 \
   if (id == i) { *R = 1; *maxw = 64; *waves = v; return 1; }
   LB_WAVE_CONFIGS(Y)
 #undef Y
@@ -83,21 +96,18 @@ extern "C" int lb_dev_variant(int id, int* R, int* maxw, int* waves) {
   return 0;
 }
 
-// 1 for the paired (two trajectories per wave) variants.
-extern "C" int lb_dev_variant_pair(int id) {
-#define Q(i, g, v) \
+// 1 for the single-wave (one trajectory per wave) variants.
+extern "C" int lb_dev_variant_wave(int id) {
+  id = lb_dev_variant_of(id);
+#define Y(i, v) \
   if (id == i) return 1;
-  LB_PAIR_CONFIGS(Q)
-#undef Q
+  LB_WAVE_CONFIGS(Y)
+#undef Y
   return 0;
 }
 
-// Gather rows a single-wave variant holds in registers (0: multi-wave variant).
+// Coupling rows a paired variant holds in registers (0: not a paired variant).
 extern "C" int lb_dev_variant_rows(int id) {
-#define Y(i, g, v) \
-  if (id == i) return g;
-  LB_WAVE_CONFIGS(Y)
-#undef Y
 #define Q(i, g, v) \
   if (id == i) return g;
   LB_PAIR_CONFIGS(Q)

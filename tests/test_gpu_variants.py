@@ -1,5 +1,6 @@
 """Kernel variants by name: ids that stored tunings and calls hold keep their
-meaning."""
+meaning, and the single-wave names are one kernel without a limit on a plan's
+rows."""
 
 from __future__ import annotations
 
@@ -43,3 +44,23 @@ def test_paired_ids_keep_their_meaning():
             assert all(bool((a == b).all()) for a, b in zip(got[:2], want[:2]))
     assert len(kernel_variants()) == 17
     assert rows[0] <= 4 and rows[1] <= 4 and 4 < rows[2] <= 8, rows
+
+
+@pytest.mark.parametrize("n", [7, 10])
+def test_single_wave_names_are_one_kernel(n):
+    """28 and 55 elements, some 13 and 19 coupling rows."""
+    torch = require_gpu()
+    system, params = dense_system(n)
+    prepared = prepare_lindblad_problem(system, params, backend="host")
+    plan = DevicePlan(prepared.flat_plan)
+    assert (plan.info["gather_rows"] > 16) == (n == 10)
+    assert [plan.launch_info(variant=v)["variant"] for v in (12, 13, 14, 15)] == [12, 13, 13, 13]
+    y0 = prepared.layout.pack(random_density(n, seed=1)) / n
+    kw = dict(output_kind="populations", n_traj=3, abstol=1e-9, reltol=1e-7, dt=1e-3)
+    want = plan.solve(y0, 0.0, 0.3, variant=1, **kw)  # the multi-wave form
+    assert int(want[1][:, 3].max()) == 0
+    for v in (0, 12, 13, 14, 15):
+        got = plan.solve(y0, 0.0, 0.3, variant=v, **kw)
+        assert all(bool((a == b).all()) for a, b in zip(got[:2], want[:2])), v
+    assert torch.isfinite(want[0]).all()
+

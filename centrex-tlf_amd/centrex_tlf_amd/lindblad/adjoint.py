@@ -30,7 +30,7 @@ import numpy as np
 
 from . import _driver as D
 from .derivatives import differentiate_flat_plan
-from .native import DevicePlan, NativeError, Tape
+from .native import SPECIALIZE_AFTER, DevicePlan, NativeError, Tape
 
 __all__ = ["DifferentiablePhotonCount", "photon_count"]
 
@@ -77,7 +77,7 @@ class DifferentiablePhotonCount:
         self.plan = DevicePlan(differentiate_flat_plan(prepared.flat_plan, self.slots, with_time=True))
         if getattr(prepared, "specialize", True):
             try:
-                self.plan.specialize()
+                self.plan.specialize(after=SPECIALIZE_AFTER)
             except NativeError:  # an instruction without a generated form: the precompiled kernels run
                 pass
 

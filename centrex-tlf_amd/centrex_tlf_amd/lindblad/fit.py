@@ -175,6 +175,9 @@ def _fit_graph(groups, parameters, *, scales, iterations, lr, solver, abstol, re
     kw = dict(solver=solver, abstol=abstol, reltol=reltol, dt=dt, maxiters=maxiters, ckpt_every=ckpt_every,
               tape_capacity=tape_capacity)
     items = _engines(groups, parameters, **kw)
+    for eng, *_ in items:  # the graph keeps the kernels that it is captured with
+        if eng.plan.specialized:
+            eng.plan.specialize()
     scale = torch.as_tensor(np.asarray(scales, dtype=np.float64), device="cuda")
     if scale.numel() != len(parameters):
         raise ValueError("one scale per fitted parameter")

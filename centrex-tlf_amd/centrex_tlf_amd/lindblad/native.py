@@ -20,6 +20,10 @@ __all__ = ["DevicePlan", "NativeError", "Tape", "library", "library_path", "torc
 
 LIB_NAME = "liblindblad_gpu.so"
 _PKG_DIR = Path(__file__).resolve().parents[1]
+# Solves of a form before a prepared problem's plan compiles it (DevicePlan.specialize):
+# a compilation takes 0.7 to 4 s and saves a solve 1 to 6 ms (n = 39), so a program
+# that solves once does not pay for it and one that goes on solving soon does.
+SPECIALIZE_AFTER = 8
 _INFO_KEYS = [
     "n_states", "dim", "upper_len", "n_terms", "n_coefficients", "time_dependent", "n_published",
     "n_gather_terms", "n_self_terms", "slot_count", "gather_rows", "flops_per_rhs",
@@ -206,12 +210,15 @@ class DevicePlan:
         self.specialized = False
         self._spec_warned = False
 
-    def specialize(self, enable: bool = True) -> "DevicePlan":
+    def specialize(self, enable: bool = True, after: int = 1) -> "DevicePlan":
         """``lb_plan_specialize``: run the one-wave kernels of this plan with its
         time-dependent coefficient programs compiled in (bitwise the values of
-        the expression machine).  Each (form, solver) compiles on its first
-        solve, about 2 s; a plan without time dependence is unchanged."""
-        _check(library().lb_plan_specialize(self._handle, 1 if enable else 0))
+        the expression machine).  Each (form, solver) compiles on the plan's
+        ``after``-th solve of it, a second or two; until then, and for plans
+        without time dependence, the precompiled kernels run."""
+        if after < 1:
+            raise ValueError("after must be at least 1")
+        _check(library().lb_plan_specialize(self._handle, int(after) if enable else 0))
         self.specialized = bool(enable)
         return self
 

@@ -42,9 +42,11 @@ class PreparedLindbladProblem:
     flat_plan: dict[str, Any]
     backend: str
     gpu_plan: Any | None = field(default=None, repr=False)
-    # Adaptive solves run kernels with the time-dependent coefficient programs
-    # compiled in (DevicePlan.specialize); False keeps the precompiled kernels
-    # with the expression machine.  Results are bitwise the same.
+    # Solves run kernels with the time-dependent coefficient programs compiled
+    # in (DevicePlan.specialize): scans with final outputs of at most 32 elements
+    # from the first on, other forms from the SPECIALIZE_AFTER-th solve of a form
+    # on.  False keeps the precompiled kernels with the expression machine.
+    # Results are bitwise the same.
     specialize: bool = True
 
     def check_execution_mode(self, execution_mode: str) -> None:
@@ -67,14 +69,14 @@ class PreparedLindbladProblem:
     def device_plan(self):
         """The device plan, created on first use."""
         if self.gpu_plan is None:
-            from .native import DevicePlan
+            from .native import SPECIALIZE_AFTER, DevicePlan
 
             self.gpu_plan = DevicePlan(self.flat_plan)
             if self.specialize:
                 from .native import NativeError
 
                 try:
-                    self.gpu_plan.specialize()
+                    self.gpu_plan.specialize(after=SPECIALIZE_AFTER)
                 except NativeError as exc:  # an instruction without a generated form
                     import warnings
 

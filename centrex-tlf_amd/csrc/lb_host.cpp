@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -178,7 +179,9 @@ struct lb_plan {
   // coefficient function, and kernel name -> compiled module
   // A failed compilation leaves a null entry (the precompiled kernel runs)
   // and its reason in spec_failure.
-  bool spec = false;
+  std::atomic<bool> spec{false};  // written under mu; launches look at it first without
+  int spec_after = 1;  // calls of a form after which it is compiled
+  std::map<std::string, int> spec_calls;
   std::string spec_source, spec_failure;
   std::map<std::string, std::shared_ptr<LbModule>> spec_kernels;
   ~lb_plan() {
@@ -1153,6 +1156,7 @@ extern "C" void lb_plan_destroy(lb_plan* p) { delete p; }
 
 extern "C" int lb_plan_specialize(lb_plan* p, int32_t enable) {
   if (!p) return fail(LB_ERR_INVALID, "null argument");
+  if (enable < 0) return fail(LB_ERR_INVALID, "enable must be 0 or a number of calls");
   std::lock_guard<std::mutex> lock(p->mu);
   if (!enable || !p->src.time_dependent) {  // nothing is evaluated per step without time dependence
     p->spec = false;
@@ -1168,6 +1172,7 @@ extern "C" int lb_plan_specialize(lb_plan* p, int32_t enable) {
     p->spec_source = lb_rtc_coef_source(p->src.prog, dyn, p->src.K, why);
     if (p->spec_source.empty()) return fail(LB_ERR_UNSUPPORTED, why);
   }
+  p->spec_after = enable;
   p->spec = true;
   return LB_OK;
 }
@@ -1641,13 +1646,16 @@ int launch_table(const lb_plan* p, const lb_solve_args* a, const DevImage* im, D
 
 namespace {
 
-// The plan-specialised kernel `name` (a template-id), compiled on first use;
-// nullptr when the plan is not specialised.  (Only the paired kernels, one
+// The plan-specialised kernel `name` (a template-id); nullptr when the plan is
+// not specialised or the form is not compiled yet.  A compilation takes 0.7 s
+// and more and saves a call 1 to 6 ms, so it is not for one call: the form is
+// compiled at the plan's spec_after-th call of it (at once where the process
+// holds it for another plan), or at the first where `at_once` says so.  (Only the paired kernels, one
 // wave per workgroup, take the generated code: a specialised multi-wave
 // kernel launched with 1024-thread workgroups had its queue aborted at
 // dispatch, cause not found, so the multi-wave kernels stay on the
 // precompiled form.)
-int spec_kernel(lb_plan* p, const std::string& name, hipStream_t stream, hipFunction_t* fn) {
+int spec_kernel(lb_plan* p, const std::string& name, bool at_once, hipStream_t stream, hipFunction_t* fn) {
   *fn = nullptr;
   std::lock_guard<std::mutex> lock(p->mu);
   if (!p->spec) return LB_OK;
@@ -1660,6 +1668,8 @@ int spec_kernel(lb_plan* p, const std::string& name, hipStream_t stream, hipFunc
     if (cs != hipStreamCaptureStatusNone) return LB_OK;
     std::shared_ptr<LbModule> mod;
     std::string why;
+    const bool wait = !at_once && ++p->spec_calls[name] < p->spec_after;
+    if (wait && !lb_rtc_held(p->spec_source, name)) return LB_OK;
     if (lb_rtc_compile(p->spec_source, name, &mod, why)) {
       // the precompiled kernel computes the same values: run it, remember
       // the failure so that later calls neither recompile nor fail
@@ -1700,7 +1710,9 @@ int launch_spec(lb_plan* p, const lb_solve_args* a, const DevImage* im, DevCall&
     std::snprintf(name, sizeof name, "lb_solve_pair_kernel<%d, %d, 2, %d, %d>", a->solver == LB_SOLVER_TSIT5 ? 1 : 0,
                   std::max(1, rows), 64 / nh, event ? LB_LANE_SAVE | LB_LANE_EVENT : save ? LB_LANE_SAVE : 0);
   hipFunction_t fn = nullptr;
-  int rc = spec_kernel(p, name, s, &fn);
+  // final outputs of at most 32 elements (scans of thousands of trajectories)
+  const bool at_once = nh == 2 && !fixed && !event && !save && !a->tape_h;
+  int rc = spec_kernel(p, name, at_once, s, &fn);
   if (rc || !fn) return rc;
   int grid = a->workgroups;
   if (grid <= 0) {

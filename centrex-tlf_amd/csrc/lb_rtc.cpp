@@ -212,10 +212,21 @@ int compile_code(const std::string& coef_source, const std::string& name_expr, C
 
 }  // namespace
 
+namespace {
+std::string code_key(const std::string& coef_source, const std::string& name_expr) {
+  const char* extra = std::getenv("CENTREX_LB_RTC_OPTIONS");
+  return std::string(extra ? extra : "") + "\n" + name_expr + "\n" + coef_source;
+}
+}  // namespace
+
+bool lb_rtc_held(const std::string& coef_source, const std::string& name_expr) {
+  std::lock_guard<std::mutex> lock(g_code_mu);
+  return g_code.count(code_key(coef_source, name_expr)) != 0;
+}
+
 int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr, std::shared_ptr<LbModule>* out,
                    std::string& why) {
-  const char* extra = std::getenv("CENTREX_LB_RTC_OPTIONS");
-  const std::string key = std::string(extra ? extra : "") + "\n" + name_expr + "\n" + coef_source;
+  const std::string key = code_key(coef_source, name_expr);
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) {
     why = "no current device";

@@ -34,3 +34,5 @@ struct LbModule {
 };
 int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr, std::shared_ptr<LbModule>* out,
                    std::string& why);
+// Whether lb_rtc_compile would compile nothing: the process holds the kernel.
+bool lb_rtc_held(const std::string& coef_source, const std::string& name_expr);

@@ -199,3 +199,42 @@ def test_failed_compilation_runs_the_precompiled_kernel(monkeypatch):
         again = spec.solve(y0, 0.0, 6.0, **kw)
     torch.cuda.synchronize()
     _same(again, want, "after the failure")
+
+
+def test_prepared_problems_compile_traces_and_gradients_after_some_solves(monkeypatch):
+    """A prepared problem's plan compiles a form at its SPECIALIZE_AFTER-th solve
+    (seen by a compilation made to fail), so a single trace or gradient does not
+    wait for the compiler; explicit specialisation compiles at the first.  The
+    solves before and after give the same bits."""
+    torch = require_gpu()
+    from centrex_tlf_amd.lindblad.adjoint import DifferentiablePhotonCount
+    from centrex_tlf_amd.lindblad.native import SPECIALIZE_AFTER
+
+    system, params, rho0, t_span, weights = tlf_n39()
+    kw = dict(output_kind="rate", trace=True, capacity=400, weights=weights, abstol=1e-9, reltol=1e-7, dt=1e-8)
+
+    def traces(prepared, count):
+        y0 = prepared.layout.pack(rho0)
+        return [prepared.device_plan().solve(y0, t_span[0], 0.3 * t_span[1], n_traj=1, **kw) for _ in range(count)]
+
+    with monkeypatch.context() as m:
+        m.setenv("CENTREX_LB_RTC_OPTIONS", "-Werror -DLB_PART=1")
+        prepared = prepare_lindblad_problem(system, params, backend="gpu")
+        traces(prepared, SPECIALIZE_AFTER - 1)
+        assert prepared.device_plan().specialize_failure() is None
+        with pytest.warns(UserWarning, match="precompiled kernel used"):
+            traces(prepared, 1)
+        assert "lb_solve_pair_kernel" in prepared.device_plan().specialize_failure()
+        engine = DifferentiablePhotonCount(prepared, ["delta0"], weights, t_span, abstol=1e-9, reltol=1e-7, dt=1e-8)
+        p = torch.zeros((1, 1), dtype=torch.float64, device="cuda")
+        for k in range(SPECIALIZE_AFTER - 1):
+            engine.forward(p, prepared.layout.pack(rho0))
+        assert engine.plan.specialize_failure() is None
+        plan = DevicePlan(prepared.flat_plan).specialize()
+        with pytest.warns(UserWarning, match="precompiled kernel used"):
+            plan.solve(prepared.layout.pack(rho0), t_span[0], 0.3 * t_span[1], n_traj=1, **kw)
+    prepared = prepare_lindblad_problem(system, params, backend="gpu")
+    results = traces(prepared, SPECIALIZE_AFTER + 1)
+    assert prepared.device_plan().specialize_failure() is None and int(results[0][4][0]) > 10
+    for got in results[1:]:
+        assert all(bool((a.nan_to_num(7.0) == b.nan_to_num(7.0)).all()) for a, b in zip(got, results[0]) if a is not None)

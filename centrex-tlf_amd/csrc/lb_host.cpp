@@ -18,7 +18,6 @@
 #include <mutex>
 #include <new>
 #include <numeric>
-#include <unordered_map>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -383,93 +382,131 @@ struct Couplings {
   int64_t dyn_terms = 0;
 };
 
+// The distinct values of a plan, numbered as they are first seen; found by hash
+// without a copy, as most couplings repeat a value.
+struct EntryTable {
+  std::vector<std::vector<EntryTerm>> values;
+  std::vector<uint64_t> hashes;
+  std::vector<int> cells = std::vector<int>(256, -1);  // open addressing, a power of two
+  int find(const EntryTerm* v, size_t n) {
+    uint64_t h = n;
+    auto mix = [&](uint64_t x) { h = (h ^ x) * 0x9E3779B97F4A7C15ull; h ^= h >> 29; };
+    for (size_t i = 0; i < n; ++i) {
+      uint64_t re, im;
+      // -0.0 and 0.0 compare equal
+      const double fr = v[i].re + 0.0, fi = v[i].im + 0.0;
+      std::memcpy(&re, &fr, 8);
+      std::memcpy(&im, &fi, 8);
+      mix(v[i].coef);
+      mix(re);
+      mix(im);
+    }
+    size_t at = h & (cells.size() - 1);
+    for (; cells[at] >= 0; at = (at + 1) & (cells.size() - 1)) {
+      const int id = cells[at];
+      if (hashes[id] == h && values[id].size() == n && std::equal(v, v + n, values[id].begin())) return id;
+    }
+    const int id = (int)values.size();
+    cells[at] = id;
+    values.emplace_back(v, v + n);
+    hashes.push_back(h);
+    if (2 * values.size() > cells.size()) {
+      cells.assign(2 * cells.size(), -1);
+      for (int k = 0; k <= id; ++k) {
+        at = hashes[k] & (cells.size() - 1);
+        while (cells[at] >= 0) at = (at + 1) & (cells.size() - 1);
+        cells[at] = k;
+      }
+    }
+    return id;
+  }
+};
+
 Couplings merge_couplings(const PlanSource& src, const std::vector<uint8_t>& act, bool merge) {
   struct Raw {
     int in;
     bool conj;
-    std::vector<EntryTerm> v;
+    int first, n;  // its terms
   };
   Couplings out;
   out.of.resize(src.U);
-  struct Hash {
-    size_t operator()(const std::vector<EntryTerm>& v) const {
-      uint64_t h = v.size();
-      auto mix = [&](uint64_t x) { h = (h ^ x) * 0x9E3779B97F4A7C15ull; h ^= h >> 29; };
-      for (const EntryTerm& t : v) {
-        uint64_t re, im;
-        // -0.0 and 0.0 compare equal
-        const double fr = t.re + 0.0, fi = t.im + 0.0;
-        std::memcpy(&re, &fr, 8);
-        std::memcpy(&im, &fi, 8);
-        mix(t.coef);
-        mix(re);
-        mix(im);
-      }
-      return h;
-    }
-  };
-  std::unordered_map<std::vector<EntryTerm>, int, Hash> dyn_id, stat_id;
-  auto is_dyn = [&](const std::vector<EntryTerm>& v) {
-    for (const EntryTerm& t : v) {
-      const uint32_t k = t.coef & 0x7FFFFFFFu;
-      if (k < (uint32_t)src.K && src.coef_dyn[k]) return true;
-    }
-    return false;
+  EntryTable dyn_id, stat_id;
+  auto is_dyn = [&](const EntryTerm& t) {
+    const uint32_t k = t.coef & 0x7FFFFFFFu;
+    return k < (uint32_t)src.K && src.coef_dyn[k];
   };
   auto conj_of = [&](const EntryTerm& t) {
     const uint32_t k = t.coef & 0x7FFFFFFFu;
     return EntryTerm{k == (uint32_t)src.K ? t.coef : t.coef ^ 0x80000000u, t.re, -t.im};
   };
-  std::vector<std::vector<std::pair<bool, int>>> ids(src.U);  // (time-dependent, index of its kind)
+  std::vector<Raw> raw;
+  std::vector<EntryTerm> terms, grouped, one, other;
+  std::vector<int> owner;
   for (int o = 0; o < src.U; ++o) {
     if (!act[o]) continue;
-    std::vector<Raw> raw;
+    raw.clear();
+    terms.clear();
+    owner.clear();
     for (int64_t k = src.output_ptrs[o]; k < src.output_ptrs[o + 1]; ++k) {
       const int in = (int)src.input_indices[k];
       const int64_t ci = src.coeff_indices[k];
       if (in == o && !(ci >= 0 && src.coef_dyn[ci]) && !src.input_conj[k]) continue;  // a self term
       const bool conj = src.up_im[in] >= 0 && src.input_conj[k];
-      EntryTerm t{ci < 0 ? (uint32_t)src.K : ((uint32_t)ci | (src.coeff_conj[k] ? 0x80000000u : 0u)),
-                  src.factors_re[k], src.factors_im[k]};
-      auto it = std::find_if(raw.begin(), raw.end(), [&](const Raw& r) { return merge && r.in == in && r.conj == conj; });
-      if (it == raw.end()) raw.push_back(Raw{in, conj, {t}});
-      else it->v.push_back(t);
+      terms.push_back(EntryTerm{ci < 0 ? (uint32_t)src.K : ((uint32_t)ci | (src.coeff_conj[k] ? 0x80000000u : 0u)),
+                                src.factors_re[k], src.factors_im[k]});
+      size_t i = merge ? 0 : raw.size();
+      while (i < raw.size() && !(raw[i].in == in && raw[i].conj == conj)) ++i;
+      if (i == raw.size()) raw.push_back(Raw{in, conj, 0, 0});
+      ++raw[i].n;
+      owner.push_back((int)i);
+    }
+    // the terms of a coupling one after the other
+    int at = 0;
+    for (Raw& r : raw) {
+      r.first = at;
+      at += r.n;
+      r.n = 0;
+    }
+    grouped.resize(terms.size());
+    for (size_t t = 0; t < terms.size(); ++t) {
+      Raw& r = raw[owner[t]];
+      grouped[r.first + r.n++] = terms[t];
     }
     if (merge && src.up_im[o] < 0) {
       // a diagonal output keeps the real part only: x v and its conjugate are twice the one
       for (size_t i = 0; i < raw.size(); ++i) {
         for (size_t j = i + 1; j < raw.size(); ++j) {
-          if (raw[i].in != raw[j].in || raw[i].conj == raw[j].conj) continue;
-          std::vector<EntryTerm> a = raw[i].v, b;
-          for (const EntryTerm& t : raw[j].v) b.push_back(conj_of(t));
-          std::sort(a.begin(), a.end());
-          std::sort(b.begin(), b.end());
-          if (!(a == b)) continue;
-          Raw& keep = raw[i].conj ? raw[j] : raw[i];
-          for (EntryTerm& t : keep.v) {
-            t.re *= 2.0;
-            t.im *= 2.0;
+          if (raw[i].in != raw[j].in || raw[i].conj == raw[j].conj || raw[i].n != raw[j].n) continue;
+          one.assign(&grouped[raw[i].first], &grouped[raw[i].first] + raw[i].n);
+          other.clear();
+          for (int t = 0; t < raw[j].n; ++t) other.push_back(conj_of(grouped[raw[j].first + t]));
+          std::sort(one.begin(), one.end());
+          std::sort(other.begin(), other.end());
+          if (!(one == other)) continue;
+          const Raw keep = raw[i].conj ? raw[j] : raw[i];
+          for (int t = 0; t < keep.n; ++t) {
+            grouped[keep.first + t].re *= 2.0;
+            grouped[keep.first + t].im *= 2.0;
           }
-          if (raw[i].conj) raw[i] = raw[j];
+          raw[i] = keep;
           raw.erase(raw.begin() + j);
           break;
         }
       }
     }
+    out.of[o].reserve(raw.size());
     for (const Raw& r : raw) {
-      const bool dyn = is_dyn(r.v);
-      auto& table = dyn ? dyn_id : stat_id;
-      const int id = table.emplace(r.v, (int)table.size()).first->second;
-      out.of[o].push_back(Coupling{r.in, r.conj, 0});
-      ids[o].push_back({dyn, id});
+      const EntryTerm* v = &grouped[r.first];
+      const bool dyn = std::any_of(v, v + r.n, is_dyn);
+      // numbered below, the time-independent ones by -1 - id until then
+      out.of[o].push_back(Coupling{r.in, r.conj, dyn ? dyn_id.find(v, r.n) : -1 - stat_id.find(v, r.n)});
     }
   }
-  out.n_dyn = (int)dyn_id.size();
-  out.entries.resize(dyn_id.size() + stat_id.size());
-  for (const auto& kv : dyn_id) {
-    out.entries[kv.second] = kv.first;
-    out.dyn_terms += (int64_t)kv.first.size();
-  }
+  const size_t n_dyn = dyn_id.values.size(), n_stat = stat_id.values.size();
+  out.n_dyn = (int)n_dyn;
+  out.entries = std::move(dyn_id.values);
+  out.entries.resize(n_dyn + n_stat);
+  for (size_t k = 0; k < n_dyn; ++k) out.dyn_terms += (int64_t)out.entries[k].size();
   // time-independent entries: those whose coefficients have derivatives first
   const int nc = src.prog.n_compounds;
   auto has_derivative = [&](const std::vector<EntryTerm>& v) {
@@ -484,20 +521,20 @@ Couplings merge_couplings(const PlanSource& src, const std::vector<uint8_t>& act
     }
     return false;
   };
-  std::vector<int> place(stat_id.size(), 0);
-  std::vector<uint8_t> derived(stat_id.size(), 0);
+  std::vector<int> place(n_stat, 0);
+  std::vector<uint8_t> derived(n_stat, 0);
   if (src.n_diff > 0)
-    for (const auto& kv : stat_id) derived[kv.second] = has_derivative(kv.first);
+    for (size_t k = 0; k < n_stat; ++k) derived[k] = has_derivative(stat_id.values[k]);
   int at = 0;
   for (int pass = 1; pass >= 0; --pass) {
     for (size_t i = 0; i < place.size(); ++i)
       if (derived[i] == pass) place[i] = at++;
     if (pass) out.n_def = out.n_dyn + at;
   }
-  for (const auto& kv : stat_id) out.entries[dyn_id.size() + place[kv.second]] = kv.first;
-  for (int o = 0; o < src.U; ++o)
-    for (size_t j = 0; j < ids[o].size(); ++j)
-      out.of[o][j].entry = ids[o][j].first ? ids[o][j].second : out.n_dyn + place[ids[o][j].second];
+  for (size_t k = 0; k < n_stat; ++k) out.entries[n_dyn + place[k]] = std::move(stat_id.values[k]);
+  for (auto& of : out.of)
+    for (Coupling& c : of)
+      if (c.entry < 0) c.entry = out.n_dyn + place[-1 - c.entry];
   return out;
 }
 
@@ -585,8 +622,9 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
     if (ex_dyn.empty()) ex_dyn.push_back(DevExpr{});
     // the same time-dependent programs in three-address form
     const std::vector<int32_t> fwd(list.begin(), list.begin() + n_dyn_fwd), fdst(dst.begin(), dst.begin() + n_dyn_fwd);
-    im->vec = lb_vector_program(src.prog, fwd, fdst, src.prog.n_slots);
-    im->vec_all = src.n_diff > 0 ? lb_vector_program(src.prog, list, dst, src.prog.n_slots) : LbVector{};
+    im->vec = lb_vector_program(src.prog, fwd, fdst, src.prog.n_slots, 8, kMaxVectorBytes);
+    im->vec_all =
+        src.n_diff > 0 ? lb_vector_program(src.prog, list, dst, src.prog.n_slots, 7, kMaxLdsBytes) : LbVector{};
   }
   P.v_steps = im->vec.steps;
   P.v_steps_all = im->vec_all.steps;
@@ -613,8 +651,7 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   P.lds_tables = 0;
   P.c_rows_total = P.g_rows = 0;
   P.v_n_const = (int32_t)im->vec.const_slot.size();
-  if (P.v_steps == 0 || 16 * 8 * (int64_t)(P.v_slots + P.v_steps) > kMaxVectorBytes)
-    drop_steps(P);  // a long program stays interpreted
+  if (P.v_steps == 0) drop_steps(P);  // none, or a long program, which stays interpreted
   const DevPlan with_steps = P;
   if (!lds_fits(P)) drop_steps(P);
   if (!couplings || P.nv_dyn + P.nv_stat > LB_MAX_ENTRIES || P.n_pub > LB_MAX_COUPLED ||
@@ -698,8 +735,10 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
     blk_rows[b] = rows;
     rows_total += rows;
   }
-  std::vector<uint32_t> g_word((size_t)rows_total * 64, lb_gword(0, true, false, false, LB_STATIC_COEF));
-  std::vector<double> g_f((size_t)rows_total * 64 * 2, 0.0);
+  // the gather tables: plans without couplings, and differentiable ones
+  const bool gather = !P.couplings || src.n_diff > 0;
+  std::vector<uint32_t> g_word(gather ? (size_t)rows_total * 64 : 0, lb_gword(0, true, false, false, LB_STATIC_COEF));
+  std::vector<double> g_f(gather ? (size_t)rows_total * 64 * 2 : 0, 0.0);
   for (int s = 0; s < S; ++s) {
     const int o = slot_el[s], b = s / 64, l = s % 64;
     if (o < 0) continue;
@@ -713,7 +752,7 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
         self_conj[e] = src.coeff_conj[k];
         self_f[2 * e] = src.factors_re[k];
         self_f[2 * e + 1] = src.factors_im[k];
-      } else {
+      } else if (gather) {
         const size_t e = (size_t)(blk_row0[b] + jg++) * 64 + l;
         g_word[e] = lb_gword((uint32_t)pub_of_upper[in], src.up_im[in] < 0, src.input_conj[k] != 0,
                              src.coeff_conj[k] != 0, ci < 0 ? LB_STATIC_COEF : (uint32_t)ci);
@@ -777,28 +816,30 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
     std::vector<int32_t> slot_of(U, -1);
     for (int s = 0; s < S; ++s)
       if (slot_el[s] >= 0) slot_of[slot_el[s]] = s;
-    std::vector<std::vector<uint32_t>> readers(S), of_entry(cpl.n_def);
+    std::vector<int> readers(S, 0);  // couplings that read a slot: counted, then placed
+    std::vector<std::vector<uint32_t>> of_entry(cpl.n_def);
+    for (int s = 0; s < S; ++s)
+      if (slot_el[s] >= 0)
+        for (const Coupling& c : cpl.of[slot_el[s]]) ++readers[slot_of[c.in]];
+    for (int b = 0; b < nblk; ++b) {
+      tc_row0[b] = tc_total;
+      tc_rows[b] = *std::max_element(&readers[64 * b], &readers[64 * b] + 64);
+      tc_total += tc_rows[b];
+    }
+    tc_word.assign((size_t)tc_total * 64, lb_cword(0, false, false, (uint32_t)(P.nv_stat - 1)));
+    readers.assign(S, 0);
     for (int s = 0; s < S; ++s) {
       const int o = slot_el[s];
       if (o < 0) continue;
       for (const Coupling& c : cpl.of[o]) {
         const bool dyn = c.entry < P.nv_dyn;
-        readers[slot_of[c.in]].push_back(
-            lb_cword((uint32_t)s, c.conj, dyn, (uint32_t)(dyn ? P.nv_stat + c.entry : c.entry - P.nv_dyn)));
+        const int r = slot_of[c.in];
+        tc_word[(size_t)(tc_row0[r / 64] + readers[r]++) * 64 + r % 64] =
+            lb_cword((uint32_t)s, c.conj, dyn, (uint32_t)(dyn ? P.nv_stat + c.entry : c.entry - P.nv_dyn));
         if (c.entry < cpl.n_def)
           of_entry[c.entry].push_back(((uint32_t)s << 20) | ((uint32_t)pub_of_upper[c.in] << 4) | (c.conj ? 2u : 0u));
       }
     }
-    for (int b = 0; b < nblk; ++b) {
-      int rows = 0;
-      for (int l = 0; l < 64; ++l) rows = std::max<int>(rows, (int)readers[64 * b + l].size());
-      tc_row0[b] = tc_total;
-      tc_rows[b] = rows;
-      tc_total += rows;
-    }
-    tc_word.assign((size_t)tc_total * 64, lb_cword(0, false, false, (uint32_t)(P.nv_stat - 1)));
-    for (int s = 0; s < S; ++s)
-      for (size_t j = 0; j < readers[s].size(); ++j) tc_word[(size_t)(tc_row0[s / 64] + (int)j) * 64 + s % 64] = readers[s][j];
     int chunks = 0;
     for (const auto& v : of_entry) chunks += ((int)v.size() + LB_Q_CHUNK - 1) / LB_Q_CHUNK;
     P.q_chunks = (chunks + 63) / 64 * 64;
@@ -823,12 +864,6 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
     }
     if (bare > kMaxLdsBytes) P.nv_def = 0;  // the gather form's adjoint
   }
-  // the gather tables: plans without couplings, and differentiable ones
-  const bool gather = !P.couplings || src.n_diff > 0;
-  if (!gather) {
-    g_word.clear();
-    g_f.clear();
-  }
   // transposed tables of a differentiable plan: for each input slot, the terms
   // that read it (self-folded terms excluded), output named by its slot
   std::vector<int32_t> t_row0(nblk, 0), t_rows(nblk, 0);
@@ -839,40 +874,35 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
     std::vector<int32_t> slot_of(U, -1);
     for (int s = 0; s < S; ++s)
       if (slot_el[s] >= 0) slot_of[slot_el[s]] = s;
-    std::vector<std::vector<int64_t>> readers(S);
-    for (int o = 0; o < U; ++o) {
-      if (!act[o]) continue;
-      for (int64_t k = src.output_ptrs[o]; k < src.output_ptrs[o + 1]; ++k) {
-        const int in = (int)src.input_indices[k];
-        if (in == o && !is_dyn(k) && !src.input_conj[k]) continue;
-        readers[slot_of[in]].push_back(k);
+    std::vector<int> readers(S, 0);  // terms that read a slot: counted, then placed
+    auto each_term = [&](auto&& f) {
+      for (int o = 0; o < U; ++o) {
+        if (!act[o]) continue;
+        for (int64_t k = src.output_ptrs[o]; k < src.output_ptrs[o + 1]; ++k) {
+          const int in = (int)src.input_indices[k];
+          if (in == o && !is_dyn(k) && !src.input_conj[k]) continue;
+          f(o, in, k);
+        }
       }
-    }
+    };
+    each_term([&](int, int in, int64_t) { ++readers[slot_of[in]]; });
     for (int b = 0; b < nblk; ++b) {
-      int rows = 0;
-      for (int l = 0; l < 64; ++l) rows = std::max<int>(rows, (int)readers[64 * b + l].size());
       t_row0[b] = t_total;
-      t_rows[b] = rows;
-      t_total += rows;
+      t_rows[b] = *std::max_element(&readers[64 * b], &readers[64 * b] + 64);
+      t_total += t_rows[b];
     }
     t_word.assign((size_t)t_total * 64, lb_gword(0, true, false, false, LB_STATIC_COEF));
     t_f.assign((size_t)t_total * 64 * 2, 0.0);
-    std::vector<int32_t> out_of(src.T, -1);
-    for (int o = 0; o < U; ++o)
-      for (int64_t k = src.output_ptrs[o]; k < src.output_ptrs[o + 1]; ++k) out_of[k] = o;
-    for (int s = 0; s < S; ++s) {
-      const int b = s / 64, l = s % 64, in = slot_el[s];
-      if (in < 0) continue;
-      int j = 0;
-      for (int64_t k : readers[s]) {
-        const int64_t ci = src.coeff_indices[k];
-        const size_t e = (size_t)(t_row0[b] + j++) * 64 + l;
-        t_word[e] = lb_gword((uint32_t)slot_of[out_of[k]], src.up_im[in] < 0, src.input_conj[k] != 0,
-                             src.coeff_conj[k] != 0, ci < 0 ? LB_STATIC_COEF : (uint32_t)ci);
-        t_f[2 * e] = src.factors_re[k];
-        t_f[2 * e + 1] = src.factors_im[k];
-      }
-    }
+    readers.assign(S, 0);
+    each_term([&](int o, int in, int64_t k) {
+      const int s = slot_of[in];
+      const int64_t ci = src.coeff_indices[k];
+      const size_t e = (size_t)(t_row0[s / 64] + readers[s]++) * 64 + s % 64;
+      t_word[e] = lb_gword((uint32_t)slot_of[o], src.up_im[in] < 0, src.input_conj[k] != 0, src.coeff_conj[k] != 0,
+                           ci < 0 ? LB_STATIC_COEF : (uint32_t)ci);
+      t_f[2 * e] = src.factors_re[k];
+      t_f[2 * e + 1] = src.factors_im[k];
+    });
   }
   // packed index -> upper index, and the active flags (outputs of dropped
   // elements are written as zeros)
@@ -1156,7 +1186,6 @@ extern "C" void lb_plan_destroy(lb_plan* p) { delete p; }
 
 extern "C" int lb_plan_specialize(lb_plan* p, int32_t enable) {
   if (!p) return fail(LB_ERR_INVALID, "null argument");
-  if (enable < 0) return fail(LB_ERR_INVALID, "enable must be 0 or a number of calls");
   std::lock_guard<std::mutex> lock(p->mu);
   if (!enable || !p->src.time_dependent) {  // nothing is evaluated per step without time dependence
     p->spec = false;
@@ -1172,7 +1201,7 @@ extern "C" int lb_plan_specialize(lb_plan* p, int32_t enable) {
     p->spec_source = lb_rtc_coef_source(p->src.prog, dyn, p->src.K, why);
     if (p->spec_source.empty()) return fail(LB_ERR_UNSUPPORTED, why);
   }
-  p->spec_after = enable;
+  p->spec_after = std::max(1, (int)enable);
   p->spec = true;
   return LB_OK;
 }

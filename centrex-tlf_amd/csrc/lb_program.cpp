@@ -305,7 +305,7 @@ struct VNode {
 }  // namespace
 
 LbVector lb_vector_program(const LbProgram& prog, const std::vector<int32_t>& list, const std::vector<int32_t>& dst,
-                           int first_slot) {
+                           int first_slot, int copies, int64_t max_bytes) {
   LbVector out;
   int next = first_slot;
   out.time_slot = next++;
@@ -414,6 +414,9 @@ LbVector lb_vector_program(const LbProgram& prog, const std::vector<int32_t>& li
   out.n_slots = next;
   // ---- steps: of the ready operations, the opcode of the one on the longest chain
   const int n = (int)nodes.size();
+  auto bytes = [&](int steps) { return 16 * ((int64_t)copies * out.n_slots + (int64_t)LB_VOP_LANES * steps); };
+  // the schedule is quadratic in the program's length: not for one that is too long
+  if (bytes((n + LB_VOP_LANES - 1) / LB_VOP_LANES) > max_bytes) return out;
   for (int k = n - 1; k >= 0; --k) {
     nodes[k].path += nodes[k].weight;
     for (int p : nodes[k].after) nodes[p].path = std::max(nodes[p].path, nodes[k].path);
@@ -437,6 +440,10 @@ LbVector lb_vector_program(const LbProgram& prog, const std::vector<int32_t>& li
       --left;
     }
     for (; used < LB_VOP_LANES; ++used) out.ops.push_back(DevVOp{0, 0, 0, 0});
+  }
+  if (bytes(out.steps) > max_bytes) {
+    out.ops.clear();
+    out.steps = 0;
   }
   return out;
 }

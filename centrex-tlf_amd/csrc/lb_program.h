@@ -30,9 +30,10 @@ struct LbVector {
 // The expressions `list` of `prog` (in evaluation order; each reads slots
 // written by earlier ones), expression e into slot dst[i] or (dst[i] < 0)
 // coefficient row entry -dst[i] - 1, as steps of independent operations of
-// one opcode.  Slots are numbered from first_slot on.
+// one opcode.  Slots are numbered from first_slot on.  A program that would take
+// more than max_bytes with `copies` copies of its slots gets no steps.
 LbVector lb_vector_program(const LbProgram& prog, const std::vector<int32_t>& list, const std::vector<int32_t>& dst,
-                           int first_slot);
+                           int first_slot, int copies, int64_t max_bytes);
 
 // Returns 0 on success, -1 (with `why`) on a malformed expression.
 int lb_build_program(const lb_plan_desc* d, const std::vector<uint8_t>& dyn_slot,

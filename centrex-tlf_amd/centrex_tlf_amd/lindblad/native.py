@@ -213,9 +213,10 @@ class DevicePlan:
     def specialize(self, enable: bool = True, after: int = 1) -> "DevicePlan":
         """``lb_plan_specialize``: run the one-wave kernels of this plan with its
         time-dependent coefficient programs compiled in (bitwise the values of
-        the expression machine).  Each (form, solver) compiles on the plan's
-        ``after``-th solve of it, a second or two; until then, and for plans
-        without time dependence, the precompiled kernels run."""
+        the expression machine).  Each (form, solver) compiles on the
+        ``after``-th solve of it by plans of these programs, a second or two;
+        until then, and for plans without time dependence, the precompiled
+        kernels run."""
         if after < 1:
             raise ValueError("after must be at least 1")
         _check(library().lb_plan_specialize(self._handle, int(after) if enable else 0))

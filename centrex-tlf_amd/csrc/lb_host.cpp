@@ -180,7 +180,6 @@ struct lb_plan {
   // and its reason in spec_failure.
   std::atomic<bool> spec{false};  // written under mu; launches look at it first without
   int spec_after = 1;  // calls of a form after which it is compiled
-  std::map<std::string, int> spec_calls;
   std::string spec_source, spec_failure;
   std::map<std::string, std::shared_ptr<LbModule>> spec_kernels;
   ~lb_plan() {
@@ -1677,13 +1676,12 @@ namespace {
 
 // The plan-specialised kernel `name` (a template-id); nullptr when the plan is
 // not specialised or the form is not compiled yet.  A compilation takes 0.7 s
-// and more and saves a call 1 to 6 ms, so it is not for one call: the form is
-// compiled at the plan's spec_after-th call of it (at once where the process
-// holds it for another plan), or at the first where `at_once` says so.  (Only the paired kernels, one
-// wave per workgroup, take the generated code: a specialised multi-wave
-// kernel launched with 1024-thread workgroups had its queue aborted at
-// dispatch, cause not found, so the multi-wave kernels stay on the
-// precompiled form.)
+// and more and saves a call 1 to 6 ms, so it is not for one call: a form is
+// compiled at the spec_after-th call of it by plans of one program, or at the
+// first where `at_once` says so.  (Only the paired kernels, one wave per
+// workgroup, take the generated code: a specialised multi-wave kernel launched
+// with 1024-thread workgroups had its queue aborted at dispatch, cause not
+// found, so the multi-wave kernels stay on the precompiled form.)
 int spec_kernel(lb_plan* p, const std::string& name, bool at_once, hipStream_t stream, hipFunction_t* fn) {
   *fn = nullptr;
   std::lock_guard<std::mutex> lock(p->mu);
@@ -1697,8 +1695,7 @@ int spec_kernel(lb_plan* p, const std::string& name, bool at_once, hipStream_t s
     if (cs != hipStreamCaptureStatusNone) return LB_OK;
     std::shared_ptr<LbModule> mod;
     std::string why;
-    const bool wait = !at_once && ++p->spec_calls[name] < p->spec_after;
-    if (wait && !lb_rtc_held(p->spec_source, name)) return LB_OK;
+    if (!at_once && !lb_rtc_ready(p->spec_source, name, p->spec_after)) return LB_OK;
     if (lb_rtc_compile(p->spec_source, name, &mod, why)) {
       // the precompiled kernel computes the same values: run it, remember
       // the failure so that later calls neither recompile nor fail

@@ -34,5 +34,6 @@ struct LbModule {
 };
 int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr, std::shared_ptr<LbModule>* out,
                    std::string& why);
-// Whether lb_rtc_compile would compile nothing: the process holds the kernel.
-bool lb_rtc_held(const std::string& coef_source, const std::string& name_expr);
+// Counts one call that would take the kernel: whether it is the `after`-th or a
+// later one in the process, or the process holds the kernel already.
+bool lb_rtc_ready(const std::string& coef_source, const std::string& name_expr, int after);

@@ -144,14 +144,13 @@ void lb_plan_destroy(lb_plan* plan);
  * Rust RHS interprets the coefficient programs on every call,
  * rust/src/lindblad/eval.rs:791-911).  With enable = k > 0, the plan's
  * time-dependent compound and coefficient programs are emitted as
- * straight-line device code; the k-th lb_solve call that takes a one-wave
- * kernel of a form (plans of at most 64 elements, persistent mode with dt
+ * straight-line device code; the k-th lb_solve call in the process, by plans
+ * of these programs, that takes a one-wave kernel of a form (plans of at most 64 elements, persistent mode with dt
  * given: final outputs, tapes, traces, save plans, stop events, fixed steps)
  * compiles that form with the code at run time (hiprtc, 0.7 to 4 s) and later
  * calls reuse it; earlier ones run the precompiled kernels.  Final outputs of
- * at most 32 elements without a tape compile at the first call whatever k, and
- * a form that the process holds for a plan of the same programs is used at
- * once.  Values are bitwise those of the expression machine.  A plan without
+ * at most 32 elements without a tape compile at the first call whatever k.
+ * Values are bitwise those of the expression machine.  A plan without
  * time dependence is left as it is.
  * Returns LB_ERR_UNSUPPORTED (with the reason) when an instruction has no
  * generated form.  When the run-time compilation or the module load of a

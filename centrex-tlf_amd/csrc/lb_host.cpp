@@ -2454,12 +2454,33 @@ extern "C" int lb_eff_solve(const lb_eff_plan* p, const lb_eff_solve_args* a, vo
   c.out_stats = a->out_stats;
   c.out_fail_t = a->out_fail_t;
   // Seats share the loads of the operators; a workgroup of one has the shorter
-  // step.  16 levels, 256 CUs: 256 trajectories 2.3 ms with one seat, 512 in
-  // 2.8 ms with two, 768 in 3.9 ms with four (with one seat a round of 256 each).
-  const int64_t per_cu_traj = (a->n_traj + std::max(1, p->cus) - 1) / std::max(1, p->cus);
-  int id, W, T, rc;
-  size_t lds;
-  if ((rc = eff_config(P, (int)std::min<int64_t>(per_cu_traj >= 3 ? 4 : per_cu_traj, 4), &id, &W, &T, &lds))) return rc;
+  // step (two seats 1.25, four 1.75 times its time), and small plans have several
+  // workgroups on a CU (eight waves of 256 registers, and the LDS).  Of one, two
+  // and four seats the number whose rounds of resident workgroups take the least
+  // time.  ms at 1, 2 and 4 seats, 256 CUs:
+  //    3 levels   1,024 trajectories  2.61  3.06  4.24    8,192  10.7  6.59  9.02
+  //    8 levels   1,024               3.53  4.52  5.71    4,096  13.4  9.07  6.84
+  //   16 levels     512               10.6  7.00  9.48    1,024  21.9  13.9  9.94
+  int id = -1, W = 0, T = 1, rc;
+  size_t lds = 0;
+  double least = 0.0;
+  for (int seats : {1, 2, 4}) {
+    int i, w, t;
+    size_t l;
+    if ((rc = eff_config(P, seats, &i, &w, &t, &l))) return rc;
+    if (t != seats) break;  // this plan has no shape of so many
+    const int64_t resident = std::max<int64_t>(1, std::min<int64_t>(8 / (w / 64), kMaxLdsBytes / (int64_t)l));
+    const int64_t groups = a->workgroups > 0 ? a->workgroups : resident * std::max(1, p->cus);
+    const double time =
+        (double)((a->n_traj + groups * t - 1) / (groups * t)) * (seats == 1 ? 1.0 : seats == 2 ? 1.25 : 1.75);
+    if (id < 0 || time < least) {
+      least = time;
+      id = i;
+      W = w;
+      T = t;
+      lds = l;
+    }
+  }
   void* fn = lb_dev_eff_kernel(id, a->solver);
   if (!fn) return fail(LB_ERR_UNSUPPORTED, "effective kernel variant is not built");
   if ((rc = set_lds_limit(fn, lds))) return rc;

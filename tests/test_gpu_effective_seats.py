@@ -1,8 +1,9 @@
 """Effective-Hamiltonian trajectories that share a workgroup give bitwise the
 results of a workgroup each: batches of one, two and four seats per workgroup
-(by the number of trajectories), fields in different grid intervals and off the
-grid, odd batches, every output kind and both ways to take the first step.
-Rows are sorted by length only where that does not pad the tables more."""
+(by the trajectories for each of a given number of workgroups), fields in
+different grid intervals and off the grid, odd batches, every output kind and
+both ways to take the first step.  Rows are sorted by length only where that
+does not pad the tables more."""
 
 from __future__ import annotations
 
@@ -36,7 +37,7 @@ def test_seats_are_bitwise_a_workgroup_each(n, density, solver, dt):
     # x(1) = x0 + 0.35: the whole grid, and some trajectories that leave it
     ov = np.stack([rng.uniform(0.3, 2.0, B), rng.uniform(-0.99, 0.75, B)], axis=1)
     slots = [plan.slot_names.index("Omega_amp"), plan.slot_names.index("x0")]
-    kw = dict(solver=solver, dt=dt, abstol=1e-8, reltol=1e-6, override_slots=slots)
+    kw = dict(solver=solver, dt=dt, abstol=1e-8, reltol=1e-6, override_slots=slots, workgroups=cus)
     save = np.asarray([0.0, 0.31, 0.77, 1.0])
     calls = [dict(output_kind="populations", save_plan=[1.0], save_start=False),
              dict(output_kind="full", save_plan=save, capacity=4),

@@ -1302,14 +1302,15 @@ int resolve_config(const DevImage* p, int variant, int threads, bool pair_ok, in
 }
 
 // The precompiled kernel of variant `id`.  pair_ok (but for the launch mode) is
-// what the lean form of a multi-wave kernel covers of a call; of a plan it needs
-// several blocks (it has their controller only), couplings and, where it is
-// time-dependent, its programs as steps: 512 + 512 trajectories, 72 levels,
-// 310 ms against 390 ms in the general form.
+// what the lean form covers of a call; of a plan it needs couplings, where it is
+// time-dependent its programs as steps, and the controller that the form has
+// (one block in one wave, several blocks in the multi-wave forms): 512 + 512
+// trajectories, 72 levels, 310 ms against 390 ms in the general form.
 void* solve_kernel(const DevImage* im, int id, int solver, bool pair_ok) {
   const DevPlan& P = im->dev;
   void* fn = nullptr;
-  if (pair_ok && P.nblk > 1 && P.couplings && (!P.time_dependent || P.v_steps > 0)) fn = lb_dev_lean_kernel(id, solver);
+  if (pair_ok && P.couplings && (!P.time_dependent || P.v_steps > 0) && (P.nblk > 1 || lb_dev_variant_wave(id)))
+    fn = lb_dev_lean_kernel(id, solver);
   return fn ? fn : lb_dev_solve_kernel(lb_dev_variant_shape(id, (int)im->rows_total), solver);
 }
 

@@ -1173,11 +1173,12 @@ __device__ __forceinline__ void write_row(const DevPlan& P, const DevCall& C, co
 // ---------------------------------------------------------------------------
 // Persistent integrator.
 // ---------------------------------------------------------------------------
-// ONE_WAVE: the single-wave form (R = 1, 64 threads), which parks the state in
-// LDS around the expression machine; otherwise the multi-wave form.  LEAN: the multi-wave form of a
-// plan with couplings (and step programs, where it is time-dependent) for a
-// call with a given initial step that pushes at accepted steps at most into
-// the weighted integral: no trace, save plan, replay or stop event.
+// ONE_WAVE: the single-wave form (R = 1, 64 threads, plans of one block), which
+// parks the state in LDS around the expression machine; otherwise the multi-wave
+// form.  LEAN: the form of a plan with couplings (and step programs, where it is
+// time-dependent; several blocks, where it is a multi-wave form) for a call with
+// a given initial step that pushes at accepted steps at most into the weighted
+// integral: no trace, save plan, replay or stop event.
 //
 // The step of a 72-level plan is 3.1k VALU instructions a wave where the
 // arithmetic needs some 700: most of the others moved spilled scalar and
@@ -1190,7 +1191,7 @@ template <int R, int SOLVER, int MAXW, int WAVES, bool ONE_WAVE = false, bool EV
 __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, const DevCall C) {
   static_assert(!ONE_WAVE || (R == 1 && MAXW == 64), "the single-wave form holds one slot per lane");
   static_assert(!EV || !ONE_WAVE, "stop events run in the multi-wave form");
-  static_assert(!LEAN || (!ONE_WAVE && !EV), "the lean form is a multi-wave form without stop events");
+  static_assert(!LEAN || !EV, "the lean form is one without stop events");
   using T = Tab<SOLVER>;
   const int tid = threadIdx.x, W = blockDim.x;
   const Lds L = carve(P);
@@ -1390,7 +1391,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         push(t0, y_r, y_i, true);
       }
       // ---- controller state (common.rs:32-70)
-      const double hmax = fabs(t1 - t0);
+      const double hmax = fabs(t1 - t0), inv_dim = 1.0 / (double)P.dim;
       double fac_old = 1.0e-4, lfo = LB_LOG_FAC_MIN;
       bool reject = false, last = false;
       int64_t ns = 0, nst = 0, ia = 0;
@@ -1413,7 +1414,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
         // The expression machine needs registers of its own: the single-wave
         // form parks its state in LDS meanwhile (the multi-wave form keeps
         // it in the other waves' registers).
-        if constexpr (ONE_WAVE) {
+        if constexpr (ONE_WAVE && !LEAN) {
           L.park[tid] = double2{y_r[0], y_i[0]};
           L.park[64 + tid] = double2{k_r[1][0], k_i[1][0]};
         }
@@ -1437,7 +1438,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           if (LEAN || P.couplings)
             fill_entries<5>(P.nv_dyn, L.eptr, L.ecoef, L.ef, L.coef + 2 * KK, KK, L.ent + P.nv_stat, tid, W);
         }
-        if constexpr (ONE_WAVE) {
+        if constexpr (ONE_WAVE && !LEAN) {
           const double2 py = L.park[tid], pk = L.park[64 + tid];
           y_r[0] = py.x;
           y_i[0] = py.y;
@@ -1533,7 +1534,7 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_solve_kernel(const DevPlan P, 
           clamped = ctl.clamped();
           hn = ctl.next(h);
         } else {
-          const StepControl ctl(e2 * (1.0 / (double)P.dim), lfo);
+          const StepControl ctl(e2 * inv_dim, lfo);
           err = ctl.err;
           accept = ctl.accept;
           clamped = ctl.clamped();
@@ -5942,6 +5943,14 @@ void* wave_solve_ptr(int solver) {
     return nullptr;
 }
 template <int I, int VV>
+void* wave_lean_ptr(int solver) {
+  if constexpr (I % LB_NPART == LB_PART)
+    return solver == 1 ? (void*)&lb_solve_kernel<1, 1, 64, VV, true, false, true>
+                       : (void*)&lb_solve_kernel<1, 0, 64, VV, true, false, true>;
+  else
+    return nullptr;
+}
+template <int I, int VV>
 void* wave_rhs_ptr() {
   if constexpr (I % LB_NPART == LB_PART)
     return (void*)&lb_rhs_kernel<1, 64, VV>;
@@ -5979,6 +5988,10 @@ extern "C" void* LB_PART_FN(lb_dev_lean_kernel)(int id, int solver) {
   if (id == i) return lean_ptr<i, r, w, v>(solver);
   LB_CONFIGS(X)
 #undef X
+#define Y(i, v) \
+  if (id == i) return wave_lean_ptr<i, v>(solver);
+  LB_WAVE_CONFIGS(Y)
+#undef Y
   return nullptr;
 }
 

@@ -129,7 +129,7 @@ extern "C" void* lb_dev_solve_kernel(int id, int solver) {
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);
 }
 
-// The lean form of a multi-wave variant (lb_solve_kernel); null for the others.
+// The lean form of a single- or multi-wave variant (lb_solve_kernel); null for the others.
 extern "C" void* lb_dev_lean_kernel(int id, int solver) {
   void* (*parts[])(int, int) = {lb_dev_lean_kernel_p0, lb_dev_lean_kernel_p1, lb_dev_lean_kernel_p2, lb_dev_lean_kernel_p3, lb_dev_lean_kernel_p4, lb_dev_lean_kernel_p5, lb_dev_lean_kernel_p6, lb_dev_lean_kernel_p7};
   return id < 0 ? nullptr : parts[id % LB_NPARTS_BUILT](id, solver);

@@ -19,10 +19,12 @@ here; all others stay exactly zero), two trajectories per wave (one per
 Also reported: the per-trajectory ("plain") GPU path on a seeded sample, the
 CPU oracle (this project's C restatement of the reference's Rust/rayon path,
 which integrates every element) timed on the host cores on a bounded seeded
-sample, a parity check of the sample against the oracle, and the FP64
-roofline of the solver kernel: `achieved` counts the reference algorithm's
-FLOPs (rhs_calls * F_rhs + attempted * dim * F_rk over the full plan), and
-`executed_*` the FLOPs of the restricted tables the kernel actually runs.
+sample, a parity check of the sample against the oracle, and the roofline of
+the solver kernel, which the latency of a step bounds: `achieved` counts the
+reference algorithm's FLOPs (rhs_calls * F_rhs + attempted * dim * F_rk over the
+full plan, most of which the restricted plan has no need of), `executed_*` the
+FLOPs of the restricted tables the kernel actually runs, and `lds_cobound` the
+LDS bytes that it moves.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W]
     python bench.py --copy-calibration   # plain 1 GiB copy kernel (HBM counter scale)
@@ -56,19 +58,12 @@ def log(msg: str) -> None:
 LDS_PEAK_TBS = 256 * 128 * 2.4e9 / 1e12
 
 
-def lds_bytes_per_rhs(prepared) -> int:
-    """Algorithmic LDS bytes of one RHS of the full plan: 8 bytes per term whose
-    input is a real (diagonal) element, 16 per complex one, plus 8*dim for
-    publishing the stage vector that the gathers read."""
-    import numpy as np
-
-    from centrex_tlf_amd.lindblad.state_layout import upper_offsets
-
-    plan = prepared.expanded_rhs_plan
-    n = int(plan["n"])
-    inputs = np.asarray(plan["input_indices"], dtype=np.int64)
-    diagonal = np.isin(inputs, upper_offsets(n))
-    return int(np.where(diagonal, 8, 16).sum()) + 8 * n * n
+def lds_bytes_per_rhs(rinfo, paired: bool) -> int:
+    """LDS bytes that the kernel moves per right-hand side of one trajectory: 16
+    published by every lane, and per lane and coupling row an entry value and an
+    input of 16 bytes each."""
+    lanes = 32 if paired else rinfo["slot_count"]
+    return lanes * 16 + (32 if paired else 64) * rinfo["gather_rows"] * 32
 
 
 def algorithmic_flops(stats, flops_per_rhs: int, dim: int, solver: str) -> float:
@@ -153,7 +148,7 @@ def uneven_leg(steps: int, warmup: int, cpu_seconds: float) -> dict:
             # roofline of the batch: the reference algorithm's FLOPs (full
             # plans) and the FLOPs of the restricted tables the kernels run,
             # over the grouped call's time; the n=72 group sets that time
-            roof = {"bound": "fp64_valu", "latency_bound": True, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+            roof = {"bound": "latency", "latency_bound": True, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                     "seconds": tuned_s, "groups": {}}
             alg_all = exe_all = 0.0
             for grp, r, label in zip(groups, res, ("n39", "n72")):
@@ -761,7 +756,7 @@ def main() -> int:
     executed = algorithmic_flops(stats_np, rinfo["flops_per_rhs"], rinfo["dim"], args.solver)
     avg_kernel_s = float(np.mean(kernel_ms)) / 1e3
     achieved_tflops = flops / avg_kernel_s / 1e12
-    lds_rhs = lds_bytes_per_rhs(prepared)
+    lds_rhs = lds_bytes_per_rhs(rinfo, rinfo["upper_len"] <= 32)
     lds_bytes = float(stats_np[:, 2].astype(np.float64).sum()) * lds_rhs
     traffic = None
     if TRAFFIC_FILE.exists():
@@ -795,7 +790,7 @@ def main() -> int:
             "threads_per_traj": args.threads_per_traj or rinfo["threads_per_traj"],
         },
         "roofline": {
-            "bound": "fp64_valu",
+            "bound": "latency",
             "latency_bound": True,
             "compute": "FP64 vector ALU (no MFMA: the sparse RHS has no dense tile); the MI355X FP64 vector "
                        "and matrix peaks are both 78.6 TFLOP/s.  Each trajectory's step chain is serial, so the "
@@ -818,8 +813,8 @@ def main() -> int:
                 "unit": "TB/s",
                 "frac": lds_bytes / avg_kernel_s / 1e12 / LDS_PEAK_TBS,
                 "bytes_per_launch": lds_bytes,
-                "definition": "sum over trajectories of rhs_calls * (sum over terms of 8 bytes per real input, 16 "
-                              f"per complex, + 8*dim), full plan: {lds_rhs} bytes per RHS; peak 256 CUs x 128 B/clk "
+                "definition": f"sum over trajectories of rhs_calls * {lds_rhs} bytes: 16 published by every lane, 32 "
+                              "read per lane and coupling row of the tables the kernel runs; peak 256 CUs x 128 B/clk "
                               "x 2.4 GHz",
             },
         },

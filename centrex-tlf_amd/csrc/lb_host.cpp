@@ -638,9 +638,13 @@ int build_image(const PlanSource& src, const std::vector<uint8_t>& act, DevImage
   // (gradients by 1e-13).  Larger plans keep a coupling per term, applied in the
   // order of the plan: flights of 10,000 steps and more through a drive that
   // jumps carry a rounding to the twelfth digit of the populations (1e-12 to
-  // 1.2e-11 in norm).  Measured: 512 + 512 uneven batch 318 against 312 ms,
-  // n=39 x/y scan 1.20 against 0.98 ms, 64 gradients at 72 levels 125 against
-  // 113 ms.
+  // 1.2e-11 in norm).  A coupling per term costs 335 against 315 ms in the
+  // 512 + 512 uneven batch (n=39 x/y scan, which merges, 1.20 against 0.98 ms;
+  // 64 gradients at 72 levels, which merge, 125 against 113 ms).
+  // Couplings leave fewer workgroups a CU than the gather tables where their
+  // entries are many, and are still no slower there: 2,048 trajectories of a
+  // dense system of 153 elements 3.2 ms both ways (3 workgroups of one wave
+  // against 8), a 40-level chain of 120 entries 0.89 against 1.42 ms.
   const Couplings cpl = merge_couplings(src, act, one_block || src.n_diff > 0);
   const int n_stat = (int)cpl.entries.size() - cpl.n_dyn + 1;  // and the zero of padding rows
   P.couplings = 1;

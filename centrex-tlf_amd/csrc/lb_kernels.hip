@@ -712,12 +712,12 @@ __device__ __forceinline__ void gather_term(uint32_t w, double2 f, const dcpx* c
   gather_apply(w, f, coef, pubbuf[2 * p], pubbuf[2 * p + 1], accr, acci);
 }
 
-// Single-wave form for plans of at most 64 elements: lane = slot, the gather
-// inputs come from the owning lanes by cross-lane permutes instead of a
-// publish / barrier / LDS-read round trip.  The publication index of a plan
-// this small is its slot, so the table words are shared with the multi-wave
-// form, and the arithmetic is the same.  All rows' table entries and inputs
-// are fetched before the first term is applied.
+// The right-hand side in the single-block adjoint's recomputation (plans of at
+// most 64 elements): lane = slot, the gather inputs come from the owning lanes by
+// cross-lane permutes instead of a publish / barrier / LDS-read round trip.  The
+// publication index of a plan this small is its slot, so the table words are
+// those of the gather tables.  All rows' table entries and inputs are fetched
+// before the first term is applied.
 template <int G>
 __device__ __forceinline__ void rhs_wave(const Lds& L, int rows, int lane, double2 selfv, bool diag, double xr,
                                          double xi, double& kr, double& ki, const dcpx* coef) {
@@ -4414,10 +4414,10 @@ __global__ __launch_bounds__(MAXW, WAVES) void lb_adjoint_block_kernel(const Dev
 // checkpoint segments: it evaluates the coefficient rows of a segment (every
 // stage time of its attempts is on the tape) in one pass, one (attempt,
 // stage) per lane, each lane with a private copy of the parameter slots and
-// its own expression stack, and recomputes the segment with the
-// register/cross-lane RHS of the single-wave solver (the same arithmetic, so
-// the stage derivatives are those of the recorded solve).  LB_AW_SWEEPERS
-// waves sweep the attempts with the same per-element state; each applies its
+// its own expression stack, and recomputes the segment with a
+// register/cross-lane RHS over gather terms (the recorded solve runs them merged
+// into couplings, so the stage derivatives are its own to rounding).
+// LB_AW_SWEEPERS waves sweep the attempts with the same per-element state; each applies its
 // share of the transposed rows of every reverse stage (kappa of other
 // elements by cross-lane permutes, each term contracted with its
 // coefficient's parameter and time derivatives), and the partial sums of mu

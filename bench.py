@@ -315,9 +315,10 @@ def adjoint_leg(steps: int, warmup: int) -> dict:
     rho0 = np.outer(psi, psi.conj())
     prepared = prepare_lindblad_problem(system, params, backend="gpu")
     engine = DifferentiablePhotonCount(prepared, names, weights, t_span, ckpt_every=16, **tol)
+    engine.plan.specialize()  # every form compiles in its first (warm-up) solve
     y0 = torch.as_tensor(prepared.layout.pack(rho0), device=dev)
     p = torch.as_tensor(p_np, device=dev)
-    plan = prepared.device_plan()
+    plan = prepared.device_plan().specialize()
     slots = [prepared.slot_names.index(m) for m in names]
     pv = p.to(torch.complex128)
 
@@ -484,7 +485,7 @@ def extras_leg(cpu_seconds: float) -> dict:
     cores = host_threads()
     system, params, rho0, t_span, weights = tlf_n39()
     prepared = prepare_lindblad_problem(system, params, backend="gpu")
-    plan = prepared.device_plan()
+    plan = prepared.device_plan().specialize()  # every form compiles in its first (warm-up) solve
     oracle = Oracle(prepared)
     names = prepared.slot_names
     slots = [names.index("delta0"), names.index("Omega0")]

@@ -1682,12 +1682,13 @@ namespace {
 // The plan-specialised kernel `name` (a template-id); nullptr when the plan is
 // not specialised or the form is not compiled yet.  A compilation takes 0.7 s
 // and more and saves a call 1 to 6 ms, so it is not for one call: a form is
-// compiled at the spec_after-th call of it by plans of one program, or at the
-// first where `at_once` says so.  (Only the paired kernels, one wave per
+// compiled at the spec_after-th call of it by plans of one program (`calls`: what
+// this one counts as), or at the first where `at_once` says so.  (Only the paired kernels, one wave per
 // workgroup, take the generated code: a specialised multi-wave kernel launched
 // with 1024-thread workgroups had its queue aborted at dispatch, cause not
 // found, so the multi-wave kernels stay on the precompiled form.)
-int spec_kernel(lb_plan* p, const std::string& name, bool at_once, hipStream_t stream, hipFunction_t* fn) {
+int spec_kernel(lb_plan* p, const std::string& name, bool at_once, int64_t calls, hipStream_t stream,
+                hipFunction_t* fn) {
   *fn = nullptr;
   std::lock_guard<std::mutex> lock(p->mu);
   if (!p->spec) return LB_OK;
@@ -1700,7 +1701,7 @@ int spec_kernel(lb_plan* p, const std::string& name, bool at_once, hipStream_t s
     if (cs != hipStreamCaptureStatusNone) return LB_OK;
     std::shared_ptr<LbModule> mod;
     std::string why;
-    if (!at_once && !lb_rtc_ready(p->spec_source, name, p->spec_after)) return LB_OK;
+    if (!at_once && !lb_rtc_ready(p->spec_source, name, calls, p->spec_after)) return LB_OK;
     if (lb_rtc_compile(p->spec_source, name, &mod, why)) {
       // the precompiled kernel computes the same values: run it, remember
       // the failure so that later calls neither recompile nor fail
@@ -1743,7 +1744,8 @@ int launch_spec(lb_plan* p, const lb_solve_args* a, const DevImage* im, DevCall&
   hipFunction_t fn = nullptr;
   // final outputs of at most 32 elements (scans of thousands of trajectories)
   const bool at_once = nh == 2 && !fixed && !event && !save && !a->tape_h;
-  int rc = spec_kernel(p, name, at_once, s, &fn);
+  // a call of 2^16 trajectories counts as two: in throughput, a trajectory saves 1 to 3 us
+  int rc = spec_kernel(p, name, at_once, 1 + (a->n_traj >> 16), s, &fn);
   if (rc || !fn) return rc;
   int grid = a->workgroups;
   if (grid <= 0) {

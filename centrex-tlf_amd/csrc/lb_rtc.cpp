@@ -157,7 +157,7 @@ struct CodeObject {
 };
 std::mutex g_code_mu;
 std::map<std::string, CodeObject> g_code;
-std::map<size_t, int> g_calls;  // calls that would take a kernel not compiled yet, by hash
+std::map<size_t, int64_t> g_calls;  // calls that would take a kernel not compiled yet, by hash
 // Loaded modules by device and code key; the most recently used ones are held
 // (a plan made again for the same system then loads nothing).  Not destroyed
 // at process exit, when the runtime may be gone.
@@ -220,11 +220,11 @@ std::string code_key(const std::string& coef_source, const std::string& name_exp
 }
 }  // namespace
 
-bool lb_rtc_ready(const std::string& coef_source, const std::string& name_expr, int after) {
+bool lb_rtc_ready(const std::string& coef_source, const std::string& name_expr, int64_t calls, int after) {
   const std::string key = code_key(coef_source, name_expr);
   std::lock_guard<std::mutex> lock(g_code_mu);
   if (g_code.count(key)) return true;
-  return ++g_calls[std::hash<std::string>()(key)] >= after;
+  return (g_calls[std::hash<std::string>()(key)] += calls) >= after;
 }
 
 int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr, std::shared_ptr<LbModule>* out,

@@ -34,6 +34,6 @@ struct LbModule {
 };
 int lb_rtc_compile(const std::string& coef_source, const std::string& name_expr, std::shared_ptr<LbModule>* out,
                    std::string& why);
-// Counts one call that would take the kernel: whether it is the `after`-th or a
-// later one in the process, or the process holds the kernel already.
-bool lb_rtc_ready(const std::string& coef_source, const std::string& name_expr, int after);
+// Counts a call (as `calls` of them) that would take the kernel: whether `after`
+// have come in the process, or it holds the kernel already.
+bool lb_rtc_ready(const std::string& coef_source, const std::string& name_expr, int64_t calls, int after);

@@ -148,7 +148,8 @@ void lb_plan_destroy(lb_plan* plan);
  * of these programs, that takes a one-wave kernel of a form (plans of at most 64 elements, persistent mode with dt
  * given: final outputs, tapes, traces, save plans, stop events, fixed steps)
  * compiles that form with the code at run time (hiprtc, 0.7 to 4 s) and later
- * calls reuse it; earlier ones run the precompiled kernels.  Final outputs of
+ * calls reuse it; earlier ones run the precompiled kernels (a call counts as
+ * one more for every 65,536 trajectories).  Final outputs of
  * at most 32 elements without a tape compile at the first call whatever k.
  * Values are bitwise those of the expression machine.  A plan without
  * time dependence is left as it is.
